@@ -15,6 +15,10 @@
 // status reads
 #define ST_SCAN_FALLBACK 0x8u
 
+// What a load notes about its triples (DevState.load_flags).
+#define LD_UNSORTED 0x1u   // the packed keys are not in order
+#define LD_NONCANON 0x2u   // duplicate coordinates or explicit zeros
+
 // Rows longer than this are counted as power-law hubs in dcsr_info.
 #define DCSR_HUB_LEN 4096
 // SpMV calls on one structure that pay for building its paneled copy
@@ -51,6 +55,7 @@ struct DevState {
     unsigned int hub_touch;         // current update: rewritten rows that were/are hubs
     unsigned int ubad_last;         // current update's batch held an out-of-range index
     unsigned int ptotal;            // current update: probe lengths of the touched rows, summed
+    unsigned int load_flags;        // current load: LD_* bits
 };
 
 // Grow-only device scratch buffers owned by a handle.
@@ -128,6 +133,7 @@ struct dcsr_matrix_s {
     int64_t ncompact;        // compactions and growths (dcsr_query reports it)
     uint32_t upd_tag;        // tag of the last update's row -> touched-row map
     bool flat_dirty;         // flat row offsets (SpMV binning) need a rebuild
+    bool flat_replayed;      // an update was captured into a graph: the row lengths may change without a call
     bool state_known;        // host mirrors valid (no NOSYNC update since last sync)
     // column-paneled copy for SpMV on matrices whose x exceeds the L2 (see
     // spmv.hip): valid until the next structural change
@@ -207,9 +213,6 @@ dcsr_status update_commit(dcsr_handle h, int64_t n, hipStream_t s, bool nosync);
 dcsr_status update_fixed_scratch(dcsr_handle h, const int32_t *rows, const int32_t *cols, const float *vals,
                                  int64_t n, uint32_t flags, hipStream_t s, uint8_t *base, size_t cap);
 size_t update_scratch_bytes(dcsr_handle h, int64_t n);
-// Flat copy of R rows (src_start[r], length dst_off[r+1]-dst_off[r]) to dst_off.
-void launch_copy_rows(const uint32_t *dst_off, int64_t R, int64_t total, const uint32_t *src_start,
-                      const int32_t *scol, const float *sval, int32_t *dcol, float *dval, hipStream_t s);
 
 // The handle's sticky status word (device): scans set ST_SCAN_FALLBACK in it.
 static inline unsigned int *fault_word(dcsr_handle h) { return &h->ds->status; }

@@ -1937,6 +1937,8 @@ dcsr_status update_fixed_scratch(dcsr_handle h, const int32_t *rows, const int32
     DCSR_TRY(upd_bufs_src(src, n, b));
     k_zero_u32<<<1, 64, 0, s>>>(b.fin, 16);
     const bool nosync = (flags & DCSR_UPDATE_NOSYNC) != 0;
+    hipStreamCaptureStatus cap_st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cap_st) == hipSuccess && cap_st != hipStreamCaptureStatusNone) h->flat_replayed = true;
     if (nosync) refresh_bounds(h);
     launch_pack(h, rows, cols, vals, n, b, s);
     DCSR_HIP(hipGetLastError());
