@@ -13,10 +13,12 @@
 //                flight per CU: a row is a chain of dependent loads);
 //   P_i <= 1024  one wave per row, LDS ESC: the row's partials are expanded
 //                with their generation index (A-entry order, then B-row
-//                order), bitonic-sorted in LDS by (column, generation), and
+//                order), bucket-sorted in LDS by (column, generation), and
 //                each run of equal columns is summed left-to-right;
 //   P_i <= 4096  the same with one 256-thread workgroup per row;
-//   P_i >  4096  (power-law hub rows, which the reference skips) a global
+//   P_i <= 16384 the same with one 1024-thread workgroup per row (8192 where
+//                the sort key needs 64 bits);
+//   larger       (power-law hub rows, which the reference skips) a global
 //                ESC: expand, stable LSD radix sort by (row, column), reduce.
 // Output rows come out column-sorted with exact zeros removed, and the
 // accumulation order is fixed, so C is deterministic.
@@ -38,11 +40,24 @@ constexpr int WAVE_GB = 10;           // generation bits of the wave kernel's ke
 constexpr int64_t WAVE_MAX_COLS32 = (1ll << (32 - WAVE_GB)) - 1;
 constexpr uint32_t WAVE_MAX = 1024;   // partials per row for the wave kernel
 constexpr uint32_t BLOCK_MAX = 4096;  // partials per row for the workgroup kernel
+constexpr int BLOCK_GB = 12;
+constexpr int64_t BLOCK_MAX_COLS32 = (1ll << (32 - BLOCK_GB)) - 1;
+// the large-row kernel: 1024 threads, most of a CU's LDS
+constexpr int BIG_TB = 1024;
+constexpr uint32_t BIG_MAX32 = 16384, BIG_MAX64 = 8192;  // partials per row by key width
+constexpr int BIG_GB = 14;
+constexpr int64_t BIG_MAX_COLS32 = (1ll << (32 - BIG_GB)) - 1;
 constexpr int SG_EX = 8;              // partials per lane whose loads are in flight together
-// row classes (list index): wave, workgroup, hub, team
+// row classes (list index): wave, workgroup, large, hub, team
 // team classes CL_TEAM + i: rows of at most 2 (i + 1) * TEAM partials, sorted
 // with 2 (i + 1) keys per lane
-enum { CL_WAVE = 0, CL_BLOCK = 1, CL_HUB = 2, CL_TEAM = 3, NTEAMCL = 4, NCLS = CL_TEAM + NTEAMCL };
+// wave classes CL_WAVE + i: rows of at most 256, 512, 1024 partials, sorted with
+// 4, 8, 16 keys per lane (the registers of the widest would hold the shorter
+// rows, which are most of them, to 3 waves per SIMD)
+enum {
+    CL_WAVE = 0, NWAVECL = 3, CL_BLOCK = CL_WAVE + NWAVECL, CL_BIG, CL_HUB, CL_TEAM, NTEAMCL = 4,
+    NCLS = CL_TEAM + NTEAMCL
+};
 
 struct SgState {
     unsigned long long total;  // sum of P_i (64-bit)
@@ -121,7 +136,8 @@ constexpr int SG_CR = 8;
 __global__ __launch_bounds__(TB) void k_sg_classify(uint32_t R, const uint32_t *__restrict__ P,
                                                     uint32_t *__restrict__ lists, uint32_t list_stride,
                                                     SgState *st, uint32_t *__restrict__ cnt,
-                                                    unsigned long long *__restrict__ bsum, uint32_t team_ok)
+                                                    unsigned long long *__restrict__ bsum, uint32_t team_ok,
+                                                    uint32_t big_max)
 {
     __shared__ unsigned long long ws[TB / 64];
     __shared__ uint32_t s_cnt[NCLS], s_base[NCLS];
@@ -147,8 +163,9 @@ __global__ __launch_bounds__(TB) void k_sg_classify(uint32_t R, const uint32_t *
             // row sizes
             cls[q] = p[q] == 0                         ? -1
                      : (p[q] <= TEAM_MAX && team_ok)   ? CL_TEAM + (int)((p[q] - 1) / (2 * TEAM))
-                     : p[q] <= WAVE_MAX                ? CL_WAVE
+                     : p[q] <= WAVE_MAX                ? CL_WAVE + (p[q] > 256u) + (p[q] > 512u)
                      : p[q] <= BLOCK_MAX               ? CL_BLOCK
+                     : p[q] <= big_max                 ? CL_BIG
                                                        : CL_HUB;
             if (p[q] == 0) cnt[r] = 0;
         }
@@ -203,9 +220,10 @@ __global__ __launch_bounds__(1024) void k_sg_total(SgState *st, const unsigned l
 
 // ---------------------------------------------------------------------------
 // Shared row routine: expand, sort, reduce.  NT threads cooperate (64 for the
-// wave kernel, 256 for the workgroup kernel); GB = generation-index bits.
+// wave kernel, 256 and 1024 for the workgroup kernels); GB = generation-index
+// bits.
 // ---------------------------------------------------------------------------
-// A team is NT threads: 16 (a quarter wave), 64 (a wave) or 256 (the
+// A team is NT threads: 16 (a quarter wave), 64 (a wave), 256 or 1024 (the
 // workgroup).  Teams inside one wave never exchange data with each other.
 template <int NT>
 __device__ __forceinline__ void team_sync()
@@ -288,26 +306,22 @@ __device__ __forceinline__ SgRowInfo sg_row_info(uint32_t row, const uint32_t *_
     return r;
 }
 
-// Rank sort of a team's P staged (key, val) pairs in LDS, for teams narrower
-// than a wave.  The keys are distinct, so a key's sorted position is the
-// number of smaller keys: lane t holds keys t, t + NT, ... in registers and
-// compares them with every key of the row, read back one at a time (the
-// team's lanes all read the same word: one broadcast per key), then every
-// pair is written to its position.  Costs P * KPL compares per lane and no
-// LDS traffic beyond the broadcasts, against a bitonic network's
-// log^2-many LDS passes.
+// Rank sort of a team's P staged keys in LDS, for teams of at most a wave.
+// The keys are distinct, so a key's sorted position is the number of smaller
+// keys: lane t holds keys t, t + NT, ... in registers and compares them with
+// every key of the row, read back one at a time (the team's lanes all read the
+// same word: one broadcast per key), then every key is written to its
+// position.  P * KPL compares per lane.
 template <int NT, int KPL, typename K>
-__device__ __forceinline__ void team_rank_sort(K *key, float *val, uint32_t P)
+__device__ __forceinline__ void team_rank_sort(K *key, uint32_t P)
 {
     const uint32_t t = threadIdx.x % NT;
     K mk[KPL];
-    float mv[KPL];
     uint32_t rk[KPL];
 #pragma unroll
     for (int r = 0; r < KPL; ++r) {
         const uint32_t i = t + (uint32_t)r * NT;
         mk[r] = i < P ? key[i] : (K)~0ull;
-        mv[r] = i < P ? val[i] : 0.0f;
         rk[r] = 0;
     }
     uint32_t j = 0;
@@ -338,23 +352,180 @@ __device__ __forceinline__ void team_rank_sort(K *key, float *val, uint32_t P)
     }
     team_sync<NT>();  // every read of the row is done before the scatter
 #pragma unroll
-    for (int r = 0; r < KPL; ++r) {
-        if (t + (uint32_t)r * NT < P) {
-            key[rk[r]] = mk[r];
-            val[rk[r]] = mv[r];
-        }
-    }
+    for (int r = 0; r < KPL; ++r)
+        if (t + (uint32_t)r * NT < P) key[rk[r]] = mk[r];
     team_sync<NT>();
 }
 
-// KPL (teams only): keys per lane of the rank sort, fixed by the row's class
-// (P <= KPL * NT); 0 picks it per row.
-template <int NT, int GB, typename K, int KPL = 0>
+// Bitonic network over LDS: the sort of the rows whose columns crowd into few
+// buckets (keys past P are padding and sort last; key holds next_pow2(P)).
+template <int NT, typename K>
+__device__ void team_bitonic_sort(K *key, uint32_t P)
+{
+    const uint32_t t = threadIdx.x % NT;
+    const uint32_t n2 = next_pow2(P < 2 * NT ? 2 * NT : P);
+    for (uint32_t p = P + t; p < n2; p += NT) key[p] = (K)~0ull;
+    team_sync<NT>();
+    for (uint32_t k = 2; k <= n2; k <<= 1) {
+        for (uint32_t js = k >> 1; js > 0; js >>= 1) {
+            for (uint32_t c = t; c < n2 / 2; c += NT) {
+                const uint32_t i1 = (c / js) * 2 * js + (c % js);
+                const uint32_t i2 = i1 + js;
+                const bool asc = (i1 & k) == 0;
+                const K ka = key[i1], kb = key[i2];
+                if ((ka > kb) == asc) {
+                    key[i1] = kb;
+                    key[i2] = ka;
+                }
+            }
+            team_sync<NT>();
+        }
+    }
+}
+
+// Bucket sort of a team's P <= NT * KPL staged keys in LDS.  A key's bucket is
+// its place between the row's smallest and largest key, in NT * BPL equal
+// steps (a float product: monotone in the key, so buckets are in key order).
+// The buckets are counted by LDS atomics, scanned, and filled in any order; a
+// key's sorted position is then its bucket's start plus the smaller keys of
+// its own bucket.  Columns that spread over the row's range leave about one
+// key per bucket, so a key costs a few LDS accesses instead of a compare with
+// every other key of the row (the rank sort) or log^2-many passes (the
+// bitonic network).  Returns false, with all keys in LDS, when a bucket of
+// the wave (of the workgroup for NT > 64) holds more than BK_CROWD keys: the
+// caller then sorts them without buckets.
+// hist: NT * BPL / 2 + 1 words, two 16-bit counters to a word.
+constexpr uint32_t BK_CROWD = 24;
+template <int KPL>
+constexpr int bucket_bpl() { return KPL > 8 ? 8 : KPL; }
+template <int NT, int KPL, int GB, typename K>
+__device__ __forceinline__ bool team_bucket_sort(K *key, uint32_t *hist, uint32_t P, uint32_t *lds_w)
+{
+    constexpr int BPL = bucket_bpl<KPL>();
+    constexpr uint32_t NB = (uint32_t)NT * BPL;
+    static_assert(BPL % 2 == 0, "whole counter words per lane");
+    const uint32_t t = threadIdx.x % NT;
+    auto place = [](K k) { return sizeof(K) == 4 ? (uint32_t)k : (uint32_t)((uint64_t)k >> GB); };
+    K mk[KPL];
+    uint32_t lo = ~0u, hi = 0u;
+#pragma unroll
+    for (int r = 0; r < KPL; ++r) {
+        const uint32_t i = t + (uint32_t)r * NT;
+        mk[r] = key[i < P ? i : 0u];
+        const uint32_t b = place(mk[r]);
+        lo = b < lo ? b : lo;
+        hi = b > hi ? b : hi;
+    }
+#pragma unroll
+    for (int i = 0; i < BPL / 2; ++i) hist[(uint32_t)i * NT + t] = 0u;
+    constexpr int W = NT < 64 ? NT : 64;
+#pragma unroll
+    for (int d = 1; d < W; d <<= 1) {
+        const uint32_t l2 = (uint32_t)__shfl_xor((int)lo, d, W), h2 = (uint32_t)__shfl_xor((int)hi, d, W);
+        lo = l2 < lo ? l2 : lo;
+        hi = h2 > hi ? h2 : hi;
+    }
+    if constexpr (NT > 64) {
+        constexpr int NW = NT / 64;
+        if (lane_id() == 0) {
+            lds_w[2 * (t >> 6)] = lo;
+            lds_w[2 * (t >> 6) + 1] = hi;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < NW; ++i) {
+            lo = lds_w[2 * i] < lo ? lds_w[2 * i] : lo;
+            hi = lds_w[2 * i + 1] > hi ? lds_w[2 * i + 1] : hi;
+        }
+    }
+    team_sync<NT>();
+    const float scale = (float)NB / ((float)(hi - lo) + 1.0f);
+    uint32_t bo[KPL];  // bucket, and the key's arrival in it << 16
+#pragma unroll
+    for (int r = 0; r < KPL; ++r) {
+        bo[r] = 0;
+        if (t + (uint32_t)r * NT < P) {
+            uint32_t b = (uint32_t)((float)(place(mk[r]) - lo) * scale);
+            b = b < NB ? b : NB - 1;
+            const uint32_t sh = (b & 1u) * 16u;
+            bo[r] = b | (((atomicAdd(&hist[b >> 1], 1u << sh) >> sh) & 0xffffu) << 16);
+        }
+    }
+    team_sync<NT>();
+    // exclusive starts, BPL consecutive buckets per lane
+    uint32_t w[BPL / 2], sum = 0;
+#pragma unroll
+    for (int i = 0; i < BPL / 2; ++i) {
+        w[i] = hist[t * (BPL / 2) + i];
+        sum += (w[i] & 0xffffu) + (w[i] >> 16);
+    }
+    uint32_t tot;
+    uint32_t run = team_excl_scan<NT>(sum, lds_w, &tot);
+#pragma unroll
+    for (int i = 0; i < BPL / 2; ++i) {
+        const uint32_t a = run + (w[i] & 0xffffu);
+        hist[t * (BPL / 2) + i] = run | (a << 16);
+        run = a + (w[i] >> 16);
+    }
+    if (t == 0) hist[NB / 2] = P;
+    team_sync<NT>();
+    const uint16_t *start = reinterpret_cast<const uint16_t *>(hist);
+    uint32_t l[KPL], n[KPL], most = 0;
+#pragma unroll
+    for (int r = 0; r < KPL; ++r) {
+        l[r] = n[r] = 0;
+        if (t + (uint32_t)r * NT < P) {
+            const uint32_t b = bo[r] & 0xffffu;
+            l[r] = start[b];
+            n[r] = start[b + 1] - l[r];
+            key[l[r] + (bo[r] >> 16)] = mk[r];
+            most = n[r] > most ? n[r] : most;
+        }
+    }
+    team_sync<NT>();
+    bool crowded;
+    if constexpr (NT > 64) crowded = __syncthreads_or(most > BK_CROWD);
+    else crowded = __any(most > BK_CROWD);
+    if (crowded) return false;
+    // smaller keys of the own bucket: the wave's fullest bucket sets the
+    // rounds, each with one independent read per key
+    uint32_t rk[KPL];
+#pragma unroll
+    for (int r = 0; r < KPL; ++r) rk[r] = l[r];
+    for (uint32_t d = 0; __any(most > 1 && d < most); ++d) {
+#pragma unroll
+        for (int r = 0; r < KPL; ++r)
+            if (d < n[r]) rk[r] += (uint32_t)(key[l[r] + d] < mk[r]);
+    }
+    team_sync<NT>();
+#pragma unroll
+    for (int r = 0; r < KPL; ++r)
+        if (n[r] > 1) key[rk[r]] = mk[r];
+    team_sync<NT>();
+    return true;
+}
+
+// Sort a team's row: buckets, with the smallest per-lane key count that holds
+// it; where they are crowded, the rank sort (teams of at most a wave and at
+// most 8 keys per lane) or the bitonic network.
+template <int NT, int KPL, int GB, typename K>
+__device__ __forceinline__ void team_sort(K *key, uint32_t *hist, uint32_t P, uint32_t *lds_w)
+{
+    if (team_bucket_sort<NT, KPL, GB, K>(key, hist, P, lds_w)) return;
+    if constexpr (NT < 64) team_rank_sort<NT, KPL, K>(key, P);
+    else if constexpr (NT == 64 && KPL <= 4) team_rank_sort<NT, KPL, K>(key, P);
+    else team_bitonic_sort<NT, K>(key, P);
+}
+
+// KPL: keys per lane of the sort, fixed by the row's class (P <= KPL * NT).  The products stay where the expansion put them
+// (generation order); only the keys are sorted, and a sorted key names its
+// product by its generation bits.
+template <int NT, int GB, typename K, int KPL>
 __device__ void sg_row(const SgRowInfo &ri, const int32_t *__restrict__ a_col, const float *__restrict__ a_val,
                        const uint32_t *__restrict__ b_start, const int32_t *__restrict__ b_len,
                        const int32_t *__restrict__ b_col, const float *__restrict__ b_val,
                        int32_t *__restrict__ tcol, float *__restrict__ tval, uint32_t *__restrict__ cnt, K *key,
-                       float *val, uint32_t *s_ex, uint32_t *s_sb, float *s_va, uint32_t *lds_w)
+                       float *val, uint32_t *hist, uint32_t *s_ex, uint32_t *s_sb, float *s_va, uint32_t *lds_w)
 {
     const uint32_t t = threadIdx.x % NT;
     const uint32_t row = ri.row, P = ri.P, ast = ri.ast, la = ri.la;
@@ -380,7 +551,7 @@ __device__ void sg_row(const SgRowInfo &ri, const int32_t *__restrict__ a_col, c
         // up to SG_EX partials per lane per round, every load of a round
         // issued before the first wait (a lane past tot reads entry 0 of B
         // and writes nothing)
-        constexpr int EX = KPL ? KPL : SG_EX;
+        constexpr int EX = KPL < SG_EX ? KPL : SG_EX;
         for (uint32_t e0 = 0; e0 < tot; e0 += EX * NT) {
             int32_t bc[EX];
             float bv[EX], av[EX];
@@ -406,44 +577,15 @@ __device__ void sg_row(const SgRowInfo &ri, const int32_t *__restrict__ a_col, c
         gbase += tot;
         team_sync<NT>();
     }
-    // 2. sort by (column, generation): rank sort for quarter-wave teams and
-    // for wave rows of up to 256 partials, bitonic network over LDS for the
-    // others (padding sorts last)
-    if constexpr (NT < 64 && KPL != 0) {
-        team_rank_sort<NT, KPL, K>(key, val, P);
-    } else if constexpr (NT < 64) {
-        if (P <= 4 * NT) team_rank_sort<NT, 4, K>(key, val, P);
-        else team_rank_sort<NT, 8, K>(key, val, P);
-    } else if (NT == 64 && P <= 4 * NT) {
-        // wave rows of up to 256 partials: the rank sort's P * 4 compares per
-        // lane cost less than the bitonic network's LDS passes (k_sg_wave
-        // 808 -> 538 us on the 2M-row Poisson(8) product); up to 512 with 8
-        // keys per lane measured the same as the network
-        team_rank_sort<NT, 4, K>(key, val, P);
+    // 2. sort by (column, generation)
+    if constexpr (KPL == 2) {
+        // 32 partials: 64 compares per lane, no more than the buckets cost
+        team_rank_sort<NT, KPL, K>(key, P);
     } else {
-        const uint32_t n2 = next_pow2(P < 2 * NT ? 2 * NT : P);
-        for (uint32_t p = P + t; p < n2; p += NT) key[p] = (K)~0ull;
-        team_sync<NT>();
-        for (uint32_t k = 2; k <= n2; k <<= 1) {
-            for (uint32_t js = k >> 1; js > 0; js >>= 1) {
-                for (uint32_t c = t; c < n2 / 2; c += NT) {
-                    const uint32_t i1 = (c / js) * 2 * js + (c % js);
-                    const uint32_t i2 = i1 + js;
-                    const bool asc = (i1 & k) == 0;
-                    const K ka = key[i1], kb = key[i2];
-                    if ((ka > kb) == asc) {
-                        key[i1] = kb;
-                        key[i2] = ka;
-                        const float va = val[i1];
-                        val[i1] = val[i2];
-                        val[i2] = va;
-                    }
-                }
-                team_sync<NT>();
-            }
-        }
+        team_sort<NT, KPL, GB, K>(key, hist, P, lds_w);
     }
     // 3. runs of equal columns, summed left to right from 0; drop exact zeros
+    constexpr uint32_t GM = (1u << GB) - 1u;
     uint32_t outc = 0;
     for (uint32_t p0 = 0; p0 < P; p0 += NT) {
         const uint32_t p = p0 + t;
@@ -451,16 +593,32 @@ __device__ void sg_row(const SgRowInfo &ri, const int32_t *__restrict__ a_col, c
         float s = 0.0f;
         uint32_t c = 0;
         if (p < P) {
-            c = (uint32_t)(key[p] >> GB);
+            const K k = key[p];
+            c = (uint32_t)(k >> GB);
             const bool head = p == 0 || (uint32_t)(key[p - 1] >> GB) != c;
             if (head) {
-                s = 0.0f + val[p];
-                for (uint32_t q = p + 1; q < P && (uint32_t)(key[q] >> GB) == c; ++q) s = s + val[q];
+                s = 0.0f + val[(uint32_t)k & GM];
+                for (uint32_t q = p + 1; q < P; ++q) {
+                    const K kq = key[q];
+                    if ((uint32_t)(kq >> GB) != c) break;
+                    s = s + val[(uint32_t)kq & GM];
+                }
                 emit = s != 0.0f;
             }
         }
-        uint32_t tot;
-        const uint32_t pos = team_excl_scan<NT>(emit ? 1u : 0u, lds_w, &tot);
+        // place among the team's emitting threads
+        uint32_t pos, tot;
+        const uint64_t m = __ballot(emit);
+        if constexpr (NT < 64) {
+            const uint32_t mt = (uint32_t)(m >> (lane_id() & ~(NT - 1))) & ((1u << NT) - 1u);
+            pos = (uint32_t)__popc(mt & ((1u << t) - 1u));
+            tot = (uint32_t)__popc(mt);
+        } else if constexpr (NT == 64) {
+            pos = (uint32_t)__popcll(m & lanemask_lt());
+            tot = (uint32_t)__popcll(m);
+        } else {
+            pos = team_excl_scan<NT>(emit ? 1u : 0u, lds_w, &tot);
+        }
         if (emit) {
             tcol[out_base + outc + pos] = (int32_t)c;
             tval[out_base + outc + pos] = s;
@@ -494,7 +652,7 @@ __device__ __forceinline__ void sg_rows(const uint32_t *__restrict__ list, uint3
 
 // Rows of at most WAVE_MAX partials: one wave per row.  K: 32-bit sort keys
 // (half the LDS per row, more rows in flight) when B's columns allow.
-template <typename K>
+template <int KPL, typename K>
 __global__ __launch_bounds__(TB) void k_sg_wave(const uint32_t *__restrict__ list, const SgState *__restrict__ st,
                                                 const uint32_t *__restrict__ P, const uint32_t *__restrict__ Poff,
                                                 const uint32_t *__restrict__ a_start, const int32_t *__restrict__ a_len,
@@ -504,16 +662,18 @@ __global__ __launch_bounds__(TB) void k_sg_wave(const uint32_t *__restrict__ lis
                                                 int32_t *__restrict__ tcol, float *__restrict__ tval,
                                                 uint32_t *__restrict__ cnt)
 {
-    __shared__ K key[TB / 64][WAVE_MAX];
-    __shared__ float val[TB / 64][WAVE_MAX];
+    static_assert(64 * KPL <= WAVE_MAX, "generations fit their key bits");
+    __shared__ __align__(16) K key[TB / 64][64 * KPL];
+    __shared__ float val[TB / 64][64 * KPL];
+    __shared__ uint32_t hist[TB / 64][64 * bucket_bpl<KPL>() / 2 + 1];
     __shared__ uint32_t s_ex[TB / 64][64], s_sb[TB / 64][64];
     __shared__ float s_va[TB / 64][64];
     const int w = threadIdx.x >> 6;
-    const uint32_t n = st->count[CL_WAVE];
+    const uint32_t n = st->count[CL_WAVE + (KPL > 4) + (KPL > 8)];
     sg_rows(list, n, blockIdx.x * (TB / 64) + w, gridDim.x * (TB / 64), P, Poff, a_start, a_len,
             [&](const SgRowInfo &ri) {
-                sg_row<64, WAVE_GB, K>(ri, a_col, a_val, b_start, b_len, b_col, b_val, tcol, tval, cnt, key[w],
-                                       val[w], s_ex[w], s_sb[w], s_va[w], nullptr);
+                sg_row<64, WAVE_GB, K, KPL>(ri, a_col, a_val, b_start, b_len, b_col, b_val, tcol, tval, cnt, key[w],
+                                       val[w], hist[w], s_ex[w], s_sb[w], s_va[w], nullptr);
             });
 }
 
@@ -532,10 +692,11 @@ __global__ __launch_bounds__(TB) void k_sg_team(const uint32_t *__restrict__ lis
     constexpr int NTEAM = TB / TEAM;
     // per-team rows padded so the four teams of a wave start on different
     // LDS banks; the pitch keeps every key row 16-byte aligned
-    constexpr uint32_t PITCH = TEAM_MAX + 20;
+    constexpr uint32_t PITCH = KPL * TEAM + 20;
     static_assert(PITCH % 4 == 0, "16-byte aligned key rows");
     __shared__ __align__(16) uint32_t key[NTEAM][PITCH];
     __shared__ float val[NTEAM][PITCH];
+    __shared__ uint32_t hist[NTEAM][KPL * TEAM / 2 + 5];
     __shared__ uint32_t s_ex[NTEAM][TEAM], s_sb[NTEAM][TEAM];
     __shared__ float s_va[NTEAM][TEAM];
     const int tm = threadIdx.x / TEAM;
@@ -544,12 +705,16 @@ __global__ __launch_bounds__(TB) void k_sg_team(const uint32_t *__restrict__ lis
     sg_rows(list, n, blockIdx.x * NTEAM + tm, gridDim.x * NTEAM, P, Poff, a_start, a_len,
             [&](const SgRowInfo &ri) {
                 sg_row<TEAM, TEAM_GB, uint32_t, KPL>(ri, a_col, a_val, b_start, b_len, b_col, b_val, tcol, tval,
-                                                     cnt, key[tm], val[tm], s_ex[tm], s_sb[tm], s_va[tm], nullptr);
+                                                     cnt, key[tm], val[tm], hist[tm], s_ex[tm], s_sb[tm], s_va[tm],
+                                                     nullptr);
             });
 }
 
-__global__ __launch_bounds__(TB) void k_sg_block(const uint32_t *__restrict__ list, const SgState *__restrict__ st,
-                                                 const uint32_t *__restrict__ P, const uint32_t *__restrict__ Poff,
+// One workgroup of NT threads per row of class `cls`, at most MAXP partials.
+template <int NT, int GB, uint32_t MAXP, typename K>
+__global__ __launch_bounds__(NT) void k_sg_block(const uint32_t *__restrict__ list, const SgState *__restrict__ st,
+                                                 int cls, const uint32_t *__restrict__ P,
+                                                 const uint32_t *__restrict__ Poff,
                                                  const uint32_t *__restrict__ a_start, const int32_t *__restrict__ a_len,
                                                  const int32_t *__restrict__ a_col, const float *__restrict__ a_val,
                                                  const uint32_t *__restrict__ b_start, const int32_t *__restrict__ b_len,
@@ -557,20 +722,22 @@ __global__ __launch_bounds__(TB) void k_sg_block(const uint32_t *__restrict__ li
                                                  int32_t *__restrict__ tcol, float *__restrict__ tval,
                                                  uint32_t *__restrict__ cnt)
 {
-    __shared__ uint64_t key[BLOCK_MAX];
-    __shared__ float val[BLOCK_MAX];
-    __shared__ uint32_t s_ex[TB], s_sb[TB];
-    __shared__ float s_va[TB];
-    __shared__ uint32_t lds_w[TB / 64];
-    const uint32_t n = st->count[CL_BLOCK];
+    constexpr int KPL = MAXP / NT;
+    __shared__ __align__(16) K key[MAXP];
+    __shared__ float val[MAXP];
+    __shared__ uint32_t hist[NT * bucket_bpl<KPL>() / 2 + 1];
+    __shared__ uint32_t s_ex[NT], s_sb[NT];
+    __shared__ float s_va[NT];
+    __shared__ uint32_t lds_w[2 * NT / 64];
+    const uint32_t n = st->count[cls];
     sg_rows(list, n, blockIdx.x, gridDim.x, P, Poff, a_start, a_len, [&](const SgRowInfo &ri) {
-        sg_row<TB, 12, uint64_t>(ri, a_col, a_val, b_start, b_len, b_col, b_val, tcol, tval, cnt, key, val, s_ex, s_sb,
-                                 s_va, lds_w);
+        sg_row<NT, GB, K, KPL>(ri, a_col, a_val, b_start, b_len, b_col, b_val, tcol, tval, cnt, key, val, hist, s_ex,
+                               s_sb, s_va, lds_w);
     });
 }
 
 // ---------------------------------------------------------------------------
-// global path for hub rows (P_i > BLOCK_MAX)
+// global path for hub rows (more partials than the large-row kernel holds)
 // ---------------------------------------------------------------------------
 // pre[2h] = len(A row), pre[2h+1] = P for hub row h (index hn: zeros)
 __global__ void k_sg_hprep(const uint32_t *__restrict__ hlist, uint32_t hn, const int32_t *__restrict__ a_len,
@@ -706,6 +873,23 @@ __global__ void k_sg_set_rows(uint32_t R, const uint32_t *__restrict__ Poff, con
     }
 }
 
+template <int NT, int GB, uint32_t MAXP, typename K>
+void launch_block(unsigned g, hipStream_t s, const uint32_t *list, const SgState *st, int cls, const uint32_t *P,
+                  const uint32_t *Poff, dcsr_handle A, dcsr_handle B, int32_t *tcol, float *tval, uint32_t *cnt)
+{
+    k_sg_block<NT, GB, MAXP, K><<<g, NT, 0, s>>>(list, st, cls, P, Poff, A->row_start, A->row_len, A->pool_col,
+                                                 A->pool_val, B->row_start, B->row_len, B->pool_col, B->pool_val, tcol,
+                                                 tval, cnt);
+}
+
+template <int KPL, typename K>
+void launch_wave(unsigned g, hipStream_t s, const uint32_t *list, const SgState *st, const uint32_t *P,
+                 const uint32_t *Poff, dcsr_handle A, dcsr_handle B, int32_t *tcol, float *tval, uint32_t *cnt)
+{
+    k_sg_wave<KPL, K><<<g, TB, 0, s>>>(list, st, P, Poff, A->row_start, A->row_len, A->pool_col, A->pool_val,
+                                       B->row_start, B->row_len, B->pool_col, B->pool_val, tcol, tval, cnt);
+}
+
 template <int KPL>
 void launch_team(unsigned g, hipStream_t s, const uint32_t *list, const SgState *st, const uint32_t *P,
                  const uint32_t *Poff, dcsr_handle A, dcsr_handle B, int32_t *tcol, float *tval, uint32_t *cnt)
@@ -743,7 +927,8 @@ dcsr_status dcsr_spgemm(dcsr_handle A, dcsr_handle B, dcsr_handle C, dcsr_stream
     k_sg_state_zero<<<1, 1, 0, s>>>(st);
     if (R > 0) {
         k_sg_count<<<grid_for(R, TB), TB, 0, s>>>(R, A->row_start, A->row_len, A->pool_col, B->row_len, P);
-        k_sg_classify<<<nbR, TB, 0, s>>>(R, P, lists, R + 1, st, cnt, bsum, B->cols <= TEAM_MAX_COLS ? 1u : 0u);
+        k_sg_classify<<<nbR, TB, 0, s>>>(R, P, lists, R + 1, st, cnt, bsum, B->cols <= TEAM_MAX_COLS ? 1u : 0u,
+                                            B->cols <= BIG_MAX_COLS32 ? BIG_MAX32 : BIG_MAX64);
         k_sg_total<<<1, 1024, 0, s>>>(st, bsum, (int)nbR);
     }
     DCSR_HIP(scan_exclusive_u32(P, Poff, R, 1, part, Poff + R, s, fault_word(C)));
@@ -777,22 +962,41 @@ dcsr_status dcsr_spgemm(dcsr_handle A, dcsr_handle B, dcsr_handle C, dcsr_stream
         default: launch_team<8>(g, s, list, st, P, Poff, A, B, tcol, tval, cnt); break;
         }
     }
-    if (hst.count[CL_WAVE]) {
-        const unsigned g = (unsigned)((hst.count[CL_WAVE] + 3) / 4 < 8192 ? (hst.count[CL_WAVE] + 3) / 4 : 8192);
-        if (B->cols <= WAVE_MAX_COLS32)
-            k_sg_wave<uint32_t><<<g, TB, 0, s>>>(lists + CL_WAVE * (uint64_t)(R + 1), st, P, Poff, A->row_start,
-                                                 A->row_len, A->pool_col, A->pool_val, B->row_start, B->row_len,
-                                                 B->pool_col, B->pool_val, tcol, tval, cnt);
-        else
-            k_sg_wave<uint64_t><<<g, TB, 0, s>>>(lists + CL_WAVE * (uint64_t)(R + 1), st, P, Poff, A->row_start,
-                                                 A->row_len, A->pool_col, A->pool_val, B->row_start, B->row_len,
-                                                 B->pool_col, B->pool_val, tcol, tval, cnt);
+    for (int c = CL_WAVE; c < CL_WAVE + NWAVECL; ++c) {
+        if (!hst.count[c]) continue;
+        const unsigned g = (hst.count[c] + 3) / 4 < 8192 ? (hst.count[c] + 3) / 4 : 8192;
+        const uint32_t *list = lists + c * (uint64_t)(R + 1);
+        const bool narrow = B->cols <= WAVE_MAX_COLS32;
+        switch (c - CL_WAVE) {
+        case 0:
+            if (narrow) launch_wave<4, uint32_t>(g, s, list, st, P, Poff, A, B, tcol, tval, cnt);
+            else launch_wave<4, uint64_t>(g, s, list, st, P, Poff, A, B, tcol, tval, cnt);
+            break;
+        case 1:
+            if (narrow) launch_wave<8, uint32_t>(g, s, list, st, P, Poff, A, B, tcol, tval, cnt);
+            else launch_wave<8, uint64_t>(g, s, list, st, P, Poff, A, B, tcol, tval, cnt);
+            break;
+        default:
+            if (narrow) launch_wave<16, uint32_t>(g, s, list, st, P, Poff, A, B, tcol, tval, cnt);
+            else launch_wave<16, uint64_t>(g, s, list, st, P, Poff, A, B, tcol, tval, cnt);
+            break;
+        }
     }
     if (hst.count[CL_BLOCK]) {
         const unsigned g = hst.count[CL_BLOCK] < 4096 ? hst.count[CL_BLOCK] : 4096;
-        k_sg_block<<<g, TB, 0, s>>>(lists + CL_BLOCK * (uint64_t)(R + 1), st, P, Poff, A->row_start, A->row_len,
-                                    A->pool_col, A->pool_val, B->row_start, B->row_len, B->pool_col, B->pool_val, tcol,
-                                    tval, cnt);
+        const uint32_t *list = lists + CL_BLOCK * (uint64_t)(R + 1);
+        if (B->cols <= BLOCK_MAX_COLS32)
+            launch_block<TB, BLOCK_GB, BLOCK_MAX, uint32_t>(g, s, list, st, CL_BLOCK, P, Poff, A, B, tcol, tval, cnt);
+        else
+            launch_block<TB, BLOCK_GB, BLOCK_MAX, uint64_t>(g, s, list, st, CL_BLOCK, P, Poff, A, B, tcol, tval, cnt);
+    }
+    if (hst.count[CL_BIG]) {
+        const unsigned g = hst.count[CL_BIG] < 1024 ? hst.count[CL_BIG] : 1024;
+        const uint32_t *list = lists + CL_BIG * (uint64_t)(R + 1);
+        if (B->cols <= BIG_MAX_COLS32)
+            launch_block<BIG_TB, BIG_GB, BIG_MAX32, uint32_t>(g, s, list, st, CL_BIG, P, Poff, A, B, tcol, tval, cnt);
+        else
+            launch_block<BIG_TB, BIG_GB, BIG_MAX64, uint64_t>(g, s, list, st, CL_BIG, P, Poff, A, B, tcol, tval, cnt);
     }
     if (hst.count[CL_HUB]) {
         const uint32_t hn = hst.count[CL_HUB];
