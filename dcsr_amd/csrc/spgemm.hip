@@ -76,35 +76,46 @@ __device__ __forceinline__ uint32_t next_pow2(uint32_t v)
     return v + 1;
 }
 
+// B's row table as one 8-byte record per row (start, length).
+__global__ void k_sg_brows(uint32_t rows, const uint32_t *__restrict__ b_start, const int32_t *__restrict__ b_len,
+                           uint2 *__restrict__ brow)
+{
+    const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
+    if (r < rows) brow[r] = make_uint2(b_start[r], (uint32_t)b_len[r]);
+}
+
 // P_i = sum over the entries of A row i of len(B row col).  One wave per 64
-// consecutive rows; entries folded per row with a DPP segmented scan.
-__global__ __launch_bounds__(TB) void k_sg_count(uint32_t R, const uint32_t *__restrict__ a_start,
-                                                 const int32_t *__restrict__ a_len, const int32_t *__restrict__ a_col,
-                                                 const int32_t *__restrict__ b_len, uint32_t *__restrict__ P)
+// consecutive rows; entries folded per row with a DPP segmented scan.  The B
+// row record of every A entry is kept in A's flat order (ent): the row
+// kernels stream it instead of gathering start and length again, each of
+// which costs a 128-byte line where B's row table exceeds an L2.
+__global__ __launch_bounds__(TB) void k_sg_count(uint32_t R, const uint32_t *__restrict__ a_foff,
+                                                 const uint32_t *__restrict__ a_start,
+                                                 const int32_t *__restrict__ a_col, const uint2 *__restrict__ brow,
+                                                 uint2 *__restrict__ ent, uint32_t *__restrict__ P)
 {
     __shared__ uint32_t s_ex[TB / 64][64];
     __shared__ uint32_t s_st[TB / 64][64];
     __shared__ uint32_t s_acc[TB / 64][64];
     const int w = threadIdx.x >> 6;
     const int lane = lane_id();
-    const uint32_t r = (blockIdx.x * (TB / 64) + w) * 64u + lane;
-    uint32_t st = 0, L = 0;
-    if (r < R) {
-        st = a_start[r];
-        L = (uint32_t)a_len[r];
-    }
-    const uint32_t inc = wave_incl_scan_u32(L);
-    const uint32_t tot = wave_read_lane_u32(inc, 63);
-    s_ex[w][lane] = inc - L;
-    s_st[w][lane] = st;
+    const uint32_t r0 = (blockIdx.x * (TB / 64) + w) * 64u;
+    const uint32_t r = r0 + lane;
+    if (r0 >= R) return;
+    const uint32_t fo = a_foff[r < R ? r : R];
+    const uint32_t f0 = wave_read_lane_u32(fo, 0);
+    const uint32_t tot = a_foff[r0 + 64u < R ? r0 + 64u : R] - f0;
+    s_ex[w][lane] = fo - f0;
+    s_st[w][lane] = r < R ? a_start[r] : 0u;
     s_acc[w][lane] = 0;
     __builtin_amdgcn_wave_barrier();
     // four 64-entry chunks per round: their A-column loads, then their B-row
-    // length loads, each issued together (two round trips per 256 entries)
+    // record loads, each issued together (two round trips per 256 entries)
     constexpr int CU = 4;
     for (uint32_t b = 0; b < tot; b += 64 * CU) {
-        uint32_t j[CU], p[CU];
+        uint32_t j[CU];
         int32_t c[CU];
+        uint2 q[CU];
 #pragma unroll
         for (int u = 0; u < CU; ++u) {
             const uint32_t e = b + (uint32_t)u * 64u + lane;
@@ -116,12 +127,13 @@ __global__ __launch_bounds__(TB) void k_sg_count(uint32_t R, const uint32_t *__r
             }
         }
 #pragma unroll
-        for (int u = 0; u < CU; ++u) p[u] = c[u] >= 0 ? (uint32_t)b_len[c[u]] : 0u;
+        for (int u = 0; u < CU; ++u) q[u] = c[u] >= 0 ? brow[c[u]] : make_uint2(0u, 0u);
 #pragma unroll
         for (int u = 0; u < CU; ++u) {
-            const uint32_t q = wave_seg_incl_scan_u32(p[u], j[u]);
+            if (c[u] >= 0) ent[(uint64_t)f0 + b + (uint32_t)u * 64u + lane] = q[u];
+            const uint32_t t = wave_seg_incl_scan_u32(q[u].y, j[u]);
             const uint32_t jn = __shfl_down(j[u], 1);
-            if (j[u] < 64 && (lane == 63 || jn != j[u])) s_acc[w][j[u]] += q;
+            if (j[u] < 64 && (lane == 63 || jn != j[u])) s_acc[w][j[u]] += t;
             __builtin_amdgcn_wave_barrier();
         }
     }
@@ -288,21 +300,37 @@ __device__ __forceinline__ uint32_t find_seg_team(const uint32_t *s, uint32_t e)
 // and A row.  Loaded one row ahead by the kernels' row loops (the loads of
 // the next row are in flight while the current row is processed).
 struct SgRowInfo {
-    uint32_t row, P, ast, la;
+    uint32_t row, P, ast, la, fo;
     uint64_t out_base;
 };
 
-__device__ __forceinline__ SgRowInfo sg_row_info(uint32_t row, const uint32_t *__restrict__ P,
-                                                 const uint32_t *__restrict__ Poff,
-                                                 const uint32_t *__restrict__ a_start,
-                                                 const int32_t *__restrict__ a_len)
+// What the row kernels read: A's row table and values, the B row record of
+// every A entry (flat order), B's pool.
+struct SgIn {
+    const uint32_t *P, *Poff, *a_start;
+    const int32_t *a_len;
+    const uint32_t *a_foff;
+    const float *a_val;
+    const uint2 *ent;
+    const int32_t *b_col;
+    const float *b_val;
+};
+// What they write: C's pool and the row's entry count.
+struct SgOut {
+    int32_t *tcol;
+    float *tval;
+    uint32_t *cnt;
+};
+
+__device__ __forceinline__ SgRowInfo sg_row_info(uint32_t row, const SgIn &in)
 {
     SgRowInfo r;
     r.row = row;
-    r.P = P[row];
-    r.out_base = Poff[row];
-    r.ast = a_start[row];
-    r.la = (uint32_t)a_len[row];
+    r.P = in.P[row];
+    r.out_base = in.Poff[row];
+    r.ast = in.a_start[row];
+    r.la = (uint32_t)in.a_len[row];
+    r.fo = in.a_foff[row];
     return r;
 }
 
@@ -521,11 +549,8 @@ __device__ __forceinline__ void team_sort(K *key, uint32_t *hist, uint32_t P, ui
 // (generation order); only the keys are sorted, and a sorted key names its
 // product by its generation bits.
 template <int NT, int GB, typename K, int KPL>
-__device__ void sg_row(const SgRowInfo &ri, const int32_t *__restrict__ a_col, const float *__restrict__ a_val,
-                       const uint32_t *__restrict__ b_start, const int32_t *__restrict__ b_len,
-                       const int32_t *__restrict__ b_col, const float *__restrict__ b_val,
-                       int32_t *__restrict__ tcol, float *__restrict__ tval, uint32_t *__restrict__ cnt, K *key,
-                       float *val, uint32_t *hist, uint32_t *s_ex, uint32_t *s_sb, float *s_va, uint32_t *lds_w)
+__device__ void sg_row(const SgRowInfo &ri, const SgIn &in, const SgOut &out, K *key, float *val, uint32_t *hist,
+                       uint32_t *s_ex, uint32_t *s_sb, float *s_va, uint32_t *lds_w)
 {
     const uint32_t t = threadIdx.x % NT;
     const uint32_t row = ri.row, P = ri.P, ast = ri.ast, la = ri.la;
@@ -537,10 +562,10 @@ __device__ void sg_row(const SgRowInfo &ri, const int32_t *__restrict__ a_col, c
         uint32_t lb = 0, sb = 0;
         float va = 0.0f;
         if (a < la) {
-            const int32_t j = a_col[(uint64_t)ast + a];
-            va = a_val[(uint64_t)ast + a];
-            lb = (uint32_t)b_len[j];
-            sb = b_start[j];
+            const uint2 q = in.ent[(uint64_t)ri.fo + a];
+            va = in.a_val[(uint64_t)ast + a];
+            sb = q.x;
+            lb = q.y;
         }
         uint32_t tot;
         const uint32_t ex = team_excl_scan<NT>(lb, lds_w, &tot);
@@ -560,8 +585,8 @@ __device__ void sg_row(const SgRowInfo &ri, const int32_t *__restrict__ a_col, c
                 const uint32_t pe = e0 + (uint32_t)i * NT + t;
                 const uint32_t q = find_seg_team<NT>(s_ex, pe < tot ? pe : 0u);
                 const uint64_t bp = pe < tot ? (uint64_t)s_sb[q] + (pe - s_ex[q]) : 0u;
-                bc[i] = b_col[bp];
-                bv[i] = b_val[bp];
+                bc[i] = in.b_col[bp];
+                bv[i] = in.b_val[bp];
                 av[i] = s_va[q];
             }
 #pragma unroll
@@ -620,12 +645,12 @@ __device__ void sg_row(const SgRowInfo &ri, const int32_t *__restrict__ a_col, c
             pos = team_excl_scan<NT>(emit ? 1u : 0u, lds_w, &tot);
         }
         if (emit) {
-            tcol[out_base + outc + pos] = (int32_t)c;
-            tval[out_base + outc + pos] = s;
+            out.tcol[out_base + outc + pos] = (int32_t)c;
+            out.tval[out_base + outc + pos] = s;
         }
         outc += tot;
     }
-    if (t == 0) cnt[row] = outc;
+    if (t == 0) out.cnt[row] = outc;
     team_sync<NT>();
 }
 
@@ -633,16 +658,14 @@ __device__ void sg_row(const SgRowInfo &ri, const int32_t *__restrict__ a_col, c
 // id and info are loaded one and two iterations ahead.
 template <typename F>
 __device__ __forceinline__ void sg_rows(const uint32_t *__restrict__ list, uint32_t n, uint32_t first, uint32_t step,
-                                        const uint32_t *__restrict__ P, const uint32_t *__restrict__ Poff,
-                                        const uint32_t *__restrict__ a_start, const int32_t *__restrict__ a_len,
-                                        F &&body)
+                                        const SgIn &in, F &&body)
 {
     if (first >= n) return;
-    SgRowInfo cur = sg_row_info(list[first], P, Poff, a_start, a_len);
+    SgRowInfo cur = sg_row_info(list[first], in);
     uint32_t next_id = first + step < n ? list[first + step] : 0u;
     for (uint32_t i = first; i < n; i += step) {
         SgRowInfo nxt{};
-        if (i + step < n) nxt = sg_row_info(next_id, P, Poff, a_start, a_len);
+        if (i + step < n) nxt = sg_row_info(next_id, in);
         const uint32_t nn_id = i + 2 * step < n ? list[i + 2 * step] : 0u;
         body(cur);
         cur = nxt;
@@ -650,17 +673,11 @@ __device__ __forceinline__ void sg_rows(const uint32_t *__restrict__ list, uint3
     }
 }
 
-// Rows of at most WAVE_MAX partials: one wave per row.  K: 32-bit sort keys
+// Wave rows: one wave per row, at most 64 * KPL partials.  K: 32-bit sort keys
 // (half the LDS per row, more rows in flight) when B's columns allow.
 template <int KPL, typename K>
 __global__ __launch_bounds__(TB) void k_sg_wave(const uint32_t *__restrict__ list, const SgState *__restrict__ st,
-                                                const uint32_t *__restrict__ P, const uint32_t *__restrict__ Poff,
-                                                const uint32_t *__restrict__ a_start, const int32_t *__restrict__ a_len,
-                                                const int32_t *__restrict__ a_col, const float *__restrict__ a_val,
-                                                const uint32_t *__restrict__ b_start, const int32_t *__restrict__ b_len,
-                                                const int32_t *__restrict__ b_col, const float *__restrict__ b_val,
-                                                int32_t *__restrict__ tcol, float *__restrict__ tval,
-                                                uint32_t *__restrict__ cnt)
+                                                SgIn in, SgOut out)
 {
     static_assert(64 * KPL <= WAVE_MAX, "generations fit their key bits");
     __shared__ __align__(16) K key[TB / 64][64 * KPL];
@@ -670,24 +687,16 @@ __global__ __launch_bounds__(TB) void k_sg_wave(const uint32_t *__restrict__ lis
     __shared__ float s_va[TB / 64][64];
     const int w = threadIdx.x >> 6;
     const uint32_t n = st->count[CL_WAVE + (KPL > 4) + (KPL > 8)];
-    sg_rows(list, n, blockIdx.x * (TB / 64) + w, gridDim.x * (TB / 64), P, Poff, a_start, a_len,
-            [&](const SgRowInfo &ri) {
-                sg_row<64, WAVE_GB, K, KPL>(ri, a_col, a_val, b_start, b_len, b_col, b_val, tcol, tval, cnt, key[w],
-                                       val[w], hist[w], s_ex[w], s_sb[w], s_va[w], nullptr);
-            });
+    sg_rows(list, n, blockIdx.x * (TB / 64) + w, gridDim.x * (TB / 64), in, [&](const SgRowInfo &ri) {
+        sg_row<64, WAVE_GB, K, KPL>(ri, in, out, key[w], val[w], hist[w], s_ex[w], s_sb[w], s_va[w], nullptr);
+    });
 }
 
 // Rows of at most KPL * TEAM partials (class CL_TEAM + KPL / 2 - 1): 16-lane
 // teams, four rows per wave.
 template <int KPL>
 __global__ __launch_bounds__(TB) void k_sg_team(const uint32_t *__restrict__ list, const SgState *__restrict__ st,
-                                                const uint32_t *__restrict__ P, const uint32_t *__restrict__ Poff,
-                                                const uint32_t *__restrict__ a_start, const int32_t *__restrict__ a_len,
-                                                const int32_t *__restrict__ a_col, const float *__restrict__ a_val,
-                                                const uint32_t *__restrict__ b_start, const int32_t *__restrict__ b_len,
-                                                const int32_t *__restrict__ b_col, const float *__restrict__ b_val,
-                                                int32_t *__restrict__ tcol, float *__restrict__ tval,
-                                                uint32_t *__restrict__ cnt)
+                                                SgIn in, SgOut out)
 {
     constexpr int NTEAM = TB / TEAM;
     // per-team rows padded so the four teams of a wave start on different
@@ -702,25 +711,16 @@ __global__ __launch_bounds__(TB) void k_sg_team(const uint32_t *__restrict__ lis
     const int tm = threadIdx.x / TEAM;
     static_assert(KPL * TEAM <= TEAM_MAX, "a team row fits its LDS row");
     const uint32_t n = st->count[CL_TEAM + KPL / 2 - 1];
-    sg_rows(list, n, blockIdx.x * NTEAM + tm, gridDim.x * NTEAM, P, Poff, a_start, a_len,
-            [&](const SgRowInfo &ri) {
-                sg_row<TEAM, TEAM_GB, uint32_t, KPL>(ri, a_col, a_val, b_start, b_len, b_col, b_val, tcol, tval,
-                                                     cnt, key[tm], val[tm], hist[tm], s_ex[tm], s_sb[tm], s_va[tm],
-                                                     nullptr);
-            });
+    sg_rows(list, n, blockIdx.x * NTEAM + tm, gridDim.x * NTEAM, in, [&](const SgRowInfo &ri) {
+        sg_row<TEAM, TEAM_GB, uint32_t, KPL>(ri, in, out, key[tm], val[tm], hist[tm], s_ex[tm], s_sb[tm], s_va[tm],
+                                             nullptr);
+    });
 }
 
 // One workgroup of NT threads per row of class `cls`, at most MAXP partials.
 template <int NT, int GB, uint32_t MAXP, typename K>
 __global__ __launch_bounds__(NT) void k_sg_block(const uint32_t *__restrict__ list, const SgState *__restrict__ st,
-                                                 int cls, const uint32_t *__restrict__ P,
-                                                 const uint32_t *__restrict__ Poff,
-                                                 const uint32_t *__restrict__ a_start, const int32_t *__restrict__ a_len,
-                                                 const int32_t *__restrict__ a_col, const float *__restrict__ a_val,
-                                                 const uint32_t *__restrict__ b_start, const int32_t *__restrict__ b_len,
-                                                 const int32_t *__restrict__ b_col, const float *__restrict__ b_val,
-                                                 int32_t *__restrict__ tcol, float *__restrict__ tval,
-                                                 uint32_t *__restrict__ cnt)
+                                                 int cls, SgIn in, SgOut out)
 {
     constexpr int KPL = MAXP / NT;
     __shared__ __align__(16) K key[MAXP];
@@ -730,9 +730,8 @@ __global__ __launch_bounds__(NT) void k_sg_block(const uint32_t *__restrict__ li
     __shared__ float s_va[NT];
     __shared__ uint32_t lds_w[2 * NT / 64];
     const uint32_t n = st->count[cls];
-    sg_rows(list, n, blockIdx.x, gridDim.x, P, Poff, a_start, a_len, [&](const SgRowInfo &ri) {
-        sg_row<NT, GB, K, KPL>(ri, a_col, a_val, b_start, b_len, b_col, b_val, tcol, tval, cnt, key, val, hist, s_ex,
-                               s_sb, s_va, lds_w);
+    sg_rows(list, n, blockIdx.x, gridDim.x, in, [&](const SgRowInfo &ri) {
+        sg_row<NT, GB, K, KPL>(ri, in, out, key, val, hist, s_ex, s_sb, s_va, lds_w);
     });
 }
 
@@ -873,31 +872,6 @@ __global__ void k_sg_set_rows(uint32_t R, const uint32_t *__restrict__ Poff, con
     }
 }
 
-template <int NT, int GB, uint32_t MAXP, typename K>
-void launch_block(unsigned g, hipStream_t s, const uint32_t *list, const SgState *st, int cls, const uint32_t *P,
-                  const uint32_t *Poff, dcsr_handle A, dcsr_handle B, int32_t *tcol, float *tval, uint32_t *cnt)
-{
-    k_sg_block<NT, GB, MAXP, K><<<g, NT, 0, s>>>(list, st, cls, P, Poff, A->row_start, A->row_len, A->pool_col,
-                                                 A->pool_val, B->row_start, B->row_len, B->pool_col, B->pool_val, tcol,
-                                                 tval, cnt);
-}
-
-template <int KPL, typename K>
-void launch_wave(unsigned g, hipStream_t s, const uint32_t *list, const SgState *st, const uint32_t *P,
-                 const uint32_t *Poff, dcsr_handle A, dcsr_handle B, int32_t *tcol, float *tval, uint32_t *cnt)
-{
-    k_sg_wave<KPL, K><<<g, TB, 0, s>>>(list, st, P, Poff, A->row_start, A->row_len, A->pool_col, A->pool_val,
-                                       B->row_start, B->row_len, B->pool_col, B->pool_val, tcol, tval, cnt);
-}
-
-template <int KPL>
-void launch_team(unsigned g, hipStream_t s, const uint32_t *list, const SgState *st, const uint32_t *P,
-                 const uint32_t *Poff, dcsr_handle A, dcsr_handle B, int32_t *tcol, float *tval, uint32_t *cnt)
-{
-    k_sg_team<KPL><<<g, TB, 0, s>>>(list, st, P, Poff, A->row_start, A->row_len, A->pool_col, A->pool_val,
-                                    B->row_start, B->row_len, B->pool_col, B->pool_val, tcol, tval, cnt);
-}
-
 }  // namespace
 
 dcsr_status dcsr_spgemm(dcsr_handle A, dcsr_handle B, dcsr_handle C, dcsr_stream_t stream)
@@ -923,10 +897,18 @@ dcsr_status dcsr_spgemm(dcsr_handle A, dcsr_handle B, dcsr_handle C, dcsr_stream
     DCSR_TRY(ws_get(C, WS_SG_BSUM, (size_t)nbR * 8, (void **)&bsum));
     DCSR_TRY(ws_get_zeroed(C, WS_PART, scan_part_words(R + 1, 2) * 4, (void **)&part, s));
 
+    DCSR_TRY(ensure_flat(A, s));
+    const uint32_t *a_foff = (const uint32_t *)A->ws.ptr[WS_FOFF];
+    uint2 *brow, *ent;
+    DCSR_TRY(ws_get(C, WS_SG_BROW, (size_t)(B->rows + 1) * 8, (void **)&brow));
+    DCSR_TRY(ws_get(C, WS_SG_ENT, (size_t)(A->nnz_h + 1) * 8, (void **)&ent));
+
     // 1. partial counts, classes, offsets
     k_sg_state_zero<<<1, 1, 0, s>>>(st);
     if (R > 0) {
-        k_sg_count<<<grid_for(R, TB), TB, 0, s>>>(R, A->row_start, A->row_len, A->pool_col, B->row_len, P);
+        if (B->rows > 0)
+            k_sg_brows<<<grid_for(B->rows, TB), TB, 0, s>>>((uint32_t)B->rows, B->row_start, B->row_len, brow);
+        k_sg_count<<<grid_for(R, TB), TB, 0, s>>>(R, a_foff, A->row_start, A->pool_col, brow, ent, P);
         k_sg_classify<<<nbR, TB, 0, s>>>(R, P, lists, R + 1, st, cnt, bsum, B->cols <= TEAM_MAX_COLS ? 1u : 0u,
                                             B->cols <= BIG_MAX_COLS32 ? BIG_MAX32 : BIG_MAX64);
         k_sg_total<<<1, 1024, 0, s>>>(st, bsum, (int)nbR);
@@ -949,55 +931,35 @@ dcsr_status dcsr_spgemm(dcsr_handle A, dcsr_handle B, dcsr_handle C, dcsr_stream
     float *tval = C->pool_val;
 
     // 2. numeric phases
-    for (int c = CL_TEAM; c < CL_TEAM + NTEAMCL; ++c) {
-        if (!hst.count[c]) continue;
-        const uint32_t per = TB / TEAM;
+    const SgIn in{P, Poff, A->row_start, A->row_len, a_foff, A->pool_val, ent, B->pool_col, B->pool_val};
+    const SgOut out{tcol, tval, cnt};
+    // launches `kernel` over the rows of class c, `per` rows to a workgroup of
+    // nt threads, on at most `most` workgroups (they stride over the rest)
+    auto run = [&](auto kernel, int c, uint32_t per, uint32_t most, int nt, auto... cls) {
         const uint32_t want = (hst.count[c] + per - 1) / per;
-        const unsigned g = want < 8192 ? want : 8192;
-        const uint32_t *list = lists + c * (uint64_t)(R + 1);
-        switch (c - CL_TEAM) {
-        case 0: launch_team<2>(g, s, list, st, P, Poff, A, B, tcol, tval, cnt); break;
-        case 1: launch_team<4>(g, s, list, st, P, Poff, A, B, tcol, tval, cnt); break;
-        case 2: launch_team<6>(g, s, list, st, P, Poff, A, B, tcol, tval, cnt); break;
-        default: launch_team<8>(g, s, list, st, P, Poff, A, B, tcol, tval, cnt); break;
-        }
+        if (want) kernel<<<want < most ? want : most, nt, 0, s>>>(lists + c * (uint64_t)(R + 1), st, cls..., in, out);
+    };
+    run(k_sg_team<2>, CL_TEAM + 0, TB / TEAM, 8192, TB);
+    run(k_sg_team<4>, CL_TEAM + 1, TB / TEAM, 8192, TB);
+    run(k_sg_team<6>, CL_TEAM + 2, TB / TEAM, 8192, TB);
+    run(k_sg_team<8>, CL_TEAM + 3, TB / TEAM, 8192, TB);
+    if (B->cols <= WAVE_MAX_COLS32) {
+        run(k_sg_wave<4, uint32_t>, CL_WAVE + 0, 4, 8192, TB);
+        run(k_sg_wave<8, uint32_t>, CL_WAVE + 1, 4, 8192, TB);
+        run(k_sg_wave<16, uint32_t>, CL_WAVE + 2, 4, 8192, TB);
+    } else {
+        run(k_sg_wave<4, uint64_t>, CL_WAVE + 0, 4, 8192, TB);
+        run(k_sg_wave<8, uint64_t>, CL_WAVE + 1, 4, 8192, TB);
+        run(k_sg_wave<16, uint64_t>, CL_WAVE + 2, 4, 8192, TB);
     }
-    for (int c = CL_WAVE; c < CL_WAVE + NWAVECL; ++c) {
-        if (!hst.count[c]) continue;
-        const unsigned g = (hst.count[c] + 3) / 4 < 8192 ? (hst.count[c] + 3) / 4 : 8192;
-        const uint32_t *list = lists + c * (uint64_t)(R + 1);
-        const bool narrow = B->cols <= WAVE_MAX_COLS32;
-        switch (c - CL_WAVE) {
-        case 0:
-            if (narrow) launch_wave<4, uint32_t>(g, s, list, st, P, Poff, A, B, tcol, tval, cnt);
-            else launch_wave<4, uint64_t>(g, s, list, st, P, Poff, A, B, tcol, tval, cnt);
-            break;
-        case 1:
-            if (narrow) launch_wave<8, uint32_t>(g, s, list, st, P, Poff, A, B, tcol, tval, cnt);
-            else launch_wave<8, uint64_t>(g, s, list, st, P, Poff, A, B, tcol, tval, cnt);
-            break;
-        default:
-            if (narrow) launch_wave<16, uint32_t>(g, s, list, st, P, Poff, A, B, tcol, tval, cnt);
-            else launch_wave<16, uint64_t>(g, s, list, st, P, Poff, A, B, tcol, tval, cnt);
-            break;
-        }
-    }
-    if (hst.count[CL_BLOCK]) {
-        const unsigned g = hst.count[CL_BLOCK] < 4096 ? hst.count[CL_BLOCK] : 4096;
-        const uint32_t *list = lists + CL_BLOCK * (uint64_t)(R + 1);
-        if (B->cols <= BLOCK_MAX_COLS32)
-            launch_block<TB, BLOCK_GB, BLOCK_MAX, uint32_t>(g, s, list, st, CL_BLOCK, P, Poff, A, B, tcol, tval, cnt);
-        else
-            launch_block<TB, BLOCK_GB, BLOCK_MAX, uint64_t>(g, s, list, st, CL_BLOCK, P, Poff, A, B, tcol, tval, cnt);
-    }
-    if (hst.count[CL_BIG]) {
-        const unsigned g = hst.count[CL_BIG] < 1024 ? hst.count[CL_BIG] : 1024;
-        const uint32_t *list = lists + CL_BIG * (uint64_t)(R + 1);
-        if (B->cols <= BIG_MAX_COLS32)
-            launch_block<BIG_TB, BIG_GB, BIG_MAX32, uint32_t>(g, s, list, st, CL_BIG, P, Poff, A, B, tcol, tval, cnt);
-        else
-            launch_block<BIG_TB, BIG_GB, BIG_MAX64, uint64_t>(g, s, list, st, CL_BIG, P, Poff, A, B, tcol, tval, cnt);
-    }
+    if (B->cols <= BLOCK_MAX_COLS32)
+        run(k_sg_block<TB, BLOCK_GB, BLOCK_MAX, uint32_t>, CL_BLOCK, 1, 4096, TB, (int)CL_BLOCK);
+    else
+        run(k_sg_block<TB, BLOCK_GB, BLOCK_MAX, uint64_t>, CL_BLOCK, 1, 4096, TB, (int)CL_BLOCK);
+    if (B->cols <= BIG_MAX_COLS32)
+        run(k_sg_block<BIG_TB, BIG_GB, BIG_MAX32, uint32_t>, CL_BIG, 1, 1024, BIG_TB, (int)CL_BIG);
+    else
+        run(k_sg_block<BIG_TB, BIG_GB, BIG_MAX64, uint64_t>, CL_BIG, 1, 1024, BIG_TB, (int)CL_BIG);
     if (hst.count[CL_HUB]) {
         const uint32_t hn = hst.count[CL_HUB];
         const uint32_t *hlist = lists + CL_HUB * (uint64_t)(R + 1);
