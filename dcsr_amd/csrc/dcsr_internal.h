@@ -69,7 +69,7 @@ enum WsSlot {
     WS_SG_HPRE, WS_SG_EA, WS_SG_APOS, WS_SG_KEY0, WS_SG_KEY1, WS_SG_VAL0, WS_SG_VAL1, WS_SG_FLAG, WS_SG_EPOS,
     WS_CANON, WS_TMP0, WS_TMP1, WS_TMP2,
     WS_PNL_OFF, WS_PNL_BND, WS_PNL_COL, WS_PNL_VAL, WS_PNL_MAP, WS_PNL_PART,
-    WS_TRS, WS_TLEN, WS_PSPAN, WS_MSPAN, WS_TCAP, WS_ROWT, WS_SG_BROW, WS_SG_ENT,
+    WS_TRS, WS_TLEN, WS_PSPAN, WS_MSPAN, WS_TCAP, WS_ROWT, WS_SG_BENT, WS_SG_ENT,
     WS_COUNT
 };
 
@@ -213,6 +213,10 @@ dcsr_status update_commit(dcsr_handle h, int64_t n, hipStream_t s, bool nosync);
 dcsr_status update_fixed_scratch(dcsr_handle h, const int32_t *rows, const int32_t *cols, const float *vals,
                                  int64_t n, uint32_t flags, hipStream_t s, uint8_t *base, size_t cap);
 size_t update_scratch_bytes(dcsr_handle h, int64_t n);
+
+// matrix.hip: the live entries as (column, value) pairs in flat order, and the
+// flat offsets (current; R+1 words).
+dcsr_status copy_rows_paired(dcsr_handle h, uint2 *dst, const uint32_t **off, hipStream_t s);
 
 // The handle's sticky status word (device): scans set ST_SCAN_FALLBACK in it.
 static inline unsigned int *fault_word(dcsr_handle h) { return &h->ds->status; }

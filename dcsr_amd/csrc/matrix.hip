@@ -202,15 +202,18 @@ __global__ void k_set_loaded(int64_t R, const uint32_t *__restrict__ foff, uint3
 // from the row map of the flat offsets (one load; a search only past a run of
 // 64 or more empty rows).  With row_offsets (an export) the kernel also stores
 // the offsets there; nothing is written when the rows hold more than `limit`
-// entries, so a caller need not know the count before the launch.
+// entries, so a caller need not know the count before the launch.  PAIR: the
+// entries go to dst_pair as (column, value bits) pairs.
 constexpr uint32_t CP_SPAN = 1024;
 constexpr uint32_t CP_PER = CP_SPAN / 64;
+template <bool PAIR>
 __global__ __launch_bounds__(TB) void k_copy_rows(const uint32_t *__restrict__ dst_off,
                                                   const uint32_t *__restrict__ rowmap, uint32_t R, uint64_t limit,
                                                   int32_t *__restrict__ row_offsets,
                                                   const uint32_t *__restrict__ src_start,
                                                   const int32_t *__restrict__ src_col, const float *__restrict__ src_val,
-                                                  int32_t *__restrict__ dst_col, float *__restrict__ dst_val)
+                                                  int32_t *__restrict__ dst_col, float *__restrict__ dst_val,
+                                                  uint2 *__restrict__ dst_pair)
 {
     struct Lds {
         uint32_t off[65];
@@ -274,8 +277,12 @@ __global__ __launch_bounds__(TB) void k_copy_rows(const uint32_t *__restrict__ d
             for (uint32_t q = 0; q < CP_PER; ++q) {
                 const uint32_t p = q * 64u + lane;
                 if (p < cnt) {
-                    dst_col[e + p] = c[q];
-                    dst_val[e + p] = v[q];
+                    if constexpr (PAIR) {
+                        dst_pair[e + p] = make_uint2((uint32_t)c[q], __float_as_uint(v[q]));
+                    } else {
+                        dst_col[e + p] = c[q];
+                        dst_val[e + p] = v[q];
+                    }
                 }
             }
             __builtin_amdgcn_wave_barrier();
@@ -858,7 +865,7 @@ static dcsr_status flat_rows(dcsr_handle h, hipStream_t s, const uint32_t **off,
 
 // total: an upper bound of the entries (sizes the grid); see k_copy_rows.
 static void launch_copy_rows(dcsr_handle h, const uint32_t *off, const uint32_t *rowmap, int64_t total, uint64_t limit,
-                             int32_t *row_offsets, int32_t *dcol, float *dval, hipStream_t s)
+                             int32_t *row_offsets, int32_t *dcol, float *dval, hipStream_t s, uint2 *dpair = nullptr)
 {
     const int64_t R = h->rows;
     if (R <= 0 || (total <= 0 && !row_offsets)) return;
@@ -867,8 +874,23 @@ static void launch_copy_rows(dcsr_handle h, const uint32_t *off, const uint32_t 
     if (row_offsets && blocks < (R + 1) / (TB * 8)) blocks = (R + 1) / (TB * 8);
     if (blocks > 2048) blocks = 2048;  // waves stride over the rest
     if (blocks < 1) blocks = 1;
-    k_copy_rows<<<(unsigned)blocks, TB, 0, s>>>(off, rowmap, (uint32_t)R, limit, row_offsets, h->row_start,
-                                                h->pool_col, h->pool_val, dcol, dval);
+    if (dpair)
+        k_copy_rows<true><<<(unsigned)blocks, TB, 0, s>>>(off, rowmap, (uint32_t)R, limit, row_offsets, h->row_start,
+                                                          h->pool_col, h->pool_val, nullptr, nullptr, dpair);
+    else
+        k_copy_rows<false><<<(unsigned)blocks, TB, 0, s>>>(off, rowmap, (uint32_t)R, limit, row_offsets, h->row_start,
+                                                           h->pool_col, h->pool_val, dcol, dval, nullptr);
+}
+
+// The live entries as (column, value) pairs in flat order; *off receives the
+// flat offsets (state known).
+dcsr_status copy_rows_paired(dcsr_handle h, uint2 *dst, const uint32_t **off, hipStream_t s)
+{
+    const uint32_t *rowmap;
+    DCSR_TRY(flat_rows(h, s, off, &rowmap));
+    launch_copy_rows(h, *off, rowmap, h->nnz_h, ~0ull, nullptr, nullptr, nullptr, s, dst);
+    DCSR_HIP(hipGetLastError());
+    return DCSR_OK;
 }
 
 // Canonical export of a matrix with duplicates / zeros (state known).

@@ -76,22 +76,14 @@ __device__ __forceinline__ uint32_t next_pow2(uint32_t v)
     return v + 1;
 }
 
-// B's row table as one 8-byte record per row (start, length).
-__global__ void k_sg_brows(uint32_t rows, const uint32_t *__restrict__ b_start, const int32_t *__restrict__ b_len,
-                           uint2 *__restrict__ brow)
-{
-    const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r < rows) brow[r] = make_uint2(b_start[r], (uint32_t)b_len[r]);
-}
-
 // P_i = sum over the entries of A row i of len(B row col).  One wave per 64
 // consecutive rows; entries folded per row with a DPP segmented scan.  The B
-// row record of every A entry is kept in A's flat order (ent): the row
-// kernels stream it instead of gathering start and length again, each of
-// which costs a 128-byte line where B's row table exceeds an L2.
+// row (flat start, length) of every A entry is kept in A's flat order (ent):
+// the row kernels stream it instead of gathering it again.
 __global__ __launch_bounds__(TB) void k_sg_count(uint32_t R, const uint32_t *__restrict__ a_foff,
                                                  const uint32_t *__restrict__ a_start,
-                                                 const int32_t *__restrict__ a_col, const uint2 *__restrict__ brow,
+                                                 const int32_t *__restrict__ a_col,
+                                                 const uint32_t *__restrict__ b_foff,
                                                  uint2 *__restrict__ ent, uint32_t *__restrict__ P)
 {
     __shared__ uint32_t s_ex[TB / 64][64];
@@ -127,7 +119,11 @@ __global__ __launch_bounds__(TB) void k_sg_count(uint32_t R, const uint32_t *__r
             }
         }
 #pragma unroll
-        for (int u = 0; u < CU; ++u) q[u] = c[u] >= 0 ? brow[c[u]] : make_uint2(0u, 0u);
+        for (int u = 0; u < CU; ++u) {
+            // neighbours in one array: one line, mostly
+            q[u] = c[u] >= 0 ? make_uint2(b_foff[c[u]], b_foff[c[u] + 1]) : make_uint2(0u, 0u);
+            q[u].y -= q[u].x;
+        }
 #pragma unroll
         for (int u = 0; u < CU; ++u) {
             if (c[u] >= 0) ent[(uint64_t)f0 + b + (uint32_t)u * 64u + lane] = q[u];
@@ -304,16 +300,19 @@ struct SgRowInfo {
     uint64_t out_base;
 };
 
-// What the row kernels read: A's row table and values, the B row record of
-// every A entry (flat order), B's pool.
+// What the row kernels read: A's row table and values, the B row of every A
+// entry (A's flat order), B's entries as (column, value) pairs in B's flat
+// order.  A short row of B is one 128-byte line of pairs where the pool's two
+// arrays cost one line each, and these lines bound the product of matrices
+// past the L2 (2M-row Poisson(8): the 16-lane kernels 1083 -> 1006 us and the
+// count 248 -> 181, the copy costs 77).
 struct SgIn {
     const uint32_t *P, *Poff, *a_start;
     const int32_t *a_len;
     const uint32_t *a_foff;
     const float *a_val;
     const uint2 *ent;
-    const int32_t *b_col;
-    const float *b_val;
+    const uint2 *b_ent;
 };
 // What they write: C's pool and the row's entry count.
 struct SgOut {
@@ -578,15 +577,14 @@ __device__ void sg_row(const SgRowInfo &ri, const SgIn &in, const SgOut &out, K 
         // and writes nothing)
         constexpr int EX = KPL < SG_EX ? KPL : SG_EX;
         for (uint32_t e0 = 0; e0 < tot; e0 += EX * NT) {
-            int32_t bc[EX];
-            float bv[EX], av[EX];
+            uint2 be[EX];
+            float av[EX];
 #pragma unroll
             for (int i = 0; i < EX; ++i) {
                 const uint32_t pe = e0 + (uint32_t)i * NT + t;
                 const uint32_t q = find_seg_team<NT>(s_ex, pe < tot ? pe : 0u);
                 const uint64_t bp = pe < tot ? (uint64_t)s_sb[q] + (pe - s_ex[q]) : 0u;
-                bc[i] = in.b_col[bp];
-                bv[i] = in.b_val[bp];
+                be[i] = in.b_ent[bp];
                 av[i] = s_va[q];
             }
 #pragma unroll
@@ -594,8 +592,8 @@ __device__ void sg_row(const SgRowInfo &ri, const SgIn &in, const SgOut &out, K 
                 const uint32_t pe = e0 + (uint32_t)i * NT + t;
                 if (pe < tot) {
                     const uint32_t g = gbase + pe;
-                    key[g] = (K)(((uint64_t)(uint32_t)bc[i] << GB) | g);
-                    val[g] = av[i] * bv[i];
+                    key[g] = (K)(((uint64_t)be[i].x << GB) | g);
+                    val[g] = av[i] * __uint_as_float(be[i].y);
                 }
             }
         }
@@ -899,16 +897,16 @@ dcsr_status dcsr_spgemm(dcsr_handle A, dcsr_handle B, dcsr_handle C, dcsr_stream
 
     DCSR_TRY(ensure_flat(A, s));
     const uint32_t *a_foff = (const uint32_t *)A->ws.ptr[WS_FOFF];
-    uint2 *brow, *ent;
-    DCSR_TRY(ws_get(C, WS_SG_BROW, (size_t)(B->rows + 1) * 8, (void **)&brow));
+    const uint32_t *b_foff;
+    uint2 *b_ent, *ent;
+    DCSR_TRY(ws_get(C, WS_SG_BENT, (size_t)(B->nnz_h + 1) * 8, (void **)&b_ent));
+    DCSR_TRY(copy_rows_paired(B, b_ent, &b_foff, s));
     DCSR_TRY(ws_get(C, WS_SG_ENT, (size_t)(A->nnz_h + 1) * 8, (void **)&ent));
 
     // 1. partial counts, classes, offsets
     k_sg_state_zero<<<1, 1, 0, s>>>(st);
     if (R > 0) {
-        if (B->rows > 0)
-            k_sg_brows<<<grid_for(B->rows, TB), TB, 0, s>>>((uint32_t)B->rows, B->row_start, B->row_len, brow);
-        k_sg_count<<<grid_for(R, TB), TB, 0, s>>>(R, a_foff, A->row_start, A->pool_col, brow, ent, P);
+        k_sg_count<<<grid_for(R, TB), TB, 0, s>>>(R, a_foff, A->row_start, A->pool_col, b_foff, ent, P);
         k_sg_classify<<<nbR, TB, 0, s>>>(R, P, lists, R + 1, st, cnt, bsum, B->cols <= TEAM_MAX_COLS ? 1u : 0u,
                                             B->cols <= BIG_MAX_COLS32 ? BIG_MAX32 : BIG_MAX64);
         k_sg_total<<<1, 1024, 0, s>>>(st, bsum, (int)nbR);
@@ -931,7 +929,7 @@ dcsr_status dcsr_spgemm(dcsr_handle A, dcsr_handle B, dcsr_handle C, dcsr_stream
     float *tval = C->pool_val;
 
     // 2. numeric phases
-    const SgIn in{P, Poff, A->row_start, A->row_len, a_foff, A->pool_val, ent, B->pool_col, B->pool_val};
+    const SgIn in{P, Poff, A->row_start, A->row_len, a_foff, A->pool_val, ent, b_ent};
     const SgOut out{tcol, tval, cnt};
     // launches `kernel` over the rows of class c, `per` rows to a workgroup of
     // nt threads, on at most `most` workgroups (they stride over the rest)
