@@ -567,30 +567,39 @@ __global__ __launch_bounds__(TB) void k_spmm_wide4(uint32_t R, const uint32_t *_
 }
 
 // Carry chains: consecutive slots (waves) carrying into the same row, added
-// to the row's head value.  A wave scans 64 slots.  Chains shorter than 64
-// slots: with one column (SpMV) a segmented wave scan sums every chain of
-// the 128 slots from the wave's base at once (a chain whose head is in the
-// wave ends within them); with KB columns, lane groups sum them (64/KB
-// groups, one lane per column, one chain per group, serially in slot
-// order).  A chain of 64 or more slots (a hub row spread over many waves) is
-// summed by the whole wave, 64 slots at a time, then reduced in a fixed
-// tree.  Either way the order depends only on the chain, so results are
-// reproducible.
+// to the row's head value.  A wave takes carry_slots_per_wave<KB>() slots.
+// Chains shorter than 64 slots: with one column (SpMV) a segmented wave scan
+// sums every chain of the 128 slots from the wave's base at once (a chain
+// whose head is in the wave ends within them); with KB columns a lane takes
+// one column of CARRY_PER slots, all their loads in flight together, and
+// follows a chain from its head in slot order.  (With 64 slots per wave, whose
+// heads were taken 64/KB at a time, the pass was a chain of 32 round trips:
+// 82 us for 62K slots of 32 columns, 24 with 8 slots.)  A chain of 64 or more slots
+// (a hub row spread over many waves) is summed by the whole wave, 64 slots at
+// a time, then reduced in a fixed tree.  Either way the order depends only on
+// the chain, so results are reproducible.
+template <int KB>
+__host__ __device__ constexpr int carry_per() { return KB < 4 ? KB : 4; }  // slots per lane (a wave has at most 64)
+template <int KB>
+__host__ __device__ constexpr uint32_t carry_slots_per_wave() { return 64u / KB * carry_per<KB>(); }
 template <int KB>
 __global__ __launch_bounds__(TB) void k_carry(uint32_t nunits, const uint32_t *__restrict__ carry_row,
                                               const float *__restrict__ carry_val, float *__restrict__ Y,
                                               int64_t ldy, float alpha)
 {
-    constexpr int G = 64 / KB;
+    constexpr int G = 64 / KB, CARRY_PER = carry_per<KB>();
     const int lane = lane_id();
     const int cl = lane % KB;
     const int g = lane / KB;
-    const uint64_t base = ((uint64_t)blockIdx.x * (TB / 64) + (threadIdx.x >> 6)) * 64;
+    const uint64_t base =
+        ((uint64_t)blockIdx.x * (TB / 64) + (threadIdx.x >> 6)) * carry_slots_per_wave<KB>();
     if (base >= nunits) return;
-    const uint64_t w = base + lane;
+    // row of the long chain whose head is this lane's slot (base + lane)
     uint32_t r = NONE;
-    bool head = false, lng = false;
+    bool lng = false;
     if constexpr (KB == 1) {
+        const uint64_t w = base + lane;
+        bool head = false;
         // every load first: this wave's slots, the next 64, the slot before
         const uint64_t w2 = w + 64;
         r = w < nunits ? carry_row[w] : NONE;
@@ -630,28 +639,48 @@ __global__ __launch_bounds__(TB) void k_carry(uint32_t nunits, const uint32_t *_
             }
         }
     } else {
-        if (w < nunits) {
-            r = carry_row[w];
-            head = r != NONE && (w == 0 || carry_row[w - 1] != r);
-            // chains are contiguous: 64+ slots iff slot w+63 still carries r
-            lng = head && w + 63 < nunits && carry_row[w + 63] == r;
+        // lane of group g: slots base + g, base + G + g, ...
+        uint32_t rw[CARRY_PER], rp[CARRY_PER], rn[CARRY_PER], r63[CARRY_PER];
+        float v[CARRY_PER];
+#pragma unroll
+        for (int u = 0; u < CARRY_PER; ++u) {
+            const uint64_t w = base + (uint64_t)(u * G + g);
+            rw[u] = w < nunits ? carry_row[w] : NONE;
+            rp[u] = w > 0 && w < nunits ? carry_row[w - 1] : NONE;
+            rn[u] = w + 1 < nunits ? carry_row[w + 1] : NONE;
+            r63[u] = w + 63 < nunits ? carry_row[w + 63] : NONE;
+            v[u] = w < nunits ? carry_val[w * KB + cl] : 0.0f;
         }
-        const uint64_t longs = __ballot(lng);
-        const uint64_t shorts = __ballot(head) & ~longs;
-        const int nshort = __popcll(shorts);
-        for (int i0 = 0; i0 < nshort; i0 += G) {
-            const int i = i0 + g;
-            // the i-th short head of this wave
-            uint64_t m = shorts;
-            for (int t = 0; t < i && m; ++t) m &= m - 1;
-            const int hl = m ? __ffsll((long long)m) - 1 : 0;
-            const uint32_t hr = (uint32_t)__shfl((int)r, hl);
-            if (i < nshort) {
-                const uint64_t hw = base + hl;
-                float acc = 0.0f;
-                for (uint64_t k = hw; k < nunits && carry_row[k] == hr; ++k) acc = acc + carry_val[k * KB + cl];
-                const uint64_t yi = (uint64_t)hr * ldy + cl;
-                Y[yi] = Y[yi] + alpha * acc;
+        float y[CARRY_PER];
+        bool sh[CARRY_PER];
+        uint32_t longs = 0;
+#pragma unroll
+        for (int u = 0; u < CARRY_PER; ++u) {
+            const bool head = rw[u] != NONE && rp[u] != rw[u];
+            // chains are contiguous: 64+ slots iff slot w+63 still carries r
+            const bool l = head && r63[u] == rw[u];
+            if (l) longs |= 1u << u;
+            sh[u] = head && !l;
+            y[u] = sh[u] ? Y[(uint64_t)rw[u] * ldy + cl] : 0.0f;
+        }
+#pragma unroll
+        for (int u = 0; u < CARRY_PER; ++u) {
+            if (!sh[u]) continue;
+            float acc = 0.0f + v[u];
+            if (rn[u] == rw[u])
+                for (uint64_t k = base + (uint64_t)(u * G + g) + 1; k < nunits && carry_row[k] == rw[u]; ++k)
+                    acc = acc + carry_val[k * KB + cl];
+            Y[(uint64_t)rw[u] * ldy + cl] = y[u] + alpha * acc;
+        }
+        // slot base + i belongs to lane i from here on
+#pragma unroll
+        for (int u = 0; u < CARRY_PER; ++u) {
+            const int src = (lane - u * G) * KB;  // a lane of group lane - u * G
+            const uint32_t l = (uint32_t)__shfl((int)longs, src & 63);
+            const uint32_t q = (uint32_t)__shfl((int)rw[u], src & 63);
+            if (lane >= u * G && lane < (u + 1) * G && ((l >> u) & 1u)) {
+                lng = true;
+                r = q;
             }
         }
     }
@@ -877,7 +906,8 @@ static dcsr_status launch_flat(dcsr_handle h, const float *X, int64_t ldx, float
     else
         k_flat<KB><<<blocks, TB, 0, s>>>(R, foff, rowmap, h->row_start, h->pool_col, h->pool_val, X, ldx, Y, ldy,
                                          alpha, beta, pw, crow, cval);
-    k_carry<KB><<<grid_for(nwaves, TB), TB, 0, s>>>((uint32_t)nwaves, crow, cval, Y, ldy, alpha);
+    k_carry<KB><<<grid_for(nwaves, TB / 64 * carry_slots_per_wave<KB>()), TB, 0, s>>>((uint32_t)nwaves, crow, cval, Y,
+                                                                                     ldy, alpha);
     DCSR_HIP(hipGetLastError());
     return DCSR_OK;
 }
@@ -912,7 +942,8 @@ static dcsr_status launch_wide(dcsr_handle h, const float *X, int64_t ldx, float
     else
         k_spmm_wide<KB><<<blocks, TB, 0, s>>>(R, foff, rowmap, h->row_start, h->pool_col, h->pool_val, X, ldx, Y,
                                               ldy, alpha, beta, crow, cval);
-    k_carry<KB><<<grid_for(nwaves, TB), TB, 0, s>>>((uint32_t)nwaves, crow, cval, Y, ldy, alpha);
+    k_carry<KB><<<grid_for(nwaves, TB / 64 * carry_slots_per_wave<KB>()), TB, 0, s>>>((uint32_t)nwaves, crow, cval, Y,
+                                                                                     ldy, alpha);
     DCSR_HIP(hipGetLastError());
     return DCSR_OK;
 }
