@@ -7,11 +7,10 @@
 // owns global rows [row_base[m], row_base[m+1]) and keeps local column
 // indices), so they share one pool and one allocator.  One persistent kernel
 // does a whole step: every workgroup takes matrix ids from a work counter and,
-// for each, applies that matrix's insert-or-add batch entirely in LDS and
-// per-workgroup scratch (stable LDS radix sort of (row, col) keys, left-to-
-// right duplicate sums, a per-row merge against the stored row for the
-// codes, prefix-sum chunk claims, a per-row merge into the new chunk,
-// commit), then
+// for each, applies that matrix's insert-or-add batch with all of its records
+// in LDS (triples bucketed by row and ranked inside their row, left-to-right
+// duplicate sums, each touched row met by 16 lanes that hold its entries in
+// registers, prefix-sum chunk claims, merge into the new chunk, commit), then
 // computes that matrix's SpMV with TEAM lanes per row and a whole wave for
 // rows longer than a threshold.  Semantics per matrix are those of
 // dcsr_update followed by dcsr_spmv.  The last workgroup to finish resets the
@@ -27,21 +26,44 @@
 
 namespace {
 
-constexpr int BT = 256;
+// 16 waves and 73 KB of LDS: two workgroups fill a CU's waves.  A matrix is a
+// chain of short phases with a barrier between them, so what bounds a step is
+// how many rows are in flight per CU: 4,096 matrices (4.0M rows, 68M entries,
+// 2,000 triples each) take 1.56 ms per step; 4 waves per matrix with the records
+// in memory and one lane per touched row took 2.44.
+constexpr int BT = 1024;
+constexpr int NW = BT / 64;
 constexpr uint32_t BMAX = 4096;  // triples per matrix per step
 constexpr int KB = 12;           // bits of a local row / column / arrival index
 constexpr uint32_t LMAX = 1u << KB;
-constexpr int ITEMS = 17;        // scan items per thread (256 * 17 >= BMAX + 1)
+constexpr int PT = BMAX / BT;    // records per thread
+constexpr int RL = 16;           // lanes per touched row
+constexpr int NTM = BT / RL;     // rows in flight per workgroup
+constexpr int RC = 2 * RL;       // entries of a row met at once (two per lane)
+static_assert(BMAX == LMAX && PT == 4, "row counters and records share their split over the threads");
 enum { C_NOP = 0, C_ADD = 1, C_DEL = 2, C_INS = 3 };
 
-// per-workgroup scratch (words)
-enum {
-    S_URC = 0, S_UVAL = S_URC + BMAX, S_UPOS = S_UVAL + BMAX, S_UCODE = S_UPOS + BMAX, S_UT = S_UCODE + BMAX,
-    S_UIP = S_UT + BMAX, S_UDP = S_UIP + BMAX + 1, S_TROW = S_UDP + BMAX + 1, S_TUB = S_TROW + BMAX,
-    S_TINS = S_TUB + BMAX + 1, S_TDEL = S_TINS + BMAX, S_TDST = S_TDEL + BMAX, S_TMP = S_TDST + BMAX + 1,
-    S_TMODE = S_TMP + BMAX + 1, S_TNL = S_TMODE + BMAX, S_HF = S_TNL + BMAX, S_RF = S_HF + BMAX + 1,
-    S_WORDS = S_RF + BMAX + 1
+// A workgroup's records.  Reused in order: buckets -> coordinates; sorted keys
+// -> positions and codes, new row lengths; sorted values -> chunk offsets; row
+// counters -> row starts in the buckets -> first coordinate of each row.
+struct BatchLds {
+    uint32_t urc[BMAX];  // bucketed column << 12 | arrival; then coordinate u: row << 12 | column
+    uint32_t sk[BMAX];   // sorted row << 12 | column; then upc and tnl
+    float sv[BMAX];      // sorted values; then tdst
+    float uval[BMAX];    // coordinate u: sum, then new value
+    uint32_t cnt[BMAX / 2 + 2];  // 16-bit: triples of each row, bucket starts; then tub
+    uint32_t lw[NW];
+    uint32_t sm[8];
+    // coordinate u: position in its old row | code << 14
+    __device__ uint16_t *upc() { return reinterpret_cast<uint16_t *>(sk); }
+    // touched row t: new length | rewritten << 15
+    __device__ uint16_t *tnl() { return reinterpret_cast<uint16_t *>(sk) + BMAX; }
+    // touched row t: its chunk's offset in the matrix's claim
+    __device__ uint32_t *tdst() { return reinterpret_cast<uint32_t *>(sv); }
+    // touched row t: first coordinate (t == touched rows: their count)
+    __device__ uint16_t *tub() { return reinterpret_cast<uint16_t *>(cnt); }
 };
+enum { SM_BAD = 0, SM_OK, SM_BASE, SM_NEXT, SM_INS, SM_ADD, SM_DEL, SM_WORDS = 8 };
 
 struct BatchState {
     unsigned int work;  // next matrix id
@@ -52,73 +74,7 @@ struct BatchState {
 #define BST_TOO_BIG 0x2u
 #define BST_EXHAUSTED 0x4u
 
-__device__ __forceinline__ uint32_t next_pow2(uint32_t v)
-{
-    v--;
-    v |= v >> 1;
-    v |= v >> 2;
-    v |= v >> 4;
-    v |= v >> 8;
-    v |= v >> 16;
-    return v + 1;
-}
-
-// In-place exclusive scan of a[0..n) (n <= 256 * ITEMS) by one workgroup;
-// returns the total.  Blocked: thread t owns [t*ITEMS, t*ITEMS+ITEMS).
-__device__ uint32_t block_scan_inplace(uint32_t *a, uint32_t n, uint32_t *lw)
-{
-    const uint32_t t = threadIdx.x;
-    uint32_t loc[ITEMS];
-    uint32_t s = 0;
-#pragma unroll
-    for (int i = 0; i < ITEMS; ++i) {
-        const uint32_t idx = t * ITEMS + i;
-        const uint32_t v = idx < n ? a[idx] : 0u;
-        loc[i] = s;
-        s += v;
-    }
-    const uint32_t inc = wave_incl_scan_u32(s);
-    if (lane_id() == 63) lw[t >> 6] = inc;
-    __syncthreads();
-    uint32_t carry = 0, tot = 0;
-#pragma unroll
-    for (int i = 0; i < BT / 64; ++i) {
-        if (i < (int)(t >> 6)) carry += lw[i];
-        tot += lw[i];
-    }
-    const uint32_t base = carry + inc - s;
-#pragma unroll
-    for (int i = 0; i < ITEMS; ++i) {
-        const uint32_t idx = t * ITEMS + i;
-        if (idx < n) a[idx] = base + loc[i];
-    }
-    __syncthreads();
-    return tot;
-}
-
-// Largest j in [0, n) with a[j] <= e (a non-decreasing, a[0] <= e).
-__device__ __forceinline__ uint32_t find_last_le(const uint32_t *a, uint32_t n, uint32_t e)
-{
-    uint32_t lo = 0, hi = n;
-    while (hi - lo > 1) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (a[mid] <= e) lo = mid; else hi = mid;
-    }
-    return lo;
-}
-
-__device__ __forceinline__ uint32_t block_sum(uint32_t v, uint32_t *lw)
-{
-    const uint32_t w = wave_sum_u32(v);
-    if (lane_id() == 0) lw[threadIdx.x >> 6] = w;
-    __syncthreads();
-    const uint32_t t = (lw[0] + lw[1]) + (lw[2] + lw[3]);
-    __syncthreads();
-    return t;
-}
-
-// Block-wide exclusive scan of one value per thread (256 threads); *total
-// receives the sum.
+// Block-wide exclusive scan of one value per thread; *total receives the sum.
 __device__ __forceinline__ uint32_t block_excl(uint32_t v, uint32_t *lw, uint32_t *total)
 {
     const uint32_t inc = wave_incl_scan_u32(v);
@@ -126,95 +82,20 @@ __device__ __forceinline__ uint32_t block_excl(uint32_t v, uint32_t *lw, uint32_
     __syncthreads();
     uint32_t carry = 0, tot = 0;
 #pragma unroll
-    for (int i = 0; i < BT / 64; ++i) {
-        if (i < (int)(threadIdx.x >> 6)) carry += lw[i];
-        tot += lw[i];
+    for (int i = 0; i < NW; ++i) {
+        const uint32_t t = lw[i];
+        if (i < (int)(threadIdx.x >> 6)) carry += t;
+        tot += t;
     }
     __syncthreads();
     *total = tot;
     return carry + inc - v;
 }
 
-// One stable pass (8-bit digit at `shift`) of an LDS radix sort of n <= BMAX
-// (key, value) pairs from (ks, vs) to (kd, vd).  Wave w ranks its contiguous
-// quarter in order (ballot digit matching, running per-digit counts in
-// wcnt[w]); digit bases come from a block scan of the digit totals.
-__device__ void lds_radix_pass(const uint32_t *ks, const float *vs, uint32_t *kd, float *vd, uint32_t n, int shift,
-                               uint32_t (*wcnt)[256], uint32_t *lw)
+// The calling lane's RL-lane team's bits of a ballot.
+__device__ __forceinline__ uint32_t team_bits(uint64_t m)
 {
-    constexpr int MAXJ = BMAX / (BT / 64) / 64;  // 64-item chunks per wave
-    const int w = threadIdx.x >> 6;
-    const int lane = lane_id();
-    const uint32_t Q = (((n + 3) / 4) + 63) & ~63u;
-    const uint32_t wb = (uint32_t)w * Q;
-    const uint32_t we = wb + Q < n ? wb + Q : n;
-    for (int i = threadIdx.x; i < (BT / 64) * 256; i += BT) (&wcnt[0][0])[i] = 0;
-    __syncthreads();
-    uint32_t key[MAXJ], rnk[MAXJ];
-    float val[MAXJ];
-    const uint64_t lt = lanemask_lt();
-    // every item read before the ranking writes the counters (the buffers
-    // arrive as generic pointers, so the compiler may not move a read past
-    // a counter write itself); indices stay below 4 * Q <= BMAX
-#pragma unroll
-    for (int j = 0; j < MAXJ; ++j) {
-        const uint32_t idx = wb + (uint32_t)j * 64 + lane;
-        key[j] = ks[idx];
-        val[j] = vs[idx];
-    }
-#pragma unroll
-    for (int j = 0; j < MAXJ; ++j) {
-        const uint32_t idx = wb + (uint32_t)j * 64 + lane;
-        const bool ok = idx < we;
-        if (!ok) {
-            key[j] = 0u;
-            val[j] = 0.0f;
-        }
-        rnk[j] = 0;
-        if (wb + (uint32_t)j * 64 < we) {  // wave-uniform
-            const uint32_t d = (key[j] >> shift) & 255u;
-            const uint64_t act = __ballot(ok);
-            const uint64_t peers = wave_match_digit8(d, act);
-            const int leader = __ffsll((long long)peers) - 1;
-            // every lane of the digit reads its count before the leader adds
-            // to it (a wave's LDS accesses complete in order): no broadcast
-            const uint32_t b = wcnt[w][d];
-            if (ok && lane == leader) wcnt[w][d] = b + (uint32_t)__popcll(peers);
-            rnk[j] = b + (uint32_t)__popcll(peers & lt);
-        }
-    }
-    __syncthreads();
-    {
-        const int d = threadIdx.x;
-        uint32_t c[BT / 64];
-        uint32_t tot = 0;
-#pragma unroll
-        for (int i = 0; i < BT / 64; ++i) {
-            c[i] = wcnt[i][d];
-            tot += c[i];
-        }
-        uint32_t all;
-        uint32_t b = block_excl(tot, lw, &all);
-#pragma unroll
-        for (int i = 0; i < BT / 64; ++i) {
-            wcnt[i][d] = b;
-            b += c[i];
-        }
-    }
-    __syncthreads();
-    // every digit base read before the first write (generic pointers again)
-    uint32_t pos[MAXJ];
-#pragma unroll
-    for (int j = 0; j < MAXJ; ++j) pos[j] = wcnt[w][(key[j] >> shift) & 255u] + rnk[j];
-#pragma unroll
-    for (int j = 0; j < MAXJ; ++j) {
-        const uint32_t idx = wb + (uint32_t)j * 64 + lane;
-        if (idx < we) {
-            kd[pos[j]] = key[j];
-            vd[pos[j]] = val[j];
-        }
-    }
-    __syncthreads();
+    return (uint32_t)(m >> (lane_id() & ~(RL - 1))) & ((1u << RL) - 1u);
 }
 
 // Counters of the matrices one workgroup updated, kept by its thread 0 and
@@ -235,9 +116,8 @@ __device__ void batch_update(uint32_t m, const uint32_t *__restrict__ row_base, 
                              const int32_t *__restrict__ tcol, const float *__restrict__ tval,
                              uint32_t *__restrict__ row_start, int32_t *__restrict__ row_len,
                              int32_t *__restrict__ row_cap, int32_t *__restrict__ pcol, float *__restrict__ pval,
-                             unsigned long long pool_cap, DevState *ds, uint32_t *__restrict__ mstat, uint32_t *sc,
-                             uint32_t (*skb)[BMAX], float (*svb)[BMAX], uint32_t (*wcnt)[256], uint32_t *lw,
-                             uint32_t *sm, bool reserved, BatchAcc &acc)
+                             unsigned long long pool_cap, DevState *ds, uint32_t *__restrict__ mstat, BatchLds &S,
+                             bool reserved, BatchAcc &acc)
 {
     const uint32_t t = threadIdx.x;
     const uint32_t gbase = row_base[m];
@@ -256,173 +136,270 @@ __device__ void batch_update(uint32_t m, const uint32_t *__restrict__ row_base, 
         return;
     }
     const uint32_t nb = (uint32_t)nb64;
-    // U1: (row, col) keys and values into LDS, stable radix sort (3 passes
-    // of 8 bits over the 24 key bits; stability keeps arrival order among
-    // duplicates)
-    if (t == 0) sm[0] = 0;
+    // U1: sort the triples by (row, column, arrival).  Row counters in LDS
+    // give every triple a place in its row's bucket, in any order; its rank
+    // among the bucket's (column, arrival) pairs is its sorted place.  A
+    // thread's triples are all loaded before the first LDS access; indices
+    // clamp to the matrix's last triple.
+    int32_t rr[PT], cc[PT];
+    float vv[PT];
+#pragma unroll
+    for (int j = 0; j < PT; ++j) {
+        const uint32_t i = t + (uint32_t)j * BT;
+        const int64_t gi = t0 + (i < nb ? i : nb - 1);
+        rr[j] = trow[gi];
+        cc[j] = tcol[gi];
+        vv[j] = tval[gi];
+    }
+    for (uint32_t i = t; i < BMAX / 2 + 2; i += BT) S.cnt[i] = 0u;
+    if (t < SM_WORDS) S.sm[t] = 0u;
     __syncthreads();
-    uint32_t bad = 0;
-    {
-        // a thread's triples (at most BMAX / BT) are all loaded before the
-        // first LDS store; indices clamp to the matrix's last triple
-        constexpr int TPT = BMAX / BT;
-        int32_t rr[TPT], cc[TPT];
-        float vv[TPT];
+    uint32_t off[PT];
+    bool bad = false;
 #pragma unroll
-        for (int j = 0; j < TPT; ++j) {
-            const uint32_t i = t + (uint32_t)j * BT;
-            const int64_t gi = t0 + (i < nb ? i : nb - 1);
-            rr[j] = trow[gi];
-            cc[j] = tcol[gi];
-            vv[j] = tval[gi];
-        }
-#pragma unroll
-        for (int j = 0; j < TPT; ++j) {
-            const uint32_t i = t + (uint32_t)j * BT;
-            if (i < nb) {
-                const int32_t r = rr[j], c = cc[j];
-                uint32_t k = 0;
-                if (r < 0 || (uint32_t)r >= Rm || c < 0 || (uint32_t)c >= Cm) bad = 1;
-                else k = ((uint32_t)r << KB) | (uint32_t)c;
-                skb[0][i] = k;
-                svb[0][i] = vv[j];
-            }
+    for (int j = 0; j < PT; ++j) {
+        const int32_t r = rr[j], c = cc[j];
+        off[j] = 0;
+        if (t + (uint32_t)j * BT >= nb) continue;
+        if (r < 0 || (uint32_t)r >= Rm || c < 0 || (uint32_t)c >= Cm) {
+            bad = true;
+        } else {
+            const uint32_t sh = ((uint32_t)r & 1u) * 16u;
+            off[j] = (atomicAdd(&S.cnt[(uint32_t)r >> 1], 1u << sh) >> sh) & 0xffffu;
         }
     }
-    if (block_sum(bad, lw)) {
+    if (__syncthreads_or(bad)) {
         if (t == 0) mstat[m] |= BST_BAD_INDEX;
         return;
     }
-    lds_radix_pass(skb[0], svb[0], skb[1], svb[1], nb, 0, wcnt, lw);
-    lds_radix_pass(skb[1], svb[1], skb[0], svb[0], nb, 8, wcnt, lw);
-    lds_radix_pass(skb[0], svb[0], skb[1], svb[1], nb, 16, wcnt, lw);
-    const uint32_t *sk = skb[1];
-    const float *sv = svb[1];
-    // U2: distinct coordinates (heads) and touched rows (row heads)
-    uint32_t *hf = sc + S_HF, *rf = sc + S_RF;
-    for (uint32_t p = t; p <= nb; p += BT) {
-        uint32_t h = 0, rh = 0;
-        if (p < nb) {
-            const uint32_t k = sk[p];
-            h = (p == 0 || sk[p - 1] != k) ? 1u : 0u;
-            rh = (p == 0 || (sk[p - 1] >> KB) != (k >> KB)) ? 1u : 0u;
-        }
-        hf[p] = h;
-        rf[p] = rh;
+    uint32_t tot;
+    {
+        // bucket starts: four rows (two counter words) per thread
+        const uint32_t w0 = S.cnt[2 * t], w1 = S.cnt[2 * t + 1];
+        const uint32_t c0 = w0 & 0xffffu, c1 = w0 >> 16, c2 = w1 & 0xffffu, c3 = w1 >> 16;
+        const uint32_t b = block_excl(c0 + c1 + c2 + c3, S.lw, &tot);
+        S.cnt[2 * t] = b | ((b + c0) << 16);
+        S.cnt[2 * t + 1] = (b + c0 + c1) | ((b + c0 + c1 + c2) << 16);
+        if (t == 0) S.cnt[BMAX / 2] = nb;
     }
     __syncthreads();
-    const uint32_t nu = block_scan_inplace(hf, nb + 1, lw);
-    const uint32_t nt = block_scan_inplace(rf, nb + 1, lw);
-    uint32_t *urc = sc + S_URC, *upos = sc + S_UPOS, *ucode = sc + S_UCODE, *ut = sc + S_UT;
-    float *uval = (float *)(sc + S_UVAL);
-    uint32_t *trw = sc + S_TROW, *tub = sc + S_TUB, *tins = sc + S_TINS, *tdel = sc + S_TDEL;
-    for (uint32_t p = t; p < nb; p += BT) {
-        const uint32_t k = sk[p];
-        const bool h = p == 0 || sk[p - 1] != k;
-        if (!h) continue;
-        const bool rh = p == 0 || (sk[p - 1] >> KB) != (k >> KB);
-        const uint32_t u = hf[p];
-        const uint32_t tt = rf[p] + (rh ? 0u : 0xffffffffu);
-        float s = 0.0f + sv[p];
-        for (uint32_t q = p + 1; q < nb && sk[q] == k; ++q) s = s + sv[q];
-        urc[u] = k;
-        uval[u] = s;
-        ut[u] = tt;
-        if (rh) {
-            trw[tt] = k >> KB;
-            tub[tt] = u;
-            tins[tt] = 0;
-            tdel[tt] = 0;
+    const uint16_t *start = reinterpret_cast<const uint16_t *>(S.cnt);
+    uint32_t lo[PT], n[PT], me[PT], most = 0;
+#pragma unroll
+    for (int j = 0; j < PT; ++j) {
+        const uint32_t i = t + (uint32_t)j * BT;
+        lo[j] = n[j] = me[j] = 0;
+        if (i < nb) {
+            lo[j] = start[rr[j]];
+            n[j] = start[rr[j] + 1] - lo[j];
+            me[j] = ((uint32_t)cc[j] << KB) | i;
+            S.urc[lo[j] + off[j]] = me[j];
+            most = n[j] > most ? n[j] : most;
         }
     }
-    if (t == 0) tub[nt] = nu;
     __syncthreads();
-    // U3: one lane per touched row merges the row's update run (sorted by
-    // column) against its old entries (sorted by column): code and new value
-    // per distinct coordinate, position of a hit, inserts / deletes per row.
-    uint32_t my_adds = 0, my_ins = 0, my_del = 0;
-    for (uint32_t tt = t; tt < nt; tt += BT) {
-        const uint32_t g = gbase + trw[tt];
-        const uint64_t st = row_start[g];
-        const int32_t L = row_len[g];
-        const uint32_t ub = tub[tt], ue = tub[tt + 1];
-        int32_t i = 0;
-        uint32_t ni = 0, nd = 0;
-        for (uint32_t u = ub; u < ue; ++u) {
-            const int32_t c = (int32_t)(urc[u] & (LMAX - 1));
-            // advance past the old columns below c, eight per step: the
-            // step's loads are issued together (indices clamp into the row)
-            // and counted with unrolled compares; the first column not below
-            // c is picked the same way
-            int32_t at = -1;  // old column at position i (-1: i == L)
-            while (i < L) {
-                int32_t pc[8];
+    {
+        uint32_t rk[PT];
 #pragma unroll
-                for (int j = 0; j < 8; ++j) pc[j] = pcol[st + (uint64_t)(i + j < L ? i + j : L - 1)];
-                int32_t below = 0;
+        for (int j = 0; j < PT; ++j) rk[j] = lo[j];
+        for (uint32_t d = 0; __any(most > 1 && d < most); ++d) {
 #pragma unroll
-                for (int j = 0; j < 8; ++j) below += (i + j < L && pc[j] < c) ? 1 : 0;
-                at = -1;
+            for (int j = 0; j < PT; ++j)
+                if (d < n[j]) rk[j] += (uint32_t)(S.urc[lo[j] + d] < me[j]);
+        }
 #pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    if (j == below && i + j < L) at = pc[j];
-                i += below;
-                if (below < 8) break;
-                at = -1;
+        for (int j = 0; j < PT; ++j) {
+            if (t + (uint32_t)j * BT < nb) {
+                S.sk[rk[j]] = ((uint32_t)rr[j] << KB) | (uint32_t)cc[j];
+                S.sv[rk[j]] = vv[j];
             }
-            const bool hit = i < L && at == c;
-            const float s = uval[u];
+        }
+    }
+    __syncthreads();
+    // U2: distinct coordinates (heads) and touched rows (row heads), four
+    // consecutive records per thread; duplicates are summed from 0 in arrival
+    // order
+    uint32_t nu, nt;
+    {
+        const uint32_t p0 = t * PT;
+        uint32_t k[PT], h = 0, rh = 0;
+        uint32_t prev = p0 > 0 && p0 - 1 < nb ? S.sk[p0 - 1] : ~0u;
+#pragma unroll
+        for (int j = 0; j < PT; ++j) {
+            k[j] = p0 + j < nb ? S.sk[p0 + j] : ~0u;
+            if (p0 + j < nb && k[j] != prev) h |= 1u << j;
+            if (p0 + j < nb && (prev == ~0u || (k[j] >> KB) != (prev >> KB))) rh |= 1u << j;
+            prev = k[j];
+        }
+        uint32_t at = block_excl((uint32_t)__popc(h) | ((uint32_t)__popc(rh) << 16), S.lw, &tot);
+        nu = tot & 0xffffu;
+        nt = tot >> 16;
+#pragma unroll
+        for (int j = 0; j < PT; ++j) {
+            if ((h >> j) & 1u) {
+                float s = 0.0f + S.sv[p0 + j];
+                for (uint32_t q = p0 + j + 1; q < nb && S.sk[q] == k[j]; ++q) s = s + S.sv[q];
+                const uint32_t u = at & 0xffffu;
+                S.urc[u] = k[j];
+                S.uval[u] = s;
+                if ((rh >> j) & 1u) {
+                    S.tub()[at >> 16] = (uint16_t)u;
+                    at += 1u << 16;
+                }
+                ++at;
+            }
+        }
+        if (t == 0) S.tub()[nt] = (uint16_t)nu;
+    }
+    __syncthreads();
+    // U3: every touched row is met by RL lanes holding RC of its entries at a
+    // time: an update's place is the count of lanes with smaller columns, its
+    // hit a lane with its own.  The columns of the team's next row, and the
+    // row table entry of the one after, are in flight meanwhile.
+    const uint32_t tm = t / RL, tl = t % RL;
+    uint16_t *upc = S.upc();
+    const uint16_t *tub = S.tub();
+    auto row_of = [&](uint32_t tt) { return gbase + (S.urc[tub[tt]] >> KB); };
+    constexpr int32_t NOCOL = 0x7fffffff;
+    {
+        uint32_t st = 0, L = 0, st1 = 0, L1 = 0;
+        int32_t c0 = NOCOL, c1 = NOCOL;
+        if (tm < nt) {
+            const uint32_t g = row_of(tm);
+            st = row_start[g];
+            L = (uint32_t)row_len[g];
+        }
+        if (tm + NTM < nt) {
+            const uint32_t g = row_of(tm + NTM);
+            st1 = row_start[g];
+            L1 = (uint32_t)row_len[g];
+        }
+        if (tl < L) c0 = pcol[(uint64_t)st + tl];
+        if (tl + RL < L) c1 = pcol[(uint64_t)st + tl + RL];
+        for (uint32_t tt = tm; tt < nt; tt += NTM) {
+            uint32_t st2 = 0, L2 = 0;
+            int32_t d0 = NOCOL, d1 = NOCOL;
+            if (tl < L1) d0 = pcol[(uint64_t)st1 + tl];
+            if (tl + RL < L1) d1 = pcol[(uint64_t)st1 + tl + RL];
+            if (tt + 2 * NTM < nt) {
+                const uint32_t g = row_of(tt + 2 * NTM);
+                st2 = row_start[g];
+                L2 = (uint32_t)row_len[g];
+            }
+            uint32_t u = tub[tt];
+            const uint32_t ue = tub[tt + 1];
+            for (uint32_t i0 = 0;;) {
+                const bool last = i0 + RC >= L;
+                const int32_t cmax = last ? NOCOL : __shfl(c1, RL - 1, RL);
+                while (u < ue) {
+                    const int32_t c = (int32_t)(S.urc[u] & (LMAX - 1));
+                    if (c > cmax) break;  // among later entries
+                    const uint32_t below =
+                        (uint32_t)(__popc(team_bits(__ballot(c0 < c))) + __popc(team_bits(__ballot(c1 < c))));
+                    const uint32_t hit = team_bits(__ballot(c0 == c || c1 == c));
+                    if (tl == 0) upc[u] = (uint16_t)((i0 + below) | (hit ? (uint32_t)C_ADD << 14 : 0u));
+                    ++u;
+                }
+                if (last || u >= ue) break;
+                i0 += RC;
+                c0 = i0 + tl < L ? pcol[(uint64_t)st + i0 + tl] : NOCOL;
+                c1 = i0 + RL + tl < L ? pcol[(uint64_t)st + i0 + RL + tl] : NOCOL;
+            }
+            st = st1;
+            L = L1;
+            c0 = d0;
+            c1 = d1;
+            st1 = st2;
+            L1 = L2;
+        }
+    }
+    __syncthreads();
+    // new value and code of every coordinate
+    uint32_t nins = 0, nadd = 0, ndel = 0;
+    {
+        uint32_t w[PT];
+        float old[PT];
+#pragma unroll
+        for (int j = 0; j < PT; ++j) {
+            const uint32_t u = t + (uint32_t)j * BT;
+            w[j] = u < nu ? upc[u] : 0u;
+            old[j] = 0.0f;
+            if (w[j] >> 14) old[j] = pval[(uint64_t)row_start[gbase + (S.urc[u] >> KB)] + (w[j] & 0x3fffu)];
+        }
+#pragma unroll
+        for (int j = 0; j < PT; ++j) {
+            const uint32_t u = t + (uint32_t)j * BT;
+            if (u >= nu) continue;
+            float v = S.uval[u];
             uint32_t code;
-            float nv;
-            if (hit) {
-                nv = pval[st + i] + s;
-                code = nv != 0.0f ? C_ADD : C_DEL;
+            if (w[j] >> 14) {
+                v = old[j] + v;
+                code = v != 0.0f ? C_ADD : C_DEL;
             } else {
-                nv = s;
-                code = s != 0.0f ? C_INS : C_NOP;
+                code = v != 0.0f ? C_INS : C_NOP;
             }
-            uval[u] = nv;
-            upos[u] = (uint32_t)i;
-            ucode[u] = code;
-            ni += code == C_INS;
-            nd += code == C_DEL;
-            my_adds += code == C_ADD;
+            S.uval[u] = v;
+            upc[u] = (uint16_t)((w[j] & 0x3fffu) | (code << 14));
+            nins += code == C_INS;
+            nadd += code == C_ADD;
+            ndel += code == C_DEL;
         }
-        tins[tt] = ni;
-        tdel[tt] = nd;
-        my_ins += ni;
-        my_del += nd;
+    }
+    nins = wave_sum_u32(nins);
+    nadd = wave_sum_u32(nadd);
+    ndel = wave_sum_u32(ndel);
+    if (lane_id() == 0) {
+        atomicAdd(&S.sm[SM_INS], nins);
+        atomicAdd(&S.sm[SM_ADD], nadd);
+        atomicAdd(&S.sm[SM_DEL], ndel);
     }
     __syncthreads();
-    const uint32_t nadd = block_sum(my_adds, lw);
-    const uint32_t nins = block_sum(my_ins, lw);
-    const uint32_t ndel = block_sum(my_del, lw);
-    // U4: plan, claim
-    uint32_t *tdst = sc + S_TDST, *tmode = sc + S_TMODE, *tnl = sc + S_TNL;
-    long long dnnz = 0, dgar = 0;
-    for (uint32_t tt = t; tt <= nt; tt += BT) {
-        uint32_t claim = 0;
-        if (tt < nt) {
-            const uint32_t g = gbase + trw[tt];
-            const uint32_t L = (uint32_t)row_len[g];
-            const uint32_t ni = tins[tt], nd = tdel[tt];
-            const uint32_t nl = L + ni - nd;
-            const uint32_t mode = (ni | nd) ? 1u : 0u;
-            if (mode) {
-                claim = chunk_round(nl);
-                dnnz += (long long)nl - (long long)L;
-                dgar += row_cap[g];
+    // U4: plan and claim, four consecutive rows per thread
+    uint16_t *tnl = S.tnl();
+    uint32_t *tdst = S.tdst();
+    uint32_t dgar = 0, claim_tot;
+    {
+        uint32_t claim[PT], sum = 0;
+        uint32_t L[PT], cap[PT];
+#pragma unroll
+        for (int j = 0; j < PT; ++j) {
+            const uint32_t tt = t * PT + j;
+            L[j] = cap[j] = 0;
+            if (tt < nt) {
+                const uint32_t g = row_of(tt);
+                L[j] = (uint32_t)row_len[g];
+                cap[j] = (uint32_t)row_cap[g];
             }
-            tmode[tt] = mode;
-            tnl[tt] = nl;
         }
-        tdst[tt] = claim;
+#pragma unroll
+        for (int j = 0; j < PT; ++j) {
+            const uint32_t tt = t * PT + j;
+            claim[j] = 0;
+            if (tt < nt) {
+                uint32_t ni = 0, nd = 0;
+                for (uint32_t u = tub[tt]; u < tub[tt + 1]; ++u) {
+                    const uint32_t code = upc[u] >> 14;
+                    ni += code == C_INS;
+                    nd += code == C_DEL;
+                }
+                const uint32_t nl = L[j] + ni - nd;
+                tnl[tt] = (uint16_t)(nl | ((ni | nd) ? 0x8000u : 0u));
+                if (ni | nd) {
+                    claim[j] = chunk_round(nl);
+                    dgar += cap[j];
+                }
+            }
+            sum += claim[j];
+        }
+        uint32_t at = block_excl(sum, S.lw, &claim_tot);
+#pragma unroll
+        for (int j = 0; j < PT; ++j) {
+            if (t * PT + j < nt) tdst[t * PT + j] = at;
+            at += claim[j];
+        }
     }
-    __syncthreads();
-    const uint32_t claim_tot = block_scan_inplace(tdst, nt + 1, lw);
-    // 64-bit deltas: per-thread values are small; reduce through 32-bit halves
-    const uint32_t dn_lo = block_sum((uint32_t)(dnnz & 0xffffffff), lw);
-    const uint32_t dg_lo = block_sum((uint32_t)(dgar & 0xffffffff), lw);
+    uint32_t dg;
+    (void)block_excl(dgar, S.lw, &dg);
     if (t == 0) {
         // claim by compare-and-swap: the bump pointer advances only when the
         // claim fits, so a matrix that does not fit leaves room for later
@@ -446,88 +423,136 @@ __device__ void batch_update(uint32_t m, const uint32_t *__restrict__ row_base, 
                 cur = seen;  // another matrix claimed first: retry from its end
             }
         }
-        sm[1] = ok ? 1u : 0u;
-        sm[2] = (uint32_t)base;
+        S.sm[SM_OK] = ok ? 1u : 0u;
+        S.sm[SM_BASE] = (uint32_t)base;
         if (!ok) mstat[m] |= BST_EXHAUSTED;
         if (ok) {
-            acc.dnnz += (long long)(int32_t)dn_lo;
-            acc.dgarbage += (long long)(int32_t)dg_lo;
-            acc.ins += nins;
-            acc.add += nadd;
-            acc.del += ndel;
+            acc.dnnz += (long long)S.sm[SM_INS] - (long long)S.sm[SM_DEL];
+            acc.dgarbage += (long long)dg;
+            acc.ins += S.sm[SM_INS];
+            acc.add += S.sm[SM_ADD];
+            acc.del += S.sm[SM_DEL];
             acc.touched += nt;
         }
     }
     __syncthreads();
-    if (!sm[1]) return;
-    const uint32_t base = sm[2];
-    // U5: one lane per touched row: rewritten rows are merged into their new
-    // chunk (old entries and the row's update run, both column-sorted);
-    // unchanged-structure rows get their added values written in place
-    for (uint32_t tt = t; tt < nt; tt += BT) {
-        const uint32_t g = gbase + trw[tt];
-        const uint64_t st = row_start[g];
-        const uint32_t ub = tub[tt], ue = tub[tt + 1];
-        if (!tmode[tt]) {
-            for (uint32_t u = ub; u < ue; ++u)
-                if (ucode[u] == C_ADD) pval[st + upos[u]] = uval[u];
-            continue;
+    if (!S.sm[SM_OK]) return;
+    const uint32_t base = S.sm[SM_BASE];
+    // U5: the same teams merge every rewritten row into its new chunk: an
+    // entry moves by the inserts less the deletes at or before its place.
+    // Rows of unchanged structure get their added values written in place.
+    {
+        uint32_t st = 0, L = 0, st1 = 0, L1 = 0;
+        int32_t c0 = 0, c1 = 0;
+        float v0 = 0.0f, v1 = 0.0f;
+        if (tm < nt) {
+            const uint32_t g = row_of(tm);
+            st = row_start[g];
+            L = (uint32_t)row_len[g];
         }
-        const int32_t L = row_len[g];
-        const uint64_t d0 = (uint64_t)base + tdst[tt];
-        uint64_t o = d0;
-        int32_t i = 0;
-        // old entries [i, to) to o.., eight at a time with all eight loads
-        // issued before their stores (source and destination share the
-        // pool arrays, so the compiler keeps each load after the stores
-        // before it); to <= L, so a clamped index stays in the row
-        auto copy_run = [&](int32_t to) {
-            for (; i < to; i += 8, o += 8) {
-                int32_t cc[8];
-                float vv[8];
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const uint64_t si = st + (uint64_t)(i + j < to ? i + j : to - 1);
-                    cc[j] = pcol[si];
-                    vv[j] = pval[si];
-                }
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    if (i + j < to) {
-                        pcol[o + j] = cc[j];
-                        pval[o + j] = vv[j];
+        if (tm + NTM < nt) {
+            const uint32_t g = row_of(tm + NTM);
+            st1 = row_start[g];
+            L1 = (uint32_t)row_len[g];
+        }
+        if (tl < L) {
+            c0 = pcol[(uint64_t)st + tl];
+            v0 = pval[(uint64_t)st + tl];
+        }
+        if (tl + RL < L) {
+            c1 = pcol[(uint64_t)st + tl + RL];
+            v1 = pval[(uint64_t)st + tl + RL];
+        }
+        for (uint32_t tt = tm; tt < nt; tt += NTM) {
+            uint32_t st2 = 0, L2 = 0;
+            int32_t d0 = 0, d1 = 0;
+            float w0 = 0.0f, w1 = 0.0f;
+            if (tl < L1) {
+                d0 = pcol[(uint64_t)st1 + tl];
+                w0 = pval[(uint64_t)st1 + tl];
+            }
+            if (tl + RL < L1) {
+                d1 = pcol[(uint64_t)st1 + tl + RL];
+                w1 = pval[(uint64_t)st1 + tl + RL];
+            }
+            if (tt + 2 * NTM < nt) {
+                const uint32_t g = row_of(tt + 2 * NTM);
+                st2 = row_start[g];
+                L2 = (uint32_t)row_len[g];
+            }
+            uint32_t u = tub[tt];
+            const uint32_t ue = tub[tt + 1];
+            const uint32_t nl = tnl[tt];
+            if (!(nl & 0x8000u)) {
+                for (uint32_t q = u + tl; q < ue; q += RL)
+                    if (upc[q] >> 14 == C_ADD) pval[(uint64_t)st + (upc[q] & 0x3fffu)] = S.uval[q];
+            } else {
+                const uint32_t g = gbase + (S.urc[u] >> KB);
+                const uint32_t dst = base + tdst[tt];
+                uint32_t sh = 0;  // inserts less deletes so far
+                for (uint32_t i0 = 0;;) {
+                    const bool last = i0 + RC >= L;
+                    const uint32_t p0 = i0 + tl, p1 = p0 + RL;
+                    uint32_t s0 = sh, s1 = sh;
+                    bool k0 = p0 < L, k1 = p1 < L;
+                    for (; u < ue; ++u) {
+                        const uint32_t w = upc[u];
+                        const uint32_t pos = w & 0x3fffu, code = w >> 14;
+                        if (!last && pos >= i0 + RC) break;  // among later entries
+                        if (code == C_INS) {
+                            if (tl == 0) {
+                                pcol[(uint64_t)dst + (pos + sh)] = (int32_t)(S.urc[u] & (LMAX - 1));
+                                pval[(uint64_t)dst + (pos + sh)] = S.uval[u];
+                            }
+                            ++sh;
+                            s0 += p0 >= pos;
+                            s1 += p1 >= pos;
+                        } else if (code == C_DEL) {
+                            --sh;
+                            k0 = k0 && p0 != pos;
+                            k1 = k1 && p1 != pos;
+                            s0 -= p0 > pos;
+                            s1 -= p1 > pos;
+                        } else if (code == C_ADD) {
+                            const float nv = S.uval[u];
+                            v0 = p0 == pos ? nv : v0;
+                            v1 = p1 == pos ? nv : v1;
+                        }
+                    }
+                    if (k0) {
+                        pcol[(uint64_t)dst + (p0 + s0)] = c0;
+                        pval[(uint64_t)dst + (p0 + s0)] = v0;
+                    }
+                    if (k1) {
+                        pcol[(uint64_t)dst + (p1 + s1)] = c1;
+                        pval[(uint64_t)dst + (p1 + s1)] = v1;
+                    }
+                    if (last) break;
+                    i0 += RC;
+                    if (i0 + tl < L) {
+                        c0 = pcol[(uint64_t)st + i0 + tl];
+                        v0 = pval[(uint64_t)st + i0 + tl];
+                    }
+                    if (i0 + RL + tl < L) {
+                        c1 = pcol[(uint64_t)st + i0 + RL + tl];
+                        v1 = pval[(uint64_t)st + i0 + RL + tl];
                     }
                 }
+                if (tl == 0) {
+                    row_start[g] = dst;
+                    row_len[g] = (int32_t)(nl & 0x7fffu);
+                    row_cap[g] = (int32_t)chunk_round(nl & 0x7fffu);
+                }
             }
-            o -= (uint64_t)(i - to);  // the last chunk stopped at to
-            i = to;
-        };
-        for (uint32_t u = ub; u < ue; ++u) {
-            const uint32_t k = upos[u];  // old entries before this coordinate
-            if (i < (int32_t)k) copy_run((int32_t)k);
-            const uint32_t code = ucode[u];
-            if (code == C_INS) {
-                pcol[o] = (int32_t)(urc[u] & (LMAX - 1));
-                pval[o] = uval[u];
-                ++o;
-            } else if (code == C_ADD) {
-                pcol[o] = pcol[st + i];
-                pval[o] = uval[u];
-                ++o;
-                ++i;
-            } else if (code == C_DEL) {
-                ++i;
-            }
+            st = st1;
+            L = L1;
+            c0 = d0;
+            c1 = d1;
+            v0 = w0;
+            v1 = w1;
+            st1 = st2;
+            L1 = L2;
         }
-        if (i < L) copy_run(L);
-    }
-    __syncthreads();
-    for (uint32_t tt = t; tt < nt; tt += BT) {
-        if (!tmode[tt]) continue;
-        const uint32_t g = gbase + trw[tt];
-        row_start[g] = base + tdst[tt];
-        row_len[g] = (int32_t)tnl[tt];
-        row_cap[g] = (int32_t)chunk_round(tnl[tt]);
     }
     __syncthreads();
 }
@@ -598,7 +623,7 @@ __device__ void batch_spmv(uint32_t m, const uint32_t *__restrict__ row_base, co
 }
 
 template <int TEAM>
-__global__ __launch_bounds__(BT) void k_batch_step(uint32_t M, const uint32_t *__restrict__ row_base,
+__global__ __launch_bounds__(BT, 8) void k_batch_step(uint32_t M, const uint32_t *__restrict__ row_base,
                                                    const uint32_t *__restrict__ col_base,
                                                    const int64_t *__restrict__ tri_off, int64_t ntri,
                                                    const int32_t *__restrict__ trow, const int32_t *__restrict__ tcol,
@@ -606,26 +631,22 @@ __global__ __launch_bounds__(BT) void k_batch_step(uint32_t M, const uint32_t *_
                                                    uint32_t *__restrict__ row_start, int32_t *__restrict__ row_len,
                                                    int32_t *__restrict__ row_cap, int32_t *__restrict__ pcol,
                                                    float *__restrict__ pval, unsigned long long pool_cap, DevState *ds,
-                                                   uint32_t *__restrict__ mstat, uint32_t *__restrict__ scratch,
+                                                   uint32_t *__restrict__ mstat,
                                                    const float *__restrict__ x, float *__restrict__ y, uint32_t thresh,
                                                    BatchState *bs, int do_update, int do_spmv, int reserved)
 {
-    __shared__ uint32_t sk[2][BMAX];
-    __shared__ float sv[2][BMAX];
-    __shared__ uint32_t wcnt[BT / 64][256];
-    __shared__ uint32_t lw[BT / 64];
-    __shared__ uint32_t sm[4];
-    uint32_t *sc = scratch + (uint64_t)blockIdx.x * S_WORDS;
-    BatchAcc acc{0, 0, 0, 0, 0, 0};
+    __shared__ BatchLds S;
+    __shared__ BatchAcc acc;
+    if (threadIdx.x == 0) acc = BatchAcc{0, 0, 0, 0, 0, 0};
     for (;;) {
-        if (threadIdx.x == 0) sm[3] = atomicAdd(&bs->work, 1u);
+        if (threadIdx.x == 0) S.sm[SM_NEXT] = atomicAdd(&bs->work, 1u);
         __syncthreads();
-        const uint32_t m = sm[3];
+        const uint32_t m = S.sm[SM_NEXT];
         __syncthreads();
         if (m >= M) break;
         if (do_update)
             batch_update(m, row_base, col_base, tri_off, ntri, trow, tcol, tval, row_start, row_len, row_cap, pcol, pval,
-                         pool_cap, ds, mstat, sc, sk, sv, wcnt, lw, sm, reserved != 0, acc);
+                         pool_cap, ds, mstat, S, reserved != 0, acc);
         if (do_spmv) batch_spmv<TEAM>(m, row_base, col_base, row_start, row_len, pcol, pval, x, y, thresh);
         __syncthreads();
     }
@@ -701,7 +722,6 @@ struct dcsr_batch_s {
     uint32_t *row_base, *col_base;  // device, M+1
     std::vector<uint32_t> row_base_h, col_base_h;
     uint32_t *mstat;                // device, per-matrix status bits
-    uint32_t *scratch;              // per-workgroup scratch
     BatchState *bs;
     int grid;
     int team, thresh;               // SpMV launch shape (autotuned)
@@ -758,7 +778,6 @@ dcsr_status dcsr_batch_create(dcsr_batch *out, int32_t count, const int32_t *row
     if ((uint32_t)b->grid > b->M) b->grid = (int)b->M;
     if (hipMalloc(&b->row_base, (count + 1) * 4) != hipSuccess || hipMalloc(&b->col_base, (count + 1) * 4) != hipSuccess ||
         hipMalloc(&b->mstat, count * 4) != hipSuccess ||
-        hipMalloc(&b->scratch, (size_t)b->grid * S_WORDS * 4) != hipSuccess ||
         hipMalloc(&b->bs, sizeof(BatchState)) != hipSuccess ||
         hipStreamCreateWithFlags(&b->cs, hipStreamNonBlocking) != hipSuccess) {
         dcsr_batch_destroy(b);
@@ -784,7 +803,6 @@ dcsr_status dcsr_batch_destroy(dcsr_batch b)
     (void)hipFree(b->row_base);
     (void)hipFree(b->col_base);
     (void)hipFree(b->mstat);
-    (void)hipFree(b->scratch);
     (void)hipFree(b->bs);
     if (b->h) dcsr_destroy(b->h);
     delete b;
@@ -829,7 +847,7 @@ static void launch_step(dcsr_batch b, const int64_t *tri_off, int64_t n, const i
     dcsr_handle h = b->h;
     k_batch_step<TEAM><<<b->grid, BT, 0, s>>>(b->M, b->row_base, b->col_base, tri_off, n, rows, cols, vals, h->row_start,
                                               h->row_len, h->row_cap, h->pool_col, h->pool_val,
-                                              (unsigned long long)h->pool_cap, h->ds, b->mstat, b->scratch, x, y,
+                                              (unsigned long long)h->pool_cap, h->ds, b->mstat, x, y,
                                               (uint32_t)b->thresh, b->bs, do_update, do_spmv, reserved);
 }
 
