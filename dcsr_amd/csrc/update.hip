@@ -27,7 +27,8 @@
 //      positions, then commit the row table.
 //
 // Cross-tile prefixes come from per-tile counts scanned by the last
-// workgroup to finish (an atomic finish counter); nothing polls.
+// workgroup to finish (an atomic finish counter); nothing polls.  Batches of
+// up to 10,240 triples take steps 1 to 5 in one workgroup (smallupd.h).
 //
 // dcsr_update is synchronous by default: the batch's status comes back with
 // the call, from one read of the device state (at the end when the host can
@@ -1458,6 +1459,8 @@ __global__ __launch_bounds__(TB) void k_upd_write(DevState *ds, uint32_t report,
     }
 }
 
+#include "smallupd.h"
+
 __global__ void k_fill_u64(uint64_t *p, int64_t n, uint64_t v)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1651,11 +1654,6 @@ dcsr_status sort_plan_launch(dcsr_handle h, int64_t n, UpdBufs &b, hipStream_t s
     const uint32_t *val = which ? b.v1 : b.v0;
     const unsigned ht = (unsigned)((n + TILE - 1) / TILE);
     const bool table = ht > HEADS_DIRECT_TILES;
-    if (b.rowt && ++h->upd_tag == 0u) {
-        // tags wrapped: clear the map, restart at 1
-        k_fill_u64<<<grid_for(h->rows, TB), TB, 0, s>>>(b.rowt, h->rows, 0ull);
-        h->upd_tag = 1u;
-    }
     k_upd_heads_count<<<ht, TB, 0, s>>>(key, n, h->cbits, h->row_len, b.tt, b.tp, b.fin, h->ds, table);
     k_upd_heads_emit<<<ht, TB, 0, s>>>(key, val, n, h->cbits, b.tt, h->ds, table, b.ucol, b.usum, b.ut, b.trow,
                                        b.tubeg, h->row_len, h->row_start, h->row_cap, b.tp, b.tlpre, b.trs, b.tlen,
@@ -1679,10 +1677,41 @@ void launch_pack(dcsr_handle h, const int32_t *rows, const int32_t *cols, const 
                                             pack_tiles(n), h->ds, b.lb, b.ndig);
 }
 
-// Pack (validate + key) the caller's triples, then sort .. offsets.
+// A batch of at most SMALL_MAX triples (smallupd.h).
+dcsr_status small_launch(dcsr_handle h, const int32_t *rows, const int32_t *cols, const float *vals, int64_t n,
+                         UpdBufs &b, hipStream_t s)
+{
+    const SmallArgs A{rows, cols, vals, (uint32_t)n, h->rows, h->cols, h->cbits, (unsigned long long)h->pool_cap, h->ds,
+                      h->row_start, h->row_len, h->row_cap, h->pool_col, h->pool_val, b.ucol, b.usum, b.uval, b.ut,
+                      b.upos, b.ucode, b.upre, b.trow, b.tubeg, b.trs, b.tlen, b.tcap, b.tins, b.tdel, b.tnewl,
+                      b.tmode, b.tmoved, b.tpre, b.mspan, b.rowt, h->upd_tag};
+    if (n <= SU_TB) {
+        k_upd_small<1, true><<<1, SU_TB, 0, s>>>(A);
+    } else if (n <= SMALL_FUSED) {
+        k_upd_small<2, true><<<1, SU_TB, 0, s>>>(A);
+    } else {
+        if (n <= 5 * SU_TB) k_upd_small<5, false><<<1, SU_TB, 0, s>>>(A);
+        else if (n <= 7 * SU_TB) k_upd_small<7, false><<<1, SU_TB, 0, s>>>(A);
+        else k_upd_small<SU_IT_MAX, false><<<1, SU_TB, 0, s>>>(A);
+        k_upd_small_probe<<<grid_for(n, TB), TB, 0, s>>>(A);
+        if (n <= 5 * SU_TB) k_upd_small_plan<5><<<1, SU_TB, 0, s>>>(A);
+        else k_upd_small_plan<SU_IT_MAX><<<1, SU_TB, 0, s>>>(A);
+    }
+    DCSR_HIP(hipGetLastError());
+    return DCSR_OK;
+}
+
+// The caller's triples to a decided plan: small batches in one workgroup, the
+// others packed (validate + key), then sort .. offsets.
 dcsr_status prepare_launch(dcsr_handle h, const int32_t *rows, const int32_t *cols, const float *vals, int64_t n,
                            UpdBufs &b, hipStream_t s)
 {
+    if (b.rowt && ++h->upd_tag == 0u) {
+        // tags wrapped: clear the map, restart at 1
+        k_fill_u64<<<grid_for(h->rows, TB), TB, 0, s>>>(b.rowt, h->rows, 0ull);
+        h->upd_tag = 1u;
+    }
+    if (n <= SMALL_MAX) return small_launch(h, rows, cols, vals, n, b, s);
     launch_pack(h, rows, cols, vals, n, b, s);
     DCSR_HIP(hipGetLastError());
     return sort_plan_launch(h, n, b, s);
@@ -1720,12 +1749,13 @@ dcsr_status commit_launch(dcsr_handle h, const UpdBufs &b, int64_t n, int64_t mo
     return DCSR_OK;
 }
 
-// Sort through commit of a packed batch of n triples (the commit kernels
-// skip themselves when the plan rejected the batch; `report`: see k_upd_write).
-// seq: a NOSYNC update's snapshot sequence number (0: no snapshot).
-dcsr_status pipeline_launch(dcsr_handle h, int64_t n, UpdBufs &b, bool report, hipStream_t s, uint64_t seq = 0)
+// The caller's triples through commit (the commit kernels skip themselves when
+// the plan rejected the batch; `report`: see k_upd_write).  seq: a NOSYNC
+// update's snapshot sequence number (0: no snapshot).
+dcsr_status pipeline_launch(dcsr_handle h, const int32_t *rows, const int32_t *cols, const float *vals, int64_t n,
+                            UpdBufs &b, bool report, hipStream_t s, uint64_t seq = 0)
 {
-    DCSR_TRY(sort_plan_launch(h, n, b, s));
+    DCSR_TRY(prepare_launch(h, rows, cols, vals, n, b, s));
     return commit_launch(h, b, n, h->pool_cap, report, s, seq);
 }
 
@@ -1847,9 +1877,7 @@ static dcsr_status update_sync(dcsr_handle h, const int32_t *rows, const int32_t
         // then holds the committed counters: write folds the deltas in)
         UpdBufs b;
         DCSR_TRY(upd_bufs(h, n, b, s));
-        launch_pack(h, rows, cols, vals, n, b, s);
-        DCSR_HIP(hipGetLastError());
-        DCSR_TRY(pipeline_launch(h, n, b, false, s));
+        DCSR_TRY(pipeline_launch(h, rows, cols, vals, n, b, false, s));
         DCSR_TRY(pull_state(h, s));
         if (h->hs->ubad_last) return DCSR_ERR_BAD_INDEX;
         if (h->hs->go) {
@@ -1895,10 +1923,8 @@ static dcsr_status update_nosync(dcsr_handle h, const int32_t *rows, const int32
     const int64_t claimed = claims_bound(h, n);
     UpdBufs b;
     DCSR_TRY(upd_bufs(h, n, b, s));
-    launch_pack(h, rows, cols, vals, n, b, s);
-    DCSR_HIP(hipGetLastError());
     const uint64_t seq = snapshot_next(h);
-    DCSR_TRY(pipeline_launch(h, n, b, true, s, seq));
+    DCSR_TRY(pipeline_launch(h, rows, cols, vals, n, b, true, s, seq));
     state_unknown(h, n, claimed);
     snapshot_note(h, seq);
     return DCSR_OK;
@@ -1940,11 +1966,9 @@ dcsr_status update_fixed_scratch(dcsr_handle h, const int32_t *rows, const int32
     hipStreamCaptureStatus cap_st = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cap_st) == hipSuccess && cap_st != hipStreamCaptureStatusNone) h->flat_replayed = true;
     if (nosync) refresh_bounds(h);
-    launch_pack(h, rows, cols, vals, n, b, s);
-    DCSR_HIP(hipGetLastError());
     const uint64_t seq = nosync ? snapshot_next(h) : 0;
     const int64_t claimed = claims_bound(h, n);
-    DCSR_TRY(pipeline_launch(h, n, b, nosync, s, seq));
+    DCSR_TRY(pipeline_launch(h, rows, cols, vals, n, b, nosync, s, seq));
     if (nosync) {
         state_unknown(h, n, claimed);
         snapshot_note(h, seq);
