@@ -56,6 +56,7 @@ struct DevState {
     unsigned int ubad_last;         // current update's batch held an out-of-range index
     unsigned int ptotal;            // current update: probe lengths of the touched rows, summed
     unsigned int load_flags;        // current load: LD_* bits
+    unsigned int load_nnz;          // current CSR load: its last offset
 };
 
 // Grow-only device scratch buffers owned by a handle.
@@ -78,6 +79,13 @@ struct HostSnap {
     uint64_t nnz, bump, seq;
 };
 constexpr int SNAP_RING = 64;
+
+// Device words the host reads back (fetch_words), stored by a kernel (seq last).
+struct HostFetch {
+    uint32_t words[126];
+    uint64_t seq;
+};
+static_assert(sizeof(DevState) <= sizeof(HostFetch::words) && sizeof(DevState) % 4 == 0, "the state is fetched whole");
 
 struct Workspace {
     void *ptr[WS_COUNT];
@@ -123,6 +131,9 @@ struct dcsr_matrix_s {
     // do not count (a read-back, load or compaction) and are ignored.
     HostSnap *hsnap;         // host view (pinned, coherent)
     HostSnap *dsnap;         // the same memory as the device addresses it
+    HostFetch *hfetch;       // host view (pinned, coherent) of words read back
+    HostFetch *dfetch;       // the same memory as the device addresses it
+    uint64_t fetch_seq;
     uint64_t snap_seq;       // last sequence number handed to an update
     uint64_t snap_valid_from;
     uint64_t snap_used;      // last snapshot folded into the bounds
@@ -170,6 +181,9 @@ dcsr_status ws_get(dcsr_handle h, WsSlot slot, size_t bytes, void **out);
 // words, finish counters): a grown buffer is zero-filled by a kernel on s.
 dcsr_status ws_get_zeroed(dcsr_handle h, WsSlot slot, size_t bytes, void **out, hipStream_t s);
 dcsr_status pull_state(dcsr_handle h, hipStream_t s);   // copy DevState to host + sync
+// A few device words to the host once everything queued on s before the call
+// has finished (whole words, at most sizeof(HostFetch::words) bytes).
+dcsr_status fetch_words(dcsr_handle h, const void *src, size_t bytes, void *dst, hipStream_t s);
 // Grow the pool in stream order, without reading the device state back:
 // the live rows are compacted into a new pool of at least new_cap entries.
 dcsr_status grow_in_order(dcsr_handle h, int64_t new_cap, hipStream_t s);

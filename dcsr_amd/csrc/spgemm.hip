@@ -913,8 +913,7 @@ dcsr_status dcsr_spgemm(dcsr_handle A, dcsr_handle B, dcsr_handle C, dcsr_stream
     }
     DCSR_HIP(scan_exclusive_u32(P, Poff, R, 1, part, Poff + R, s, fault_word(C)));
     SgState hst;
-    DCSR_HIP(hipMemcpyAsync(&hst, st, sizeof(SgState), hipMemcpyDeviceToHost, s));
-    DCSR_HIP(hipStreamSynchronize(s));
+    DCSR_TRY(fetch_words(C, st, sizeof(SgState), &hst, s));
     if (hst.total >= 0xfffffff0ull) return DCSR_ERR_UNSUPPORTED;
     const uint32_t Ptot = (uint32_t)hst.total;
 
@@ -971,8 +970,7 @@ dcsr_status dcsr_spgemm(dcsr_handle A, dcsr_handle B, dcsr_handle C, dcsr_stream
         uint32_t *htot_d;
         DCSR_TRY(ws_get(C, WS_TMP2, 64, (void **)&htot_d));
         DCSR_HIP(scan_exclusive_u32(hpre_in, hpre, hn + 1, 2, part, htot_d, s, fault_word(C)));
-        DCSR_HIP(hipMemcpyAsync(htot, htot_d, 8, hipMemcpyDeviceToHost, s));
-        DCSR_HIP(hipStreamSynchronize(s));
+        DCSR_TRY(fetch_words(C, htot_d, 8, htot, s));
         const uint32_t nent = htot[0], np = htot[1];
         DCSR_TRY(ws_get(C, WS_SG_EA, (size_t)(nent + 1) * sizeof(EA), (void **)&ea));
         DCSR_TRY(ws_get(C, WS_SG_APOS, (size_t)(nent + 2) * 8, (void **)&blen));
