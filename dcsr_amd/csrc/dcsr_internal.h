@@ -63,7 +63,7 @@ struct DevState {
 enum WsSlot {
     WS_KEY_A, WS_KEY_B, WS_VAL_A, WS_VAL_B, WS_FLAGS, WS_SCAN, WS_PART, WS_HIST,
     WS_UCOL, WS_UVAL, WS_UT, WS_UPOS, WS_UCODE, WS_UPRE,
-    WS_TROW, WS_TUBEG, WS_TINS, WS_TDEL, WS_TOLDS, WS_TMOVED, WS_TDEST, WS_TNEWL, WS_TMODE, WS_TOLDPRE,
+    WS_TROW, WS_TUBEG, WS_TINS, WS_TDEL, WS_TMOVED, WS_TDEST, WS_TNEWL, WS_TMODE, WS_TOLDPRE,
     WS_HUB_ROWS, WS_HUB_PRE, WS_HUB_PART, WS_HUB_DONE,
     WS_PPROBE, WS_PPLAN, WS_UROW, WS_TPAIRPRE, WS_FOFF, WS_ROWMAP, WS_CARRY_ROW, WS_CARRY_VAL, WS_SPMM_CROW, WS_SPMM_CVAL,
     WS_SG_P, WS_SG_POFF, WS_SG_CNT, WS_SG_COFF, WS_SG_LIST, WS_SG_STATE, WS_SG_BSUM,

@@ -17,17 +17,17 @@
 //   4. plan per touched row: rows whose structure is unchanged get their
 //      values written in place; the others claim a new chunk of the pool's
 //      bump region.  Claims are slot offsets from a prefix sum, so no two
-//      rows contend on an atomic.  The last workgroup of the plan launch
-//      turns every per-tile count into offsets and decides the batch: a bad
-//      index or pool exhaustion rejects it whole (no-op), otherwise the bump
-//      pointer advances;
+//      rows contend on an atomic.  The per-tile counts become offsets and the
+//      batch is decided: a bad index or pool exhaustion rejects it whole
+//      (no-op), otherwise the bump pointer advances;
 //   5. offsets: per-entry exclusive counts (inserts / deletes before each
 //      coordinate, claims / moved entries before each row);
 //   6. move surviving old entries and write inserted ones at their merged
 //      positions, then commit the row table.
 //
-// Cross-tile prefixes come from per-tile counts scanned by the last
-// workgroup to finish (an atomic finish counter); nothing polls.  Batches of
+// Cross-tile prefixes come from per-tile counts, summed where they are used
+// (up to 1,024 tiles) or scanned by a launch of one workgroup; nothing polls.
+// Batches of
 // up to 10,240 triples take steps 1 to 5 in one workgroup (smallupd.h).
 //
 // dcsr_update is synchronous by default: the batch's status comes back with
@@ -132,10 +132,14 @@ __device__ __forceinline__ long long wave_sum_i64(long long v)
 
 // ---------------------------------------------------------------------------
 // Tile tables.  The per-element passes work on tiles of 2048 entries (8 per
-// thread, blocked).  Each tile writes its counts to a table; the last
-// workgroup of the launch to finish (an atomic finish counter: nothing ever
-// waits) turns the table's columns into exclusive offsets, and a later
-// kernel adds them to the in-tile prefixes.
+// thread, blocked).  Each tile writes its counts to a table; where a batch has
+// too many tiles for every workgroup to sum the counts before its own, a
+// launch of one workgroup turns the table's columns into exclusive offsets,
+// and a later kernel adds them to the in-tile prefixes.  (The last workgroup
+// of the counting launch to finish did that before: the release that each
+// workgroup needs ahead of its finish counter writes its XCD's L2 back, and
+// over the 1,954 tiles of a 4M-triple batch the two counting passes took 47 and
+// 115 us; they take 13 and 40, and the scans 8 and 15.)
 // ---------------------------------------------------------------------------
 constexpr int IPT = 8;
 constexpr int TILE = TB * IPT;
@@ -148,29 +152,6 @@ enum { TT_H = 0, TT_R, TT_HX, TT_RX, TT_C, TT_M, TT_CX, TT_MX, TT_WORDS };
 // probe tile table: inserts, adds, deletes; insert / delete offsets; probe
 // lengths of the tile's touched rows (sum, offset)
 enum { TP_I = 0, TP_A, TP_D, TP_IX, TP_DX, TP_L, TP_LX, TP_WORDS = 8 };
-// finish counters (self-resetting)
-enum { FC_HEADS = 0, FC_PLAN = 1 };
-
-// True in every thread of the last workgroup of the launch to finish; it then
-// sees what every other workgroup wrote before finishing.  Each workgroup
-// releases (L2 write-back) before it is counted and only the last one
-// acquires (L2 invalidate): a full fence in every workgroup would also
-// invalidate the L2 under the workgroups still running.
-__device__ __forceinline__ bool last_block(unsigned int *ctr, uint32_t *s_flag)
-{
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-        const bool last = atomicAdd(ctr, 1u) == gridDim.x - 1;
-        if (last) atomicExch(ctr, 0u);
-        *s_flag = last ? 1u : 0u;
-    }
-    __syncthreads();
-    const bool last = *s_flag != 0u;
-    if (last) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    return last;
-}
-
 // One workgroup: exclusive scans of NC columns of tile tables with 8 words
 // per row, tab[c][i * 8 + src[c]] -> tab[c][i * 8 + dst[c]] for i < cnt;
 // tot[c] receives column c's total.  Every load of a 2048-row chunk (all
@@ -265,17 +246,15 @@ __device__ __forceinline__ uint32_t head_rows_len(const uint64_t (&k)[IPT], uint
 }
 
 // Pass 1 of the heads: per-tile counts (coordinates, touched rows, and the
-// rows' probe lengths).  With `table` the last workgroup makes them offsets
-// and stores nuniq / ntouched / ptotal; without it (batches of at most
-// HEADS_DIRECT_TILES tiles) pass 2 sums the counts before each tile itself,
-// and this kernel ends at the counts.
+// rows' probe lengths).  Pass 2 sums the counts before each tile itself for
+// batches of at most HEADS_DIRECT_TILES tiles; k_upd_heads_scan makes them
+// offsets for larger ones.
 constexpr int64_t HEADS_DIRECT_TILES = 4 * TB;
 __global__ __launch_bounds__(TB) void k_upd_heads_count(const uint64_t *__restrict__ key, int64_t n, int cbits,
                                                         const int32_t *__restrict__ row_len,
-                                                        uint32_t *__restrict__ tt, uint32_t *__restrict__ tp,
-                                                        unsigned int *fin, DevState *ds, bool table)
+                                                        uint32_t *__restrict__ tt, uint32_t *__restrict__ tp)
 {
-    __shared__ uint32_t lds4[4], s_flag;
+    __shared__ uint32_t lds4[4];
     const int64_t tile = blockIdx.x;
     uint64_t k[IPT], prev;
     load_keys(key, n, tile * TILE + (int64_t)threadIdx.x * IPT, k, prev);
@@ -290,16 +269,19 @@ __global__ __launch_bounds__(TB) void k_upd_heads_count(const uint64_t *__restri
         tt[tile * TT_WORDS + TT_R] = rc;
         tp[tile * TP_WORDS + TP_L] = lc;
     }
-    if (!table) return;
-    if (last_block(&fin[FC_HEADS], &s_flag)) {
-        uint32_t *const tabs[3] = {tt, tt, tp};
-        uint32_t tot[3];
-        block_scan_columns<3>(tabs, {TT_H, TT_R, TP_L}, {TT_HX, TT_RX, TP_LX}, gridDim.x, lds4, tot);
-        if (threadIdx.x == 0) {
-            ds->nuniq = tot[0];
-            ds->ntouched = tot[1];
-            ds->ptotal = tot[2];
-        }
+}
+
+// The heads' tile counts to offsets and totals, by one workgroup.
+__global__ __launch_bounds__(TB) void k_upd_heads_scan(uint32_t *tt, uint32_t *tp, int64_t ntiles, DevState *ds)
+{
+    __shared__ uint32_t lds4[4];
+    uint32_t *const tabs[3] = {tt, tt, tp};
+    uint32_t tot[3];
+    block_scan_columns<3>(tabs, {TT_H, TT_R, TP_L}, {TT_HX, TT_RX, TP_LX}, ntiles, lds4, tot);
+    if (threadIdx.x == 0) {
+        ds->nuniq = tot[0];
+        ds->ntouched = tot[1];
+        ds->ptotal = tot[2];
     }
 }
 
@@ -805,10 +787,7 @@ __device__ void plan_totals_decide(DevState *ds, unsigned long long pool_cap, co
 // recorded (tlen, tcap) still hold, so every load is one coalesced round
 // trip; otherwise (a re-plan after the pool was compacted or grown) they
 // and the row's pool start are re-read from the row table and trs is
-// rewritten.  The last workgroup to finish then decides the batch: it makes the
-// claim / moved / insert / delete columns exclusive offsets, totals every
-// counter, rejects the batch (no-op) on a bad index or when the claims do
-// not fit the pool, and otherwise advances the bump pointer.
+// rewritten.
 __global__ __launch_bounds__(TB) void k_upd_plan(DevState *ds, unsigned long long pool_cap,
                                                  const uint32_t *__restrict__ trow, const uint32_t *__restrict__ tins,
                                                  const uint32_t *__restrict__ tdel, const uint32_t *__restrict__ ucode,
@@ -818,12 +797,11 @@ __global__ __launch_bounds__(TB) void k_upd_plan(DevState *ds, unsigned long lon
                                                  uint32_t *__restrict__ tnewl,
                                                  uint32_t *__restrict__ tmode, uint32_t *__restrict__ tmoved,
                                                  uint32_t *__restrict__ tt,
-                                                 uint32_t *__restrict__ tp, long long *__restrict__ pplan,
-                                                 unsigned int *fin, bool table, bool fresh,
+                                                 uint32_t *__restrict__ tp, long long *__restrict__ pplan, bool fresh,
                                                  const uint32_t *__restrict__ tlen, const uint32_t *__restrict__ tcap)
 {
     __shared__ long long lds[4][8];
-    __shared__ uint32_t lds4[4], lds44[4][4], s_flag;
+    __shared__ uint32_t lds44[4][4];
     const int64_t tile = blockIdx.x;
     const int64_t t0 = tile * TILE + (int64_t)threadIdx.x * IPT;
     const uint32_t nt = ds->ntouched, nu = ds->nuniq;
@@ -911,16 +889,20 @@ __global__ __launch_bounds__(TB) void k_upd_plan(DevState *ds, unsigned long lon
         tp[tile * TP_WORDS + TP_A] = cia >> 16;
         tp[tile * TP_WORDS + TP_D] = cdl;
     }
-    // without a table scan (at most HEADS_DIRECT_TILES tiles) the offsets
-    // pass sums the counts before each tile and decides the batch
-    if (!table || !last_block(&fin[FC_PLAN], &s_flag)) return;
+}
 
-    const int64_t ntiles = gridDim.x;
+// The plan's tile counts to offsets, then the decision (plan_totals_decide),
+// by one workgroup; without a table the offsets pass does both.
+__global__ __launch_bounds__(TB) void k_upd_plan_scan(DevState *ds, unsigned long long pool_cap, uint32_t *tt,
+                                                      uint32_t *tp, const long long *__restrict__ pplan,
+                                                      int64_t ntiles)
+{
+    __shared__ long long lds[4][8];
+    __shared__ uint32_t lds4[4];
     uint32_t *const tabs[4] = {tt, tt, tp, tp};
     uint32_t ctot[4];
     block_scan_columns<4>(tabs, {TT_C, TT_M, TP_I, TP_D}, {TT_CX, TT_MX, TP_IX, TP_DX}, ntiles, lds4, ctot);
-    const uint32_t claim_total = ctot[0], moved_total = ctot[1], ins_total = ctot[2], del_total = ctot[3];
-    plan_totals_decide(ds, pool_cap, pplan, tp, ntiles, claim_total, moved_total, ins_total, del_total, lds);
+    plan_totals_decide(ds, pool_cap, pplan, tp, ntiles, ctot[0], ctot[1], ctot[2], ctot[3], lds);
 }
 
 // Exclusive offsets per entry: upre[2u], upre[2u+1] = inserts / deletes
@@ -942,7 +924,7 @@ __global__ __launch_bounds__(TB) void k_upd_offsets(DevState *__restrict__ ds,
     __shared__ long long lds[4][8];
     const int64_t tile = blockIdx.x;
     const int64_t e0 = tile * TILE + (int64_t)threadIdx.x * IPT;
-    // tile bases: scanned by the plan's last workgroup (table), or summed
+    // tile bases: scanned by k_upd_plan_scan (table), or summed
     // here from the counts of the tiles before this one (loaded with the
     // entries: up to four tiles per thread, index clamped to tile 0, masked)
     constexpr int QT = HEADS_DIRECT_TILES / TB;
@@ -1474,7 +1456,7 @@ struct UpdBufs {
     float *usum, *uval;
     uint32_t *ut, *upos, *ucode, *upre;
     uint32_t *trow, *tubeg, *tlpre, *trs, *tlen, *tcap, *tins, *tdel, *tnewl, *tmode, *tmoved, *tpre;
-    uint32_t *tt, *tp, *fin;
+    uint32_t *tt, *tp;
     // first touched row of every probe / move span (null: searched for)
     uint32_t *pspan, *mspan;
     // tagged row -> touched-row map for the move kernel's row scan (null: no
@@ -1531,7 +1513,7 @@ struct BufSrc {
 dcsr_status take(BufSrc &src, WsSlot slot, size_t bytes, void **out)
 {
     if (!src.base && !src.measure) {
-        if (slot == WS_SCAN || slot == WS_TOLDS) return ws_get_zeroed(src.h, slot, bytes, out, src.s);
+        if (slot == WS_SCAN) return ws_get_zeroed(src.h, slot, bytes, out, src.s);
         return ws_get(src.h, slot, bytes, out);
     }
     const size_t at = (src.used + 255) & ~size_t(255);
@@ -1581,8 +1563,6 @@ dcsr_status upd_bufs_src(BufSrc &src, int64_t n, UpdBufs &b)
     DCSR_TRY(take(src, WS_TDEST, nt * TT_WORDS * 4, (void **)&b.tt));
     DCSR_TRY(take(src, WS_PPROBE, nt * TP_WORDS * 4, (void **)&b.tp));
     DCSR_TRY(take(src, WS_PPLAN, nt * NPLAN * 8, (void **)&b.pplan));
-    // finish counters: zero-filled on allocation, reset by their last user
-    DCSR_TRY(take(src, WS_TOLDS, 64, (void **)&b.fin));
     // span tables grow with the matrix, so a fixed region goes without them
     b.pspan = b.mspan = nullptr;
     b.rowt = nullptr;
@@ -1604,8 +1584,8 @@ dcsr_status upd_bufs(dcsr_handle h, int64_t n, UpdBufs &b, hipStream_t s)
     return DCSR_OK;
 }
 
-// Tile tables scanned by a last workgroup (table) only for batches of more
-// than HEADS_DIRECT_TILES tiles; smaller ones sum them where they are used.
+// Tile tables are scanned (table) only for batches of more than
+// HEADS_DIRECT_TILES tiles; smaller ones sum them where they are used.
 static inline bool use_tables(int64_t n) { return ptiles(n) > HEADS_DIRECT_TILES; }
 
 static void launch_offsets(dcsr_handle h, UpdBufs &b, int64_t n, hipStream_t s)
@@ -1614,8 +1594,8 @@ static void launch_offsets(dcsr_handle h, UpdBufs &b, int64_t n, hipStream_t s)
                                            b.pplan, (unsigned long long)h->pool_cap, use_tables(n), b.mspan);
 }
 
-// Plan and decision.  With tile tables the plan's last workgroup decides;
-// without them the offsets pass does (its last tile), so it runs here.
+// Plan and decision.  With tile tables their scan decides; without them the
+// offsets pass does (its last tile), so it runs here.
 // fresh: straight after the heads pass (false for a re-plan after the pool
 // was compacted or grown).
 dcsr_status plan_and_check(dcsr_handle h, UpdBufs &b, int64_t n, hipStream_t s, bool fresh)
@@ -1623,8 +1603,9 @@ dcsr_status plan_and_check(dcsr_handle h, UpdBufs &b, int64_t n, hipStream_t s, 
     const bool table = use_tables(n);
     k_upd_plan<<<ptiles(n), TB, 0, s>>>(h->ds, (unsigned long long)h->pool_cap, b.trow, b.tins, b.tdel, b.ucode, h->row_len,
                                         h->row_cap, h->row_start, b.trs, b.tnewl, b.tmode, b.tmoved, b.tt, b.tp,
-                                        b.pplan, b.fin, table, fresh, b.tlen, b.tcap);
-    if (!table) launch_offsets(h, b, n, s);
+                                        b.pplan, fresh, b.tlen, b.tcap);
+    if (table) k_upd_plan_scan<<<1, TB, 0, s>>>(h->ds, (unsigned long long)h->pool_cap, b.tt, b.tp, b.pplan, ptiles(n));
+    else launch_offsets(h, b, n, s);
     return hipGetLastError() == hipSuccess ? DCSR_OK : DCSR_ERR_HIP;
 }
 
@@ -1654,7 +1635,8 @@ dcsr_status sort_plan_launch(dcsr_handle h, int64_t n, UpdBufs &b, hipStream_t s
     const uint32_t *val = which ? b.v1 : b.v0;
     const unsigned ht = (unsigned)((n + TILE - 1) / TILE);
     const bool table = ht > HEADS_DIRECT_TILES;
-    k_upd_heads_count<<<ht, TB, 0, s>>>(key, n, h->cbits, h->row_len, b.tt, b.tp, b.fin, h->ds, table);
+    k_upd_heads_count<<<ht, TB, 0, s>>>(key, n, h->cbits, h->row_len, b.tt, b.tp);
+    if (table) k_upd_heads_scan<<<1, TB, 0, s>>>(b.tt, b.tp, ht, h->ds);
     k_upd_heads_emit<<<ht, TB, 0, s>>>(key, val, n, h->cbits, b.tt, h->ds, table, b.ucol, b.usum, b.ut, b.trow,
                                        b.tubeg, h->row_len, h->row_start, h->row_cap, b.tp, b.tlpre, b.trs, b.tlen,
                                        b.tcap, b.tins, b.tdel, b.pspan, b.rowt, h->upd_tag);
@@ -1930,13 +1912,6 @@ static dcsr_status update_nosync(dcsr_handle h, const int32_t *rows, const int32
     return DCSR_OK;
 }
 
-namespace {
-__global__ void k_zero_u32(uint32_t *p, int n)
-{
-    for (int i = threadIdx.x; i < n; i += blockDim.x) p[i] = 0;
-}
-}  // namespace
-
 // Bytes of scratch an update of n triples on h carves from a fixed region.
 size_t update_scratch_bytes(dcsr_handle h, int64_t n)
 {
@@ -1950,8 +1925,7 @@ size_t update_scratch_bytes(dcsr_handle h, int64_t n)
 // base + cap) instead of the handle's workspace: nothing is allocated, the
 // pool is never grown or compacted (a batch whose claims do not fit is
 // rejected whole: DCSR_ERR_POOL_EXHAUSTED, or with NOSYNC the sticky bit),
-// and the matrix must be canonical (canonicalizing allocates).  The region's
-// finish counters are cleared first (a fill kernel: safe under capture).
+// and the matrix must be canonical (canonicalizing allocates).
 dcsr_status update_fixed_scratch(dcsr_handle h, const int32_t *rows, const int32_t *cols, const float *vals,
                                  int64_t n, uint32_t flags, hipStream_t s, uint8_t *base, size_t cap)
 {
@@ -1961,7 +1935,6 @@ dcsr_status update_fixed_scratch(dcsr_handle h, const int32_t *rows, const int32
     BufSrc src{h, base, cap, 0, false, s};
     UpdBufs b;
     DCSR_TRY(upd_bufs_src(src, n, b));
-    k_zero_u32<<<1, 64, 0, s>>>(b.fin, 16);
     const bool nosync = (flags & DCSR_UPDATE_NOSYNC) != 0;
     hipStreamCaptureStatus cap_st = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cap_st) == hipSuccess && cap_st != hipStreamCaptureStatusNone) h->flat_replayed = true;
