@@ -152,7 +152,7 @@ struct dcsr_matrix_s {
     int pnl_calls;           // SpMV calls since the last structural change
     int pnl_prev_calls;      // the same for the last structure that had any
     int pnl_count;           // panels in the current copy
-    int64_t pnl_cols;        // panel width (columns)
+    int64_t pnl_cols;        // widest panel (columns)
     int64_t pnl_min_nnz;     // smallest nnz worth a paneled copy
     dcsr_config cfg;
     Workspace ws;

@@ -688,13 +688,13 @@ dcsr_status dcsr_create(dcsr_handle *out, int64_t rows, int64_t cols, const dcsr
     h->hubs_dirty = false;
     h->flat_dirty = true;
     state_exact(h);
-    // SpMV column panels: 1.5M columns (6 MB of x; measured best on a 10M x
-    // 10M power-law matrix among 1M, 1.25M, 1.5M, 2M and 3M with non-temporal
-    // entry loads: 1.91, 1.76, 1.74, 1.80, 2.13 ms) for matrices of at least
-    // 16M entries; both can be overridden for testing
-    h->pnl_cols = 1536 << 10;
+    // SpMV column panels: at most 1.25M columns (5 MB of x; a 10M x 10M
+    // power-law matrix with 160M entries takes 1.56, 1.50, 1.46, 1.53, 1.73 ms
+    // with 0.75M, 1M, 1.25M, 1.5M and 2M) for matrices of at least 8M entries;
+    // both can be overridden for testing
+    h->pnl_cols = 1280 << 10;
     h->pnl_prev_calls = DCSR_PNL_REUSE;  // no evidence yet: a fresh matrix is assumed to be reused
-    h->pnl_min_nnz = 16ll << 20;
+    h->pnl_min_nnz = 8ll << 20;
     if (const char *e = getenv("DCSR_SPMV_PANEL_COLS")) h->pnl_cols = atoll(e) > 0 ? atoll(e) : h->pnl_cols;
     if (const char *e = getenv("DCSR_SPMV_PANEL_MIN_NNZ")) h->pnl_min_nnz = atoll(e) >= 0 ? atoll(e) : h->pnl_min_nnz;
     // the update tag's starting value (a test of its wrap-around)

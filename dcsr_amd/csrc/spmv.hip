@@ -92,10 +92,192 @@ __device__ __forceinline__ float combine(float alpha, float acc, float beta, con
     return beta == 0.0f ? alpha * acc : alpha * acc + beta * y[i];
 }
 
-// Flat kernel for a column block of width KB (1: SpMV, 2 or 4: narrow SpMM).
-// X is row-major with leading dimension ldx, Y with ldy (SpMV: both 1).
-// NT: non-temporal entry loads (ld_entry); on the paneled copy of a
-// 10M-row / 160M-entry matrix 1.87 -> 1.80 ms per SpMV.
+// Flat kernel for one column: y[r * ldy] = alpha * (A X[., 0])_r + beta * y.
+//
+// A wave owns PW1 = 256 entries of the flat order.  The rows that start in
+// them leave a bit each in a 256-bit map and, by their rank among the starts
+// (a ballot count), their pool displacement and row number in a table; slot 0
+// is the row that runs into the range.  An entry's row is then a bit count of
+// the map (two instructions), the loads go 64 entries at a time, and the
+// products pass through LDS so that a lane sums four consecutive ones by
+// itself (in double, rounded once: the error against 64 bits is a tenth below
+// that of a scan over all entries, rms 3.5-3.9e-8 against 4.0-4.4e-8 over
+// 256 to 2.5M rows): one segmented scan over the lanes' open sums serves all
+// 256 entries.
+// The kernel issues about 270 vector instructions per 256 entries where a
+// search of 64 offsets per entry and a scan per 64 took 500 (860 on the
+// paneled copy, whose rows hold two entries each), half and more of its time.
+// Per SpMV, before and after: 1M rows / 16M entries 110 -> 101 us, 325K / 3M
+// 27 -> 23, 10M / 160M (paneled, with the narrower panels) 1695 -> 1330.
+// What is left is the gathers of x (228 G/s from L2, measured).
+//
+// UNIT: ldx == 1.  CONTIG: the entries lie in flat order (the paneled copy),
+// so an entry's slot is its flat index.  WR: rows per lane and window (4 for the
+// paneled copy, whose short rows would take three windows of 64).  NT:
+// non-temporal entry loads (ld_entry); on the paneled copy of a 10M-row /
+// 160M-entry matrix 1.87 -> 1.80 ms per SpMV.
+constexpr uint32_t PW1 = DCSR_SPMV_PW;
+struct Flat1Lds {
+    uint32_t delta[PW1 + 4];  // pool slot less flat index, per start (slot 0: the row running in)
+    uint32_t row[PW1 + 4];
+    float sum[PW1 + 4];       // products, then per start its sum in the wave
+    uint64_t map[PW1 / 64];
+};
+template <bool UNIT, bool CONTIG, int WR, bool NT>
+__global__ __launch_bounds__(TB) void k_flat1(uint32_t R, const uint32_t *__restrict__ foff,
+                                              const uint32_t *__restrict__ rowmap,
+                                              const uint32_t *__restrict__ row_start, const int32_t *__restrict__ col,
+                                              const float *__restrict__ val, const float *__restrict__ X, int64_t ldx,
+                                              float *__restrict__ Y, int64_t ldy, float alpha, float beta,
+                                              uint32_t *__restrict__ carry_row, float *__restrict__ carry_val)
+{
+    constexpr int CH = PW1 / 64;
+    static_assert(CH == 4, "a lane sums four consecutive products");
+    __shared__ __align__(16) Flat1Lds sh[TB / 64];
+    Flat1Lds &S = sh[threadIdx.x >> 6];
+    const uint32_t lane = (uint32_t)lane_id();
+    const uint32_t wave = blockIdx.x * (TB / 64) + (threadIdx.x >> 6);
+    const uint32_t total = foff[R];
+    const uint32_t lastw = total ? (total - 1) / PW1 : 0;
+    if (wave > lastw) {
+        if (lane == 0) carry_row[wave] = NONE;
+        return;
+    }
+    const uint32_t e0 = wave * PW1;
+    const uint32_t e1 = total - e0 < PW1 ? total : e0 + PW1;
+    const bool last = wave == lastw;
+    const uint64_t lt = lanemask_lt();
+    if (lane < CH) S.map[lane] = 0ull;
+    __builtin_amdgcn_wave_barrier();
+    // the rows of the range, WR * 64 at a time (row map granules divide PW1)
+    uint32_t nst = 0, carried = NONE;
+    for (uint32_t j = rowmap[e0 / GRAN];;) {
+        uint32_t rs[WR], re[WR], st[WR];
+#pragma unroll
+        for (int q = 0; q < WR; ++q) {
+            const uint32_t r = j + (uint32_t)q * 64u + lane;
+            rs[q] = foff[r < R ? r : R];
+            re[q] = foff[r < R ? r + 1 : R];
+            st[q] = 0;
+            if constexpr (!CONTIG) st[q] = r < R ? row_start[r] : 0u;
+        }
+#pragma unroll
+        for (int q = 0; q < WR; ++q) {
+            const uint32_t r = j + (uint32_t)q * 64u + lane;
+            const bool starts = re[q] > rs[q] && rs[q] >= e0 && rs[q] < e1;
+            const uint64_t b = __ballot(starts);
+            if (starts) {
+                const uint32_t k = nst + 1u + (uint32_t)__popcll(b & lt);
+                const uint32_t p = rs[q] - e0;
+                if constexpr (!CONTIG) S.delta[k] = st[q] - rs[q];
+                S.row[k] = r;
+                atomicOr(reinterpret_cast<uint32_t *>(S.map) + (p >> 5), 1u << (p & 31u));
+            }
+            nst += (uint32_t)__popcll(b);
+            if (re[q] > e0 && rs[q] < e0) {
+                carried = r;
+                if constexpr (!CONTIG) S.delta[0] = st[q] - rs[q];
+            }
+            // empty rows of the range (and trailing ones)
+            if (r < R && re[q] == rs[q] && ((rs[q] >= e0 && rs[q] < e1) || (last && rs[q] == total))) {
+                const uint64_t i = (uint64_t)r * ldy;
+                Y[i] = beta == 0.0f ? 0.0f : beta * Y[i];
+            }
+        }
+        const uint32_t next = wave_read_lane_u32(re[WR - 1], 63);
+        j += 64u * WR;
+        if (!(next < e1 || (last && j < R))) break;
+    }
+    __builtin_amdgcn_wave_barrier();
+    uint64_t m[CH];
+#pragma unroll
+    for (int u = 0; u < CH; ++u)
+        m[u] = ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(S.map[u] >> 32)) << 32) |
+               (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)S.map[u]);
+    const uint32_t cnt = e1 - e0;
+    uint32_t pre[CH];  // starts before word u
+    pre[0] = 0;
+#pragma unroll
+    for (int u = 1; u < CH; ++u) pre[u] = pre[u - 1] + (uint32_t)__popcll(m[u - 1]);
+    int32_t c[CH];
+    float v[CH], xv[CH];
+#pragma unroll
+    for (int u = 0; u < CH; ++u) {
+        const uint32_t i = (uint32_t)u * 64u + lane;
+        c[u] = 0;
+        v[u] = 0.0f;
+        if (i < cnt) {
+            uint32_t pos = e0 + i;
+            if constexpr (!CONTIG) {
+                // starts at or before the entry
+                const uint64_t w = m[u] >> 1;
+                pos += S.delta[__builtin_amdgcn_mbcnt_hi(
+                    (uint32_t)(w >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)w, pre[u] + (uint32_t)(m[u] & 1ull)))];
+            }
+            c[u] = ld_entry<NT>(&col[pos]);
+            v[u] = ld_entry<NT>(&val[pos]);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < CH; ++u) {
+        xv[u] = 0.0f;
+        if ((uint32_t)u * 64u + lane < cnt) xv[u] = UNIT ? X[c[u]] : X[(int64_t)c[u] * ldx];
+    }
+#pragma unroll
+    for (int u = 0; u < CH; ++u) S.sum[u * 64 + lane] = v[u] * xv[u];
+    __builtin_amdgcn_wave_barrier();
+    // four consecutive products per lane
+    const float4 p4 = *reinterpret_cast<const float4 *>(&S.sum[4 * lane]);
+    const float p[4] = {p4.x, p4.y, p4.z, p4.w};
+    const uint64_t mw = S.map[lane >> 4];
+    const uint32_t sft = (lane & 15u) * 4u;
+    const uint32_t bits = (uint32_t)(mw >> sft) & 15u;
+    const uint32_t kb = (lane < 32 ? (lane < 16 ? pre[0] : pre[1]) : (lane < 48 ? pre[2] : pre[3])) +
+                        (uint32_t)__popcll(mw & ((1ull << sft) - 1ull));
+    __builtin_amdgcn_wave_barrier();  // every product is read before the first sum is stored
+    double acc = 0.0, head = 0.0;  // one rounding per lane and row
+    uint32_t k = kb;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if ((bits >> i) & 1u) {
+            if (k == kb) head = acc;          // ends the row open at the lane's first entry
+            else S.sum[k] = (float)acc;       // a row inside the lane
+            ++k;
+            acc = p[i];
+        } else {
+            acc = acc + p[i];
+        }
+    }
+    // a row that ends inside the next lane takes that lane's share here, so that
+    // the scan's tree covers all of it; lanes with the same k at their end
+    // continue one row
+    const uint64_t eb = (__ballot(bits != 0u) >> 1) | (1ull << 63);  // by every lane
+    const bool ends = (eb >> lane) & 1ull;
+    const float first = (float)head;
+    const float share = __shfl_down(first, 1);
+    if (ends && lane < 63) acc = acc + share;
+    const float run = wave_seg_incl_scan_f32((float)acc, k);
+    if (ends) S.sum[k] = run;
+    if (lane == 0 && bits) S.sum[0] = first;  // the row running in ends in the first lane
+    __builtin_amdgcn_wave_barrier();
+    for (uint32_t i = 1u + lane; i <= nst; i += 64u) {
+        const uint64_t y = (uint64_t)S.row[i] * ldy;
+        Y[y] = combine(alpha, S.sum[i], beta, Y, y);
+    }
+    const uint64_t cb = __ballot(carried != NONE);
+    if (cb) {
+        if (carried != NONE) {
+            carry_row[wave] = carried;
+            carry_val[wave] = S.sum[0];
+        }
+    } else if (lane == 0) {
+        carry_row[wave] = NONE;
+    }
+}
+
+// Flat kernel for a column block of width KB (2 or 4: narrow SpMM).
+// X is row-major with leading dimension ldx, Y with ldy.  NT: non-temporal
+// entry loads (ld_entry).
 template <int KB, bool NT = false>
 __global__ __launch_bounds__(TB) void k_flat(uint32_t R, const uint32_t *__restrict__ foff,
                                              const uint32_t *__restrict__ rowmap,
@@ -817,15 +999,23 @@ __global__ void k_pnl_fill(uint32_t nnz, uint32_t R, int64_t panel, const uint32
     pval[dst] = val[pos];
 }
 
-// y[r] = alpha * (sum of row r's panel partials, in panel order) + beta * y[r]
+// y[r] = alpha * (sum of row r's panel partials) + beta * y[r]; the partials are
+// added in panel order, four at a time in pairs
 __global__ void k_pnl_reduce(uint32_t R, int P, const float *__restrict__ part, float *__restrict__ y, float alpha,
                              float beta)
 {
     const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= R) return;
-    float acc = 0.0f;
-    for (int p = 0; p < P; ++p) acc = acc + part[(uint64_t)p * (R + 1) + r];
-    y[r] = combine(alpha, acc, beta, y, r);
+    double acc = 0.0;  // one rounding for all panels
+    int p = 0;
+    for (; p + 4 <= P; p += 4) {
+        float q[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) q[i] = part[(uint64_t)(p + i) * (R + 1) + r];
+        acc = acc + (((double)q[0] + q[1]) + ((double)q[2] + q[3]));
+    }
+    for (; p < P; ++p) acc = acc + part[(uint64_t)p * (R + 1) + r];
+    y[r] = combine(alpha, (float)acc, beta, y, r);
 }
 
 }  // namespace
@@ -900,7 +1090,15 @@ static dcsr_status launch_flat(dcsr_handle h, const float *X, int64_t ldx, float
     DCSR_TRY(ws_get(h, WS_CARRY_VAL, cap_slots * 4 * KB, (void **)&cval));
     const uint32_t *foff = (const uint32_t *)h->ws.ptr[WS_FOFF];
     const uint32_t *rowmap = (const uint32_t *)h->ws.ptr[WS_ROWMAP];
-    if (stream_entries(h, KB))
+    const bool nt = stream_entries(h, KB);
+    if constexpr (KB == 1) {
+        auto run = [&](auto kernel) {
+            kernel<<<blocks, TB, 0, s>>>(R, foff, rowmap, h->row_start, h->pool_col, h->pool_val, X, ldx, Y, ldy, alpha,
+                                         beta, crow, cval);
+        };
+        if (ldx == 1) nt ? run(k_flat1<true, false, 1, true>) : run(k_flat1<true, false, 1, false>);
+        else nt ? run(k_flat1<false, false, 1, true>) : run(k_flat1<false, false, 1, false>);
+    } else if (nt)
         k_flat<KB, true><<<blocks, TB, 0, s>>>(R, foff, rowmap, h->row_start, h->pool_col, h->pool_val, X, ldx, Y,
                                                ldy, alpha, beta, pw, crow, cval);
     else
@@ -954,19 +1152,31 @@ static dcsr_status prepare_compute(dcsr_handle h, hipStream_t s)
     return ensure_flat(h, s);
 }
 
-// Paneled copy worth building: column-sorted rows, x several panels wide, a
-// large matrix, and the virtual row count within 32 bits.
+// Panels of a matrix: as few as keep them within pnl_cols columns, equally
+// wide (whole 64s).
+static int64_t pnl_panels(dcsr_handle h) { return (h->cols + h->pnl_cols - 1) / h->pnl_cols; }
+static int64_t pnl_width(dcsr_handle h)
+{
+    const int64_t P = pnl_panels(h);
+    return ((h->cols + P - 1) / P + 63) / 64 * 64;
+}
+
+// Paneled copy worth building: column-sorted rows, x past one panel by a
+// quarter, a large matrix, and the virtual row count within 32 bits.  Per SpMV
+// with and without the copy: 1.4M columns / 17M entries 122 / 129 us, 1.7M / 20M
+// 146 / 174, 2M / 8M 78 / 93, 2M / 32M 233 / 315, 3M / 9M 105 / 128, 5M / 20M 227
+// / 305, 10M / 160M 1,427 / 2,601; 1.5M / 6M 58 / 59.
 static bool pnl_eligible(dcsr_handle h)
 {
-    if (!h->state_known || !h->canonical || h->cols < 2 * h->pnl_cols || h->nnz_h < h->pnl_min_nnz) return false;
-    const int64_t P = (h->cols + h->pnl_cols - 1) / h->pnl_cols;
-    return P * (h->rows + 1) < (1ll << 31);
+    if (!h->state_known || !h->canonical || h->cols * 4 < h->pnl_cols * 5 || h->nnz_h < h->pnl_min_nnz) return false;
+    return pnl_panels(h) * (h->rows + 1) < (1ll << 31);
 }
 
 static dcsr_status build_panels(dcsr_handle h, hipStream_t s)
 {
     const int64_t R = h->rows;
-    const int P = (int)((h->cols + h->pnl_cols - 1) / h->pnl_cols);
+    const int P = (int)pnl_panels(h);
+    const int64_t width = pnl_width(h);
     const int64_t Rv = (int64_t)P * (R + 1);
     const int64_t nnz = h->nnz_h;
     uint32_t *poff, *bnd, *pmap, *part;
@@ -984,11 +1194,11 @@ static dcsr_status build_panels(dcsr_handle h, hipStream_t s)
     // per-(panel, row) counts go to the partial buffer (free until the first
     // paneled SpMV), then are scanned into poff
     uint32_t *pcnt = (uint32_t *)ppart;
-    k_pnl_bounds<<<grid_for(R, TB), TB, 0, s>>>((uint32_t)R, P, h->pnl_cols, h->row_start, h->row_len, h->pool_col,
+    k_pnl_bounds<<<grid_for(R, TB), TB, 0, s>>>((uint32_t)R, P, width, h->row_start, h->row_len, h->pool_col,
                                                 pcnt, bnd);
     DCSR_HIP(scan_exclusive_u32(pcnt, poff, Rv, 1, part, poff + Rv, s, fault_word(h)));
     if (nnz > 0)
-        k_pnl_fill<<<grid_for(nnz, TB), TB, 0, s>>>((uint32_t)nnz, (uint32_t)R, h->pnl_cols, foff, rowmap,
+        k_pnl_fill<<<grid_for(nnz, TB), TB, 0, s>>>((uint32_t)nnz, (uint32_t)R, width, foff, rowmap,
                                                     h->row_start, h->pool_col, h->pool_val, poff, bnd, pcol, pval);
     const int64_t ng = nnz / GRAN + 1;
     k_rowmap<<<grid_for(ng, TB), TB, 0, s>>>((uint32_t)Rv, poff, pmap, (uint32_t)ng);
@@ -1018,8 +1228,9 @@ static dcsr_status spmv_paneled(dcsr_handle h, const float *x, float *y, float a
     const int32_t *pcol = (const int32_t *)h->ws.ptr[WS_PNL_COL];
     const float *pval = (const float *)h->ws.ptr[WS_PNL_VAL];
     float *ppart = (float *)h->ws.ptr[WS_PNL_PART];
-    // the copy is contiguous in flat order: a virtual row starts at its offset
-    k_flat<1, true><<<blocks, TB, 0, s>>>(Rv, poff, pmap, poff, pcol, pval, x, 1, ppart, 1, 1.0f, 0.0f, pw, crow, cval);
+    // the copy is contiguous in flat order; its rows hold two entries or so
+    k_flat1<true, true, 4, true><<<blocks, TB, 0, s>>>(Rv, poff, pmap, poff, pcol, pval, x, 1, ppart, 1, 1.0f, 0.0f,
+                                                       crow, cval);
     k_carry<1><<<grid_for(nwaves, TB), TB, 0, s>>>((uint32_t)nwaves, crow, cval, ppart, 1, 1.0f);
     k_pnl_reduce<<<grid_for(R, TB), TB, 0, s>>>((uint32_t)R, P, ppart, y, alpha, beta);
     DCSR_HIP(hipGetLastError());
