@@ -112,37 +112,37 @@ __global__ __launch_bounds__(TB) void k_upd_pack(const int32_t *__restrict__ row
 
 static inline unsigned pack_tiles(int64_t n) { return (unsigned)((n + RADIX_TILE - 1) / RADIX_TILE); }
 
-// Sum of one 32-bit counter over the 256 threads of a block (fixed order).
-__device__ __forceinline__ uint32_t block_sum_u32(uint32_t v, uint32_t *lds4)
-{
-    const uint32_t w = wave_sum_u32(v);
-    if (lane_id() == 0) lds4[threadIdx.x >> 6] = w;
-    __syncthreads();
-    const uint32_t t = lds4[0] + lds4[1] + lds4[2] + lds4[3];
-    __syncthreads();
-    return t;
-}
-
 __device__ __forceinline__ long long wave_sum_i64(long long v)
 {
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
-    return v;
+    // three 32-bit scans across the lanes (DPP) instead of twelve LDS permutes
+    const uint32_t a = wave_sum_u32((uint32_t)v & 0xffffu), b = wave_sum_u32((uint32_t)v >> 16);
+    const uint32_t c = wave_sum_u32((uint32_t)((uint64_t)v >> 32));
+    return (long long)(((uint64_t)c << 32) + ((uint64_t)b << 16) + a);
 }
 
 // ---------------------------------------------------------------------------
-// Tile tables.  The per-element passes work on tiles of 2048 entries (8 per
-// thread, blocked).  Each tile writes its counts to a table; where a batch has
-// too many tiles for every workgroup to sum the counts before its own, a
-// launch of one workgroup turns the table's columns into exclusive offsets,
-// and a later kernel adds them to the in-tile prefixes.  (The last workgroup
-// of the counting launch to finish did that before: the release that each
-// workgroup needs ahead of its finish counter writes its XCD's L2 back, and
-// over the 1,954 tiles of a 4M-triple batch the two counting passes took 47 and
-// 115 us; they take 13 and 40, and the scans 8 and 15.)
+// Tile tables.  The per-element passes work on tiles of two entries per thread.
+// Each tile writes its counts to a table; where a batch has too many tiles for
+// every workgroup to sum the counts before its own, a launch of one workgroup
+// turns the table's columns into exclusive offsets, and a later kernel adds
+// them to the in-tile prefixes.  (The last workgroup of the counting launch to
+// finish did that before: the release that each workgroup needs ahead of its
+// finish counter writes its XCD's L2 back, and over the 1,954 tiles of a
+// 4M-triple batch the two counting passes took 47 and 115 us; they take 12 and
+// 18, and the scans 8 and 15.)
+//
+// Short code and little work per CU are what a pass of a few microseconds is
+// made of: with 256 threads and eight unrolled entries each, heads emit, plan
+// and offsets took 16, 10 and 8 us for 100K triples (17, 19, 19 for 1M; 61, 28,
+// 38 for 4M); with two they take 7, 4 and 6 (17, 9, 13; 41, 18, 20).  Workgroups
+// of 1,024 threads keep the tiles few; up to SPREAD_TILES tiles of a 256-thread
+// workgroup, the smaller ones put a batch's gathers (one line per clock and CU)
+// on more CUs: emit 12.8 -> 6.3 us for 10,300 triples.
 // ---------------------------------------------------------------------------
-constexpr int IPT = 8;
-constexpr int TILE = TB * IPT;
+constexpr int IPT = 2;
+constexpr int SIPT = 8;  // rows per thread of a table scan (TB threads)
+constexpr int TTB_MAX = 1024, TTB_SPREAD = 256;
+constexpr int64_t SPREAD_TILES = TTB_SPREAD;  // a tile's counts per thread
 // Positions of the probe space (touched rows end to end) and of the move
 // space (old entries of rewritten rows end to end) owned by one wave.
 constexpr uint32_t PR_SPAN = 1024;
@@ -164,23 +164,23 @@ __device__ void block_scan_columns(uint32_t *const (&tab)[NC], const int (&src)[
 {
 #pragma unroll
     for (int c = 0; c < NC; ++c) tot[c] = 0;
-    for (int64_t base = 0; base < cnt; base += TILE) {
-        const int64_t i0 = base + (int64_t)threadIdx.x * IPT;
-        uint32_t v[NC][IPT];
+    for (int64_t base = 0; base < cnt; base += TB * SIPT) {
+        const int64_t i0 = base + (int64_t)threadIdx.x * SIPT;
+        uint32_t v[NC][SIPT];
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
 #pragma unroll
-            for (int j = 0; j < IPT; ++j) v[c][j] = i0 + j < cnt ? tab[c][(i0 + j) * 8 + src[c]] : 0u;
+            for (int j = 0; j < SIPT; ++j) v[c][j] = i0 + j < cnt ? tab[c][(i0 + j) * 8 + src[c]] : 0u;
         }
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
             uint32_t sum = 0;
 #pragma unroll
-            for (int j = 0; j < IPT; ++j) sum += v[c][j];
+            for (int j = 0; j < SIPT; ++j) sum += v[c][j];
             uint32_t t;
             uint32_t p = tot[c] + block_excl_scan_256(sum, lds4, &t);
 #pragma unroll
-            for (int j = 0; j < IPT; ++j) {
+            for (int j = 0; j < SIPT; ++j) {
                 if (i0 + j < cnt) tab[c][(i0 + j) * 8 + dst[c]] = p;
                 p += v[c][j];
             }
@@ -189,85 +189,85 @@ __device__ void block_scan_columns(uint32_t *const (&tab)[NC], const int (&src)[
     }
 }
 
-// The thread's IPT blocked keys (~0 past n) and the key before them (~0
-// before item 0: it differs from every valid key and, shifted, from every
-// valid row).
-__device__ __forceinline__ void load_keys(const uint64_t *__restrict__ key, int64_t n, int64_t i0,
-                                          uint64_t (&k)[IPT], uint64_t &prev)
-{
-    // unconditional loads (a tail item reads the last key and becomes ~0),
-    // all in flight together
-    prev = key[i0 > 0 ? (i0 - 1 < n ? i0 - 1 : n - 1) : 0];
-#pragma unroll
-    for (int j = 0; j < IPT; ++j) k[j] = key[i0 + j < n ? i0 + j : n - 1];
-    if (!(i0 > 0 && i0 - 1 < n)) prev = ~0ull;
-#pragma unroll
-    for (int j = 0; j < IPT; ++j)
-        if (i0 + j >= n) k[j] = ~0ull;
-}
-
-// Heads of the sorted batch: an item is a coordinate head if it is the
-// first of its (row, col) run and a row head if the first of its row; items
-// past n and invalid keys (~0) are neither.
-struct HeadFlags {
-    uint32_t h, r;  // bit j: item j of the thread
+// Heads of a tile of the sorted batch: an item is a coordinate head if it is
+// the first of its (row, col) run and a row head if the first of its row; items
+// past n and invalid keys (~0) are neither.  Wave w holds the tile's items from
+// w * 64 * IPT, 64 consecutive ones at a time, so that ranks are ballot counts
+// and the records of one step leave in whole lines without a stop in LDS (48 KB
+// of it per workgroup when a thread held eight consecutive items).
+struct HeadTile {
+    uint64_t k[IPT];
+    uint64_t h[IPT], r[IPT], v[IPT];  // per step: coordinate heads, row heads, valid items
 };
-__device__ __forceinline__ HeadFlags head_flags(const uint64_t (&k)[IPT], uint64_t prev, int cbits)
+template <int TTB>
+__device__ __forceinline__ int64_t head_item(int j)
 {
-    HeadFlags f{0u, 0u};
+    return (int64_t)blockIdx.x * (TTB * IPT) + (threadIdx.x >> 6) * (64 * IPT) + j * 64 + lane_id();
+}
+template <int TTB>
+__device__ __forceinline__ void load_heads(const uint64_t *__restrict__ key, int64_t n, int cbits, HeadTile &T)
+{
+    // unconditional loads (a tail item reads the last key), all in flight
+    uint64_t prev[IPT];
 #pragma unroll
     for (int j = 0; j < IPT; ++j) {
-        const bool valid = k[j] != ~0ull;
-        if (valid && prev != k[j]) f.h |= 1u << j;
-        if (valid && (prev >> cbits) != (k[j] >> cbits)) f.r |= 1u << j;
-        prev = k[j];
+        const int64_t i = head_item<TTB>(j);
+        T.k[j] = key[i < n ? i : n - 1];
+        prev[j] = key[i > 0 && i < n ? i - 1 : 0];
     }
-    return f;
+#pragma unroll
+    for (int j = 0; j < IPT; ++j) {
+        const int64_t i = head_item<TTB>(j);
+        const bool valid = i < n && T.k[j] != ~0ull;
+        T.v[j] = __ballot(valid);
+        T.h[j] = __ballot(valid && (i == 0 || prev[j] != T.k[j]));
+        T.r[j] = __ballot(valid && (i == 0 || (prev[j] >> cbits) != (T.k[j] >> cbits)));
+    }
 }
 
 // Probe length of a touched row: its entries, at least 1 (a row without
 // entries still owns one position, where its records are probed).
 __device__ __forceinline__ uint32_t probe_len(int32_t len) { return len > 1 ? (uint32_t)len : 1u; }
 
-// Sum of the probe lengths of the row heads among the thread's items, and
-// their row lengths (one round trip: every row length is loaded at once).
-__device__ __forceinline__ uint32_t head_rows_len(const uint64_t (&k)[IPT], uint32_t rflags, int cbits,
-                                                  const int32_t *__restrict__ row_len, int32_t (&lj)[IPT])
+// Row lengths of the row heads among the thread's items (0 elsewhere; one
+// round trip: every length is loaded at once).
+__device__ __forceinline__ void head_rows_len(const HeadTile &T, int cbits, const int32_t *__restrict__ row_len,
+                                              int32_t (&lj)[IPT])
 {
-    uint32_t sum = 0;
 #pragma unroll
     for (int j = 0; j < IPT; ++j) {
         lj[j] = 0;
-        if ((rflags >> j) & 1u) lj[j] = row_len[(uint32_t)(k[j] >> cbits)];
+        if ((T.r[j] >> lane_id()) & 1u) lj[j] = row_len[(uint32_t)(T.k[j] >> cbits)];
     }
-#pragma unroll
-    for (int j = 0; j < IPT; ++j) sum += (rflags >> j) & 1u ? probe_len(lj[j]) : 0u;
-    return sum;
 }
 
 // Pass 1 of the heads: per-tile counts (coordinates, touched rows, and the
-// rows' probe lengths).  Pass 2 sums the counts before each tile itself for
-// batches of at most HEADS_DIRECT_TILES tiles; k_upd_heads_scan makes them
-// offsets for larger ones.
-constexpr int64_t HEADS_DIRECT_TILES = 4 * TB;
-__global__ __launch_bounds__(TB) void k_upd_heads_count(const uint64_t *__restrict__ key, int64_t n, int cbits,
+// rows' probe lengths).  Pass 2 sums the counts before each tile itself, a
+// tile per thread; k_upd_heads_scan makes them offsets for batches of more
+// tiles.
+template <int TTB>
+__global__ __launch_bounds__(TTB) void k_upd_heads_count(const uint64_t *__restrict__ key, int64_t n, int cbits,
                                                         const int32_t *__restrict__ row_len,
                                                         uint32_t *__restrict__ tt, uint32_t *__restrict__ tp)
 {
-    __shared__ uint32_t lds4[4];
+    __shared__ uint32_t lds3[TTB / 64][3];
     const int64_t tile = blockIdx.x;
-    uint64_t k[IPT], prev;
-    load_keys(key, n, tile * TILE + (int64_t)threadIdx.x * IPT, k, prev);
-    const HeadFlags f = head_flags(k, prev, cbits);
+    HeadTile T;
+    load_heads<TTB>(key, n, cbits, T);
     int32_t lj[IPT];
-    const uint32_t ls = head_rows_len(k, f.r, cbits, row_len, lj);
-    const uint32_t hc = block_sum_u32(__popc(f.h), lds4);
-    const uint32_t rc = block_sum_u32(__popc(f.r), lds4);
-    const uint32_t lc = block_sum_u32(ls, lds4);
+    head_rows_len(T, cbits, row_len, lj);
+    uint32_t sum[3] = {0, 0, 0};  // heads and row heads: lane 0's, once per wave
+#pragma unroll
+    for (int j = 0; j < IPT; ++j) {
+        sum[0] += lane_id() == 0 ? (uint32_t)__popcll(T.h[j]) : 0u;
+        sum[1] += lane_id() == 0 ? (uint32_t)__popcll(T.r[j]) : 0u;
+        sum[2] += (T.r[j] >> lane_id()) & 1u ? probe_len(lj[j]) : 0u;
+    }
+    block_sum_n<TTB / 64>(sum, lds3);
     if (threadIdx.x == 0) {
-        tt[tile * TT_WORDS + TT_H] = hc;
-        tt[tile * TT_WORDS + TT_R] = rc;
-        tp[tile * TP_WORDS + TP_L] = lc;
+        tt[tile * TT_WORDS + TT_H] = sum[0];
+        tt[tile * TT_WORDS + TT_R] = sum[1];
+        tp[tile * TP_WORDS + TP_L] = sum[2];
     }
 }
 
@@ -292,12 +292,11 @@ __global__ __launch_bounds__(TB) void k_upd_heads_scan(uint32_t *tt, uint32_t *t
 // rowt[row] = rtag << 32 | t, the update's tag beside the row's touched
 // index, for the move kernel's scan of the new row lengths (entries of
 // earlier updates carry older tags).  Sums run left to right from 0 in batch order, as the host path
-// accumulates B_row[j]; a run is summed from the thread's registers and
-// only a run that continues past the thread's items reads memory.  A tile's
-// records are contiguous, so they are staged in LDS and written out
-// coalesced.  The tubeg[ntouched] = nuniq sentinel is stored by workgroup 0
+// accumulates B_row[j]; a run is summed from the tile's items in LDS and
+// only one that continues past them reads memory.  The tubeg[ntouched] = nuniq sentinel is stored by workgroup 0
 // (table) or by the last tile, which then also stores nuniq / ntouched.
-__global__ __launch_bounds__(TB) void k_upd_heads_emit(const uint64_t *__restrict__ key,
+template <int TTB>
+__global__ __launch_bounds__(TTB) void k_upd_heads_emit(const uint64_t *__restrict__ key,
                                                        const uint32_t *__restrict__ val, int64_t n, int cbits,
                                                        const uint32_t *__restrict__ tt, DevState *ds, bool table,
                                                        int32_t *__restrict__ ucol, float *__restrict__ usum,
@@ -312,109 +311,90 @@ __global__ __launch_bounds__(TB) void k_upd_heads_emit(const uint64_t *__restric
                                                        uint32_t *__restrict__ pspan, uint64_t *__restrict__ rowt,
                                                        uint32_t rtag)
 {
-    __shared__ uint32_t lds3[4][3];
-    __shared__ int32_t s_ucol[TILE];
-    __shared__ float s_usum[TILE];
-    __shared__ uint32_t s_ut[TILE], s_trow[TILE], s_tub[TILE], s_tl[TILE];
+    constexpr int TILE = TTB * IPT;
+    __shared__ uint32_t lds6[TTB / 64][6];
+    __shared__ float s_val[TILE];
+    __shared__ uint64_t s_more[TILE / 64];  // items that continue the run before them
     const int64_t tile = blockIdx.x;
-    const int64_t i0 = tile * TILE + (int64_t)threadIdx.x * IPT;
-    // counts of the tiles before this one (loaded with the keys): each
-    // thread sums up to four of them (index clamped to tile 0, masked)
-    uint32_t ch[HEADS_DIRECT_TILES / TB], cr[HEADS_DIRECT_TILES / TB], cl[HEADS_DIRECT_TILES / TB];
-    uint32_t ubase = 0, tbase = 0, lbase = 0;
-    if (table) {
-        ubase = tt[tile * TT_WORDS + TT_HX];
-        tbase = tt[tile * TT_WORDS + TT_RX];
-        lbase = tp[tile * TP_WORDS + TP_LX];
-    } else {
+    const uint32_t lane = (uint32_t)lane_id(), w = threadIdx.x >> 6;
+    const uint64_t lt_mask = lanemask_lt(), le_mask = lt_mask | (1ull << lane);
+    // counts of the tiles before this one (loaded with the keys): a tile per
+    // thread (index clamped to tile 0, masked), or the scanned offsets in thread 0
+    const bool mine = table ? threadIdx.x == 0 : (int64_t)threadIdx.x < tile;
+    const int64_t pt = mine ? (table ? tile : (int64_t)threadIdx.x) : 0;
+    const uint32_t th = tt[pt * TT_WORDS + (table ? TT_HX : TT_H)], tr = tt[pt * TT_WORDS + (table ? TT_RX : TT_R)];
+    const uint32_t tl = tp[pt * TP_WORDS + (table ? TP_LX : TP_L)];
+    HeadTile T;
+    load_heads<TTB>(key, n, cbits, T);
+    float vb[IPT];
 #pragma unroll
-        for (int q = 0; q < HEADS_DIRECT_TILES / TB; ++q) {
-            const int64_t pt = (int64_t)threadIdx.x + q * TB;
-            ch[q] = tt[(pt < tile ? pt : 0) * TT_WORDS + TT_H];
-            cr[q] = tt[(pt < tile ? pt : 0) * TT_WORDS + TT_R];
-            cl[q] = tp[(pt < tile ? pt : 0) * TP_WORDS + TP_L];
-        }
-    }
-    uint64_t k[IPT], prev;
-    load_keys(key, n, i0, k, prev);
-    uint32_t vb[IPT];
-#pragma unroll
-    for (int j = 0; j < IPT; ++j) vb[j] = val[i0 + j < n ? i0 + j : n - 1];
-    const HeadFlags f = head_flags(k, prev, cbits);
+    for (int j = 0; j < IPT; ++j) vb[j] = __uint_as_float(val[head_item<TTB>(j) < n ? head_item<TTB>(j) : n - 1]);
     int32_t lj[IPT];
     uint32_t rsj[IPT], rcj[IPT];
 #pragma unroll
     for (int j = 0; j < IPT; ++j) {
-        const bool rh = (f.r >> j) & 1u;
-        rsj[j] = rh ? row_start[(uint32_t)(k[j] >> cbits)] : 0u;
-        rcj[j] = rh ? (uint32_t)row_cap[(uint32_t)(k[j] >> cbits)] : 0u;
+        const bool rh = (T.r[j] >> lane) & 1u;
+        rsj[j] = rh ? row_start[(uint32_t)(T.k[j] >> cbits)] : 0u;
+        rcj[j] = rh ? (uint32_t)row_cap[(uint32_t)(T.k[j] >> cbits)] : 0u;
     }
-    const uint32_t ls = head_rows_len(k, f.r, cbits, row_len, lj);
-    if (!table) {
-        uint32_t sb[3] = {0, 0, 0};
-#pragma unroll
-        for (int q = 0; q < HEADS_DIRECT_TILES / TB; ++q) {
-            const bool in = (int64_t)threadIdx.x + q * TB < tile;
-            sb[0] += in ? ch[q] : 0u;
-            sb[1] += in ? cr[q] : 0u;
-            sb[2] += in ? cl[q] : 0u;
-        }
-        block_sum_n<3>(sb, lds3);
-        ubase = sb[0];
-        tbase = sb[1];
-        lbase = sb[2];
-    }
-    uint32_t sc[3] = {(uint32_t)__popc(f.h), (uint32_t)__popc(f.r), ls}, stot[3];
-    block_excl_scan_n<3>(sc, lds3, stot);
-    const uint32_t htot = stot[0], rtot = stot[1], ltot = stot[2];
-    uint32_t lu = sc[0], lt = sc[1], ll = sc[2] + lbase;
+    head_rows_len(T, cbits, row_len, lj);
 #pragma unroll
     for (int j = 0; j < IPT; ++j) {
-        if (!((f.h >> j) & 1u)) continue;
-        const bool rh = (f.r >> j) & 1u;
-        float s = 0.0f + __uint_as_float(vb[j]);
-        bool open = true;
+        s_val[w * (64 * IPT) + j * 64 + lane] = vb[j];
+        if (lane == 0) s_more[w * IPT + j] = T.v[j] & ~T.h[j];
+    }
+    // probe lengths before each of the wave's row heads
+    uint32_t lp[IPT], lsum = 0, hc = 0, rc = 0;
 #pragma unroll
-        for (int m = j + 1; m < IPT; ++m) {
-            if (open && k[m] == k[j]) s = s + __uint_as_float(vb[m]);
-            else open = false;
-        }
-        if (open)
-            for (int64_t m = i0 + IPT; m < n && key[m] == k[j]; ++m) s = s + __uint_as_float(val[m]);
-        const uint32_t r = (uint32_t)(k[j] >> cbits);
-        s_ucol[lu] = (int32_t)(k[j] & ((1ull << cbits) - 1ull));
-        s_usum[lu] = s;
-        // a coordinate that is not a row head belongs to the last row head
-        // before it (possibly in an earlier tile)
-        s_ut[lu] = tbase + lt - (rh ? 0u : 1u);
-        if (rh) {
-            s_trow[lt] = r;
-            s_tub[lt] = ubase + lu;
-            s_tl[lt] = ll;
+    for (int j = 0; j < IPT; ++j) {
+        const uint32_t pl = (T.r[j] >> lane) & 1u ? probe_len(lj[j]) : 0u;
+        const uint32_t inc = wave_incl_scan_u32(pl);
+        lp[j] = lsum + inc - pl;
+        lsum += wave_read_lane_u32(inc, 63);
+        hc += (uint32_t)__popcll(T.h[j]);
+        rc += (uint32_t)__popcll(T.r[j]);
+    }
+    // the wave's offsets in the tile (its totals count once, in lane 0) and the
+    // tile's own
+    uint32_t sc[6] = {lane == 0 ? hc : 0u, lane == 0 ? rc : 0u, lane == 0 ? lsum : 0u,
+                      mine ? th : 0u, mine ? tr : 0u, mine ? tl : 0u};
+    uint32_t tot[6];
+    block_excl_scan_n<TTB / 64>(sc, lds6, tot);
+    const uint32_t ubase = tot[3], tbase = tot[4], lbase = tot[5];
+    uint32_t ub = ubase + wave_read_lane_u32(sc[0], 0), tb = tbase + wave_read_lane_u32(sc[1], 0);
+    const uint32_t lb = lbase + wave_read_lane_u32(sc[2], 0);
+#pragma unroll
+    for (int j = 0; j < IPT; ++j) {
+        const uint64_t k = T.k[j];
+        const uint32_t u = ub + (uint32_t)__popcll(T.h[j] & lt_mask);
+        // the last row head up to here (possibly in an earlier tile)
+        const uint32_t t = tb + (uint32_t)__popcll(T.r[j] & le_mask) - 1u;
+        if ((T.r[j] >> lane) & 1u) {
+            const uint32_t r = (uint32_t)(k >> cbits), ll = lb + lp[j];
+            trow[t] = r;
+            tubeg[t] = u;
+            tlpre[t] = ll;
+            trs[t] = rsj[j];
+            tlen[t] = (uint32_t)lj[j];
+            tcap[t] = rcj[j];
+            tins[t] = 0;
+            tdel[t] = 0;
             if (pspan)
-                for (uint32_t k = (ll + PR_SPAN - 1u) / PR_SPAN; k * PR_SPAN < ll + probe_len(lj[j]); ++k)
-                    pspan[k] = tbase + lt;
-            ll += probe_len(lj[j]);
-            trs[tbase + lt] = rsj[j];
-            tlen[tbase + lt] = (uint32_t)lj[j];
-            tcap[tbase + lt] = rcj[j];
-            if (rowt) rowt[r] = ((uint64_t)rtag << 32) | (uint64_t)(tbase + lt);
-            ++lt;
+                for (uint32_t q = (ll + PR_SPAN - 1u) / PR_SPAN; q * PR_SPAN < ll + probe_len(lj[j]); ++q) pspan[q] = t;
+            if (rowt) rowt[r] = ((uint64_t)rtag << 32) | (uint64_t)t;
         }
-        ++lu;
-    }
-    __syncthreads();
-    for (uint32_t i = threadIdx.x; i < htot; i += TB) {
-        ucol[ubase + i] = s_ucol[i];
-        usum[ubase + i] = s_usum[i];
-        ut[ubase + i] = s_ut[i];
-    }
-    for (uint32_t i = threadIdx.x; i < rtot; i += TB) {
-        trow[tbase + i] = s_trow[i];
-        tubeg[tbase + i] = s_tub[i];
-        tlpre[tbase + i] = s_tl[i];
-        tins[tbase + i] = 0;
-        tdel[tbase + i] = 0;
+        if ((T.h[j] >> lane) & 1u) {
+            float s = 0.0f + vb[j];
+            uint32_t m = w * (64 * IPT) + j * 64 + lane + 1;
+            for (; m < TILE && ((s_more[m >> 6] >> (m & 63u)) & 1u); ++m) s = s + s_val[m];
+            if (m == TILE)
+                for (int64_t i = tile * TILE + TILE; i < n && key[i] == k; ++i) s = s + __uint_as_float(val[i]);
+            ucol[u] = (int32_t)(k & ((1ull << cbits) - 1ull));
+            usum[u] = s;
+            ut[u] = t;
+        }
+        ub += (uint32_t)__popcll(T.h[j]);
+        tb += (uint32_t)__popcll(T.r[j]);
     }
     if (threadIdx.x == 0) {
         if (table) {
@@ -423,11 +403,11 @@ __global__ __launch_bounds__(TB) void k_upd_heads_emit(const uint64_t *__restric
                 tlpre[ds->ntouched] = ds->ptotal;
             }
         } else if (tile == gridDim.x - 1) {
-            ds->nuniq = ubase + htot;
-            ds->ntouched = tbase + rtot;
-            ds->ptotal = lbase + ltot;
-            tubeg[tbase + rtot] = ubase + htot;
-            tlpre[tbase + rtot] = lbase + ltot;
+            ds->nuniq = ubase + tot[0];
+            ds->ntouched = tbase + tot[1];
+            ds->ptotal = lbase + tot[2];
+            tubeg[tbase + tot[1]] = ubase + tot[0];
+            tlpre[tbase + tot[1]] = lbase + tot[2];
         }
     }
 }
@@ -731,29 +711,23 @@ __global__ __launch_bounds__(TB) void k_upd_probe(const DevState *__restrict__ d
 // are summed over all ntiles tiles, the claims / moved / inserts / deletes
 // totals come in.  The batch goes ahead only if every index was valid and
 // bump + claims fits the pool; only then does the bump pointer advance.
+template <int NW>
 __device__ void plan_totals_decide(DevState *ds, unsigned long long pool_cap, const long long *__restrict__ pplan,
                                    const uint32_t *__restrict__ tp, int64_t ntiles, uint32_t claim_total,
                                    uint32_t moved_total, uint32_t ins_total, uint32_t del_total,
-                                   long long (*lds)[8])
+                                   long long *tot)
 {
-    long long acc[NPLAN + 1] = {0, 0, 0, 0, 0, 0};
-#pragma unroll 4
-    for (int64_t b = threadIdx.x; b < ntiles; b += TB) {
-#pragma unroll
-        for (int i = 0; i < NPLAN; ++i) acc[i] += pplan[b * NPLAN + i];
-        acc[NPLAN] += tp[b * TP_WORDS + TP_A];
-    }
     __syncthreads();
-#pragma unroll
-    for (int i = 0; i < NPLAN + 1; ++i) {
-        const long long w = wave_sum_i64(acc[i]);
-        if (lane_id() == 0) lds[threadIdx.x >> 6][i] = w;
+    for (int i = (int)(threadIdx.x >> 6); i <= NPLAN; i += NW) {  // a wave per column
+        long long acc = 0;
+#pragma unroll 8
+        for (int64_t b = lane_id(); b < ntiles; b += 64)
+            acc += i < NPLAN ? pplan[b * NPLAN + i] : (long long)tp[b * TP_WORDS + TP_A];
+        acc = wave_sum_i64(acc);
+        if (lane_id() == 0) tot[i] = acc;
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        long long tot[NPLAN + 1];
-#pragma unroll
-        for (int i = 0; i < NPLAN + 1; ++i) tot[i] = (lds[0][i] + lds[1][i]) + (lds[2][i] + lds[3][i]);
         ds->claim_total = claim_total;
         ds->nrewrite_old = moved_total;
         ds->n_ins = ins_total;
@@ -788,7 +762,8 @@ __device__ void plan_totals_decide(DevState *ds, unsigned long long pool_cap, co
 // trip; otherwise (a re-plan after the pool was compacted or grown) they
 // and the row's pool start are re-read from the row table and trs is
 // rewritten.
-__global__ __launch_bounds__(TB) void k_upd_plan(DevState *ds, unsigned long long pool_cap,
+template <int TTB>
+__global__ __launch_bounds__(TTB) void k_upd_plan(DevState *ds, unsigned long long pool_cap,
                                                  const uint32_t *__restrict__ trow, const uint32_t *__restrict__ tins,
                                                  const uint32_t *__restrict__ tdel, const uint32_t *__restrict__ ucode,
                                                  const int32_t *__restrict__ row_len,
@@ -800,15 +775,17 @@ __global__ __launch_bounds__(TB) void k_upd_plan(DevState *ds, unsigned long lon
                                                  uint32_t *__restrict__ tp, long long *__restrict__ pplan, bool fresh,
                                                  const uint32_t *__restrict__ tlen, const uint32_t *__restrict__ tcap)
 {
-    __shared__ long long lds[4][8];
-    __shared__ uint32_t lds44[4][4];
+    constexpr int TILE = TTB * IPT;
+    __shared__ uint32_t lds9[TTB / 64][4 + NPLAN];
     const int64_t tile = blockIdx.x;
     const int64_t t0 = tile * TILE + (int64_t)threadIdx.x * IPT;
     const uint32_t nt = ds->ntouched, nu = ds->nuniq;
-    uint32_t csum = 0, msum = 0;
-    long long v[NPLAN] = {0, 0, 0, 0, 0};
+    // claims, moved, inserts | adds << 16 (each at most TILE), deletes, then the
+    // plan counters: the pool bounds a tile's capacities and the batch the
+    // others, so 32 bits hold them (differences wrap to their sign)
+    uint32_t sums[4 + NPLAN] = {};
     // loads in two phases (row ids, counts and the tile's codes, then row
-    // lengths), so each phase is one memory round trip for all eight rows
+    // lengths), so each phase is one memory round trip
     uint32_t rr[IPT], ti[IPT], td[IPT], rl[IPT], rc[IPT], cd[IPT];
     uint32_t rsv[IPT];
 #pragma unroll
@@ -846,48 +823,38 @@ __global__ __launch_bounds__(TB) void k_upd_plan(DevState *ds, unsigned long lon
         const uint32_t nl = L + ni - nd;
         const uint32_t mode = (ni | nd) ? M_REWRITE : M_VALUES;
         if (mode == M_REWRITE) {
-            csum += chunk_round(nl);
-            msum += L;
-            const int hub_now = nl > DCSR_HUB_LEN, hub_was = L > DCSR_HUB_LEN;
-            v[0] += (long long)nl - (long long)L;
-            v[1] += (long long)cap;
-            v[2] += hub_now - hub_was;
-            v[3] += (hub_now ? ((long long)nl + DCSR_HUB_CHUNK - 1) / DCSR_HUB_CHUNK : 0) -
-                    (hub_was ? ((long long)L + DCSR_HUB_CHUNK - 1) / DCSR_HUB_CHUNK : 0);
-            v[4] += hub_now | hub_was;
+            sums[0] += chunk_round(nl);
+            sums[1] += L;
+            const uint32_t hub_now = nl > DCSR_HUB_LEN, hub_was = L > DCSR_HUB_LEN;
+            sums[4] += nl - L;
+            sums[5] += cap;
+            sums[6] += hub_now - hub_was;
+            sums[7] += (hub_now ? (nl + (DCSR_HUB_CHUNK - 1)) / DCSR_HUB_CHUNK : 0u) -
+                       (hub_was ? (L + (DCSR_HUB_CHUNK - 1)) / DCSR_HUB_CHUNK : 0u);
+            sums[8] += hub_now | hub_was;
         }
         tnewl[t] = nl;
         tmode[t] = mode;
         if (!fresh) trs[t] = rsv[j];
         tmoved[t] = mode == M_REWRITE ? L : 0u;
     }
-    // claims, moved, inserts | adds << 16 (each at most TILE), deletes
-    uint32_t sums[4] = {csum, msum, 0u, 0u};
 #pragma unroll
     for (int j = 0; j < IPT; ++j) {
         sums[2] += (cd[j] == C_INS ? 1u : 0u) + (cd[j] == C_ADD ? 0x10000u : 0u);
         sums[3] += cd[j] == C_DEL ? 1u : 0u;
     }
-    block_sum_n<4>(sums, lds44);
-    csum = sums[0];
-    msum = sums[1];
-    const uint32_t cia = sums[2], cdl = sums[3];
-#pragma unroll
-    for (int i = 0; i < NPLAN; ++i) {
-        const long long w = wave_sum_i64(v[i]);
-        if (lane_id() == 0) lds[threadIdx.x >> 6][i] = w;
-    }
-    __syncthreads();
-    if (threadIdx.x < NPLAN) {
-        const int i = threadIdx.x;
-        pplan[tile * NPLAN + i] = ((lds[0][i] + lds[1][i]) + (lds[2][i] + lds[3][i]));
-    }
+    block_sum_n<TTB / 64>(sums, lds9);
     if (threadIdx.x == 0) {
-        tt[tile * TT_WORDS + TT_C] = csum;
-        tt[tile * TT_WORDS + TT_M] = msum;
-        tp[tile * TP_WORDS + TP_I] = cia & 0xffffu;
-        tp[tile * TP_WORDS + TP_A] = cia >> 16;
-        tp[tile * TP_WORDS + TP_D] = cdl;
+        tt[tile * TT_WORDS + TT_C] = sums[0];
+        tt[tile * TT_WORDS + TT_M] = sums[1];
+        tp[tile * TP_WORDS + TP_I] = sums[2] & 0xffffu;
+        tp[tile * TP_WORDS + TP_A] = sums[2] >> 16;
+        tp[tile * TP_WORDS + TP_D] = sums[3];
+        pplan[tile * NPLAN + 0] = (int32_t)sums[4];
+        pplan[tile * NPLAN + 1] = sums[5];
+        pplan[tile * NPLAN + 2] = (int32_t)sums[6];
+        pplan[tile * NPLAN + 3] = (int32_t)sums[7];
+        pplan[tile * NPLAN + 4] = sums[8];
     }
 }
 
@@ -897,12 +864,12 @@ __global__ __launch_bounds__(TB) void k_upd_plan_scan(DevState *ds, unsigned lon
                                                       uint32_t *tp, const long long *__restrict__ pplan,
                                                       int64_t ntiles)
 {
-    __shared__ long long lds[4][8];
+    __shared__ long long lds[NPLAN + 1];
     __shared__ uint32_t lds4[4];
     uint32_t *const tabs[4] = {tt, tt, tp, tp};
     uint32_t ctot[4];
     block_scan_columns<4>(tabs, {TT_C, TT_M, TP_I, TP_D}, {TT_CX, TT_MX, TP_IX, TP_DX}, ntiles, lds4, ctot);
-    plan_totals_decide(ds, pool_cap, pplan, tp, ntiles, ctot[0], ctot[1], ctot[2], ctot[3], lds);
+    plan_totals_decide<TB / 64>(ds, pool_cap, pplan, tp, ntiles, ctot[0], ctot[1], ctot[2], ctot[3], lds);
 }
 
 // Exclusive offsets per entry: upre[2u], upre[2u+1] = inserts / deletes
@@ -910,7 +877,8 @@ __global__ __launch_bounds__(TB) void k_upd_plan_scan(DevState *ds, unsigned lon
 // tpre[2t], tpre[2t+1] = chunk slots claimed / old entries moved before
 // touched row t (t <= ntouched), from the in-tile prefixes plus the tile
 // offsets; (mspan) touched row t for every move span that starts in it.
-__global__ __launch_bounds__(TB) void k_upd_offsets(DevState *__restrict__ ds,
+template <int TTB>
+__global__ __launch_bounds__(TTB) void k_upd_offsets(DevState *__restrict__ ds,
                                                     const uint32_t *__restrict__ ucode,
                                                     const uint32_t *__restrict__ tmode,
                                                     const uint32_t *__restrict__ tnewl,
@@ -920,26 +888,18 @@ __global__ __launch_bounds__(TB) void k_upd_offsets(DevState *__restrict__ ds,
                                                     const long long *__restrict__ pplan, unsigned long long pool_cap,
                                                     bool table, uint32_t *__restrict__ mspan)
 {
-    __shared__ uint32_t lds44[4][4];
-    __shared__ long long lds[4][8];
+    constexpr int TILE = TTB * IPT;
+    __shared__ uint32_t lds8[TTB / 64][8];
+    __shared__ long long lds[NPLAN + 1];
     const int64_t tile = blockIdx.x;
     const int64_t e0 = tile * TILE + (int64_t)threadIdx.x * IPT;
-    // tile bases: scanned by k_upd_plan_scan (table), or summed
-    // here from the counts of the tiles before this one (loaded with the
-    // entries: up to four tiles per thread, index clamped to tile 0, masked)
-    constexpr int QT = HEADS_DIRECT_TILES / TB;
-    uint32_t qc[QT], qm[QT], qi[QT], qd[QT];
-    if (!table) {
-#pragma unroll
-        for (int q = 0; q < QT; ++q) {
-            const int64_t pt = (int64_t)threadIdx.x + q * TB;
-            const int64_t ix = pt < tile ? pt : 0;
-            qc[q] = tt[ix * TT_WORDS + TT_C];
-            qm[q] = tt[ix * TT_WORDS + TT_M];
-            qi[q] = tp[ix * TP_WORDS + TP_I];
-            qd[q] = tp[ix * TP_WORDS + TP_D];
-        }
-    }
+    // tile bases (claims, moved, inserts, deletes): scanned by k_upd_plan_scan
+    // (table), or summed here from the counts of the tiles before this one
+    // (loaded with the entries: a tile per thread, clamped to tile 0, masked)
+    const bool mine = table ? threadIdx.x == 0 : (int64_t)threadIdx.x < tile;
+    const int64_t bt = mine ? (table ? tile : (int64_t)threadIdx.x) : 0;
+    const uint32_t a[4] = {tt[bt * TT_WORDS + (table ? TT_CX : TT_C)], tt[bt * TT_WORDS + (table ? TT_MX : TT_M)],
+                     tp[bt * TP_WORDS + (table ? TP_IX : TP_I)], tp[bt * TP_WORDS + (table ? TP_DX : TP_D)]};
     const uint32_t nu = ds->nuniq, nt = ds->ntouched;
     uint32_t ins[IPT], del[IPT], cl[IPT], mv[IPT];
     uint32_t code[IPT], md[IPT], nl[IPT];
@@ -968,35 +928,13 @@ __global__ __launch_bounds__(TB) void k_upd_offsets(DevState *__restrict__ ds,
         sc += cl[j];
         sm += mv[j];
     }
-    uint32_t bi, bd, bc, bm;
-    if (table) {
-        bi = tp[tile * TP_WORDS + TP_IX];
-        bd = tp[tile * TP_WORDS + TP_DX];
-        bc = tt[tile * TT_WORDS + TT_CX];
-        bm = tt[tile * TT_WORDS + TT_MX];
-    } else {
-        uint32_t a[4] = {0, 0, 0, 0};
-#pragma unroll
-        for (int q = 0; q < QT; ++q) {
-            const bool in = (int64_t)threadIdx.x + q * TB < tile;
-            a[0] += in ? qi[q] : 0u;
-            a[1] += in ? qd[q] : 0u;
-            a[2] += in ? qc[q] : 0u;
-            a[3] += in ? qm[q] : 0u;
-        }
-        block_sum_n<4>(a, lds44);
-        bi = a[0];
-        bd = a[1];
-        bc = a[2];
-        bm = a[3];
-    }
-    uint32_t sv[4] = {si, sd, sc, sm}, stot[4];
-    block_excl_scan_n<4>(sv, lds44, stot);
-    const uint32_t ti = stot[0], td = stot[1], tc = stot[2], tm = stot[3];
-    si = sv[0] + bi;
-    sd = sv[1] + bd;
-    sc = sv[2] + bc;
-    sm = sv[3] + bm;
+    uint32_t sv[8] = {si, sd, sc, sm, mine ? a[2] : 0u, mine ? a[3] : 0u, mine ? a[0] : 0u, mine ? a[1] : 0u};
+    uint32_t tot[8];
+    block_excl_scan_n<TTB / 64>(sv, lds8, tot);
+    si = sv[0] + tot[4];
+    sd = sv[1] + tot[5];
+    sc = sv[2] + tot[6];
+    sm = sv[3] + tot[7];
 #pragma unroll
     for (int j = 0; j < IPT; ++j) {
         const int64_t e = e0 + j;
@@ -1017,7 +955,8 @@ __global__ __launch_bounds__(TB) void k_upd_offsets(DevState *__restrict__ ds,
     }
     // the last tile knows every total: its bases plus its own counts
     if (!table && tile == gridDim.x - 1)
-        plan_totals_decide(ds, pool_cap, pplan, tp, gridDim.x, bc + tc, bm + tm, bi + ti, bd + td, lds);
+        plan_totals_decide<TTB / 64>(ds, pool_cap, pplan, tp, gridDim.x, tot[6] + tot[2], tot[7] + tot[3], tot[4] + tot[0],
+                                tot[5] + tot[1], lds);
 }
 
 // Move surviving old entries of rewritten rows to their merged positions
@@ -1472,7 +1411,9 @@ __global__ void k_upd_validate_begin(DevState *ds) { ds->ubad = 0; }
 
 
 // Tiles of the per-entry kernels (entries 0..n: index n carries totals).
-static inline unsigned ptiles(int64_t n) { return (unsigned)((n + 1 + TILE - 1) / TILE); }
+static inline bool spread(int64_t n) { return n < SPREAD_TILES * (TTB_SPREAD * IPT); }
+static inline int64_t tile_size(int64_t n) { return (spread(n) ? TTB_SPREAD : TTB_MAX) * IPT; }
+static inline unsigned ptiles(int64_t n) { return (unsigned)((n + 1 + tile_size(n) - 1) / tile_size(n)); }
 
 // Row-group sort plan of a batch of n triples: groups of 2^gshift rows, as
 // few rows per group as keeps the group count within GS_MAX_DIGITS - 1 and
@@ -1531,7 +1472,7 @@ dcsr_status upd_bufs_src(BufSrc &src, int64_t n, UpdBufs &b)
 {
     dcsr_handle h = src.h;
     const size_t n4 = (size_t)(n + 2) * 4, n8 = (size_t)(n + 2) * 8;
-    const size_t nt = ptiles(n);
+    const size_t nt = (size_t)(n + 1 + TTB_MAX * IPT - 1) / (TTB_MAX * IPT);
     sort_plan(h, n, b.lb, b.ndig);
     size_t hw = radix_hist_words(n);
     if (b.lb > 0 && gs_hist_words(n, b.ndig) > hw) hw = gs_hist_words(n, b.ndig);
@@ -1563,6 +1504,15 @@ dcsr_status upd_bufs_src(BufSrc &src, int64_t n, UpdBufs &b)
     DCSR_TRY(take(src, WS_TDEST, nt * TT_WORDS * 4, (void **)&b.tt));
     DCSR_TRY(take(src, WS_PPROBE, nt * TP_WORDS * 4, (void **)&b.tp));
     DCSR_TRY(take(src, WS_PPLAN, nt * NPLAN * 8, (void **)&b.pplan));
+    if (spread(n)) {
+        // the smaller tiles' tables take the place of the sort's, which are no
+        // longer read once the heads are counted (26 words per 512 triples of
+        // at least 64, so the scratch that an update needs stays what it was)
+        static_assert(2 * NPLAN + TT_WORDS + TP_WORDS <= TTB_SPREAD * IPT * 256 / RADIX_TILE, "the tables fit");
+        b.pplan = (long long *)b.hist;
+        b.tt = b.hist + (size_t)ptiles(n) * (2 * NPLAN);
+        b.tp = b.tt + (size_t)ptiles(n) * TT_WORDS;
+    }
     // span tables grow with the matrix, so a fixed region goes without them
     b.pspan = b.mspan = nullptr;
     b.rowt = nullptr;
@@ -1585,13 +1535,21 @@ dcsr_status upd_bufs(dcsr_handle h, int64_t n, UpdBufs &b, hipStream_t s)
 }
 
 // Tile tables are scanned (table) only for batches of more than
-// HEADS_DIRECT_TILES tiles; smaller ones sum them where they are used.
-static inline bool use_tables(int64_t n) { return ptiles(n) > HEADS_DIRECT_TILES; }
+// a tile per thread; smaller ones sum them where they are used.
+static inline bool use_tables(int64_t n) { return ptiles(n) > TTB_MAX; }
+
+// Launches f<TTB> over the tiles of a batch of n, with the workgroup size of
+// its tiles.
+#define LAUNCH_TILES(f, tiles, n, s, ...)                                  \
+    do {                                                                   \
+        if (spread(n)) f<TTB_SPREAD><<<tiles, TTB_SPREAD, 0, s>>>(__VA_ARGS__); \
+        else f<TTB_MAX><<<tiles, TTB_MAX, 0, s>>>(__VA_ARGS__);            \
+    } while (0)
 
 static void launch_offsets(dcsr_handle h, UpdBufs &b, int64_t n, hipStream_t s)
 {
-    k_upd_offsets<<<ptiles(n), TB, 0, s>>>(h->ds, b.ucode, b.tmode, b.tnewl, b.tmoved, b.tt, b.tp, b.upre, b.tpre,
-                                           b.pplan, (unsigned long long)h->pool_cap, use_tables(n), b.mspan);
+    LAUNCH_TILES(k_upd_offsets, ptiles(n), n, s, h->ds, b.ucode, b.tmode, b.tnewl, b.tmoved, b.tt, b.tp, b.upre, b.tpre,
+                 b.pplan, (unsigned long long)h->pool_cap, use_tables(n), b.mspan);
 }
 
 // Plan and decision.  With tile tables their scan decides; without them the
@@ -1601,9 +1559,9 @@ static void launch_offsets(dcsr_handle h, UpdBufs &b, int64_t n, hipStream_t s)
 dcsr_status plan_and_check(dcsr_handle h, UpdBufs &b, int64_t n, hipStream_t s, bool fresh)
 {
     const bool table = use_tables(n);
-    k_upd_plan<<<ptiles(n), TB, 0, s>>>(h->ds, (unsigned long long)h->pool_cap, b.trow, b.tins, b.tdel, b.ucode, h->row_len,
-                                        h->row_cap, h->row_start, b.trs, b.tnewl, b.tmode, b.tmoved, b.tt, b.tp,
-                                        b.pplan, fresh, b.tlen, b.tcap);
+    LAUNCH_TILES(k_upd_plan, ptiles(n), n, s, h->ds, (unsigned long long)h->pool_cap, b.trow, b.tins, b.tdel, b.ucode,
+                 h->row_len, h->row_cap, h->row_start, b.trs, b.tnewl, b.tmode, b.tmoved, b.tt, b.tp, b.pplan, fresh,
+                 b.tlen, b.tcap);
     if (table) k_upd_plan_scan<<<1, TB, 0, s>>>(h->ds, (unsigned long long)h->pool_cap, b.tt, b.tp, b.pplan, ptiles(n));
     else launch_offsets(h, b, n, s);
     return hipGetLastError() == hipSuccess ? DCSR_OK : DCSR_ERR_HIP;
@@ -1633,13 +1591,13 @@ dcsr_status sort_plan_launch(dcsr_handle h, int64_t n, UpdBufs &b, hipStream_t s
         DCSR_HIP(radix_sort_pairs(b.k0, b.v0, b.k1, b.v1, n, nbits, b.hist, b.part, &which, s, true));
     const uint64_t *key = which ? b.k1 : b.k0;
     const uint32_t *val = which ? b.v1 : b.v0;
-    const unsigned ht = (unsigned)((n + TILE - 1) / TILE);
-    const bool table = ht > HEADS_DIRECT_TILES;
-    k_upd_heads_count<<<ht, TB, 0, s>>>(key, n, h->cbits, h->row_len, b.tt, b.tp);
+    const unsigned ht = (unsigned)((n + tile_size(n) - 1) / tile_size(n));
+    const bool table = ht > TTB_MAX;
+    LAUNCH_TILES(k_upd_heads_count, ht, n, s, key, n, h->cbits, h->row_len, b.tt, b.tp);
     if (table) k_upd_heads_scan<<<1, TB, 0, s>>>(b.tt, b.tp, ht, h->ds);
-    k_upd_heads_emit<<<ht, TB, 0, s>>>(key, val, n, h->cbits, b.tt, h->ds, table, b.ucol, b.usum, b.ut, b.trow,
-                                       b.tubeg, h->row_len, h->row_start, h->row_cap, b.tp, b.tlpre, b.trs, b.tlen,
-                                       b.tcap, b.tins, b.tdel, b.pspan, b.rowt, h->upd_tag);
+    LAUNCH_TILES(k_upd_heads_emit, ht, n, s, key, val, n, h->cbits, b.tt, h->ds, table, b.ucol, b.usum, b.ut, b.trow,
+                 b.tubeg, h->row_len, h->row_start, h->row_cap, b.tp, b.tlpre, b.trs, b.tlen,
+                 b.tcap, b.tins, b.tdel, b.pspan, b.rowt, h->upd_tag);
     k_upd_probe<<<probe_blocks(h, n), TB, 0, s>>>(h->ds, h->row_start, h->row_len, h->pool_col, h->pool_val,
                                                   b.tubeg, b.tlpre, b.trs, b.tlen, b.ucol, b.usum, b.uval, b.upos,
                                                   b.ucode, b.tins, b.tdel, b.pspan);

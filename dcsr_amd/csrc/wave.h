@@ -118,50 +118,44 @@ __device__ __forceinline__ uint32_t block_excl_scan_256(uint32_t v, uint32_t *ld
     return carry + inc - v;
 }
 
-// block_excl_scan_256 for N columns at once (one LDS exchange and one pair
-// of barriers for all of them): v[i] becomes the exclusive prefix of column
-// i over the workgroup, tot[i] its total.  lds: [4][N] words.
-template <int N>
+// Exclusive scan of N columns over a workgroup of NW waves (one LDS exchange
+// and one pair of barriers for all of them): v[i] becomes the exclusive prefix
+// of column i, tot[i] its total.  lds: [NW][N] words.  The waves' totals are
+// scanned by a wave, not read out one by one: short code (see TTB, update.hip).
+template <int NW, int N>
 __device__ __forceinline__ void block_excl_scan_n(uint32_t (&v)[N], uint32_t (*lds)[N], uint32_t (&tot)[N])
 {
-    const int w = threadIdx.x >> 6;
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = lane_id();
     uint32_t inc[N];
 #pragma unroll
-    for (int i = 0; i < N; ++i) inc[i] = wave_incl_scan_u32(v[i]);
-    if (lane_id() == 63) {
-#pragma unroll
-        for (int i = 0; i < N; ++i) lds[w][i] = inc[i];
+    for (int i = 0; i < N; ++i) {
+        inc[i] = wave_incl_scan_u32(v[i]);
+        if (lane == 63) lds[w][i] = inc[i];
     }
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < N; ++i) {
-        uint32_t carry = 0, t = 0;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const uint32_t x = lds[q][i];
-            if (q < w) carry += x;
-            t += x;
-        }
-        tot[i] = t;
-        v[i] = carry + inc[i] - v[i];
+        const uint32_t t = lane < NW ? lds[lane][i] : 0u;
+        const uint32_t sc = wave_incl_scan_u32(t);
+        tot[i] = wave_read_lane_u32(sc, 63);
+        v[i] = wave_read_lane_u32(sc - t, w) + inc[i] - v[i];
     }
     __syncthreads();
 }
 
 // Workgroup totals of N columns at once: v[i] becomes column i's total.
-template <int N>
+template <int NW, int N>
 __device__ __forceinline__ void block_sum_n(uint32_t (&v)[N], uint32_t (*lds)[N])
 {
-    uint32_t t[N];
+    const int lane = lane_id();
 #pragma unroll
-    for (int i = 0; i < N; ++i) t[i] = wave_read_lane_u32(wave_incl_scan_u32(v[i]), 63);
-    if (lane_id() == 0) {
-#pragma unroll
-        for (int i = 0; i < N; ++i) lds[threadIdx.x >> 6][i] = t[i];
+    for (int i = 0; i < N; ++i) {
+        const uint32_t t = wave_incl_scan_u32(v[i]);
+        if (lane == 63) lds[threadIdx.x >> 6][i] = t;
     }
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < N; ++i) v[i] = (lds[0][i] + lds[1][i]) + (lds[2][i] + lds[3][i]);
+    for (int i = 0; i < N; ++i) v[i] = wave_sum_u32(lane < NW ? lds[lane][i] : 0u);
     __syncthreads();
 }
 
