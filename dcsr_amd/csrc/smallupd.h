@@ -1,10 +1,10 @@
 // smallupd.h -- sort, heads, probe, plan and offsets of a small update batch
 // in one workgroup (included by update.hip).
 //
-// The update pipeline's passes over tiles of a batch are launches of a few
-// microseconds with a gap between them; below some ten thousand triples the
-// launches and gaps are the time (1,000 triples: nine launches, 56 us of kernels
-// and as much between them; 5,000: 67 us; 10,000: 91 us).
+// The update pipeline's passes over tiles of a batch are launches of four to
+// twelve microseconds each; below some thousands of triples the launches are the
+// time (1,000 triples: 56 us of kernels and as much between them when there
+// were nine; 5,000: 67 us).
 // Here one workgroup of 1,024 threads
 //   1. packs and sorts the triples in LDS: a key's bucket is its place between
 //      the batch's smallest and largest key, buckets are counted by LDS
@@ -17,18 +17,20 @@
 //      not streamed, so its length costs a logarithm) and gives it its code;
 //   4. takes the prefix sums, plans the rows and decides the batch.
 // Up to SMALL_FUSED triples the steps are one launch (17 us for 1,000); above,
-// step 3 runs on the whole device between a launch of steps 1-2 and one of
-// step 4, because one CU's gathers (one line per clock) would take longer than
-// two more launches (5,000 triples: 20 + 6 + 11 us; 10,000 on 1M rows: 64 + 10
-// + 22, where the tiled passes are level).  Every array and DevState field is the pipeline's own, so the move,
-// write and re-plan kernels that follow are the same.
+// steps 1 and 2 are (14 us for 3,000, 25 for 7,000), and the device-wide
+// bisection, plan and offsets passes follow (5 + 4 + 5), because one CU's gathers
+// (one line per clock) would take longer.  Above SMALL_MAX the tiled passes sort
+// and emit in the time that this workgroup needs (a whole update: 72 us for 7,000
+// here, 83 for 7,300 there, 105 for 10,000 in one workgroup).  Every array and
+// DevState field is the pipeline's own, so the move, write and re-plan kernels
+// that follow are the same.
 #pragma once
 
 constexpr int SU_TB = 1024;
 constexpr int SU_NW = SU_TB / 64;
 constexpr int64_t SMALL_FUSED = 2048;
-constexpr int SU_IT_MAX = 10;                               // triples per thread
-constexpr int64_t SMALL_MAX = (int64_t)SU_IT_MAX * SU_TB;   // 10,240: 136 KB of LDS
+constexpr int SU_IT_MAX = 7;                                // triples per thread
+constexpr int64_t SMALL_MAX = (int64_t)SU_IT_MAX * SU_TB;
 constexpr uint32_t SU_CROWD = 64;                           // keys per bucket before the radix sort takes over
 constexpr int SU_RADIX_WORDS = SU_NW * 256;
 
@@ -184,7 +186,7 @@ __device__ __forceinline__ void su_radix_sort(SmallLds<IT> &S, uint32_t n, int b
 
 // Steps 1 and 2.  Returns (every thread) whether the batch is valid; *nu and
 // *nt receive its coordinates and touched rows.
-template <int IT>
+template <int IT, bool FUSED>
 __device__ __forceinline__ bool su_heads(const SmallArgs &A, SmallLds<IT> &S, uint32_t *nu, uint32_t *nt)
 {
     constexpr uint32_t NB = SmallLds<IT>::NB;
@@ -344,6 +346,10 @@ __device__ __forceinline__ bool su_heads(const SmallArgs &A, SmallLds<IT> &S, ui
         if ((rm[j] >> lane) & 1u) {
             A.trow[tt] = r;
             A.tubeg[tt] = u;
+            if constexpr (!FUSED) {
+                A.tins[tt] = 0u;
+                A.tdel[tt] = 0u;
+            }
             if (A.rowt) A.rowt[r] = ((uint64_t)A.rtag << 32) | (uint64_t)tt;
         }
         if ((hm[j] >> lane) & 1u) {
@@ -364,9 +370,13 @@ __device__ __forceinline__ bool su_heads(const SmallArgs &A, SmallLds<IT> &S, ui
     return true;
 }
 
-// Step 3 for coordinates u0 + q * step < nu, PT of them.  A row's first
-// coordinate also records the row's table entry for the later steps.
-template <int PT>
+// Step 3 for coordinates u0 + q * step < nu, PT of them.  FROM: where a row's
+// pool start and length come from and what else is recorded.  P_FUSED: the row
+// table; a row's first coordinate records its entry for step 4.  P_SPLIT: the
+// same, and the rows' insert and delete counts for the plan pass.  P_TILES: the
+// records of the heads pass, and the counts.
+enum { P_FUSED, P_SPLIT, P_TILES };
+template <int PT, int FROM>
 __device__ __forceinline__ void su_probe(const SmallArgs &A, uint32_t u0, uint32_t step, uint32_t nu)
 {
     uint32_t st[PT], len[PT], pos[PT], tq[PT], rq[PT], most = 0;
@@ -387,30 +397,40 @@ __device__ __forceinline__ void su_probe(const SmallArgs &A, uint32_t u0, uint32
             sum[q] = A.usum[u];
         }
     }
-    uint32_t first[PT];
+    if constexpr (FROM == P_TILES) {
 #pragma unroll
-    for (int q = 0; q < PT; ++q) {
-        first[q] = ~0u;
-        if (u0 + (uint32_t)q * step < nu) {
-            rq[q] = A.trow[tq[q]];
-            first[q] = A.tubeg[tq[q]];
+        for (int q = 0; q < PT; ++q) {
+            if (u0 + (uint32_t)q * step < nu) {
+                st[q] = A.trs[tq[q]];
+                len[q] = A.tlen[tq[q]];
+            }
         }
-    }
+    } else {
+        uint32_t first[PT];
 #pragma unroll
-    for (int q = 0; q < PT; ++q) {
-        const uint32_t u = u0 + (uint32_t)q * step;
-        if (u < nu) {
-            st[q] = A.row_start[rq[q]];
-            len[q] = (uint32_t)A.row_len[rq[q]];
-            rq[q] = first[q] == u ? (uint32_t)A.row_cap[rq[q]] : 0u;
+        for (int q = 0; q < PT; ++q) {
+            first[q] = ~0u;
+            if (u0 + (uint32_t)q * step < nu) {
+                rq[q] = A.trow[tq[q]];
+                first[q] = A.tubeg[tq[q]];
+            }
         }
-    }
 #pragma unroll
-    for (int q = 0; q < PT; ++q) {
-        if (first[q] == u0 + (uint32_t)q * step) {
-            A.trs[tq[q]] = st[q];
-            A.tlen[tq[q]] = len[q];
-            A.tcap[tq[q]] = rq[q];
+        for (int q = 0; q < PT; ++q) {
+            const uint32_t u = u0 + (uint32_t)q * step;
+            if (u < nu) {
+                st[q] = A.row_start[rq[q]];
+                len[q] = (uint32_t)A.row_len[rq[q]];
+                rq[q] = first[q] == u ? (uint32_t)A.row_cap[rq[q]] : 0u;
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < PT; ++q) {
+            if (first[q] == u0 + (uint32_t)q * step) {
+                A.trs[tq[q]] = st[q];
+                A.tlen[tq[q]] = len[q];
+                A.tcap[tq[q]] = rq[q];
+            }
         }
     }
 #pragma unroll
@@ -449,6 +469,10 @@ __device__ __forceinline__ void su_probe(const SmallArgs &A, uint32_t u0, uint32
         A.uval[u] = v;
         A.upos[u] = pos[q];
         A.ucode[u] = code;
+        if constexpr (FROM != P_FUSED) {
+            if (code == C_INS) atomicAdd(&A.tins[tq[q]], 1u);
+            else if (code == C_DEL) atomicAdd(&A.tdel[tq[q]], 1u);
+        }
     }
 }
 
@@ -574,51 +598,39 @@ __device__ __forceinline__ void su_plan(const SmallArgs &A, uint32_t nu, uint32_
     }
 }
 
-// A batch with an index outside the matrix: rejected whole.
-__device__ __forceinline__ void su_reject(DevState *ds)
-{
-    ds->nuniq = ds->ntouched = 0;
-    ds->nrewrite_old = 0;
-    ds->ubad = 0;
-    ds->ubad_last = 1;
-    ds->go = 0;
-}
-
+// FUSED: all steps.  Else steps 1 and 2; a batch with an index outside the
+// matrix goes on without coordinates to the decision, which rejects it.
 template <int IT, bool FUSED>
 __global__ __launch_bounds__(SU_TB) void k_upd_small(SmallArgs A)
 {
     __shared__ SmallLds<IT> S;
     uint32_t nu, nt;
-    const bool ok = su_heads<IT>(A, S, &nu, &nt);
+    const bool ok = su_heads<IT, FUSED>(A, S, &nu, &nt);
     if (threadIdx.x == 0) {
-        if (ok) {
-            A.ds->nuniq = nu;
-            A.ds->ntouched = nt;
+        A.ds->nuniq = ok ? nu : 0u;
+        A.ds->ntouched = ok ? nt : 0u;
+        if constexpr (FUSED) {
             A.ds->ubad = 0;
-            A.ds->ubad_last = 0;
-        } else {
-            su_reject(A.ds);
+            A.ds->ubad_last = ok ? 0 : 1;
+            if (!ok) {  // rejected whole
+                A.ds->nrewrite_old = 0;
+                A.ds->go = 0;
+            }
+        } else if (!ok) {
+            A.ds->ubad = 1;
         }
     }
     if constexpr (FUSED) {
         if (!ok) return;
         __syncthreads();
-        su_probe<IT>(A, threadIdx.x, SU_TB, nu);
+        su_probe<IT, P_FUSED>(A, threadIdx.x, SU_TB, nu);
         __syncthreads();
         su_plan<IT>(A, nu, nt, S.lw, S.mm);
     }
 }
 
-__global__ __launch_bounds__(TB) void k_upd_small_probe(SmallArgs A)
+template <int FROM>
+__global__ __launch_bounds__(TB) void k_upd_bisect(SmallArgs A)
 {
-    su_probe<1>(A, blockIdx.x * TB + threadIdx.x, 0u, A.ds->nuniq);
-}
-
-template <int IT>
-__global__ __launch_bounds__(SU_TB) void k_upd_small_plan(SmallArgs A)
-{
-    __shared__ uint32_t lw[SU_NW];
-    __shared__ uint64_t lds64[NPLAN * SU_NW];
-    if (A.ds->ubad_last) return;
-    su_plan<IT>(A, A.ds->nuniq, A.ds->ntouched, lw, lds64);
+    su_probe<1, FROM>(A, blockIdx.x * TB + threadIdx.x, 0u, A.ds->nuniq);
 }

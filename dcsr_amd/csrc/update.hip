@@ -9,11 +9,12 @@
 //
 //   1. pack (row, col) keys (counting the sort's first digit per tile on
 //      the way), stable LSD radix sort of (key, value) pairs;
-//   2. heads (two passes over 2048-entry tiles): one record per distinct
+//   2. heads (two passes over tiles): one record per distinct
 //      coordinate, summed left-to-right in batch order starting from 0 (the
 //      host path's B_row[j] accumulation), one per touched row;
 //   3. probe every distinct coordinate in its (column-sorted) row: existing
-//      -> new = old + sum, removed when == 0; missing -> inserted when != 0;
+//      -> new = old + sum, removed when == 0; missing -> inserted when != 0
+//      (by bisection, or for many coordinates per row by streaming the rows);
 //   4. plan per touched row: rows whose structure is unchanged get their
 //      values written in place; the others claim a new chunk of the pool's
 //      bump region.  Claims are slot offsets from a prefix sum, so no two
@@ -27,8 +28,8 @@
 //
 // Cross-tile prefixes come from per-tile counts, summed where they are used
 // (up to 1,024 tiles) or scanned by a launch of one workgroup; nothing polls.
-// Batches of
-// up to 10,240 triples take steps 1 to 5 in one workgroup (smallupd.h).
+// Batches of up to 2,048 triples take steps 1 to 5 in one workgroup, of up to
+// 7,168 steps 1 and 2 (smallupd.h).
 //
 // dcsr_update is synchronous by default: the batch's status comes back with
 // the call, from one read of the device state (at the end when the host can
@@ -1578,6 +1579,14 @@ static inline unsigned probe_blocks(dcsr_handle h, int64_t n)
     return (unsigned)(b < 1 ? 1 : (b > PR_BLOCKS ? PR_BLOCKS : b));
 }
 
+SmallArgs small_args(dcsr_handle h, int64_t n, UpdBufs &b)
+{
+    return SmallArgs{nullptr, nullptr, nullptr, (uint32_t)n, h->rows, h->cols, h->cbits,
+                     (unsigned long long)h->pool_cap, h->ds, h->row_start, h->row_len, h->row_cap, h->pool_col,
+                     h->pool_val, b.ucol, b.usum, b.uval, b.ut, b.upos, b.ucode, b.upre, b.trow, b.tubeg, b.trs,
+                     b.tlen, b.tcap, b.tins, b.tdel, b.tnewl, b.tmode, b.tmoved, b.tpre, b.mspan, b.rowt, h->upd_tag};
+}
+
 // Sort, heads, probe, plan (+ decision), offsets of a packed batch: the
 // launches shared by every update path (the matrix is only read).  They
 // read and write workspace only, never the caller's triples.
@@ -1598,9 +1607,18 @@ dcsr_status sort_plan_launch(dcsr_handle h, int64_t n, UpdBufs &b, hipStream_t s
     LAUNCH_TILES(k_upd_heads_emit, ht, n, s, key, val, n, h->cbits, b.tt, h->ds, table, b.ucol, b.usum, b.ut, b.trow,
                  b.tubeg, h->row_len, h->row_start, h->row_cap, b.tp, b.tlpre, b.trs, b.tlen,
                  b.tcap, b.tins, b.tdel, b.pspan, b.rowt, h->upd_tag);
-    k_upd_probe<<<probe_blocks(h, n), TB, 0, s>>>(h->ds, h->row_start, h->row_len, h->pool_col, h->pool_val,
-                                                  b.tubeg, b.tlpre, b.trs, b.tlen, b.ucol, b.usum, b.uval, b.upos,
-                                                  b.ucode, b.tins, b.tdel, b.pspan);
+    // A bisection per coordinate takes 36 us per million coordinates and about 5
+    // below 100,000; the pass that streams the touched rows once costs a row, not
+    // a coordinate, and 13 us at least.  With 0.3, 1, 2, 3.1 and 4 coordinates per
+    // row of the matrix (300K to 4M triples): 12, 35, 76, 37, 139 us by bisection,
+    // 20, 42, 101, 27, 87 streamed.
+    if (spread(n) || 2 * n <= 5 * h->rows) {
+        k_upd_bisect<P_TILES><<<grid_for(n, TB), TB, 0, s>>>(small_args(h, n, b));
+    } else {
+        k_upd_probe<<<probe_blocks(h, n), TB, 0, s>>>(h->ds, h->row_start, h->row_len, h->pool_col, h->pool_val,
+                                                      b.tubeg, b.tlpre, b.trs, b.tlen, b.ucol, b.usum, b.uval, b.upos,
+                                                      b.ucode, b.tins, b.tdel, b.pspan);
+    }
     DCSR_HIP(hipGetLastError());
     DCSR_TRY(plan_and_check(h, b, n, s, true));
     if (use_tables(n)) launch_offsets(h, b, n, s);
@@ -1621,21 +1639,19 @@ void launch_pack(dcsr_handle h, const int32_t *rows, const int32_t *cols, const 
 dcsr_status small_launch(dcsr_handle h, const int32_t *rows, const int32_t *cols, const float *vals, int64_t n,
                          UpdBufs &b, hipStream_t s)
 {
-    const SmallArgs A{rows, cols, vals, (uint32_t)n, h->rows, h->cols, h->cbits, (unsigned long long)h->pool_cap, h->ds,
-                      h->row_start, h->row_len, h->row_cap, h->pool_col, h->pool_val, b.ucol, b.usum, b.uval, b.ut,
-                      b.upos, b.ucode, b.upre, b.trow, b.tubeg, b.trs, b.tlen, b.tcap, b.tins, b.tdel, b.tnewl,
-                      b.tmode, b.tmoved, b.tpre, b.mspan, b.rowt, h->upd_tag};
+    SmallArgs A = small_args(h, n, b);
+    A.rows = rows;
+    A.cols = cols;
+    A.vals = vals;
     if (n <= SU_TB) {
         k_upd_small<1, true><<<1, SU_TB, 0, s>>>(A);
     } else if (n <= SMALL_FUSED) {
         k_upd_small<2, true><<<1, SU_TB, 0, s>>>(A);
     } else {
         if (n <= 5 * SU_TB) k_upd_small<5, false><<<1, SU_TB, 0, s>>>(A);
-        else if (n <= 7 * SU_TB) k_upd_small<7, false><<<1, SU_TB, 0, s>>>(A);
         else k_upd_small<SU_IT_MAX, false><<<1, SU_TB, 0, s>>>(A);
-        k_upd_small_probe<<<grid_for(n, TB), TB, 0, s>>>(A);
-        if (n <= 5 * SU_TB) k_upd_small_plan<5><<<1, SU_TB, 0, s>>>(A);
-        else k_upd_small_plan<SU_IT_MAX><<<1, SU_TB, 0, s>>>(A);
+        k_upd_bisect<P_SPLIT><<<grid_for(n, TB), TB, 0, s>>>(A);
+        return plan_and_check(h, b, n, s, true);
     }
     DCSR_HIP(hipGetLastError());
     return DCSR_OK;

@@ -12,10 +12,20 @@ from tests.helpers import assert_same_structure, check_healthy, check_layout, to
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [10_241, 12_799, 12_800, 12_801, 65_536, 131_070, 131_071, 131_072, 133_120, 300_001])
+@pytest.mark.parametrize("n", [7_169, 10_241, 12_799, 12_800, 12_801, 65_536, 131_070, 131_071, 131_072, 133_120, 300_001])
 def test_tiles(n):
+    check(40_003, n)
+
+
+@pytest.mark.parametrize("R,n", [(52_428, 131_072), (52_430, 131_072), (300_007, 140_001)])
+def test_coordinates_per_row(R, n):
+    """Both probes on both sides of five coordinates per two rows."""
+    check(R, n)
+
+
+def check(R, n):
     import dcsr_amd
-    R, C = 40_003, 30_000
+    C = 30_000
     rng = np.random.default_rng(n)
     key = np.unique(rng.integers(0, R, 400_000) * np.int64(C) + rng.integers(0, C, 400_000))
     r, c = (key // C).astype(np.int32), (key % C).astype(np.int32)
