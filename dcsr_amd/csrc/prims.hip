@@ -27,7 +27,7 @@ __global__ void k_fill_u32(uint32_t *p, int64_t n, uint32_t v)
 }
 
 constexpr int SCAN_THREADS = 256;
-constexpr int SCAN_IPT = 8;
+constexpr int SCAN_IPT = 16;
 constexpr int SCAN_TILE = SCAN_THREADS * SCAN_IPT;
 
 // Single-pass exclusive scan of NC interleaved components: tile = ticket,
@@ -46,7 +46,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_scan1(const uint32_t *__restri
     unsigned int *ctl = part;
     uint64_t *st = (uint64_t *)(part + 4);
     uint32_t tag;
-    const int64_t tile = lb_ticket(ctl, s_ticket, &tag);
+    const int64_t tile = lb_ticket(ctl, s_ticket, &tag, gridDim.x);
     const int64_t ntiles = (n + SCAN_TILE - 1) / SCAN_TILE;
     const int64_t base = tile * SCAN_TILE;
     // all loads in flight first (a tail item reads the tile's first element
@@ -97,8 +97,6 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_scan1(const uint32_t *__restri
             if (idx < n) out[idx * NC + c] = p + tile_s[c][i * SCAN_THREADS + threadIdx.x];
         }
     }
-    __syncthreads();
-    if (threadIdx.x == 0) lb_finish(ctl);
 }
 
 // ---------------------------------------------------------------------------

@@ -37,8 +37,7 @@ struct RowScanLds {
 // threads.  lens(r0, full, v) loads the lengths of rows r0 .. r0+15 (full:
 // all of them exist; else rows past R read 0); prefix(n) is the exact sum of
 // the lengths of rows [0, n) by one whole wave (the look-back fallback).
-// ntiles: the workgroups that run this function in the launch (the last one
-// to finish resets the control words).
+// ntiles: the workgroups that run this function in the launch.
 template <class Lens, class Prefix>
 __device__ void rowscan_tile(uint32_t R, Lens &&lens, Prefix &&prefix, uint32_t *__restrict__ foff,
                              uint32_t *__restrict__ rowmap, uint32_t *__restrict__ part, unsigned int *fault,
@@ -47,7 +46,7 @@ __device__ void rowscan_tile(uint32_t R, Lens &&lens, Prefix &&prefix, uint32_t 
     unsigned int *ctl = part;
     uint64_t *st = (uint64_t *)(part + 4);
     uint32_t tag;
-    const int64_t tile = lb_ticket(ctl, L.tk, &tag);
+    const int64_t tile = lb_ticket(ctl, L.tk, &tag, ntiles);
     const int64_t r0 = tile * RS_TILE + (int64_t)threadIdx.x * RS_IPT;
     const bool full = r0 + RS_IPT <= (int64_t)R;
     uint32_t v[RS_IPT];
@@ -108,6 +107,4 @@ __device__ void rowscan_tile(uint32_t R, Lens &&lens, Prefix &&prefix, uint32_t 
     // the thread holding row R-1 stores the total
     if (r0 < (int64_t)R && r0 + RS_IPT >= (int64_t)R) foff[R] = a;
     if (tile == 0 && threadIdx.x == 0) rowmap[0] = 0u;
-    __syncthreads();
-    if (threadIdx.x == 0) lb_finish_n(ctl, ntiles);
 }
