@@ -13,12 +13,9 @@
 //      contiguously, in arrival order (digits ranked by wave ballots, staged
 //      in LDS so runs are written together);
 //   3. k_gs_sort: one workgroup per group sorts the group's pairs by their
-//      low lb key bits (all of its keys share the bits above), a stable LSD
-//      sort with 8- or 9-bit digits (whichever takes fewer passes); groups of
-//      up to GS_CAP pairs sort in LDS (one 32-bit word per pair where the
-//      local key's unranked bits and the pair's position fit one, else a
-//      key and a position array), larger ones out of global memory with the
-//      same ranking.
+//      low lb key bits (all of its keys share the bits above): groups of up to
+//      GS_CAP pairs in LDS by buckets, larger ones out of global memory by
+//      stable LSD passes.
 //
 // The result is exactly the stable sort of the batch by key, which the LSD
 // radix sort (prims.hip) gives in one count/scan/scatter round per 8 key
@@ -30,8 +27,8 @@
 
 namespace {
 
-constexpr int GT = 256;              // threads of the scan-free kernels
-constexpr int GIPT = 8;              // pairs per lane in a scatter tile
+constexpr int GT = 512;              // threads of the scatter
+constexpr int GIPT = 4;              // pairs per lane in a scatter tile
 constexpr int GTILE = GT * GIPT;     // 2048 == RADIX_TILE
 static_assert(GTILE == RADIX_TILE, "pack counts tiles of the scatter's size");
 constexpr int GS_SCAN_T = 1024;      // k_gs_scan: 16 waves per 64 digits
@@ -102,18 +99,20 @@ __global__ __launch_bounds__(GS_SCAN_T) void k_gs_scan(uint32_t *__restrict__ hi
 
 // Stable scatter of one 2048-pair tile into the group order.  gbase_out
 // (block 0) receives the exclusive offsets of the ndig digits plus the total.
+// A tile's ranking is a serial chain per wave, so eight waves take four pairs per
+// lane (four took eight: 22.7 us for 1M triples, 8.6 for 100K; now 19.7 and 6.4).
 __global__ __launch_bounds__(GT) void k_gs_scatter(const uint64_t *__restrict__ kin, const uint32_t *__restrict__ vin,
                                                    uint64_t *__restrict__ kout, uint32_t *__restrict__ vout,
                                                    int64_t n, int lb, int ndig, int dbits,
                                                    const uint32_t *__restrict__ hist, int64_t nb,
                                                    const uint32_t *__restrict__ dtot, uint32_t *__restrict__ gbase_out)
 {
-    __shared__ uint32_t wcnt[GT / 64][GS_MAX_DIGITS];
+    __shared__ uint16_t wcnt[GT / 64][GS_MAX_DIGITS];  // at most a tile
     __shared__ uint32_t lofs[GS_MAX_DIGITS];
     __shared__ uint32_t gofs[GS_MAX_DIGITS];
     __shared__ uint64_t skey[GTILE];
     __shared__ uint32_t sval[GTILE];
-    __shared__ uint32_t lds4[4];
+    __shared__ uint32_t lds2[GT / 64][2];
     constexpr int DPT = GS_MAX_DIGITS / GT;  // digits per thread in the offset phase
     const int w = threadIdx.x >> 6, lane = lane_id();
     const int64_t tile = blockIdx.x;
@@ -156,7 +155,7 @@ __global__ __launch_bounds__(GT) void k_gs_scatter(const uint64_t *__restrict__ 
         // every lane of the digit reads its count before the leader adds to
         // it (a wave's LDS accesses complete in order): no broadcast needed
         const uint32_t b = wcnt[w][d];
-        if (lane == leader) wcnt[w][d] = b + (uint32_t)__popcll(peers);
+        if (lane == leader) wcnt[w][d] = (uint16_t)(b + (uint32_t)__popcll(peers));
         rnk[j] = b + (uint32_t)__popcll(peers & lt);
         dg[j] = d;
     }
@@ -172,7 +171,7 @@ __global__ __launch_bounds__(GT) void k_gs_scatter(const uint64_t *__restrict__ 
 #pragma unroll
                 for (int i = 0; i < GT / 64; ++i) {
                     const uint32_t x = wcnt[i][d];
-                    wcnt[i][d] = c;
+                    wcnt[i][d] = (uint16_t)c;
                     c += x;
                 }
             }
@@ -181,9 +180,9 @@ __global__ __launch_bounds__(GT) void k_gs_scatter(const uint64_t *__restrict__ 
             gs[q] = gsum;
             gsum += dt[q];
         }
-        uint32_t tot;
-        const uint32_t lp = block_excl_scan_256(csum, lds4, &tot);
-        const uint32_t gp = block_excl_scan_256(gsum, lds4, &tot);
+        uint32_t pre[2] = {csum, gsum}, tot[2];
+        block_excl_scan_n<GT / 64>(pre, lds2, tot);
+        const uint32_t lp = pre[0], gp = pre[1];
 #pragma unroll
         for (int q = 0; q < DPT; ++q) {
             const int d = d0 + q;
@@ -193,7 +192,7 @@ __global__ __launch_bounds__(GT) void k_gs_scatter(const uint64_t *__restrict__ 
                 if (tile == 0) gbase_out[d] = gp + gs[q];
             }
         }
-        if (tile == 0 && threadIdx.x == 0) gbase_out[ndig] = tot;
+        if (tile == 0 && threadIdx.x == 0) gbase_out[ndig] = tot[1];
     }
     __syncthreads();
 #pragma unroll
@@ -225,20 +224,22 @@ __global__ __launch_bounds__(GT) void k_gs_scatter(const uint64_t *__restrict__ 
 // wcnt[w][d] = items of digit d in waves before w, loff[d] = items of the
 // chunk with a smaller digit, cnt_out[d] (if not null) = items of digit d.
 // ---------------------------------------------------------------------------
-constexpr int SJ = GS_CAP / GT;  // items per lane in a full LDS group
+constexpr int ST = 512;          // threads of a group's workgroup
+constexpr int SNW = ST / 64;
+constexpr int SJ = GS_CAP / ST;  // items per lane in a full LDS group
+constexpr int SD_BITS = 9;       // digits of the stable passes: one per thread
+constexpr int SD = 1 << SD_BITS;
+static_assert(SD == ST && GS_CAP % ST == 0, "a digit per thread");
 
-template <int J, int DB = 8, typename C = uint32_t>
+template <int J>
 __device__ __forceinline__ void rank_chunk(const uint32_t (&dg)[J], const bool (&real)[J], int jmax,
-                                           uint32_t (&rnk)[J], C (*wcnt)[1 << DB], uint32_t *loff,
-                                           uint32_t *lds4)
+                                           uint32_t (&rnk)[J], uint16_t (*wcnt)[SD], uint32_t *loff,
+                                           uint32_t (*lds)[1])
 {
-    constexpr int ND = 1 << DB;     // digits
-    constexpr int DPT = ND / GT;    // digits per thread in the offset scan
-    static_assert(DPT >= 1 && ND % GT == 0, "at least one digit per thread");
     const int w = threadIdx.x >> 6, lane = lane_id();
     const uint64_t lt = lanemask_lt();
 #pragma unroll
-    for (int i = 0; i < ND / 64; ++i) wcnt[w][lane + 64 * i] = 0;
+    for (int i = 0; i < SD / 64; ++i) wcnt[w][lane + 64 * i] = 0;
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
     for (int j = 0; j < J; ++j) {
@@ -248,7 +249,7 @@ __device__ __forceinline__ void rank_chunk(const uint32_t (&dg)[J], const bool (
         if (!real[j]) continue;
         uint64_t peers = act;
 #pragma unroll
-        for (int b = 0; b < DB; ++b) {
+        for (int b = 0; b < SD_BITS; ++b) {
             const uint64_t m = __ballot((dg[j] >> b) & 1u);
             peers &= ((dg[j] >> b) & 1u) ? m : ~m;
         }
@@ -256,210 +257,239 @@ __device__ __forceinline__ void rank_chunk(const uint32_t (&dg)[J], const bool (
         // every lane of the digit reads its count before the leader adds to
         // it (a wave's LDS accesses complete in order): no broadcast needed
         const uint32_t c = wcnt[w][dg[j]];
-        if (lane == leader) wcnt[w][dg[j]] = (C)(c + (uint32_t)__popcll(peers));
+        if (lane == leader) wcnt[w][dg[j]] = (uint16_t)(c + (uint32_t)__popcll(peers));
         rnk[j] = c + (uint32_t)__popcll(peers & lt);
     }
     __syncthreads();
-    {
-        // digits threadIdx.x * DPT .. + DPT - 1 (contiguous: the scan stays
-        // in digit order)
-        uint32_t sd[DPT], st = 0;
+    uint32_t s[1] = {0}, tot[1];
 #pragma unroll
-        for (int k = 0; k < DPT; ++k) {
-            const int d = threadIdx.x * DPT + k;
-            uint32_t s = 0;
-#pragma unroll
-            for (int i = 0; i < GT / 64; ++i) {
-                const uint32_t x = wcnt[i][d];
-                wcnt[i][d] = (C)s;
-                s += x;
-            }
-            sd[k] = s;
-            st += s;
-        }
-        uint32_t tot;
-        uint32_t pre = block_excl_scan_256(st, lds4, &tot);
-#pragma unroll
-        for (int k = 0; k < DPT; ++k) {
-            loff[threadIdx.x * DPT + k] = pre;
-            pre += sd[k];
-        }
+    for (int i = 0; i < SNW; ++i) {
+        const uint32_t x = wcnt[i][threadIdx.x];
+        wcnt[i][threadIdx.x] = (uint16_t)s[0];
+        s[0] += x;
     }
+    block_excl_scan_n<SNW>(s, lds, tot);
+    loff[threadIdx.x] = s[0];
     __syncthreads();
 }
 
-// LDS sort of cnt <= GS_CAP pairs of group g: keys (local bits) and the
-// pairs' indices ping-pong between two LDS arrays; digits of DB bits (9 when
-// that takes fewer passes over the lb local bits than 8).
-template <typename K, int DB>
+// LDS sort of n <= GS_CAP pairs of a group.  A pair is one word, its local key
+// above its position in the group (GS_POS bits: ties keep their arrival order).
+//
+// A key's bucket is its top GS_NBB local bits.  Buckets are counted by LDS
+// atomics, their starts scanned, the words placed in bucket order, and a pair is
+// ranked among its own bucket's words.  Keys and values stay in registers and go
+// straight to their places.  The ranking's LDS reads are the cost (they conflict:
+// a microsecond for every two words in the fullest bucket with the chip's groups
+// in flight), so where a bucket holds more than GS_FEW pairs every bucket is
+// split first; a group that still has more than GS_CROWD pairs in a part (a
+// coordinate repeated, columns that crowd) takes stable digit passes.
+// For 10,000, 100,000 and 1M triples spread over 1M rows the groups take 5.2, 6
+// and 19 us; in digit passes alone (nine ballots per pair and pass, three to five
+// passes) 12, 13 and 30.  1M power-law triples on 325K rows: 23 and 26.
+constexpr int GS_POS = 12;  // position bits (GS_CAP <= 4096)
+static_assert(GS_CAP <= (1 << GS_POS), "a position fits its field");
+constexpr int GS_NBB = 11;
+constexpr int GS_NB = 1 << GS_NBB;
+constexpr uint32_t GS_FEW = 6;     // pairs in a bucket before the buckets are split
+constexpr uint32_t GS_CROWD = 64;  // pairs in a part before the digit passes
+constexpr uint32_t GS_PARTS = 2 * GS_CAP + GS_NB;
+static_assert(GS_PARTS / 2 + 1 <= 2 * GS_CAP && GS_PARTS % (2 * ST) == 0, "16-bit part counters fit the words");
+
 struct GsLds {
-    K key[2][GS_CAP];
-    uint16_t idx[2][GS_CAP];
-    uint32_t wcnt[GT / 64][1 << DB];
-    uint32_t loff[1 << DB];
-    uint32_t lds4[4];
+    uint64_t word[GS_CAP];
+    union {
+        uint32_t start[GS_NB + 1];
+        struct {
+            uint16_t wcnt[SNW][SD];
+            uint32_t loff[SD];
+        } r;
+    };
+    uint32_t lds[SNW][1];
 };
 
-template <typename K, int DB>
-__device__ void group_sort_lds(GsLds<K, DB> &S, const uint64_t *__restrict__ kin, const uint32_t *__restrict__ vin,
-                               uint64_t *__restrict__ kout, uint32_t *__restrict__ vout, int64_t s0, int cnt, int lb,
-                               uint64_t high)
+// A crowded group of n pairs (lb + GS_POS <= 64): digit passes over its words.
+__device__ void group_sort_crowded(GsLds &S, const uint64_t *__restrict__ kin, const uint32_t *__restrict__ vin,
+                                   uint64_t *__restrict__ kout, uint32_t *__restrict__ vout, uint32_t n, int lb)
 {
-    const int w = threadIdx.x >> 6, lane = lane_id();
-    const uint64_t lmask = lb >= 64 ? ~0ull : ((1ull << lb) - 1ull);
-    // every key load in flight before the first store (indices clamped into
-    // the group, extra items dropped)
-    {
-        uint64_t kl[SJ];
-#pragma unroll
-        for (int j = 0; j < SJ; ++j) {
-            const int i = j * GT + threadIdx.x;
-            kl[j] = kin[s0 + (i < cnt ? i : cnt - 1)];
-        }
-#pragma unroll
-        for (int j = 0; j < SJ; ++j) {
-            const int i = j * GT + threadIdx.x;
-            if (i < cnt) {
-                S.key[0][i] = (K)(kl[j] & lmask);
-                S.idx[0][i] = (uint16_t)i;
-            }
-        }
-    }
+    const uint64_t lmask = (1ull << lb) - 1ull;
+    const int cnt = (int)n;
+    for (uint32_t i = threadIdx.x; i < n; i += ST) S.word[i] = ((kin[i] & lmask) << GS_POS) | (uint64_t)i;
     __syncthreads();
-    // positions per wave: a multiple of 64 covering cnt / 4
-    const int jmax = (cnt + GT - 1) / GT;
-    const int pw = jmax * 64;
-    int cur = 0;
-    for (int sh = 0; sh < lb; sh += DB) {
-        // only the ranks stay in registers; keys are read again from LDS for
-        // the scatter
+    const int w = threadIdx.x >> 6, lane = lane_id();
+    const int jmax = (cnt + ST - 1) / ST, pw = jmax * 64;  // positions per wave
+    for (int sh = GS_POS; sh < lb + GS_POS; sh += SD_BITS) {
         uint32_t dg[SJ], rnk[SJ];
+        uint64_t wd[SJ];
         bool real[SJ];
 #pragma unroll
         for (int j = 0; j < SJ; ++j) {
             const int p = w * pw + j * 64 + lane;
             real[j] = j < jmax && p < cnt;
-            dg[j] = real[j] ? (uint32_t)(S.key[cur][p] >> sh) & ((1u << DB) - 1u) : 0u;
+            wd[j] = real[j] ? S.word[p] : 0ull;
+            dg[j] = (uint32_t)(wd[j] >> sh) & (SD - 1u);
         }
-        rank_chunk<SJ, DB>(dg, real, jmax, rnk, S.wcnt, S.loff, S.lds4);
+        rank_chunk<SJ>(dg, real, jmax, rnk, S.r.wcnt, S.r.loff, S.lds);  // its barriers: every word is read
 #pragma unroll
-        for (int j = 0; j < SJ; ++j) {
-            if (!real[j]) continue;
-            const int p = w * pw + j * 64 + lane;
-            const uint32_t q = S.loff[dg[j]] + S.wcnt[w][dg[j]] + rnk[j];
-            S.key[cur ^ 1][q] = S.key[cur][p];
-            S.idx[cur ^ 1][q] = S.idx[cur][p];
-        }
+        for (int j = 0; j < SJ; ++j)
+            if (real[j]) S.word[S.r.loff[dg[j]] + S.r.wcnt[w][dg[j]] + rnk[j]] = wd[j];
         __syncthreads();
-        cur ^= 1;
     }
-    // the value gather: every load in flight before the first store
-    uint32_t vv[SJ];
-#pragma unroll
-    for (int j = 0; j < SJ; ++j) {
-        const int i = j * GT + threadIdx.x;
-        vv[j] = vin[s0 + (i < cnt ? S.idx[cur][i] : 0)];
-    }
-#pragma unroll
-    for (int j = 0; j < SJ; ++j) {
-        const int i = j * GT + threadIdx.x;
-        if (i < cnt) {
-            kout[s0 + i] = high | (uint64_t)S.key[cur][i];
-            vout[s0 + i] = vv[j];
-        }
+    for (uint32_t i = threadIdx.x; i < n; i += ST) {
+        const uint32_t src = (uint32_t)S.word[i] & ((1u << GS_POS) - 1u);
+        kout[i] = kin[src];
+        vout[i] = vin[src];
     }
 }
 
-// LDS sort of cnt <= GS_CAP pairs of a group whose local keys have at most
-// GS_PK_BITS + DB bits: one 32-bit word per pair and pass, the key bits not
-// yet ranked above the pair's position in the group (GS_PK_POS bits).  The
-// first pass ranks the digits straight from the loaded keys; the last one
-// leaves the positions in sorted order, and each pair's key and value are
-// gathered from the group's input by position.  Half the LDS of the
-// two-array sort (16-bit per-wave digit counts too): five workgroups fit a
-// CU, so the bench-sized batch of ~1,270 groups runs in one round.
-constexpr int GS_PK_POS = 12;                 // position bits (GS_CAP <= 4096)
-constexpr int GS_PK_BITS = 32 - GS_PK_POS;    // key bits a word carries
-static_assert(GS_CAP <= (1 << GS_PK_POS), "a position fits its field");
-static_assert(GS_CAP <= 65535, "16-bit digit counts");
-
-template <int DB>
-struct GsPacked {
-    uint32_t w[2][GS_CAP];
-    uint16_t wcnt[GT / 64][1 << DB];
-    uint32_t loff[1 << DB];
-    uint32_t lds4[4];
-};
-
-template <int DB>
-__device__ void group_sort_packed(GsPacked<DB> &S, const uint64_t *__restrict__ kin,
-                                  const uint32_t *__restrict__ vin, uint64_t *__restrict__ kout,
-                                  uint32_t *__restrict__ vout, int64_t s0, int cnt, int lb)
+// Returns (every thread) false, with nothing written, for a crowded group.
+__device__ bool group_sort_lds(GsLds &S, const uint64_t *__restrict__ kin, const uint32_t *__restrict__ vin,
+                               uint64_t *__restrict__ kout, uint32_t *__restrict__ vout, uint32_t n, int lb)
 {
-    constexpr uint32_t DM = (1u << DB) - 1u;
-    constexpr uint32_t PM = (1u << GS_PK_POS) - 1u;
-    const int w = threadIdx.x >> 6, lane = lane_id();
     const uint64_t lmask = (1ull << lb) - 1ull;
-    // positions per wave: a multiple of 64 covering cnt / 4; item j of a
-    // lane sits at w * pw + 64 j + lane in every pass
-    const int jmax = (cnt + GT - 1) / GT;
-    const int pw = jmax * 64;
-    uint32_t dg[SJ], rnk[SJ], wd[SJ];
-    bool real[SJ];
-    {
-        uint64_t kl[SJ];
+    const int bs = lb > GS_NBB ? lb - GS_NBB : 0;  // key bits below the bucket's
+    const uint64_t rest = (1ull << bs) - 1ull;
+    // every load in flight before the first use (indices clamped into the group)
+    uint64_t k[SJ];
+    uint32_t v[SJ];
 #pragma unroll
-        for (int j = 0; j < SJ; ++j) {
-            const int p = w * pw + j * 64 + lane;
-            real[j] = j < jmax && p < cnt;
-            kl[j] = real[j] ? kin[s0 + p] : 0ull;
-        }
-#pragma unroll
-        for (int j = 0; j < SJ; ++j) {
-            const uint64_t lk = kl[j] & lmask;
-            dg[j] = (uint32_t)lk & DM;
-            wd[j] = ((uint32_t)(lk >> DB) << GS_PK_POS) | (uint32_t)(w * pw + j * 64 + lane);
-        }
+    for (int j = 0; j < SJ; ++j) {
+        const uint32_t i = j * ST + threadIdx.x;
+        if (j * ST >= n) break;
+        k[j] = kin[i < n ? i : n - 1];
+        v[j] = vin[i < n ? i : n - 1];
     }
-    int cur = 0;
-    for (int sh = 0;; sh += DB) {
-        rank_chunk<SJ, DB, uint16_t>(dg, real, jmax, rnk, S.wcnt, S.loff, S.lds4);
+    for (int i = threadIdx.x; i < GS_NB; i += ST) S.start[i] = 0u;
+    __syncthreads();
+    uint32_t at[SJ];  // arrival in the bucket
 #pragma unroll
-        for (int j = 0; j < SJ; ++j) {
-            if (!real[j]) continue;
-            S.w[cur][S.loff[dg[j]] + S.wcnt[w][dg[j]] + rnk[j]] = wd[j];
+    for (int j = 0; j < SJ; ++j) {
+        const uint32_t i = j * ST + threadIdx.x;
+        if (j * ST >= n) break;
+        at[j] = i < n ? atomicAdd(&S.start[(uint32_t)((k[j] & lmask) >> bs)], 1u) : 0u;
+    }
+    __syncthreads();
+    {
+        constexpr int BPT = GS_NB / ST;
+        uint32_t c[BPT], sum[1] = {0}, tot[1];
+#pragma unroll
+        for (int q = 0; q < BPT; ++q) {
+            c[q] = S.start[threadIdx.x * BPT + q];
+            sum[0] += c[q];
+        }
+        block_excl_scan_n<SNW>(sum, S.lds, tot);
+#pragma unroll
+        for (int q = 0; q < BPT; ++q) {
+            S.start[threadIdx.x * BPT + q] = sum[0];
+            sum[0] += c[q];
+        }
+        if (threadIdx.x == 0) S.start[GS_NB] = n;
+    }
+    __syncthreads();
+    uint32_t lc[SJ], most = 0;  // bucket start, pairs in it << 16
+#pragma unroll
+    for (int j = 0; j < SJ; ++j) {
+        const uint32_t i = j * ST + threadIdx.x;
+        if (j * ST >= n) break;
+        const uint32_t b = (uint32_t)((k[j] & lmask) >> bs);
+        const uint32_t l = S.start[b], c = i < n ? S.start[b + 1] - l : 0u;
+        lc[j] = l | (c << 16);
+        most = c > most ? c : most;
+    }
+    if (__syncthreads_or(most > GS_FEW)) {
+        // a long row: every bucket is split into at least as many equal parts as it
+        // has pairs, and the parts are counted (16 bits each, in the words'
+        // place) and scanned like the buckets before
+        uint32_t *parts = reinterpret_cast<uint32_t *>(S.word);
+        constexpr int BPT = GS_NB / ST, PPT = GS_PARTS / 2 / ST;
+        uint32_t lg[BPT], sum[1] = {0}, tot[1];
+#pragma unroll
+        for (int q = 0; q < BPT; ++q) {
+            const uint32_t c = S.start[threadIdx.x * BPT + q + 1] - S.start[threadIdx.x * BPT + q];
+            lg[q] = c > 1 ? 32u - (uint32_t)__clz(c - 1u) : 0u;
+            lg[q] = lg[q] < (uint32_t)bs ? lg[q] : (uint32_t)bs;
+            sum[0] += 1u << lg[q];
+        }
+        for (uint32_t i = threadIdx.x; i < GS_PARTS / 2; i += ST) parts[i] = 0u;
+        block_excl_scan_n<SNW>(sum, S.lds, tot);
+#pragma unroll
+        for (int q = 0; q < BPT; ++q) {
+            S.start[threadIdx.x * BPT + q] = sum[0] | (lg[q] << 16);
+            sum[0] += 1u << lg[q];
         }
         __syncthreads();
-        if (sh + DB >= lb) break;
-        // the next digit: the lowest key bits the words still carry
 #pragma unroll
         for (int j = 0; j < SJ; ++j) {
-            const int p = w * pw + j * 64 + lane;
-            wd[j] = real[j] ? S.w[cur][p] : 0u;
-            dg[j] = (wd[j] >> GS_PK_POS) & DM;
-            wd[j] = (((wd[j] >> GS_PK_POS) >> DB) << GS_PK_POS) | (wd[j] & PM);
+            const uint32_t i = j * ST + threadIdx.x;
+            if (j * ST >= n) break;
+            const uint32_t e = S.start[(uint32_t)((k[j] & lmask) >> bs)];
+            lc[j] = (e & 0xffffu) + (uint32_t)((k[j] & rest) >> (bs - (int)(e >> 16)));
+            const uint32_t sh = (lc[j] & 1u) * 16u;
+            at[j] = i < n ? (atomicAdd(&parts[lc[j] >> 1], 1u << sh) >> sh) & 0xffffu : 0u;
         }
-        cur ^= 1;
+        __syncthreads();
+        uint32_t pc[PPT];
+        sum[0] = 0;
+#pragma unroll
+        for (int q = 0; q < PPT; ++q) {
+            pc[q] = parts[threadIdx.x * PPT + q];
+            sum[0] += (pc[q] & 0xffffu) + (pc[q] >> 16);
+        }
+        block_excl_scan_n<SNW>(sum, S.lds, tot);
+#pragma unroll
+        for (int q = 0; q < PPT; ++q) {
+            const uint32_t a = sum[0] + (pc[q] & 0xffffu);
+            parts[threadIdx.x * PPT + q] = sum[0] | (a << 16);
+            sum[0] = a + (pc[q] >> 16);
+        }
+        if (threadIdx.x == 0) parts[GS_PARTS / 2] = n;
+        __syncthreads();
+        const uint16_t *ps = reinterpret_cast<const uint16_t *>(S.word);
+        most = 0;
+#pragma unroll
+        for (int j = 0; j < SJ; ++j) {
+            const uint32_t i = j * ST + threadIdx.x;
+            if (j * ST >= n) break;
+            const uint32_t l = ps[lc[j]], c = i < n ? ps[lc[j] + 1] - l : 0u;
+            lc[j] = l | (c << 16);
+            most = c > most ? c : most;
+        }
+        if (__syncthreads_or(most > GS_CROWD)) return false;
     }
-    // S.w[cur]: the positions in sorted order; the key and value gathers of
-    // every item in flight before the first store
-    uint64_t kk[SJ];
-    uint32_t vv[SJ];
 #pragma unroll
     for (int j = 0; j < SJ; ++j) {
-        const int i = j * GT + threadIdx.x;
-        const uint32_t src = i < cnt ? (S.w[cur][i] & PM) : 0u;
-        kk[j] = kin[s0 + src];
-        vv[j] = vin[s0 + src];
+        const uint32_t i = j * ST + threadIdx.x;
+        if (j * ST >= n) break;
+        if (i < n) S.word[(lc[j] & 0xffffu) + at[j]] = ((k[j] & rest) << GS_POS) | (uint64_t)i;
+        at[j] = lc[j] & 0xffffu;  // from here on the pair's place
+    }
+    __syncthreads();
+    for (uint32_t d = 0; __any(d < most); ++d) {
+        // all reads in flight before the first use
+        uint64_t o[SJ];
+#pragma unroll
+        for (int j = 0; j < SJ; ++j) {
+            if (j * ST >= n) break;
+            o[j] = ~0ull;
+            if (d < (lc[j] >> 16)) o[j] = S.word[(lc[j] & 0xffffu) + d];
+        }
+#pragma unroll
+        for (int j = 0; j < SJ; ++j) {
+            const uint64_t mine = ((k[j] & rest) << GS_POS) | (uint64_t)(j * ST + threadIdx.x);
+            if (j * ST >= n) break;
+            at[j] += o[j] < mine ? 1u : 0u;
+        }
     }
 #pragma unroll
     for (int j = 0; j < SJ; ++j) {
-        const int i = j * GT + threadIdx.x;
-        if (i < cnt) {
-            kout[s0 + i] = kk[j];
-            vout[s0 + i] = vv[j];
+        const uint32_t i = j * ST + threadIdx.x;
+        if (j * ST >= n) break;
+        if (i < n) {
+            kout[at[j]] = k[j];
+            vout[at[j]] = v[j];
         }
     }
+    return true;
 }
 
 // A group larger than GS_CAP: stable LSD passes out of global memory by this
@@ -467,10 +497,10 @@ __device__ void group_sort_packed(GsPacked<DB> &S, const uint64_t *__restrict__ 
 // digit's running offset carried in LDS).  Ping-pongs between the group's
 // ranges of (a_k, a_v) (input) and (b_k, b_v) and ends in (b_k, b_v).
 struct GsBig {
-    uint32_t wcnt[GT / 64][256];
-    uint32_t loff[256];
-    uint32_t run[256];
-    uint32_t lds4[4];
+    uint16_t wcnt[SNW][SD];
+    uint32_t loff[SD];
+    uint32_t run[SD];
+    uint32_t lds[SNW][1];
 };
 
 __device__ void group_sort_big(GsBig &S, uint64_t *__restrict__ a_k, uint32_t *__restrict__ a_v,
@@ -478,27 +508,26 @@ __device__ void group_sort_big(GsBig &S, uint64_t *__restrict__ a_k, uint32_t *_
                                int lb)
 {
     constexpr int BJ = 2;                 // items per lane per chunk
-    constexpr int CH = GT * BJ;           // 512 pairs per chunk
+    constexpr int CH = ST * BJ;           // pairs per chunk
     const int w = threadIdx.x >> 6, lane = lane_id();
     uint64_t *sk = a_k, *dk = b_k;
     uint32_t *sv = a_v, *dv = b_v;
     bool in_b = false;
-    for (int sh = 0; sh < lb; sh += 8) {
+    for (int sh = 0; sh < lb; sh += SD_BITS) {
         // digit counts of the whole group
         S.run[threadIdx.x] = 0;
         __syncthreads();
-        for (int64_t i = threadIdx.x; i < cnt; i += GT) atomicAdd(&S.run[(uint32_t)(sk[s0 + i] >> sh) & 255u], 1u);
+        for (int64_t i = threadIdx.x; i < cnt; i += ST) atomicAdd(&S.run[(uint32_t)(sk[s0 + i] >> sh) & (SD - 1u)], 1u);
         __syncthreads();
         {
-            uint32_t tot;
-            const uint32_t c = S.run[threadIdx.x];
-            __syncthreads();
-            S.run[threadIdx.x] = block_excl_scan_256(c, S.lds4, &tot);
+            uint32_t c[1] = {S.run[threadIdx.x]}, tot[1];
+            block_excl_scan_n<SNW>(c, S.lds, tot);
+            S.run[threadIdx.x] = c[0];
         }
         __syncthreads();
         for (int64_t c0 = 0; c0 < cnt; c0 += CH) {
             const int64_t left = cnt - c0;
-            const int jmax = left >= CH ? BJ : (int)((left + GT - 1) / GT);
+            const int jmax = left >= CH ? BJ : (int)((left + ST - 1) / ST);
             const int pw = jmax * 64;
             // only digits and ranks stay in registers; the pairs are read
             // again for the scatter (L2 hits)
@@ -508,9 +537,9 @@ __device__ void group_sort_big(GsBig &S, uint64_t *__restrict__ a_k, uint32_t *_
             for (int j = 0; j < BJ; ++j) {
                 const int64_t p = (int64_t)w * pw + j * 64 + lane;
                 real[j] = j < jmax && p < left;
-                dg[j] = real[j] ? (uint32_t)(sk[s0 + c0 + p] >> sh) & 255u : 0u;
+                dg[j] = real[j] ? (uint32_t)(sk[s0 + c0 + p] >> sh) & (SD - 1u) : 0u;
             }
-            rank_chunk<BJ>(dg, real, jmax, rnk, S.wcnt, S.loff, S.lds4);
+            rank_chunk<BJ>(dg, real, jmax, rnk, S.wcnt, S.loff, S.lds);
 #pragma unroll
             for (int j = 0; j < BJ; ++j) {
                 if (!real[j]) continue;
@@ -523,7 +552,7 @@ __device__ void group_sort_big(GsBig &S, uint64_t *__restrict__ a_k, uint32_t *_
             // the chunk's count of digit d: loff[d + 1] - loff[d]
             {
                 const int d = threadIdx.x;
-                const uint32_t c = (d == 255 ? (uint32_t)(left < CH ? left : CH) : S.loff[d + 1]) - S.loff[d];
+                const uint32_t c = (d == SD - 1 ? (uint32_t)(left < CH ? left : CH) : S.loff[d + 1]) - S.loff[d];
                 S.run[d] += c;
             }
             __syncthreads();
@@ -533,7 +562,7 @@ __device__ void group_sort_big(GsBig &S, uint64_t *__restrict__ a_k, uint32_t *_
         in_b = !in_b;
     }
     if (!in_b) {
-        for (int64_t i = threadIdx.x; i < cnt; i += GT) {
+        for (int64_t i = threadIdx.x; i < cnt; i += ST) {
             b_k[s0 + i] = a_k[s0 + i];
             b_v[s0 + i] = a_v[s0 + i];
         }
@@ -543,13 +572,12 @@ __device__ void group_sort_big(GsBig &S, uint64_t *__restrict__ a_k, uint32_t *_
 // One workgroup per digit (group); the last digit holds the invalid keys,
 // copied as they are.  In: (kin, vin) in group order; out: (kout, vout)
 // sorted.  gbase: ndig + 1 exclusive group offsets.
-template <typename K, int DB>
-__global__ __launch_bounds__(GT) void k_gs_sort(uint64_t *__restrict__ kin, uint32_t *__restrict__ vin,
+__global__ __launch_bounds__(ST) __attribute__((amdgpu_waves_per_eu(6))) void k_gs_sort(uint64_t *__restrict__ kin, uint32_t *__restrict__ vin,
                                                 uint64_t *__restrict__ kout, uint32_t *__restrict__ vout, int lb,
                                                 int ndig, const uint32_t *__restrict__ gbase)
 {
     __shared__ union {
-        GsLds<K, DB> lds;
+        GsLds lds;
         GsBig big;
     } S;
     const int g = blockIdx.x;
@@ -557,45 +585,21 @@ __global__ __launch_bounds__(GT) void k_gs_sort(uint64_t *__restrict__ kin, uint
     const int64_t cnt = (int64_t)gbase[g + 1] - s0;
     if (cnt <= 0) return;
     if (g == ndig - 1) {
-        for (int64_t i = threadIdx.x; i < cnt; i += GT) {
+        for (int64_t i = threadIdx.x; i < cnt; i += ST) {
             kout[s0 + i] = kin[s0 + i];
             vout[s0 + i] = vin[s0 + i];
         }
         return;
     }
     if (cnt <= GS_CAP) {
-        group_sort_lds<K, DB>(S.lds, kin, vin, kout, vout, s0, (int)cnt, lb, (uint64_t)g << lb);
-    } else {
-        group_sort_big(S.big, kin, vin, kout, vout, s0, cnt, lb);
-    }
-}
-
-// The same with the one-word LDS sort (lb <= GS_PK_BITS + DB).
-template <int DB>
-__global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(5))) void k_gs_sort_packed(
-    uint64_t *__restrict__ kin, uint32_t *__restrict__ vin, uint64_t *__restrict__ kout, uint32_t *__restrict__ vout,
-    int lb, int ndig, const uint32_t *__restrict__ gbase)
-{
-    __shared__ union {
-        GsPacked<DB> pk;
-        GsBig big;
-    } S;
-    const int g = blockIdx.x;
-    const int64_t s0 = gbase[g];
-    const int64_t cnt = (int64_t)gbase[g + 1] - s0;
-    if (cnt <= 0) return;
-    if (g == ndig - 1) {
-        for (int64_t i = threadIdx.x; i < cnt; i += GT) {
-            kout[s0 + i] = kin[s0 + i];
-            vout[s0 + i] = vin[s0 + i];
+        if (group_sort_lds(S.lds, kin + s0, vin + s0, kout + s0, vout + s0, (uint32_t)cnt, lb)) return;
+        __syncthreads();
+        if (lb + GS_POS <= 64) {
+            group_sort_crowded(S.lds, kin + s0, vin + s0, kout + s0, vout + s0, (uint32_t)cnt, lb);
+            return;
         }
-        return;
     }
-    if (cnt <= GS_CAP) {
-        group_sort_packed<DB>(S.pk, kin, vin, kout, vout, s0, (int)cnt, lb);
-    } else {
-        group_sort_big(S.big, kin, vin, kout, vout, s0, cnt, lb);
-    }
+    group_sort_big(S.big, kin, vin, kout, vout, s0, cnt, lb);
 }
 
 }  // namespace
@@ -620,17 +624,6 @@ hipError_t group_sort_pairs(uint64_t *k0, uint32_t *v0, uint64_t *k1, uint32_t *
     while ((1 << dbits) < ndig) ++dbits;
     k_gs_scan<<<blocks, GS_SCAN_T, 0, s>>>(hist, nb, dtot);
     k_gs_scatter<<<(unsigned)nb, GT, 0, s>>>(k0, v0, k1, v1, n, lb, ndig, dbits, hist, nb, dtot, gbase);
-    // 9-bit digits where they save a pass over the lb local bits
-    const bool nine = (lb + 8) / 9 < (lb + 7) / 8;
-    if (lb <= GS_PK_BITS + (nine ? 9 : 8)) {
-        if (nine) k_gs_sort_packed<9><<<ndig, GT, 0, s>>>(k1, v1, k0, v0, lb, ndig, gbase);
-        else k_gs_sort_packed<8><<<ndig, GT, 0, s>>>(k1, v1, k0, v0, lb, ndig, gbase);
-    } else if (lb <= 32) {
-        // lb in 29..32 here, where 9-bit digits take as many passes as 8-bit
-        k_gs_sort<uint32_t, 8><<<ndig, GT, 0, s>>>(k1, v1, k0, v0, lb, ndig, gbase);
-    } else {
-        if (nine) k_gs_sort<uint64_t, 9><<<ndig, GT, 0, s>>>(k1, v1, k0, v0, lb, ndig, gbase);
-        else k_gs_sort<uint64_t, 8><<<ndig, GT, 0, s>>>(k1, v1, k0, v0, lb, ndig, gbase);
-    }
+    k_gs_sort<<<ndig, ST, 0, s>>>(k1, v1, k0, v0, lb, ndig, gbase);
     return hipGetLastError();
 }
