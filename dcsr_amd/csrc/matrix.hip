@@ -199,7 +199,7 @@ __global__ void k_set_loaded(int64_t R, const uint32_t *__restrict__ foff, uint3
 
 // Flat copy of every row into destination offsets (compaction / export).
 // dst_off[r] is the row's new start; src rows are (start, len).  Each wave
-// owns CP_SPAN destination entries, in chunks of at most 64 rows: a start
+// owns SPAN destination entries, in chunks of at most 64 rows: a start
 // map of the chunk's rows (ranked to rows through `tab`: empty rows share a
 // start) gives every entry its row without a search, and all of a lane's
 // loads are in flight before its first store.  The wave's first row comes
@@ -208,9 +208,14 @@ __global__ void k_set_loaded(int64_t R, const uint32_t *__restrict__ foff, uint3
 // the offsets there; nothing is written when the rows hold more than `limit`
 // entries, so a caller need not know the count before the launch.  PAIR: the
 // entries go to dst_pair as (column, value bits) pairs.
-constexpr uint32_t CP_SPAN = 1024;
-constexpr uint32_t CP_PER = CP_SPAN / 64;
-template <bool PAIR>
+//
+// A wave's pass over its entries is one chain of loads, so up to CP_SHORT_MAX
+// entries (fewer workgroups than CUs at CP_SPAN) the waves own CP_SHORT: 3,000
+// entries 7.4 -> 3.8 us, 200,000 11.7 -> 5.1, 1M (as pairs) 10 -> 8.3; 4M takes
+// 18 either way, and 16M (57 us) moves 4.5 TB/s.
+constexpr uint32_t CP_SPAN = 1024, CP_SHORT = 256;
+constexpr int64_t CP_SHORT_MAX = 1 << 20;
+template <bool PAIR, uint32_t SPAN>
 __global__ __launch_bounds__(TB) void k_copy_rows(const uint32_t *__restrict__ dst_off,
                                                   const uint32_t *__restrict__ rowmap, uint32_t R, uint64_t limit,
                                                   int32_t *__restrict__ row_offsets,
@@ -219,10 +224,11 @@ __global__ __launch_bounds__(TB) void k_copy_rows(const uint32_t *__restrict__ d
                                                   int32_t *__restrict__ dst_col, float *__restrict__ dst_val,
                                                   uint2 *__restrict__ dst_pair)
 {
+    constexpr uint32_t PER = SPAN / 64;
     struct Lds {
         uint32_t off[65];
         uint32_t src[64];
-        uint32_t pmap[CP_SPAN / 32];
+        uint32_t pmap[SPAN / 32];
         uint32_t tab[64];
     };
     __shared__ Lds sh[TB / 64];
@@ -234,10 +240,10 @@ __global__ __launch_bounds__(TB) void k_copy_rows(const uint32_t *__restrict__ d
         for (uint64_t r = (uint64_t)blockIdx.x * TB + threadIdx.x; r <= R; r += (uint64_t)gridDim.x * TB)
             row_offsets[r] = (int32_t)dst_off[r];
     const uint64_t nwaves = (uint64_t)gridDim.x * (TB / 64);
-    for (uint64_t wave = (uint64_t)blockIdx.x * (TB / 64) + (threadIdx.x >> 6); wave * CP_SPAN < total;
+    for (uint64_t wave = (uint64_t)blockIdx.x * (TB / 64) + (threadIdx.x >> 6); wave * SPAN < total;
          wave += nwaves) {
-        const uint32_t e0 = (uint32_t)(wave * CP_SPAN);
-        const uint32_t e1 = total - e0 < CP_SPAN ? total : e0 + CP_SPAN;
+        const uint32_t e0 = (uint32_t)(wave * SPAN);
+        const uint32_t e1 = total - e0 < SPAN ? total : e0 + SPAN;
         uint32_t j = rowmap[e0 / RS_GRAN];
         if (j + 64u <= R && dst_off[j + 64u] <= e0) j = wave_find_last_le(dst_off, R, e0);
         uint32_t e = e0;
@@ -249,7 +255,7 @@ __global__ __launch_bounds__(TB) void k_copy_rows(const uint32_t *__restrict__ d
             S.off[lane] = off_t;
             if (lane == 0) S.off[64] = off_64;
             S.src[lane] = src;
-            if (lane < CP_SPAN / 32) S.pmap[lane] = 0u;
+            if (lane < SPAN / 32) S.pmap[lane] = 0u;
             __builtin_amdgcn_wave_barrier();
             const uint32_t wend = S.off[64] < e1 ? S.off[64] : e1;
             const uint32_t cnt = wend - e;
@@ -258,14 +264,14 @@ __global__ __launch_bounds__(TB) void k_copy_rows(const uint32_t *__restrict__ d
             const bool starts_here = t < R && off_t >= e && off_t < wend && S.off[lane + 1] > off_t;
             if (starts_here) atomicOr(&S.pmap[(off_t - e) >> 5], 1u << ((off_t - e) & 31u));
             __builtin_amdgcn_wave_barrier();
-            const StartMap pm = start_map_load(S.pmap, CP_SPAN / 64);
+            const StartMap pm = start_map_load(S.pmap, SPAN / 64);
             const uint32_t rank = start_map_rank(pm, starts_here ? off_t - e : 0u);  // every lane takes part
             if (starts_here) S.tab[rank] = lane;
             __builtin_amdgcn_wave_barrier();
-            int32_t c[CP_PER];
-            float v[CP_PER];
+            int32_t c[PER];
+            float v[PER];
 #pragma unroll
-            for (uint32_t q = 0; q < CP_PER; ++q) {
+            for (uint32_t q = 0; q < PER; ++q) {
                 const uint32_t p = q * 64u + lane;
                 const uint32_t nst = start_map_count(pm, (int)q);
                 c[q] = 0;
@@ -278,7 +284,7 @@ __global__ __launch_bounds__(TB) void k_copy_rows(const uint32_t *__restrict__ d
                 }
             }
 #pragma unroll
-            for (uint32_t q = 0; q < CP_PER; ++q) {
+            for (uint32_t q = 0; q < PER; ++q) {
                 const uint32_t p = q * 64u + lane;
                 if (p < cnt) {
                     if constexpr (PAIR) {
@@ -917,17 +923,19 @@ static void launch_copy_rows(dcsr_handle h, const uint32_t *off, const uint32_t 
 {
     const int64_t R = h->rows;
     if (R <= 0 || (total <= 0 && !row_offsets)) return;
-    const int64_t waves = (total + CP_SPAN - 1) / CP_SPAN;
+    const bool small = total <= CP_SHORT_MAX;
+    const int64_t span = small ? CP_SHORT : CP_SPAN;
+    const int64_t waves = (total + span - 1) / span;
     int64_t blocks = (waves + 3) / 4;
     if (row_offsets && blocks < (R + 1) / (TB * 8)) blocks = (R + 1) / (TB * 8);
     if (blocks > 2048) blocks = 2048;  // waves stride over the rest
     if (blocks < 1) blocks = 1;
-    if (dpair)
-        k_copy_rows<true><<<(unsigned)blocks, TB, 0, s>>>(off, rowmap, (uint32_t)R, limit, row_offsets, h->row_start,
-                                                          h->pool_col, h->pool_val, nullptr, nullptr, dpair);
-    else
-        k_copy_rows<false><<<(unsigned)blocks, TB, 0, s>>>(off, rowmap, (uint32_t)R, limit, row_offsets, h->row_start,
-                                                           h->pool_col, h->pool_val, dcol, dval, nullptr);
+    auto run = [&](auto *k) {
+        k<<<(unsigned)blocks, TB, 0, s>>>(off, rowmap, (uint32_t)R, limit, row_offsets, h->row_start, h->pool_col,
+                                          h->pool_val, dcol, dval, dpair);
+    };
+    if (dpair) small ? run(k_copy_rows<true, CP_SHORT>) : run(k_copy_rows<true, CP_SPAN>);
+    else small ? run(k_copy_rows<false, CP_SHORT>) : run(k_copy_rows<false, CP_SPAN>);
 }
 
 // The live entries as (column, value) pairs in flat order; *off receives the

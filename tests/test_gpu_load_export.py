@@ -121,3 +121,19 @@ def test_export_after_nosync_updates_checks_the_capacity():
     got = np.repeat(np.arange(R), np.diff(off.cpu().numpy())).astype(np.int64) * R + col.cpu().numpy()
     np.testing.assert_array_equal(got, np.union1d(key, bkey))
     m.close()
+
+
+@pytest.mark.parametrize("n", [255, 256, 257, 2**20 - 1, 2**20, 2**20 + 1, 1_300_003])
+def test_export_on_both_sides_of_the_copy_span(n):
+    import dcsr_amd
+    R, C = 150_000, 40_000
+    rng = np.random.default_rng(n)
+    r = rng.integers(0, R, n).astype(np.int32)
+    r[: n // 8] = R // 2  # a long row
+    c, v = rng.integers(0, C, n).astype(np.int32), rng.random(n, np.float32)
+    m = dcsr_amd.DcsrMatrix(R, C, pool_factor=1.2)
+    m.LoadMatrix(r, c, v)
+    m.SortMatrixRow()  # the same copy, into the pool
+    same(m.to_csr(), stored(R, r, c, v)[:3])
+    check_healthy(m)
+    m.close()
