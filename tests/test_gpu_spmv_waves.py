@@ -63,3 +63,40 @@ def test_rows_and_ranges(name, paneled, monkeypatch):
     D[br, bc] += 7
     check()
     m.close()
+
+
+@pytest.mark.parametrize("narrow", [False, True])
+def test_captured_product_follows_updates(narrow, monkeypatch):
+    """A product captured after the copy exists replays the rows as they are."""
+    import torch
+    import dcsr_amd
+    monkeypatch.setenv("DCSR_SPMV_PANEL_COLS", "1000" if narrow else "1500")
+    monkeypatch.setenv("DCSR_SPMV_PANEL_MIN_NNZ", "1500" if narrow else "0")
+    R, C, n = 400, 2000 + 500 * narrow, 2000
+    rng = np.random.default_rng(3)
+    key = rng.permutation(R * C)[:n]
+    r, c = (key // C).astype(np.int32), (key % C).astype(np.int32)
+    v = rng.integers(1, 9, n).astype(np.float32)
+    m = dcsr_amd.DcsrMatrix(R, C, pool_factor=4.0)
+    m.LoadMatrix(r, c, v)
+    xh = rng.integers(-4, 5, C).astype(np.float32)
+    x, y = torch.from_numpy(xh).cuda(), torch.empty(R, device="cuda")
+    for _ in range(5):  # the copy is built on the way
+        m.spmv(x, y)
+    torch.cuda.synchronize()
+    s, g = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.stream(s):
+        m.spmv(x, y)  # eager, on the capture's stream
+        s.synchronize()
+        with torch.cuda.graph(g, stream=s):
+            m.spmv(x, y)
+    want = np.zeros(R)
+    np.add.at(want, r, v * xh[c])
+    for k in range(3):
+        y.fill_(7.0)
+        g.replay()
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(y.cpu().numpy(), want.astype(np.float32))
+        m.UpdateMatrix(r, c, np.full(n, k + 1.0, np.float32))  # in place: the rows stay where they are
+        np.add.at(want, r, (k + 1.0) * xh[c])
+    m.close()
