@@ -544,6 +544,60 @@ __device__ __forceinline__ void team_sort(K *key, uint32_t *hist, uint32_t P, ui
     else team_bitonic_sort<NT, K>(key, P);
 }
 
+// The expansion of up to TEAM entries of a team's row (tot partials from
+// generation gbase): the entries with partials leave a bit each at their first
+// one in a map of the row's at most 32 * KPL / 2 partials (in hist, free until the sort)
+// and, by their rank, their displacement and value in a table, so a partial's
+// entry is a bit count; a search of the entries' offsets took four dependent LDS
+// reads and 24 instructions per partial (the four classes on 2M Poisson rows with
+// 8 entries: 994 -> 907 us, 30 of it k_sg_team's registers).
+template <int GB, int KPL>
+__device__ __forceinline__ void sg_expand_team(const SgIn &in, uint32_t lb, uint32_t sb, float va, uint32_t ex,
+                                               uint32_t tot, uint32_t gbase, uint32_t *key, float *val,
+                                               uint32_t *map, uint32_t *s_sb, float *s_va)
+{
+    constexpr int W = KPL / 2;  // words of 32 partials
+    static_assert(KPL % 2 == 0 && TEAM == 16, "two partials per lane and word");
+    const uint32_t t = threadIdx.x % TEAM;
+    if (t < W) map[t] = 0u;
+    const uint32_t some = (uint32_t)(__ballot(lb > 0u) >> (lane_id() & ~(TEAM - 1))) & 0xffffu;
+    team_sync<TEAM>();
+    if (lb > 0u) {
+        const uint32_t k = (uint32_t)__popc(some & ((1u << t) - 1u));
+        s_sb[k] = sb - ex;  // B's entry of a partial less the partial
+        s_va[k] = va;
+        atomicOr(&map[ex >> 5], 1u << (ex & 31u));
+    }
+    team_sync<TEAM>();
+    if (tot == 0u) return;
+    uint32_t m[W], before[W];
+#pragma unroll
+    for (int i = 0; i < W; ++i) {
+        m[i] = map[i];
+        before[i] = i ? before[i - 1] + (uint32_t)__popc(m[i - 1]) : ~0u;
+    }
+    // every load before the first use (a lane past tot reads entry 0 of B and
+    // writes nothing)
+    uint2 be[KPL];
+    float av[KPL];
+#pragma unroll
+    for (int i = 0; i < KPL; ++i) {
+        const uint32_t pe = (uint32_t)i * TEAM + t;
+        const uint32_t q = before[i / 2] + (uint32_t)__popc(m[i / 2] & ((2u << ((i & 1) * TEAM + t)) - 1u));
+        be[i] = in.b_ent[pe < tot ? s_sb[q] + pe : 0u];
+        av[i] = s_va[q];
+    }
+#pragma unroll
+    for (int i = 0; i < KPL; ++i) {
+        const uint32_t pe = (uint32_t)i * TEAM + t;
+        if (pe < tot) {
+            const uint32_t g = gbase + pe;
+            key[g] = (be[i].x << GB) | g;
+            val[g] = av[i] * __uint_as_float(be[i].y);
+        }
+    }
+}
+
 // KPL: keys per lane of the sort, fixed by the row's class (P <= KPL * NT).  The products stay where the expansion put them
 // (generation order); only the keys are sorted, and a sorted key names its
 // product by its generation bits.
@@ -568,6 +622,12 @@ __device__ void sg_row(const SgRowInfo &ri, const SgIn &in, const SgOut &out, K 
         }
         uint32_t tot;
         const uint32_t ex = team_excl_scan<NT>(lb, lds_w, &tot);
+        if constexpr (NT == TEAM) {
+            sg_expand_team<GB, KPL>(in, lb, sb, va, ex, tot, gbase, key, val, hist, s_sb, s_va);
+            gbase += tot;
+            team_sync<NT>();
+            continue;
+        }
         s_ex[t] = ex;
         s_sb[t] = sb;
         s_va[t] = va;
@@ -691,9 +751,11 @@ __global__ __launch_bounds__(TB) void k_sg_wave(const uint32_t *__restrict__ lis
 }
 
 // Rows of at most KPL * TEAM partials (class CL_TEAM + KPL / 2 - 1): 16-lane
-// teams, four rows per wave.
+// teams, four rows per wave.  Six keys per lane take 90 registers, five waves per
+// SIMD; held to 80 they fit six, 400 -> 370 us.  Eight would spill (154 -> 177 at
+// five waves), as four at eight waves (325 -> 340).
 template <int KPL>
-__global__ __launch_bounds__(TB) void k_sg_team(const uint32_t *__restrict__ list, const SgState *__restrict__ st,
+__global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(KPL == 6 ? 6 : 4))) void k_sg_team(const uint32_t *__restrict__ list, const SgState *__restrict__ st,
                                                 SgIn in, SgOut out)
 {
     constexpr int NTEAM = TB / TEAM;
