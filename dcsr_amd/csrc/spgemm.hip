@@ -245,15 +245,17 @@ template <int NT>
 __device__ __forceinline__ uint32_t team_excl_scan(uint32_t v, uint32_t *lds_w, uint32_t *total)
 {
     if (NT < 64) {
-        // within the team's aligned NT-lane slice of the wave
-        const int t = lane_id() % NT;
-        uint32_t inc = v;
-#pragma unroll
-        for (int d = 1; d < NT; d <<= 1) {
-            const uint32_t u = __shfl_up(inc, d, NT);
-            if (t >= d) inc += u;
-        }
-        *total = __shfl(inc, NT - 1, NT);
+        static_assert(NT >= 64 || NT == 16, "a team is a DPP row");
+        uint32_t inc = v, tot = v;
+        inc += dpp_u32<DPP_ROW_SHR(1)>(0u, inc);
+        inc += dpp_u32<DPP_ROW_SHR(2)>(0u, inc);
+        inc += dpp_u32<DPP_ROW_SHR(4)>(0u, inc);
+        inc += dpp_u32<DPP_ROW_SHR(8)>(0u, inc);
+        tot += dpp_u32<DPP_ROW_ROR(8)>(0u, tot);
+        tot += dpp_u32<DPP_ROW_ROR(4)>(0u, tot);
+        tot += dpp_u32<DPP_ROW_ROR(2)>(0u, tot);
+        tot += dpp_u32<DPP_ROW_ROR(1)>(0u, tot);
+        *total = tot;
         return inc - v;
     }
     const uint32_t inc = wave_incl_scan_u32(v);
@@ -297,7 +299,7 @@ __device__ __forceinline__ uint32_t find_seg_team(const uint32_t *s, uint32_t e)
 // the next row are in flight while the current row is processed).
 struct SgRowInfo {
     uint32_t row, P, ast, la, fo;
-    uint64_t out_base;
+    uint32_t out_base;
 };
 
 // What the row kernels read: A's row table and values, the B row of every A
@@ -445,12 +447,18 @@ __device__ __forceinline__ bool team_bucket_sort(K *key, uint32_t *hist, uint32_
     }
 #pragma unroll
     for (int i = 0; i < BPL / 2; ++i) hist[(uint32_t)i * NT + t] = 0u;
-    constexpr int W = NT < 64 ? NT : 64;
-#pragma unroll
-    for (int d = 1; d < W; d <<= 1) {
-        const uint32_t l2 = (uint32_t)__shfl_xor((int)lo, d, W), h2 = (uint32_t)__shfl_xor((int)hi, d, W);
+    // over the 16 lanes of a DPP row by rotations, across rows by permutes
+    auto both = [&](uint32_t l2, uint32_t h2) {
         lo = l2 < lo ? l2 : lo;
         hi = h2 > hi ? h2 : hi;
+    };
+    both(dpp_u32<DPP_ROW_ROR(8)>(lo, lo), dpp_u32<DPP_ROW_ROR(8)>(hi, hi));
+    both(dpp_u32<DPP_ROW_ROR(4)>(lo, lo), dpp_u32<DPP_ROW_ROR(4)>(hi, hi));
+    both(dpp_u32<DPP_ROW_ROR(2)>(lo, lo), dpp_u32<DPP_ROW_ROR(2)>(hi, hi));
+    both(dpp_u32<DPP_ROW_ROR(1)>(lo, lo), dpp_u32<DPP_ROW_ROR(1)>(hi, hi));
+    if constexpr (NT >= 64) {
+#pragma unroll
+        for (int d = 16; d < 64; d <<= 1) both((uint32_t)__shfl_xor((int)lo, d), (uint32_t)__shfl_xor((int)hi, d));
     }
     if constexpr (NT > 64) {
         constexpr int NW = NT / 64;
@@ -550,7 +558,7 @@ __device__ __forceinline__ void team_sort(K *key, uint32_t *hist, uint32_t P, ui
 // and, by their rank, their displacement and value in a table, so a partial's
 // entry is a bit count; a search of the entries' offsets took four dependent LDS
 // reads and 24 instructions per partial (the four classes on 2M Poisson rows with
-// 8 entries: 994 -> 907 us, 30 of it k_sg_team's registers).
+// 8 entries: 994 -> 937 us).
 template <int GB, int KPL>
 __device__ __forceinline__ void sg_expand_team(const SgIn &in, uint32_t lb, uint32_t sb, float va, uint32_t ex,
                                                uint32_t tot, uint32_t gbase, uint32_t *key, float *val,
@@ -675,19 +683,21 @@ __device__ void sg_row(const SgRowInfo &ri, const SgIn &in, const SgOut &out, K 
         bool emit = false;
         float s = 0.0f;
         uint32_t c = 0;
-        if (p < P) {
-            const K k = key[p];
-            c = (uint32_t)(k >> GB);
-            const bool head = p == 0 || (uint32_t)(key[p - 1] >> GB) != c;
-            if (head) {
-                s = 0.0f + val[(uint32_t)k & GM];
-                for (uint32_t q = p + 1; q < P; ++q) {
+        // the key, its neighbours and its product without a branch: most runs
+        // are one key
+        const uint32_t pc = p < P ? p : 0u;
+        const K k = key[pc], kp = key[pc > 0u ? pc - 1u : 0u], kn = key[pc + 1u < P ? pc + 1u : pc];
+        c = (uint32_t)(k >> GB);
+        if (p < P && (p == 0u || (uint32_t)(kp >> GB) != c)) {
+            s = 0.0f + val[(uint32_t)k & GM];
+            if (p + 1u < P && (uint32_t)(kn >> GB) == c) {
+                for (uint32_t q = p + 1u; q < P; ++q) {
                     const K kq = key[q];
                     if ((uint32_t)(kq >> GB) != c) break;
                     s = s + val[(uint32_t)kq & GM];
                 }
-                emit = s != 0.0f;
             }
+            emit = s != 0.0f;
         }
         // place among the team's emitting threads
         uint32_t pos, tot;
@@ -751,11 +761,14 @@ __global__ __launch_bounds__(TB) void k_sg_wave(const uint32_t *__restrict__ lis
 }
 
 // Rows of at most KPL * TEAM partials (class CL_TEAM + KPL / 2 - 1): 16-lane
-// teams, four rows per wave.  Six keys per lane take 90 registers, five waves per
-// SIMD; held to 80 they fit six, 400 -> 370 us.  Eight would spill (154 -> 177 at
-// five waves), as four at eight waves (325 -> 340).
+// teams, four rows per wave.  A row is a chain of round trips, so waves in flight
+// are what counts: a team is a DPP row, its scans and bounds stay in registers
+// (44, 64, 72 and 96 of them for 2, 4, 6 and 8 keys per lane; with permutes 54, 72,
+// 90 and 106), and six keys are held to the 72 that let seven waves share a SIMD.
+// The four classes on 2M Poisson rows with 8 entries: 907 -> 866 us.  Loading the
+// next row's A entries a row ahead cost more registers than it gave (866 -> 912).
 template <int KPL>
-__global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(KPL == 6 ? 6 : 4))) void k_sg_team(const uint32_t *__restrict__ list, const SgState *__restrict__ st,
+__global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(KPL == 6 ? 7 : 4))) void k_sg_team(const uint32_t *__restrict__ list, const SgState *__restrict__ st,
                                                 SgIn in, SgOut out)
 {
     constexpr int NTEAM = TB / TEAM;
