@@ -616,8 +616,8 @@ __global__ __launch_bounds__(SU_TB) void k_upd_small(SmallArgs A)
                 A.ds->nrewrite_old = 0;
                 A.ds->go = 0;
             }
-        } else if (!ok) {
-            A.ds->ubad = 1;
+        } else {
+            A.ds->ubad = ok ? 0 : 1;
         }
     }
     if constexpr (FUSED) {
