@@ -147,7 +147,7 @@ constexpr int64_t SPREAD_TILES = TTB_SPREAD;  // a tile's counts per thread
 // Positions of the probe space (touched rows end to end) and of the move
 // space (old entries of rewritten rows end to end) owned by one wave.
 constexpr uint32_t PR_SPAN = 1024;
-constexpr uint32_t MV_SPAN = 512;
+constexpr uint32_t MV_SPAN = 256;
 // batch tile table: heads / row heads (count, offset), claims / moved (sum, offset)
 enum { TT_H = 0, TT_R, TT_HX, TT_RX, TT_C, TT_M, TT_CX, TT_MX, TT_WORDS };
 // probe tile table: inserts, adds, deletes; insert / delete offsets; probe
@@ -974,6 +974,10 @@ __global__ __launch_bounds__(TTB) void k_upd_offsets(DevState *__restrict__ ds,
 // every entry its shift.  So the copy is a coalesced stream with no
 // per-entry search.  A row cut by the chunk's start begins from the shift
 // of its records before the cut, located by a search on their positions.
+// A span is a chain of dependent phases, so waves in flight are what counts:
+// 256 entries per wave take 72 registers (seven waves per SIMD; 512 took four
+// waves), 107 -> 89 us for 16M entries and a 4M-triple batch, 33 -> 30 for 3.2M
+// and 1M.
 constexpr uint32_t MV_PER = MV_SPAN / 64;  // entries per lane
 constexpr int MV_RU = 4;                   // record rounds of 64 in flight
 // The SpMV's flat row scan (rowscan.h) run by the first `ntiles`
@@ -1676,7 +1680,7 @@ dcsr_status prepare_launch(dcsr_handle h, const int32_t *rows, const int32_t *co
 // Move + write launches.  move_bound bounds the old entries to move: the
 // move kernel strides over them with at most MV_BLOCKS workgroups (waves
 // past the device's count exit at once).
-constexpr int64_t MV_BLOCKS = 1280;
+constexpr int64_t MV_BLOCKS = 4096;
 dcsr_status commit_launch(dcsr_handle h, const UpdBufs &b, int64_t n, int64_t move_bound, bool report,
                           hipStream_t s, uint64_t seq = 0)
 {
