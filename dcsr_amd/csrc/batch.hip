@@ -921,7 +921,11 @@ dcsr_status dcsr_batch_step(dcsr_batch b, const int64_t *tri_off, const int32_t 
     h->last_stream = s;
     if (!h->canonical) DCSR_TRY(canonicalize(h, s));
     int reserved = 0;
-    if (do_update) DCSR_TRY(batch_reserve(b, n, s, &reserved));
+    if (do_update) {
+        if (capturing(s)) h->replayed = true;
+        else DCSR_TRY(refresh_replayed(h, s));
+        DCSR_TRY(batch_reserve(b, n, s, &reserved));
+    }
     k_batch_zero_stat<<<grid_for(b->M, 256), 256, 0, s>>>(b->mstat, b->M, h->ds);
     if (flags & DCSR_BATCH_GRAPH) {
         const void *key[13] = {tri_off, rows, cols, vals, x, y, h->pool_col, (const void *)(intptr_t)b->team,

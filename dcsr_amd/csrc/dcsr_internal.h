@@ -144,7 +144,7 @@ struct dcsr_matrix_s {
     int64_t ncompact;        // compactions and growths (dcsr_query reports it)
     uint32_t upd_tag;        // tag of the last update's row -> touched-row map
     bool flat_dirty;         // flat row offsets (SpMV binning) need a rebuild
-    bool flat_replayed;      // an update was captured into a graph: the row lengths may change without a call
+    bool replayed;           // an update was captured into a graph: rows and counters may change without a call
     bool state_known;        // host mirrors valid (no NOSYNC update since last sync)
     // column-paneled copy for SpMV on matrices whose x exceeds the L2 (see
     // spmv.hip): valid until the next structural change
@@ -203,6 +203,12 @@ void refresh_bounds(dcsr_handle h);
 static inline int64_t live_bound(dcsr_handle h) { return h->state_known ? h->nnz_h : h->nnz_ub; }
 static inline int64_t bump_bound(dcsr_handle h) { return h->state_known ? h->bump_h : h->bump_ub; }
 dcsr_status ensure_flat(dcsr_handle h, hipStream_t s);  // spmv.hip
+bool capturing(hipStream_t s);
+// Before a call relies on the host mirrors, their bounds or the flat offsets:
+// a matrix that a replayed graph may have changed (h->replayed) has its state
+// read back and its offsets scanned again; one call in the graph's own capture
+// takes the pool's capacity as the bound of every later replay.
+dcsr_status refresh_replayed(dcsr_handle h, hipStream_t s);
 // The SpMV's flat offsets, row map and row-scan look-back block (sized for
 // the current pool), and the bookkeeping once a stream-ordered scan has
 // rebuilt them (the update's move kernel can run that scan).
@@ -228,9 +234,9 @@ dcsr_status update_fixed_scratch(dcsr_handle h, const int32_t *rows, const int32
                                  int64_t n, uint32_t flags, hipStream_t s, uint8_t *base, size_t cap);
 size_t update_scratch_bytes(dcsr_handle h, int64_t n);
 
-// matrix.hip: the live entries as (column, value) pairs in flat order, and the
-// flat offsets (current; R+1 words).
-dcsr_status copy_rows_paired(dcsr_handle h, uint2 *dst, const uint32_t **off, hipStream_t s);
+// matrix.hip: the live entries as (column, value) pairs in flat order (at most
+// cap of them), and the flat offsets (current; R+1 words).
+dcsr_status copy_rows_paired(dcsr_handle h, uint2 *dst, int64_t cap, const uint32_t **off, hipStream_t s);
 
 // The handle's sticky status word (device): scans set ST_SCAN_FALLBACK in it.
 static inline unsigned int *fault_word(dcsr_handle h) { return &h->ds->status; }

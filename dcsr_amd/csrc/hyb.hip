@@ -107,6 +107,7 @@ dcsr_status dcsr_export_hyb(dcsr_handle h, int32_t width, int64_t pitch, int32_t
     if (width > 0 && h->rows > 0 && (!ell_col || !ell_val)) return DCSR_ERR_INVALID;
     hipStream_t s = (hipStream_t)stream;
     h->last_stream = s;
+    DCSR_TRY(refresh_replayed(h, s));
     if (!h->state_known) DCSR_TRY(pull_state(h, s));
     DCSR_TRY(ensure_flat(h, s));
     const uint32_t R = (uint32_t)h->rows;

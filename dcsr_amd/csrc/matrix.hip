@@ -574,6 +574,27 @@ dcsr_status pull_state(dcsr_handle h, hipStream_t s)
     return DCSR_OK;
 }
 
+bool capturing(hipStream_t s)
+{
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+        (void)hipGetLastError();  // the null stream beside another stream's capture
+        return false;
+    }
+    return st != hipStreamCaptureStatusNone;
+}
+
+dcsr_status refresh_replayed(dcsr_handle h, hipStream_t s)
+{
+    if (!h->replayed) return DCSR_OK;
+    h->flat_dirty = true;
+    if (!capturing(s)) return pull_state(h, s);
+    h->state_known = false;
+    h->nnz_ub = h->bump_ub = h->pool_cap;
+    h->snap_valid_from = h->snap_seq + 1;
+    return DCSR_OK;
+}
+
 void state_exact(dcsr_handle h)
 {
     h->state_known = true;
@@ -906,11 +927,9 @@ dcsr_status dcsr_load_csr(dcsr_handle h, const int32_t *row_offsets, const int32
 
 // Flat exclusive offsets of the live rows (u32, R+1 entries) and their row
 // map: the SpMV's own, scanned again only where they are not known to be
-// current (a structural change outside the update pipeline, or an update that
-// may be replayed from a captured graph without this library being called).
+// current (a structural change outside the update pipeline; refresh_replayed).
 static dcsr_status flat_rows(dcsr_handle h, hipStream_t s, const uint32_t **off, const uint32_t **rowmap)
 {
-    if (h->flat_replayed) h->flat_dirty = true;
     DCSR_TRY(ensure_flat(h, s));
     *off = (const uint32_t *)h->ws.ptr[WS_FOFF];
     *rowmap = (const uint32_t *)h->ws.ptr[WS_ROWMAP];
@@ -939,12 +958,12 @@ static void launch_copy_rows(dcsr_handle h, const uint32_t *off, const uint32_t 
 }
 
 // The live entries as (column, value) pairs in flat order; *off receives the
-// flat offsets (state known).
-dcsr_status copy_rows_paired(dcsr_handle h, uint2 *dst, const uint32_t **off, hipStream_t s)
+// flat offsets (state known; cap: the entries that dst holds).
+dcsr_status copy_rows_paired(dcsr_handle h, uint2 *dst, int64_t cap, const uint32_t **off, hipStream_t s)
 {
     const uint32_t *rowmap;
     DCSR_TRY(flat_rows(h, s, off, &rowmap));
-    launch_copy_rows(h, *off, rowmap, h->nnz_h, ~0ull, nullptr, nullptr, nullptr, s, dst);
+    launch_copy_rows(h, *off, rowmap, h->nnz_h, (uint64_t)cap, nullptr, nullptr, nullptr, s, dst);
     DCSR_HIP(hipGetLastError());
     return DCSR_OK;
 }
@@ -1000,6 +1019,7 @@ dcsr_status dcsr_export_csr(dcsr_handle h, int32_t *row_offsets, int32_t *cols, 
     hipStream_t s = (hipStream_t)stream;
     h->last_stream = s;
     const int64_t R = h->rows;
+    DCSR_TRY(refresh_replayed(h, s));
     const bool canon = (flags & DCSR_EXPORT_CANONICAL) && !h->canonical;
     if (canon || !cols || !vals || cap < 0) {
         if (!h->state_known) DCSR_TRY(pull_state(h, s));
@@ -1104,6 +1124,7 @@ dcsr_status dcsr_compact(dcsr_handle h, dcsr_stream_t stream)
     if (!h) return DCSR_ERR_INVALID;
     hipStream_t s = (hipStream_t)stream;
     h->last_stream = s;
+    DCSR_TRY(refresh_replayed(h, s));
     if (!h->state_known) DCSR_TRY(pull_state(h, s));
     // keep the capacity, release retired chunks
     return compact_into(h, h->pool_cap, s);

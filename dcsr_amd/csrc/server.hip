@@ -484,14 +484,15 @@ dcsr_status dcsr_server_create(dcsr_server *out, dcsr_handle h, int32_t max_cols
     // (the first update would otherwise rewrite every row under running
     // queries)
     (void)hipDeviceSynchronize();
-    if (!h->canonical) {
+    st = refresh_replayed(h, S->su);
+    if (st == DCSR_OK && !h->canonical) {
         if (!h->state_known) st = pull_state(h, S->su);
         if (st == DCSR_OK) st = canonicalize(h, S->su);
         (void)hipStreamSynchronize(S->su);
-        if (st != DCSR_OK) {
-            dcsr_server_destroy(S);
-            return st;
-        }
+    }
+    if (st != DCSR_OK) {
+        dcsr_server_destroy(S);
+        return st;
     }
     memset(&S->stats, 0, sizeof(S->stats));
     S->sched = std::thread(scheduler_loop, S);

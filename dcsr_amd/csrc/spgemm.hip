@@ -953,6 +953,8 @@ dcsr_status dcsr_spgemm(dcsr_handle A, dcsr_handle B, dcsr_handle C, dcsr_stream
     if (A->cols != B->rows || C->rows != A->rows || C->cols != B->cols) return DCSR_ERR_INVALID;
     hipStream_t s = (hipStream_t)stream;
     A->last_stream = B->last_stream = C->last_stream = s;
+    DCSR_TRY(refresh_replayed(A, s));
+    DCSR_TRY(refresh_replayed(B, s));
     if (!A->state_known) DCSR_TRY(pull_state(A, s));
     if (!B->state_known) DCSR_TRY(pull_state(B, s));
     const uint32_t R = (uint32_t)A->rows;
@@ -975,7 +977,7 @@ dcsr_status dcsr_spgemm(dcsr_handle A, dcsr_handle B, dcsr_handle C, dcsr_stream
     const uint32_t *b_foff;
     uint2 *b_ent, *ent;
     DCSR_TRY(ws_get(C, WS_SG_BENT, (size_t)(B->nnz_h + 1) * 8, (void **)&b_ent));
-    DCSR_TRY(copy_rows_paired(B, b_ent, &b_foff, s));
+    DCSR_TRY(copy_rows_paired(B, b_ent, B->nnz_h, &b_foff, s));
     DCSR_TRY(ws_get(C, WS_SG_ENT, (size_t)(A->nnz_h + 1) * 8, (void **)&ent));
 
     // 1. partial counts, classes, offsets

@@ -1149,6 +1149,7 @@ static dcsr_status launch_wide(dcsr_handle h, const float *X, int64_t ldx, float
 static dcsr_status prepare_compute(dcsr_handle h, hipStream_t s)
 {
     h->last_stream = s;
+    DCSR_TRY(refresh_replayed(h, s));
     return ensure_flat(h, s);
 }
 
@@ -1179,8 +1180,7 @@ static bool pnl_eligible(dcsr_handle h)
 // record it, and a copy is never built in a capture (it allocates).
 static bool pnl_allowed(dcsr_handle h, hipStream_t s)
 {
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap == hipStreamCaptureStatusNone) return true;
+    if (!capturing(s)) return true;
     return h->pnl_valid && h->nnz_h >= 2 * h->pnl_min_nnz && h->cols * 5 >= h->pnl_cols * 12;
 }
 

@@ -1454,6 +1454,7 @@ struct BufSrc {
     size_t cap, used;
     bool measure;
     hipStream_t s;  // orders the zero fill of grown control-word slots
+    bool recorded;  // under capture
 };
 
 dcsr_status take(BufSrc &src, WsSlot slot, size_t bytes, void **out)
@@ -1518,10 +1519,11 @@ dcsr_status upd_bufs_src(BufSrc &src, int64_t n, UpdBufs &b)
         b.tt = b.hist + (size_t)ptiles(n) * (2 * NPLAN);
         b.tp = b.tt + (size_t)ptiles(n) * TT_WORDS;
     }
-    // span tables grow with the matrix, so a fixed region goes without them
+    // span tables grow with the matrix, so a fixed region goes without them, and
+    // so does a capture, whose replays may meet a larger one
     b.pspan = b.mspan = nullptr;
     b.rowt = nullptr;
-    if (!src.base && !src.measure) {
+    if (!src.base && !src.measure && !src.recorded) {
         const int64_t live = live_bound(h);
         DCSR_TRY(take(src, WS_PSPAN, (size_t)((live + n) / PR_SPAN + 2) * 4, (void **)&b.pspan));
         DCSR_TRY(take(src, WS_MSPAN, (size_t)(live / MV_SPAN + 2) * 4, (void **)&b.mspan));
@@ -1531,8 +1533,13 @@ dcsr_status upd_bufs_src(BufSrc &src, int64_t n, UpdBufs &b)
 
 dcsr_status upd_bufs(dcsr_handle h, int64_t n, UpdBufs &b, hipStream_t s)
 {
-    BufSrc src{h, nullptr, 0, 0, false, s};
+    BufSrc src{h, nullptr, 0, 0, false, s, capturing(s)};
     DCSR_TRY(upd_bufs_src(src, n, b));
+    if (src.recorded) {
+        // every replay would write the same tag: no row map
+        h->replayed = true;
+        return DCSR_OK;
+    }
     // zeroed when first allocated: no entry carries a tag before the first
     // update's
     if (h->rows > 0) DCSR_TRY(ws_get_zeroed(h, WS_ROWT, (size_t)h->rows * 8, (void **)&b.rowt, s));
@@ -1893,7 +1900,7 @@ static dcsr_status update_nosync(dcsr_handle h, const int32_t *rows, const int32
 // Bytes of scratch an update of n triples on h carves from a fixed region.
 size_t update_scratch_bytes(dcsr_handle h, int64_t n)
 {
-    BufSrc src{h, nullptr, 0, 0, true, nullptr};
+    BufSrc src{h, nullptr, 0, 0, true, nullptr, false};
     UpdBufs b;
     if (upd_bufs_src(src, n, b) != DCSR_OK) return ~size_t(0);
     return src.used;
@@ -1910,12 +1917,11 @@ dcsr_status update_fixed_scratch(dcsr_handle h, const int32_t *rows, const int32
     if (!h->canonical) return DCSR_ERR_INVALID;
     h->last_stream = s;
     if (n == 0) return DCSR_OK;
-    BufSrc src{h, base, cap, 0, false, s};
+    BufSrc src{h, base, cap, 0, false, s, capturing(s)};
     UpdBufs b;
     DCSR_TRY(upd_bufs_src(src, n, b));
     const bool nosync = (flags & DCSR_UPDATE_NOSYNC) != 0;
-    hipStreamCaptureStatus cap_st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &cap_st) == hipSuccess && cap_st != hipStreamCaptureStatusNone) h->flat_replayed = true;
+    if (src.recorded) h->replayed = true;
     if (nosync) refresh_bounds(h);
     const uint64_t seq = nosync ? snapshot_next(h) : 0;
     const int64_t claimed = claims_bound(h, n);
@@ -1939,6 +1945,7 @@ dcsr_status dcsr_update(dcsr_handle h, const int32_t *rows, const int32_t *cols,
     if (n >= (int64_t)0x7ffffff0ll) return DCSR_ERR_INVALID;
     hipStream_t s = (hipStream_t)stream;
     h->last_stream = s;
+    if (h->replayed && !capturing(s)) DCSR_TRY(refresh_replayed(h, s));
     if (flags & DCSR_UPDATE_NOSYNC) return update_nosync(h, rows, cols, vals, n, flags, s);
     return update_sync(h, rows, cols, vals, n, flags, s);
 }

@@ -372,7 +372,10 @@ void dcsr_set_scan_wait_limit(int32_t polls);
  * with DCSR_UPDATE_NOSYNC).  The scratch is one fixed device array per GPU
  * (8 MiB, held until the process ends) shared by every call on that GPU:
  * calls that overlap on one GPU (two streams, two threads) race, so callers
- * serialize them. */
+ * serialize them.  Replays change a matrix without a call, so once an update
+ * of it has been captured, later calls on it outside a capture read its state
+ * back first (they sync), and a product captured afterwards covers whatever
+ * its pool can hold. */
 dcsr_status dcsr_update_noalloc(dcsr_handle h, const int32_t *rows, const int32_t *cols, const float *vals,
                                 int64_t n, uint32_t flags, dcsr_stream_t stream);
 int64_t dcsr_update_noalloc_max_triples(void);
