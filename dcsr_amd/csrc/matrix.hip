@@ -1025,6 +1025,7 @@ dcsr_status dcsr_export_csr(dcsr_handle h, int32_t *row_offsets, int32_t *cols, 
         if (!h->state_known) DCSR_TRY(pull_state(h, s));
         if (!canon && cap < h->nnz_h) return DCSR_ERR_CAPACITY;
         if (h->nnz_h > 0 && (!cols || !vals)) return DCSR_ERR_INVALID;
+        if (canon && cap < 0) return DCSR_ERR_CAPACITY;  // the kernels compare it unsigned
         if (canon) return export_canonical(h, row_offsets, cols, vals, cap, nnz_out, s);
     }
     if (h->state_known && cap < h->nnz_h) return DCSR_ERR_CAPACITY;
