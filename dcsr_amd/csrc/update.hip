@@ -1749,7 +1749,11 @@ dcsr_status update_prepare(dcsr_handle h, const int32_t *rows, const int32_t *co
                                                     pack_tiles(n), h->ds, 0, 0);
             DCSR_HIP(hipGetLastError());
             DCSR_TRY(pull_state(h, s));
-            if (h->hs->ubad) return DCSR_ERR_BAD_INDEX;
+            if (h->hs->ubad) {
+                // the next batch may be one that only adds to the flag
+                k_upd_validate_begin<<<1, 1, 0, s>>>(h->ds);
+                return DCSR_ERR_BAD_INDEX;
+            }
         }
         if (!h->state_known) DCSR_TRY(pull_state(h, s));
         DCSR_TRY(canonicalize(h, s));
