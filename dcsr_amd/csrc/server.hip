@@ -331,21 +331,19 @@ static dcsr_status run_queries(dcsr_server_s *S, const std::vector<Req> &g)
     dcsr_handle h = S->h;
     hipStream_t s = S->sq;
     dcsr_status st = DCSR_OK;
-    std::vector<const dcsr_request *> pack;
+    std::vector<const dcsr_request *> pack, whole;
     for (const Req &q : g) {
         // whole lines already: a request of 32-column blocks whose rows start
         // on lines is its own packed operand (packing would move it four
         // times and run the same passes over A)
-        if (g.size() > 1 && q.r.kind == DCSR_REQ_SPMM && q.r.k % 32 == 0 && q.r.ldx % 32 == 0 && q.r.ldy % 4 == 0 &&
-            (uintptr_t)q.r.x % 128 == 0 && (uintptr_t)q.r.y % 16 == 0) {
-            if (st == DCSR_OK) st = run_one(S, q.r);
-        } else {
-            pack.push_back(&q.r);
-        }
+        const bool lines = q.r.kind == DCSR_REQ_SPMM && q.r.k % 32 == 0 && q.r.ldx % 32 == 0 && q.r.ldy % 4 == 0 &&
+                           (uintptr_t)q.r.x % 128 == 0 && (uintptr_t)q.r.y % 16 == 0;
+        (lines ? whole : pack).push_back(&q.r);
     }
-    if (pack.size() == 1) {
-        if (st == DCSR_OK) st = run_one(S, *pack[0]);
-    } else if (pack.size() > 1 && st == DCSR_OK) {
+    if (pack.size() < 2) {
+        for (const Req &q : g)
+            if (st == DCSR_OK) st = run_one(S, q.r);
+    } else {
         const int slot = S->slot;
         S->slot = (S->slot + 1) % S->nslots;
         // the host must not rewrite a slot whose previous copy is pending
@@ -367,8 +365,13 @@ static dcsr_status run_queries(dcsr_server_s *S, const std::vector<Req> &g)
         const unsigned nb = (unsigned)((Kp + 31) / 32);
         const auto tiles = [](int64_t n) { return (unsigned)((n + PK_ROWS - 1) / PK_ROWS < 2048 ? (n + PK_ROWS - 1) / PK_ROWS : 2048); };
         if (C > 0) k_pack<<<dim3(tiles(C), nb), PK_TB, 0, s>>>(dd, (int)pack.size(), C, K, Kp, ld, S->X);
-        st = dcsr_spmm_dense(h, S->X, Kp, ld, S->Y, ld, 1.0f, 0.0f, s);
-        if (R > 0) k_unpack<<<dim3(tiles(R), nb), PK_TB, 0, s>>>(dd, (int)pack.size(), R, K, Kp, ld, S->Y);
+        // the others between the last read of a packed operand and the first
+        // write of a packed result: a request may write what an earlier one
+        // reads
+        for (const dcsr_request *r : whole)
+            if (st == DCSR_OK) st = run_one(S, *r);
+        if (st == DCSR_OK) st = dcsr_spmm_dense(h, S->X, Kp, ld, S->Y, ld, 1.0f, 0.0f, s);
+        if (R > 0 && st == DCSR_OK) k_unpack<<<dim3(tiles(R), nb), PK_TB, 0, s>>>(dd, (int)pack.size(), R, K, Kp, ld, S->Y);
         if (hipGetLastError() != hipSuccess) st = DCSR_ERR_HIP;
         (void)hipEventRecord(S->slot_ev[slot], s);
         S->slot_used[slot] = 1;
