@@ -1173,17 +1173,6 @@ static bool pnl_eligible(dcsr_handle h)
     return pnl_panels(h) * (h->rows + 1) < (1ll << 31);
 }
 
-// Whether a product on s may go through the copy.  A captured product replays
-// the copy that it was recorded with, where the direct kernel follows later
-// updates: only matrices of twice the entries and of 2.4 panels, on which the
-// direct kernel costs the most (2.6 against 1.4 ms at 10M columns / 160M entries),
-// record it, and a copy is never built in a capture (it allocates).
-static bool pnl_allowed(dcsr_handle h, hipStream_t s)
-{
-    if (!capturing(s)) return true;
-    return h->pnl_valid && h->nnz_h >= 2 * h->pnl_min_nnz && h->cols * 5 >= h->pnl_cols * 12;
-}
-
 static dcsr_status build_panels(dcsr_handle h, hipStream_t s)
 {
     const int64_t R = h->rows;
@@ -1260,7 +1249,9 @@ dcsr_status dcsr_spmv(dcsr_handle h, const float *x, float *y, float alpha, floa
     h->last_stream = s;
     if (h->rows == 0) return DCSR_OK;
     DCSR_TRY(prepare_compute(h, s));
-    if (pnl_eligible(h) && pnl_allowed(h, s)) {
+    // a capture records the direct kernel, which follows later updates; the copy
+    // would replay the values it was made from, and may be freed
+    if (pnl_eligible(h) && !capturing(s)) {
         // the copy costs about two thirds of a direct SpMV and saves about a
         // third of one per later call: build it on the second call of a
         // structure when the last structure that saw SpMVs saw

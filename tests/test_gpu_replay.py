@@ -137,3 +137,39 @@ def test_a_product_in_the_graph_follows_the_rows(entry):
         t.y.fill_(7.0)
     check_healthy(t.m)
     t.m.close()
+
+
+def test_a_captured_product_of_a_paneled_matrix_follows_updates(monkeypatch):
+    """Many panels and many entries per panel: the copy that an eager product
+    takes is not what a capture records."""
+    import torch
+    import dcsr_amd
+    monkeypatch.setenv("DCSR_SPMV_PANEL_COLS", "300")
+    monkeypatch.setenv("DCSR_SPMV_PANEL_MIN_NNZ", "500")
+    C, n = 3_000, 4_000
+    rng = np.random.default_rng(7)
+    key = np.sort(rng.permutation(R * C)[:n])
+    r, c = (key // C).astype(np.int32), (key % C).astype(np.int32)
+    v = rng.integers(1, 9, n).astype(np.float32)
+    m = dcsr_amd.DcsrMatrix(R, C, pool_factor=8.0)
+    m.LoadMatrix(r, c, v)
+    xh = rng.integers(-4, 5, C).astype(np.float32)
+    x, y = torch.from_numpy(xh).cuda(), torch.empty(R, device="cuda")
+    s, g = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(s):
+        for _ in range(5):
+            m.spmv(x, y)
+        assert m.info()["spmv_paneled"] == 1
+        with torch.cuda.graph(g, stream=s):
+            m.spmv(x, y)
+    want = np.zeros(R)
+    np.add.at(want, r, v * xh[c])
+    for k in range(3):
+        y.fill_(7.0)
+        g.replay()
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(y.cpu().numpy(), want.astype(np.float32))
+        m.UpdateMatrix(r, c, np.full(n, k + 1.0, np.float32))  # in place: the rows stay where they are
+        np.add.at(want, r, (k + 1.0) * xh[c])
+    m.close()
