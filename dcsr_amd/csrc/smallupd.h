@@ -457,21 +457,35 @@ __device__ __forceinline__ void su_probe(const SmallArgs &A, uint32_t u0, uint32
 #pragma unroll
     for (int q = 0; q < PT; ++q) {
         const uint32_t u = u0 + (uint32_t)q * step;
-        if (u >= nu) continue;
         float v = sum[q];
-        uint32_t code;
-        if (hit[q]) {
-            v = old[q] + v;
-            code = v != 0.0f ? C_ADD : C_DEL;
-        } else {
-            code = v != 0.0f ? C_INS : C_NOP;
+        uint32_t code = C_NOP;
+        if (u < nu) {
+            if (hit[q]) {
+                v = old[q] + v;
+                code = v != 0.0f ? C_ADD : C_DEL;
+            } else {
+                code = v != 0.0f ? C_INS : C_NOP;
+            }
+            A.uval[u] = v;
+            A.upos[u] = pos[q];
+            A.ucode[u] = code;
         }
-        A.uval[u] = v;
-        A.upos[u] = pos[q];
-        A.ucode[u] = code;
         if constexpr (FROM != P_FUSED) {
-            if (code == C_INS) atomicAdd(&A.tins[tq[q]], 1u);
-            else if (code == C_DEL) atomicAdd(&A.tdel[tq[q]], 1u);
+            // the wave's coordinates are in row order: the first one of a row adds
+            // the row's counts.  One atomic per coordinate took 5,583 us where
+            // 500,000 of them fall into four rows (93 so) and 117 for 10,000 (6)
+            static_assert(PT == 1, "a wave's coordinates are consecutive");
+            const int lane = lane_id();
+            const uint32_t before = (uint32_t)__shfl_up((int)tq[q], 1);
+            const uint64_t heads = __ballot(u < nu && (lane == 0 || before != tq[q]));
+            const uint64_t im = __ballot(code == C_INS), dm = __ballot(code == C_DEL);
+            if ((heads >> lane) & 1u) {
+                const uint64_t next = heads & ~((2ull << lane) - 1ull);
+                const uint64_t own = (next ? (next & (0ull - next)) - 1ull : ~0ull) & ~((1ull << lane) - 1ull);
+                const uint32_t ni = (uint32_t)__popcll(im & own), nd = (uint32_t)__popcll(dm & own);
+                if (ni) atomicAdd(&A.tins[tq[q]], ni);
+                if (nd) atomicAdd(&A.tdel[tq[q]], nd);
+            }
         }
     }
 }
