@@ -39,13 +39,18 @@ constexpr uint32_t BMAX = 4096;  // triples per matrix per step
 constexpr int KB = 12;           // bits of a local row / column / arrival index
 constexpr uint32_t LMAX = 1u << KB;
 constexpr int PT = BMAX / BT;    // records per thread
+// Triples of one row before the batch is sorted by digits instead of ranked inside
+// its rows, a round per triple of the fullest.  600 matrices, two steps: 4,096
+// triples at one coordinate 6,554 -> 1,648 us, 1,000 in one row 1,885 -> 1,214; 100 in
+// one row 409 -> 404.  Limits of 16 to 128 differ by less than the runs do.
+constexpr uint32_t BT_CROWD = 64;
 constexpr int RL = 16;           // lanes per touched row
 constexpr int NTM = BT / RL;     // rows in flight per workgroup
 constexpr int RC = 2 * RL;       // entries of a row met at once (two per lane)
 static_assert(BMAX == LMAX && PT % 2 == 0, "row counters and records share their split over the threads");
 enum { C_NOP = 0, C_ADD = 1, C_DEL = 2, C_INS = 3 };
 
-enum { SM_BAD = 0, SM_OK, SM_BASE, SM_INS, SM_ADD, SM_DEL, SM_LONG, SM_WORDS };
+enum { SM_CROWD = 0, SM_OK, SM_BASE, SM_INS, SM_ADD, SM_DEL, SM_LONG, SM_WORDS };
 // A workgroup's records.  Reused in order: buckets -> coordinates; sorted keys
 // -> positions and codes, new row lengths; sorted values -> chunk offsets; row
 // counters -> row starts in the buckets -> first coordinate of each row.
@@ -94,6 +99,69 @@ __device__ __forceinline__ uint32_t block_excl(uint32_t v, uint32_t *lw, uint32_
     __syncthreads();
     *total = tot;
     return carry + inc - v;
+}
+
+// Stable sort of the nb keys in S.sk (below 2^24, in arrival order) with S.sv
+// along: LSD passes of 8 bits in place, a pass's records in registers, wave w
+// ranking those from w * 64 * PT.  The 16-bit counters of every wave and digit
+// lie in S.cnt.  The caller has synchronized.
+__device__ __forceinline__ void batch_radix_sort(BatchLds &S, uint32_t nb)
+{
+    static_assert(NW * 256 <= 2 * (BMAX / 2 + 2), "the counters fit the row counters");
+    uint16_t *cnt = reinterpret_cast<uint16_t *>(S.cnt);
+    // opaque to the compiler: what follows from it is computed here, not kept in
+    // registers across the matrices (18 registers spilled, not 22)
+    uint32_t t = threadIdx.x;
+    asm volatile("" : "+v"(t));
+    const uint32_t lane = t & 63u, w = t >> 6, wb = w * (64 * PT);
+    const uint64_t lt = (1ull << lane) - 1ull;
+#pragma unroll 1
+    for (int shift = 0; shift < 2 * KB; shift += 8) {
+        for (uint32_t i = t; i < NW * 128; i += BT) S.cnt[i] = 0u;
+        __syncthreads();
+#pragma unroll 1
+        for (uint32_t i = wb + lane; i < wb + 64 * PT; i += 64) {
+            const bool ok = i < nb;
+            const uint32_t d = ok ? (S.sk[i] >> shift) & 255u : 0u;
+            const uint64_t peers = wave_match_digit8(d, __ballot(ok));
+            const int leader = __ffsll((long long)peers) - 1;
+            const uint32_t b = cnt[w * 256 + d];
+            if (ok && (int)lane == leader) cnt[w * 256 + d] = (uint16_t)(b + (uint32_t)__popcll(peers));
+            S.urc[i] = b + (uint32_t)__popcll(peers & lt);
+        }
+        __syncthreads();
+        uint32_t sum = 0, tot;
+        if (t < 256)
+#pragma unroll 1
+            for (int i = 0; i < NW; ++i) sum += cnt[i * 256 + t];
+        uint32_t base = block_excl(sum, S.lw, &tot);
+        if (t < 256) {
+#pragma unroll 1
+            for (int i = 0; i < NW; ++i) {
+                const uint32_t c = cnt[i * 256 + t];
+                cnt[i * 256 + t] = (uint16_t)base;
+                base += c;
+            }
+        }
+        __syncthreads();
+        uint32_t k[PT], p[PT];
+        float v[PT];
+#pragma unroll
+        for (int j = 0; j < PT; ++j) {
+            const uint32_t i = wb + (uint32_t)j * 64 + lane;
+            k[j] = S.sk[i];
+            v[j] = S.sv[i];
+            p[j] = cnt[w * 256 + ((k[j] >> shift) & 255u)] + S.urc[i];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < PT; ++j) {
+            if (wb + (uint32_t)j * 64 + lane >= nb) continue;
+            S.sk[p[j]] = k[j];
+            S.sv[p[j]] = v[j];
+        }
+        __syncthreads();
+    }
 }
 
 // Counters of the matrices one workgroup updated, kept by its thread 0 and
@@ -165,6 +233,7 @@ __device__ __forceinline__ void batch_update(uint32_t m, const uint32_t *__restr
         } else {
             const uint32_t sh = ((uint32_t)r & 1u) * 16u;
             off[j] = (atomicAdd(&S.cnt[(uint32_t)r >> 1], 1u << sh) >> sh) & 0xffffu;
+            if (off[j] == BT_CROWD) S.sm[SM_CROWD] = 1u;
         }
     }
     if (__syncthreads_or(bad)) {
@@ -172,40 +241,51 @@ __device__ __forceinline__ void batch_update(uint32_t m, const uint32_t *__restr
         return;
     }
     uint32_t tot;
-    {
+    if (S.sm[SM_CROWD]) {
+#pragma unroll
+        for (int j = 0; j < PT; ++j) {
+            const uint32_t i = t + (uint32_t)j * BT;
+            if (i < nb) {
+                S.sk[i] = ((uint32_t)rr[j] << KB) | (uint32_t)cc[j];
+                S.sv[i] = vv[j];
+            }
+        }
+        __syncthreads();
+        batch_radix_sort(S, nb);
+    } else {
         // bucket starts: PT rows (two to a counter word) per thread
-        uint32_t w[PT / 2], sum = 0;
+        {
+            uint32_t w[PT / 2], sum = 0;
 #pragma unroll
-        for (int i = 0; i < PT / 2; ++i) {
-            w[i] = S.cnt[t * (PT / 2) + i];
-            sum += (w[i] & 0xffffu) + (w[i] >> 16);
-        }
-        uint32_t b = block_excl(sum, S.lw, &tot);
+            for (int i = 0; i < PT / 2; ++i) {
+                w[i] = S.cnt[t * (PT / 2) + i];
+                sum += (w[i] & 0xffffu) + (w[i] >> 16);
+            }
+            uint32_t b = block_excl(sum, S.lw, &tot);
 #pragma unroll
-        for (int i = 0; i < PT / 2; ++i) {
-            const uint32_t a = b + (w[i] & 0xffffu);
-            S.cnt[t * (PT / 2) + i] = b | (a << 16);
-            b = a + (w[i] >> 16);
+            for (int i = 0; i < PT / 2; ++i) {
+                const uint32_t a = b + (w[i] & 0xffffu);
+                S.cnt[t * (PT / 2) + i] = b | (a << 16);
+                b = a + (w[i] >> 16);
+            }
+            if (t == 0) S.cnt[BMAX / 2] = nb;
         }
-        if (t == 0) S.cnt[BMAX / 2] = nb;
-    }
-    __syncthreads();
-    const uint16_t *start = reinterpret_cast<const uint16_t *>(S.cnt);
-    uint32_t lo[PT], n[PT], me[PT], most = 0;
+        __syncthreads();
+        const uint16_t *start = reinterpret_cast<const uint16_t *>(S.cnt);
+        uint32_t lo[PT], n[PT], me[PT], most = 0;
 #pragma unroll
-    for (int j = 0; j < PT; ++j) {
-        const uint32_t i = t + (uint32_t)j * BT;
-        lo[j] = n[j] = me[j] = 0;
-        if (i < nb) {
-            lo[j] = start[rr[j]];
-            n[j] = start[rr[j] + 1] - lo[j];
-            me[j] = ((uint32_t)cc[j] << KB) | i;
-            S.urc[lo[j] + off[j]] = me[j];
-            most = n[j] > most ? n[j] : most;
+        for (int j = 0; j < PT; ++j) {
+            const uint32_t i = t + (uint32_t)j * BT;
+            lo[j] = n[j] = me[j] = 0;
+            if (i < nb) {
+                lo[j] = start[rr[j]];
+                n[j] = start[rr[j] + 1] - lo[j];
+                me[j] = ((uint32_t)cc[j] << KB) | i;
+                S.urc[lo[j] + off[j]] = me[j];
+                most = n[j] > most ? n[j] : most;
+            }
         }
-    }
-    __syncthreads();
-    {
+        __syncthreads();
         uint32_t rk[PT];
 #pragma unroll
         for (int j = 0; j < PT; ++j) rk[j] = lo[j];
@@ -221,8 +301,8 @@ __device__ __forceinline__ void batch_update(uint32_t m, const uint32_t *__restr
                 S.sv[rk[j]] = vv[j];
             }
         }
+        __syncthreads();
     }
-    __syncthreads();
     // U2: distinct coordinates (heads) and touched rows (row heads), four
     // consecutive records per thread; duplicates are summed from 0 in arrival
     // order
