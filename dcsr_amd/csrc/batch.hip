@@ -506,7 +506,9 @@ __device__ __forceinline__ void batch_update(uint32_t m, const uint32_t *__restr
     // unchanged structure get their added values written in place.  With x, the
     // row's product is taken from the entries at hand (each lane's in order, then
     // a fixed tree): reading the rewritten rows again for it would be a third of
-    // the step's bytes.
+    // the step's bytes.  It is summed in double, whatever the row's length: 16
+    // chains in float were 7.4e-8 rms off over 4,096 entries, where batch_spmv's 64
+    // lanes were 4.3e-8; now 3.4e-8 at most from 4 to 4,000
     {
         uint32_t st = 0, L = 0, st1 = 0, L1 = 0;
         int32_t c0 = 0, c1 = 0;
@@ -555,14 +557,14 @@ __device__ __forceinline__ void batch_update(uint32_t m, const uint32_t *__restr
             } else {
                 const uint32_t g = gbase + (S.urc[u] >> KB);
                 const uint32_t dst = base + tdst[tt];
-                float prod = 0.0f;
+                double prod = 0.0;
                 for (uint32_t q = u + tl; q < ue; q += RL) {
                     if (upc[q] >> 14 != C_INS) continue;
                     const uint64_t d = (uint64_t)dst + (upc[q] & 0x3fffu);
                     const int32_t c = (int32_t)(S.urc[q] & (LMAX - 1));
                     pcol[d] = c;
                     pval[d] = S.uval[q];
-                    if (x) prod = prod + S.uval[q] * x[c];
+                    if (x) prod = prod + (double)(S.uval[q] * x[c]);
                 }
                 uint32_t sh = 0;  // inserts less deletes so far
                 for (uint32_t i0 = 0;;) {
@@ -591,12 +593,12 @@ __device__ __forceinline__ void batch_update(uint32_t m, const uint32_t *__restr
                     if (k0) {
                         pcol[(uint64_t)dst + (p0 + s0)] = c0;
                         pval[(uint64_t)dst + (p0 + s0)] = v0;
-                        prod = prod + v0 * x0;
+                        prod = prod + (double)(v0 * x0);
                     }
                     if (k1) {
                         pcol[(uint64_t)dst + (p1 + s1)] = c1;
                         pval[(uint64_t)dst + (p1 + s1)] = v1;
-                        prod = prod + v1 * x1;
+                        prod = prod + (double)(v1 * x1);
                     }
                     if (last) break;
                     i0 += RC;
@@ -609,11 +611,10 @@ __device__ __forceinline__ void batch_update(uint32_t m, const uint32_t *__restr
                         v1 = pval[(uint64_t)st + i0 + RL + tl];
                     }
                 }
-#pragma unroll
-                for (int o = RL / 2; o >= 1; o >>= 1) prod += __shfl_xor(prod, o);
+                prod = dpp_row_sum_f64(prod);
                 if (tl == 0) {
                     if (x) {
-                        y[g] = prod;
+                        y[g] = (float)prod;
                         atomicOr(&S.done[(g - gbase) >> 5], 1u << ((g - gbase) & 31u));
                     }
                     row_start[g] = dst;

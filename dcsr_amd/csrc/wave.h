@@ -160,6 +160,23 @@ __device__ __forceinline__ void block_sum_n(uint32_t (&v)[N], uint32_t (*lds)[N]
     __syncthreads();
 }
 
+// Sum over the 16 lanes of a DPP row (in every lane; the row's lanes are active).
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double v)
+{
+    const uint64_t b = (uint64_t)__double_as_longlong(v);
+    const uint32_t lo = dpp_u32<CTRL>((uint32_t)b, (uint32_t)b), hi = dpp_u32<CTRL>((uint32_t)(b >> 32), (uint32_t)(b >> 32));
+    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+__device__ __forceinline__ double dpp_row_sum_f64(double v)
+{
+    v += dpp_f64<DPP_ROW_ROR(8)>(v);
+    v += dpp_f64<DPP_ROW_ROR(4)>(v);
+    v += dpp_f64<DPP_ROW_ROR(2)>(v);
+    v += dpp_f64<DPP_ROW_ROR(1)>(v);
+    return v;
+}
+
 // Fixed-order float sum over the wave (tree over lane index).
 __device__ __forceinline__ float wave_sum_f32(float v)
 {
