@@ -160,20 +160,36 @@ __device__ __forceinline__ void block_sum_n(uint32_t (&v)[N], uint32_t (*lds)[N]
     __syncthreads();
 }
 
-// Sum over the 16 lanes of a DPP row (in every lane; the row's lanes are active).
-template <int CTRL>
-__device__ __forceinline__ double dpp_f64(double v)
+template <int CTRL, int ROW_MASK = 0xf>
+__device__ __forceinline__ double dpp_f64(double old, double src)
 {
-    const uint64_t b = (uint64_t)__double_as_longlong(v);
-    const uint32_t lo = dpp_u32<CTRL>((uint32_t)b, (uint32_t)b), hi = dpp_u32<CTRL>((uint32_t)(b >> 32), (uint32_t)(b >> 32));
+    const uint64_t o = (uint64_t)__double_as_longlong(old), v = (uint64_t)__double_as_longlong(src);
+    const uint32_t lo = dpp_u32<CTRL, ROW_MASK>((uint32_t)o, (uint32_t)v);
+    const uint32_t hi = dpp_u32<CTRL, ROW_MASK>((uint32_t)(o >> 32), (uint32_t)(v >> 32));
     return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
 }
+
+// Sum over the 16 lanes of a DPP row (in every lane; the row's lanes are active).
 __device__ __forceinline__ double dpp_row_sum_f64(double v)
 {
-    v += dpp_f64<DPP_ROW_ROR(8)>(v);
-    v += dpp_f64<DPP_ROW_ROR(4)>(v);
-    v += dpp_f64<DPP_ROW_ROR(2)>(v);
-    v += dpp_f64<DPP_ROW_ROR(1)>(v);
+    v += dpp_f64<DPP_ROW_ROR(8)>(v, v);
+    v += dpp_f64<DPP_ROW_ROR(4)>(v, v);
+    v += dpp_f64<DPP_ROW_ROR(2)>(v, v);
+    v += dpp_f64<DPP_ROW_ROR(1)>(v, v);
+    return v;
+}
+
+// wave_seg_incl_scan_f32 in double.
+__device__ __forceinline__ double wave_seg_incl_scan_f64(double v, uint32_t seg)
+{
+    double t;
+    uint32_t s;
+    t = dpp_f64<DPP_ROW_SHR(1)>(0.0, v); s = dpp_u32<DPP_ROW_SHR(1)>(0xffffffffu, seg); v += (s == seg) ? t : 0.0;
+    t = dpp_f64<DPP_ROW_SHR(2)>(0.0, v); s = dpp_u32<DPP_ROW_SHR(2)>(0xffffffffu, seg); v += (s == seg) ? t : 0.0;
+    t = dpp_f64<DPP_ROW_SHR(4)>(0.0, v); s = dpp_u32<DPP_ROW_SHR(4)>(0xffffffffu, seg); v += (s == seg) ? t : 0.0;
+    t = dpp_f64<DPP_ROW_SHR(8)>(0.0, v); s = dpp_u32<DPP_ROW_SHR(8)>(0xffffffffu, seg); v += (s == seg) ? t : 0.0;
+    t = dpp_f64<DPP_ROW_BCAST15, 0xa>(0.0, v); s = dpp_u32<DPP_ROW_BCAST15, 0xa>(0xffffffffu, seg); v += (s == seg) ? t : 0.0;
+    t = dpp_f64<DPP_ROW_BCAST31, 0xc>(0.0, v); s = dpp_u32<DPP_ROW_BCAST31, 0xc>(0xffffffffu, seg); v += (s == seg) ? t : 0.0;
     return v;
 }
 
