@@ -99,8 +99,12 @@ __global__ __launch_bounds__(TB) void k_pack_keys(const int32_t *__restrict__ ro
 
 // The same keys for a CSR matrix: a wave owns KEY_SPAN consecutive entries and
 // walks the rows they belong to 64 at a time (wave_visit), so an entry costs a
-// search of 64 offsets in LDS instead of one of all R offsets in memory.
-constexpr uint32_t KEY_SPAN = 512;
+// search of 64 offsets in LDS instead of one of all R offsets in memory.  Entries
+// that lie further apart than KEY_WALK rows (a matrix of mostly empty rows) are
+// searched for instead, a lane's eight together: a load into 10M rows took 86 ms
+// where one wave's entries were the first row's and the last's (now 0.2), 856 us for
+// 100,000 entries a hundred rows apart (214).
+constexpr uint32_t KEY_SPAN = 512, KEY_WALK = 1024;
 __global__ __launch_bounds__(TB) void k_pack_keys_csr(const int32_t *__restrict__ off, uint32_t R,
                                                       const int32_t *__restrict__ cols,
                                                       const float *__restrict__ vals, uint32_t n, int64_t C, int cbits,
@@ -108,20 +112,50 @@ __global__ __launch_bounds__(TB) void k_pack_keys_csr(const int32_t *__restrict_
                                                       DevState *ds)
 {
     __shared__ uint32_t s_off[TB / 64][65];
+    const uint32_t *uoff = (const uint32_t *)off;
     uint64_t e0 = ((uint64_t)blockIdx.x * (TB / 64) + (threadIdx.x >> 6)) * KEY_SPAN;
     if (e0 > n) e0 = n;
     const uint32_t e1 = n - (uint32_t)e0 < KEY_SPAN ? n : (uint32_t)e0 + KEY_SPAN;
     bool bad = false, down = false;
-    wave_visit((const uint32_t *)off, R, (uint32_t)e0, e1, s_off[threadIdx.x >> 6],
-               [&](bool valid, uint32_t r, uint32_t k, uint32_t e) {
-                   if (!valid) return;
-                   const int32_t c = cols[e];
-                   if (k > 0) down |= cols[e - 1] > c;
-                   const bool b = (c < 0) | (c >= C);
-                   key[e] = b ? ~0ull : (((uint64_t)r << cbits) | (uint32_t)c);
-                   val[e] = __float_as_uint(vals[e]);
-                   bad |= b;
-               });
+    auto pack = [&](bool valid, uint32_t r, uint32_t k, uint32_t e) {
+        if (!valid) return;
+        const int32_t c = cols[e];
+        if (k > 0) down |= cols[e - 1] > c;
+        const bool b = (c < 0) | (c >= C);
+        key[e] = b ? ~0ull : (((uint64_t)r << cbits) | (uint32_t)c);
+        val[e] = __float_as_uint(vals[e]);
+        bad |= b;
+    };
+    if (e0 < e1) {
+        const uint32_t j = wave_find_last_le(uoff, R, (uint32_t)e0);
+        if (R - j <= KEY_WALK || uoff[j + KEY_WALK] >= e1) {
+            wave_visit_from(uoff, R, j, (uint32_t)e0, e1, s_off[threadIdx.x >> 6], pack);
+        } else {
+            constexpr int PER = KEY_SPAN / 64;
+            uint32_t lo[PER], hi[PER];  // off[lo] <= e < off[hi]
+            const uint32_t j1 = wave_find_last_le(uoff, R, e1 - 1) + 1;
+#pragma unroll
+            for (int q = 0; q < PER; ++q) {
+                lo[q] = j;
+                hi[q] = j1;
+            }
+            for (uint32_t span = j1 - j; span > 1; span = (span + 1) >> 1) {  // no interval is longer
+#pragma unroll
+                for (int q = 0; q < PER; ++q) {
+                    const uint32_t e = (uint32_t)e0 + (uint32_t)q * 64 + lane_id();
+                    const uint32_t mid = lo[q] + ((hi[q] - lo[q]) >> 1);
+                    const bool left = uoff[mid] > e;  // mid == lo: it is not
+                    hi[q] = left ? mid : hi[q];
+                    lo[q] = left ? lo[q] : mid;
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < PER; ++q) {
+                const uint32_t e = (uint32_t)e0 + (uint32_t)q * 64 + lane_id();
+                pack(e < e1, lo[q], e < e1 ? e - uoff[lo[q]] : 0u, e);
+            }
+        }
+    }
     if (__ballot(bad) && lane_id() == 0) atomicOr(&ds->status, ST_BAD_INDEX);
     raise_load_flag(ds, LD_UNSORTED, down);
 }

@@ -48,14 +48,13 @@ __device__ __forceinline__ uint32_t wave_find_last_le(const uint32_t *off, uint3
 // off[0..nseg] (element j at off[j*S]; off[nseg*S] = total).  For every entry, calls
 //   f(seg, k, e)   with k = e - off[seg]   (all lanes of the wave call
 // into the loop together; lanes without an entry get valid == false).
-// s_off: 65 words of LDS owned by this wave.
+// s_off: 65 words of LDS owned by this wave.  wave_visit_from: j, the segment that
+// holds e0, is known.
 template <int S = 1, class F>
-__device__ __forceinline__ void wave_visit(const uint32_t *__restrict__ off, uint32_t nseg, uint32_t e0, uint32_t e1,
-                                           uint32_t *s_off, F &&f)
+__device__ __forceinline__ void wave_visit_from(const uint32_t *__restrict__ off, uint32_t nseg, uint32_t j, uint32_t e0,
+                                                uint32_t e1, uint32_t *s_off, F &&f)
 {
     const int lane = lane_id();
-    if (e0 >= e1) return;
-    uint32_t j = wave_find_last_le<S>(off, nseg, e0);
     uint32_t e = e0;
     while (e < e1) {
         // window: segments j .. j+63, boundaries off[j .. j+64]
@@ -75,6 +74,13 @@ __device__ __forceinline__ void wave_visit(const uint32_t *__restrict__ off, uin
         j += 64;
         __builtin_amdgcn_wave_barrier();
     }
+}
+
+template <int S = 1, class F>
+__device__ __forceinline__ void wave_visit(const uint32_t *__restrict__ off, uint32_t nseg, uint32_t e0, uint32_t e1,
+                                           uint32_t *s_off, F &&f)
+{
+    if (e0 < e1) wave_visit_from<S>(off, nseg, wave_find_last_le<S>(off, nseg, e0), e0, e1, s_off, f);
 }
 
 // Start map of up to 64 * 64 items: bit i set when item i starts a segment
