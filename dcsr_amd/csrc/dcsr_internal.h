@@ -202,7 +202,8 @@ void refresh_bounds(dcsr_handle h);
 // state is known).
 static inline int64_t live_bound(dcsr_handle h) { return h->state_known ? h->nnz_h : h->nnz_ub; }
 static inline int64_t bump_bound(dcsr_handle h) { return h->state_known ? h->bump_h : h->bump_ub; }
-dcsr_status ensure_flat(dcsr_handle h, hipStream_t s);  // spmv.hip
+// spmv.hip; entries: how many rows hold, where the host's bound is not theirs yet
+dcsr_status ensure_flat(dcsr_handle h, hipStream_t s, int64_t entries = -1);
 bool capturing(hipStream_t s);
 // Before a call relies on the host mirrors, their bounds or the flat offsets:
 // a matrix that a replayed graph may have changed (h->replayed) has its state
@@ -214,6 +215,7 @@ dcsr_status refresh_replayed(dcsr_handle h, hipStream_t s);
 // rebuilt them (the update's move kernel can run that scan).
 struct FlatBufs {
     uint32_t *foff, *rowmap, *part;
+    int64_t mapcap;  // words of rowmap
 };
 dcsr_status flat_buffers(dcsr_handle h, hipStream_t s, FlatBufs *fb);  // spmv.hip
 void flat_rebuilt(dcsr_handle h);                                      // spmv.hip

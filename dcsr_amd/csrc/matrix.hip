@@ -874,7 +874,7 @@ static dcsr_status load_sorted(dcsr_handle h, const uint64_t *key, const uint32_
     // natural order, no slack: the row starts are the SpMV's flat offsets,
     // which the next product finds ready
     h->flat_dirty = true;
-    DCSR_TRY(ensure_flat(h, s));
+    DCSR_TRY(ensure_flat(h, s, n));
     k_set_loaded<<<grid_for(R > 0 ? R : 1, TB), TB, 0, s>>>(R, (const uint32_t *)h->ws.ptr[WS_FOFF], h->row_start,
                                                             h->row_len, h->row_cap, h->ds, (uint64_t)n);
     DCSR_HIP(hipGetLastError());

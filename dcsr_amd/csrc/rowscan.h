@@ -9,7 +9,8 @@
 // matrix of a few hundred thousand rows resolves in one or two rounds.  The
 // tile's granules are filled by the whole workgroup, one granule per thread
 // and a search of the tile's offsets in LDS, so that a long row does not
-// leave one thread storing its granules one by one.
+// leave one thread storing its granules one by one.  rowmap may be null: offsets
+// only.
 //
 // Used by the SpMV's own scan kernel (spmv.hip) over the row lengths, and by
 // the update's move kernel (update.hip), whose extra workgroups scan the
@@ -79,7 +80,7 @@ __device__ void rowscan_tile(uint32_t R, Lens &&lens, Prefix &&prefix, uint32_t 
     }
     if (threadIdx.x == 0) L.off[n] = L.pre + tot;
     __syncthreads();
-    {
+    if (rowmap) {
         // granules g with off[0] < g*RS_GRAN <= off[n]: the tile's row i
         // with off[i] < g*RS_GRAN <= off[i+1] (the last i with off[i] <
         // g*RS_GRAN, found by bisection)
@@ -106,5 +107,5 @@ __device__ void rowscan_tile(uint32_t R, Lens &&lens, Prefix &&prefix, uint32_t 
     }
     // the thread holding row R-1 stores the total
     if (r0 < (int64_t)R && r0 + RS_IPT >= (int64_t)R) foff[R] = a;
-    if (tile == 0 && threadIdx.x == 0) rowmap[0] = 0u;
+    if (rowmap && tile == 0 && threadIdx.x == 0) rowmap[0] = 0u;
 }

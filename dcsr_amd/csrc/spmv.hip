@@ -37,16 +37,16 @@ constexpr uint32_t GRAN = RS_GRAN;  // row-map granule (nonzeros)
 __global__ void k_rowmap(uint32_t R, const uint32_t *__restrict__ foff, uint32_t *__restrict__ rowmap, uint32_t cap)
 {
     const uint32_t total = foff[R];
-    const uint32_t ng = total / GRAN + 1;
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= ng || i >= cap) return;
-    const uint32_t e = i * GRAN;
-    uint32_t lo = 0, hi = R;  // smallest r in [0, R) with foff[r+1] >= e
-    while (lo < hi) {
-        uint32_t mid = (lo + hi) >> 1;
-        if (foff[mid + 1] >= e) hi = mid; else lo = mid + 1;
+    const uint32_t ng = total / GRAN + 1 < cap ? total / GRAN + 1 : cap;  // the offsets decide, not the grid
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < ng; i += gridDim.x * blockDim.x) {
+        const uint32_t e = i * GRAN;
+        uint32_t lo = 0, hi = R;  // smallest r in [0, R) with foff[r+1] >= e
+        while (lo < hi) {
+            uint32_t mid = (lo + hi) >> 1;
+            if (foff[mid + 1] >= e) hi = mid; else lo = mid + 1;
+        }
+        rowmap[i] = lo;
     }
-    rowmap[i] = lo;
 }
 
 // Flat offsets and row map of the row lengths (rowscan.h), one tile per
@@ -1055,6 +1055,7 @@ dcsr_status flat_buffers(dcsr_handle h, hipStream_t s, FlatBufs *fb)
     const int64_t live = live_bound(h);
     const int64_t ngcap = (h->pool_cap > live ? h->pool_cap : live) / GRAN + 1;
     DCSR_TRY(ws_get(h, WS_ROWMAP, (size_t)ngcap * 4, (void **)&fb->rowmap));
+    fb->mapcap = ngcap;
     return DCSR_OK;
 }
 
@@ -1066,15 +1067,26 @@ void flat_rebuilt(dcsr_handle h)
     h->flat_dirty = false;
 }
 
-dcsr_status ensure_flat(dcsr_handle h, hipStream_t s)
+// Granules of the row map per scan tile (4,096 rows) past which a launch of their
+// own fills them: a tile fills 256 at a time, each by a search in LDS, so few rows
+// with many entries leave the chip idle.  Offsets and map of 3,000 rows of 512 and
+// 4,096 entries: 90 and 585 us in the scan, 26 and 23 apart; level at 32 entries
+// per row from 300 to 409,600 rows, which is this line.
+constexpr int64_t MAP_APART = 2048;
+dcsr_status ensure_flat(dcsr_handle h, hipStream_t s, int64_t entries)
 {
     if (!h->flat_dirty) return DCSR_OK;
     const int64_t R = h->rows;
     FlatBufs fb;
     DCSR_TRY(flat_buffers(h, s, &fb));
-    if (R > 0)
-        k_scan_rows<<<(unsigned)rowscan_tiles(R), TB, 0, s>>>((uint32_t)R, h->row_len, fb.foff, fb.rowmap, fb.part,
-                                                              fault_word(h), lb_spin_limit());
+    if (R > 0) {
+        const int64_t tiles = rowscan_tiles(R), granules = (entries < 0 ? live_bound(h) : entries) / GRAN + 1;
+        const bool apart = granules > MAP_APART * tiles;
+        k_scan_rows<<<(unsigned)tiles, TB, 0, s>>>((uint32_t)R, h->row_len, fb.foff, apart ? nullptr : fb.rowmap, fb.part,
+                                                   fault_word(h), lb_spin_limit());
+        if (apart)
+            k_rowmap<<<grid_for(granules, TB), TB, 0, s>>>((uint32_t)R, fb.foff, fb.rowmap, (uint32_t)fb.mapcap);
+    }
     DCSR_HIP(hipGetLastError());
     flat_rebuilt(h);
     return DCSR_OK;
