@@ -1071,8 +1071,10 @@ void flat_rebuilt(dcsr_handle h)
 // own fills them: a tile fills 256 at a time, each by a search in LDS, so few rows
 // with many entries leave the chip idle.  Offsets and map of 3,000 rows of 512 and
 // 4,096 entries: 90 and 585 us in the scan, 26 and 23 apart; level at 32 entries
-// per row from 300 to 409,600 rows, which is this line.
-constexpr int64_t MAP_APART = 2048;
+// per row from 300 to 409,600 rows, which is this line.  With tiles for half of the
+// CUs the scan fills the chip: 64 entries in each of 409,600 / 600,000 / 2M rows take
+// 33 / 34 / 44 us in it and 28 / 35 / 63 apart.
+constexpr int64_t MAP_APART = 2048, MAP_APART_TILES = 128;
 dcsr_status ensure_flat(dcsr_handle h, hipStream_t s, int64_t entries)
 {
     if (!h->flat_dirty) return DCSR_OK;
@@ -1081,7 +1083,7 @@ dcsr_status ensure_flat(dcsr_handle h, hipStream_t s, int64_t entries)
     DCSR_TRY(flat_buffers(h, s, &fb));
     if (R > 0) {
         const int64_t tiles = rowscan_tiles(R), granules = (entries < 0 ? live_bound(h) : entries) / GRAN + 1;
-        const bool apart = granules > MAP_APART * tiles;
+        const bool apart = tiles <= MAP_APART_TILES && granules > MAP_APART * tiles;
         k_scan_rows<<<(unsigned)tiles, TB, 0, s>>>((uint32_t)R, h->row_len, fb.foff, apart ? nullptr : fb.rowmap, fb.part,
                                                    fault_word(h), lb_spin_limit());
         if (apart)
