@@ -27,6 +27,9 @@
 // Nonzeros owned by one wave in the flat SpMV / SpMM kernels.
 #define DCSR_SPMV_PW 256u
 
+// Entries of both SpGEMM operands from which the product copies them (spgemm.hip).
+#define SG_PAIR_MIN (3 << 19)
+
 // Pool chunk granularity: chunk starts stay 16-byte aligned.
 #define DCSR_CHUNK_ALIGN 4u
 
@@ -154,6 +157,7 @@ struct dcsr_matrix_s {
     int pnl_count;           // panels in the current copy
     int64_t pnl_cols;        // widest panel (columns)
     int64_t pnl_min_nnz;     // smallest nnz worth a paneled copy
+    int64_t sg_pair_min;     // as the output of SpGEMM: entries of both operands from which they are copied
     dcsr_config cfg;
     Workspace ws;
     hipStream_t last_stream;
@@ -180,6 +184,8 @@ dcsr_status ws_get(dcsr_handle h, WsSlot slot, size_t bytes, void **out);
 // For slots whose words must start at zero (look-back control and status
 // words, finish counters): a grown buffer is zero-filled by a kernel on s.
 dcsr_status ws_get_zeroed(dcsr_handle h, WsSlot slot, size_t bytes, void **out, hipStream_t s);
+// Free a slot (waits for s and for whatever else uses it).
+dcsr_status ws_release(dcsr_handle h, WsSlot slot, hipStream_t s);
 dcsr_status pull_state(dcsr_handle h, hipStream_t s);   // copy DevState to host + sync
 // A few device words to the host once everything queued on s before the call
 // has finished (whole words, at most sizeof(HostFetch::words) bytes).

@@ -569,6 +569,16 @@ dcsr_status ws_get(dcsr_handle h, WsSlot slot, size_t bytes, void **out)
     return DCSR_OK;
 }
 
+dcsr_status ws_release(dcsr_handle h, WsSlot slot, hipStream_t s)
+{
+    DCSR_HIP(hipStreamSynchronize(s));
+    release_retired(h);
+    if (h->ws.ptr[slot]) DCSR_HIP(hipFree(h->ws.ptr[slot]));
+    h->ws.ptr[slot] = nullptr;
+    h->ws.bytes[slot] = 0;
+    return DCSR_OK;
+}
+
 dcsr_status ws_get_zeroed(dcsr_handle h, WsSlot slot, size_t bytes, void **out, hipStream_t s)
 {
     if (bytes == 0) bytes = 16;
@@ -784,6 +794,10 @@ dcsr_status dcsr_create(dcsr_handle *out, int64_t rows, int64_t cols, const dcsr
     h->pnl_min_nnz = 8ll << 20;
     if (const char *e = getenv("DCSR_SPMV_PANEL_COLS")) h->pnl_cols = atoll(e) > 0 ? atoll(e) : h->pnl_cols;
     if (const char *e = getenv("DCSR_SPMV_PANEL_MIN_NNZ")) h->pnl_min_nnz = atoll(e) >= 0 ? atoll(e) : h->pnl_min_nnz;
+    // SpGEMM: entries of both operands from which it takes copies of them
+    // (spgemm.hip); overridden for testing
+    h->sg_pair_min = SG_PAIR_MIN;
+    if (const char *e = getenv("DCSR_SPGEMM_PAIR_MIN")) h->sg_pair_min = atoll(e) >= 0 ? atoll(e) : h->sg_pair_min;
     // the update tag's starting value (a test of its wrap-around)
     if (const char *e = getenv("DCSR_UPDATE_TAG_START")) h->upd_tag = (uint32_t)strtoul(e, nullptr, 0);
     dcsr_status st = alloc_rows(h);

@@ -48,15 +48,23 @@ constexpr uint32_t BIG_MAX32 = 16384, BIG_MAX64 = 8192;  // partials per row by 
 constexpr int BIG_GB = 14;
 constexpr int64_t BIG_MAX_COLS32 = (1ll << (32 - BIG_GB)) - 1;
 constexpr int SG_EX = 8;              // partials per lane whose loads are in flight together
-// row classes (list index): wave, workgroup, large, hub, team
-// team classes CL_TEAM + i: rows of at most 2 (i + 1) * TEAM partials, sorted
-// with 2 (i + 1) keys per lane
-// wave classes CL_WAVE + i: rows of at most 256, 512, 1024 partials, sorted with
+// row classes: hub, large, workgroup;
+// team classes CL_TEAM + 2 i: rows of at most 2 (i + 1) * TEAM partials, sorted
+// with 2 (i + 1) keys per lane;
+// wave classes CL_WAVE + 2 i: rows of at most 256, 512, 1024 partials, sorted with
 // 4, 8, 16 keys per lane (the registers of the widest would hold the shorter
 // rows, which are most of them, to 3 waves per SIMD)
-enum {
-    CL_WAVE = 0, NWAVECL = 3, CL_BLOCK = CL_WAVE + NWAVECL, CL_BIG, CL_HUB, CL_TEAM, NTEAMCL = 4,
-    NCLS = CL_TEAM + NTEAMCL
+enum { CL_HUB = 0, CL_BIG = 1, CL_TEAM = 2, CL_BLOCK = 3, CL_WAVE = 5, NCLS = 10 };
+constexpr int cl_team(int kpl) { return CL_TEAM + 2 * (kpl / 2 - 1); }
+constexpr int cl_wave(int kpl) { return CL_WAVE + 2 * ((kpl > 4) + (kpl > 8)); }
+
+// The rows of one class.  A row is in one class at most, so two classes share an
+// array of R rows: the even one fills it from the front, the odd one from the back.
+template <int CLS>
+struct SgList {
+    const uint32_t *p;
+    SgList(const uint32_t *lists, uint32_t R) : p(lists + (uint64_t)(CLS / 2) * R + (CLS % 2 ? R - 1 : 0)) {}
+    __device__ __forceinline__ uint32_t operator[](uint32_t i) const { return CLS % 2 ? *(p - i) : p[i]; }
 };
 
 struct SgState {
@@ -76,15 +84,35 @@ __device__ __forceinline__ uint32_t next_pow2(uint32_t v)
     return v + 1;
 }
 
+// What the kernels read: the operands' row tables and pools, and in a PAIRED
+// product the B row of every A entry (A's flat order) and B's entries as (column,
+// value) pairs in B's flat order.  A short row of B is one 128-byte line of pairs
+// where the pool's two arrays cost one line each, and these lines bound the product
+// of matrices past the L2 (2M-row Poisson(8): the 16-lane kernels 1083 -> 1006 us
+// and the count 248 -> 181, the copy costs 77).  Small products read the operands
+// as they are, for the copy is a launch: squares of 0.3M / 0.6M / 0.8M / 1.2M / 1.6M /
+// 3.2M / 16M entries (Poisson rows of 3 and 8) take 99 / 113 / 163 / 160 / 224 / 382 /
+// 1,879 us so and 104 / 124 / 164 / 161 / 207 / 302 / 1,260 with the copies, power-law
+// squares of 0.1M / 0.4M / 0.8M / 1.6M / 2M 191 / 273 / 321 / 508 / 590 and 195 / 276 /
+// 314 / 493 / 579: the line is at 1.6M entries of both operands.  So do products for
+// which the copies do not fit the memory.
+struct SgIn {
+    const uint32_t *P, *Poff, *a_start;
+    const int32_t *a_len, *a_col;
+    const float *a_val;
+    const uint32_t *b_start;
+    const int32_t *b_len, *b_col;
+    const float *b_val;
+    const uint32_t *a_foff, *b_foff;
+    const uint2 *ent, *b_ent;
+};
+
 // P_i = sum over the entries of A row i of len(B row col).  One wave per 64
-// consecutive rows; entries folded per row with a DPP segmented scan.  The B
-// row (flat start, length) of every A entry is kept in A's flat order (ent):
-// the row kernels stream it instead of gathering it again.
-__global__ __launch_bounds__(TB) void k_sg_count(uint32_t R, const uint32_t *__restrict__ a_foff,
-                                                 const uint32_t *__restrict__ a_start,
-                                                 const int32_t *__restrict__ a_col,
-                                                 const uint32_t *__restrict__ b_foff,
-                                                 uint2 *__restrict__ ent, uint32_t *__restrict__ P)
+// consecutive rows; entries folded per row with a DPP segmented scan.  PAIRED: the
+// B row (flat start, length) of every A entry is kept in A's flat order (ent): the
+// row kernels stream it instead of gathering it again.
+template <bool PAIRED>
+__global__ __launch_bounds__(TB) void k_sg_count(uint32_t R, SgIn in, uint2 *__restrict__ ent, uint32_t *__restrict__ P)
 {
     __shared__ uint32_t s_ex[TB / 64][64];
     __shared__ uint32_t s_st[TB / 64][64];
@@ -94,11 +122,19 @@ __global__ __launch_bounds__(TB) void k_sg_count(uint32_t R, const uint32_t *__r
     const uint32_t r0 = (blockIdx.x * (TB / 64) + w) * 64u;
     const uint32_t r = r0 + lane;
     if (r0 >= R) return;
-    const uint32_t fo = a_foff[r < R ? r : R];
-    const uint32_t f0 = wave_read_lane_u32(fo, 0);
-    const uint32_t tot = a_foff[r0 + 64u < R ? r0 + 64u : R] - f0;
-    s_ex[w][lane] = fo - f0;
-    s_st[w][lane] = r < R ? a_start[r] : 0u;
+    uint32_t f0 = 0, tot, ex;
+    if constexpr (PAIRED) {
+        const uint32_t fo = in.a_foff[r < R ? r : R];
+        f0 = wave_read_lane_u32(fo, 0);
+        tot = in.a_foff[r0 + 64u < R ? r0 + 64u : R] - f0;
+        ex = fo - f0;
+    } else {
+        const uint32_t L = r < R ? (uint32_t)in.a_len[r] : 0u, inc = wave_incl_scan_u32(L);
+        tot = wave_read_lane_u32(inc, 63);
+        ex = inc - L;
+    }
+    s_ex[w][lane] = ex;
+    s_st[w][lane] = r < R ? in.a_start[r] : 0u;
     s_acc[w][lane] = 0;
     __builtin_amdgcn_wave_barrier();
     // four 64-entry chunks per round: their A-column loads, then their B-row
@@ -115,18 +151,22 @@ __global__ __launch_bounds__(TB) void k_sg_count(uint32_t R, const uint32_t *__r
             c[u] = -1;
             if (e < tot) {
                 j[u] = (uint32_t)find_seg64(s_ex[w], e);
-                c[u] = a_col[(uint64_t)s_st[w][j[u]] + (e - s_ex[w][j[u]])];
+                c[u] = in.a_col[(uint64_t)s_st[w][j[u]] + (e - s_ex[w][j[u]])];
             }
         }
 #pragma unroll
         for (int u = 0; u < CU; ++u) {
-            // neighbours in one array: one line, mostly
-            q[u] = c[u] >= 0 ? make_uint2(b_foff[c[u]], b_foff[c[u] + 1]) : make_uint2(0u, 0u);
-            q[u].y -= q[u].x;
+            if constexpr (PAIRED) {
+                // neighbours in one array: one line, mostly
+                q[u] = c[u] >= 0 ? make_uint2(in.b_foff[c[u]], in.b_foff[c[u] + 1]) : make_uint2(0u, 0u);
+                q[u].y -= q[u].x;
+            } else {
+                q[u] = make_uint2(0u, c[u] >= 0 ? (uint32_t)in.b_len[c[u]] : 0u);
+            }
         }
 #pragma unroll
         for (int u = 0; u < CU; ++u) {
-            if (c[u] >= 0) ent[(uint64_t)f0 + b + (uint32_t)u * 64u + lane] = q[u];
+            if (PAIRED && c[u] >= 0) ent[(uint64_t)f0 + b + (uint32_t)u * 64u + lane] = q[u];
             const uint32_t t = wave_seg_incl_scan_u32(q[u].y, j[u]);
             const uint32_t jn = __shfl_down(j[u], 1);
             if (j[u] < 64 && (lane == 63 || jn != j[u])) s_acc[w][j[u]] += t;
@@ -142,8 +182,7 @@ __global__ __launch_bounds__(TB) void k_sg_count(uint32_t R, const uint32_t *__r
 // counters took ~60K contended atomics per product (94 us on 2M rows).
 constexpr int SG_CR = 8;
 __global__ __launch_bounds__(TB) void k_sg_classify(uint32_t R, const uint32_t *__restrict__ P,
-                                                    uint32_t *__restrict__ lists, uint32_t list_stride,
-                                                    SgState *st, uint32_t *__restrict__ cnt,
+                                                    uint32_t *__restrict__ lists, SgState *st, uint32_t *__restrict__ cnt,
                                                     unsigned long long *__restrict__ bsum, uint32_t team_ok,
                                                     uint32_t big_max)
 {
@@ -170,8 +209,8 @@ __global__ __launch_bounds__(TB) void k_sg_classify(uint32_t R, const uint32_t *
             // lane), so the four teams of a wave run the same sort over similar
             // row sizes
             cls[q] = p[q] == 0                         ? -1
-                     : (p[q] <= TEAM_MAX && team_ok)   ? CL_TEAM + (int)((p[q] - 1) / (2 * TEAM))
-                     : p[q] <= WAVE_MAX                ? CL_WAVE + (p[q] > 256u) + (p[q] > 512u)
+                     : (p[q] <= TEAM_MAX && team_ok)   ? CL_TEAM + 2 * (int)((p[q] - 1) / (2 * TEAM))
+                     : p[q] <= WAVE_MAX                ? CL_WAVE + 2 * ((p[q] > 256u) + (p[q] > 512u))
                      : p[q] <= BLOCK_MAX               ? CL_BLOCK
                      : p[q] <= big_max                 ? CL_BIG
                                                        : CL_HUB;
@@ -196,7 +235,10 @@ __global__ __launch_bounds__(TB) void k_sg_classify(uint32_t R, const uint32_t *
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < SG_CR; ++q)
-        if (cls[q] >= 0) lists[(uint64_t)cls[q] * list_stride + s_base[cls[q]] + slot[q]] = r0 + (uint32_t)q * TB;
+        if (cls[q] >= 0) {
+            const uint32_t i = s_base[cls[q]] + slot[q];
+            lists[(uint64_t)(cls[q] >> 1) * R + (cls[q] & 1 ? R - 1u - i : i)] = r0 + (uint32_t)q * TB;
+        }
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
     if (lane_id() == 0) ws[threadIdx.x >> 6] = v;
@@ -302,20 +344,6 @@ struct SgRowInfo {
     uint32_t out_base;
 };
 
-// What the row kernels read: A's row table and values, the B row of every A
-// entry (A's flat order), B's entries as (column, value) pairs in B's flat
-// order.  A short row of B is one 128-byte line of pairs where the pool's two
-// arrays cost one line each, and these lines bound the product of matrices
-// past the L2 (2M-row Poisson(8): the 16-lane kernels 1083 -> 1006 us and the
-// count 248 -> 181, the copy costs 77).
-struct SgIn {
-    const uint32_t *P, *Poff, *a_start;
-    const int32_t *a_len;
-    const uint32_t *a_foff;
-    const float *a_val;
-    const uint2 *ent;
-    const uint2 *b_ent;
-};
 // What they write: C's pool and the row's entry count.
 struct SgOut {
     int32_t *tcol;
@@ -323,6 +351,24 @@ struct SgOut {
     uint32_t *cnt;
 };
 
+// B's row (start in B's entries, length) of entry a of A's row.
+template <bool PAIRED>
+__device__ __forceinline__ uint2 sg_b_row(const SgIn &in, const SgRowInfo &ri, uint32_t a)
+{
+    if constexpr (PAIRED) return in.ent[(uint64_t)ri.fo + a];
+    const int32_t c = in.a_col[(uint64_t)ri.ast + a];
+    return make_uint2(in.b_start[c], (uint32_t)in.b_len[c]);
+}
+
+// Entry p of B: column and value bits.
+template <bool PAIRED>
+__device__ __forceinline__ uint2 sg_b_entry(const SgIn &in, uint32_t p)
+{
+    if constexpr (PAIRED) return in.b_ent[p];
+    return make_uint2((uint32_t)in.b_col[p], __float_as_uint(in.b_val[p]));
+}
+
+template <bool PAIRED>
 __device__ __forceinline__ SgRowInfo sg_row_info(uint32_t row, const SgIn &in)
 {
     SgRowInfo r;
@@ -331,7 +377,7 @@ __device__ __forceinline__ SgRowInfo sg_row_info(uint32_t row, const SgIn &in)
     r.out_base = in.Poff[row];
     r.ast = in.a_start[row];
     r.la = (uint32_t)in.a_len[row];
-    r.fo = in.a_foff[row];
+    r.fo = PAIRED ? in.a_foff[row] : 0u;
     return r;
 }
 
@@ -559,7 +605,7 @@ __device__ __forceinline__ void team_sort(K *key, uint32_t *hist, uint32_t P, ui
 // entry is a bit count; a search of the entries' offsets took four dependent LDS
 // reads and 24 instructions per partial (the four classes on 2M Poisson rows with
 // 8 entries: 994 -> 937 us).
-template <int GB, int KPL>
+template <bool PAIRED, int GB, int KPL>
 __device__ __forceinline__ void sg_expand_team(const SgIn &in, uint32_t lb, uint32_t sb, float va, uint32_t ex,
                                                uint32_t tot, uint32_t gbase, uint32_t *key, float *val,
                                                uint32_t *map, uint32_t *s_sb, float *s_va)
@@ -592,7 +638,7 @@ __device__ __forceinline__ void sg_expand_team(const SgIn &in, uint32_t lb, uint
     for (int i = 0; i < KPL; ++i) {
         const uint32_t pe = (uint32_t)i * TEAM + t;
         const uint32_t q = before[i / 2] + (uint32_t)__popc(m[i / 2] & ((2u << ((i & 1) * TEAM + t)) - 1u));
-        be[i] = in.b_ent[pe < tot ? s_sb[q] + pe : 0u];
+        be[i] = sg_b_entry<PAIRED>(in, pe < tot ? s_sb[q] + pe : 0u);
         av[i] = s_va[q];
     }
 #pragma unroll
@@ -609,7 +655,7 @@ __device__ __forceinline__ void sg_expand_team(const SgIn &in, uint32_t lb, uint
 // KPL: keys per lane of the sort, fixed by the row's class (P <= KPL * NT).  The products stay where the expansion put them
 // (generation order); only the keys are sorted, and a sorted key names its
 // product by its generation bits.
-template <int NT, int GB, typename K, int KPL>
+template <bool PAIRED, int NT, int GB, typename K, int KPL>
 __device__ void sg_row(const SgRowInfo &ri, const SgIn &in, const SgOut &out, K *key, float *val, uint32_t *hist,
                        uint32_t *s_ex, uint32_t *s_sb, float *s_va, uint32_t *lds_w)
 {
@@ -623,7 +669,7 @@ __device__ void sg_row(const SgRowInfo &ri, const SgIn &in, const SgOut &out, K 
         uint32_t lb = 0, sb = 0;
         float va = 0.0f;
         if (a < la) {
-            const uint2 q = in.ent[(uint64_t)ri.fo + a];
+            const uint2 q = sg_b_row<PAIRED>(in, ri, a);
             va = in.a_val[(uint64_t)ast + a];
             sb = q.x;
             lb = q.y;
@@ -631,7 +677,7 @@ __device__ void sg_row(const SgRowInfo &ri, const SgIn &in, const SgOut &out, K 
         uint32_t tot;
         const uint32_t ex = team_excl_scan<NT>(lb, lds_w, &tot);
         if constexpr (NT == TEAM) {
-            sg_expand_team<GB, KPL>(in, lb, sb, va, ex, tot, gbase, key, val, hist, s_sb, s_va);
+            sg_expand_team<PAIRED, GB, KPL>(in, lb, sb, va, ex, tot, gbase, key, val, hist, s_sb, s_va);
             gbase += tot;
             team_sync<NT>();
             continue;
@@ -651,8 +697,7 @@ __device__ void sg_row(const SgRowInfo &ri, const SgIn &in, const SgOut &out, K 
             for (int i = 0; i < EX; ++i) {
                 const uint32_t pe = e0 + (uint32_t)i * NT + t;
                 const uint32_t q = find_seg_team<NT>(s_ex, pe < tot ? pe : 0u);
-                const uint64_t bp = pe < tot ? (uint64_t)s_sb[q] + (pe - s_ex[q]) : 0u;
-                be[i] = in.b_ent[bp];
+                be[i] = sg_b_entry<PAIRED>(in, pe < tot ? s_sb[q] + (pe - s_ex[q]) : 0u);
                 av[i] = s_va[q];
             }
 #pragma unroll
@@ -724,16 +769,15 @@ __device__ void sg_row(const SgRowInfo &ri, const SgIn &in, const SgOut &out, K 
 
 // Team loop over a class list: team `first`, stride `step`.  The next row's
 // id and info are loaded one and two iterations ahead.
-template <typename F>
-__device__ __forceinline__ void sg_rows(const uint32_t *__restrict__ list, uint32_t n, uint32_t first, uint32_t step,
-                                        const SgIn &in, F &&body)
+template <bool PAIRED, int CLS, typename F>
+__device__ __forceinline__ void sg_rows(SgList<CLS> list, uint32_t n, uint32_t first, uint32_t step, const SgIn &in, F &&body)
 {
     if (first >= n) return;
-    SgRowInfo cur = sg_row_info(list[first], in);
+    SgRowInfo cur = sg_row_info<PAIRED>(list[first], in);
     uint32_t next_id = first + step < n ? list[first + step] : 0u;
     for (uint32_t i = first; i < n; i += step) {
         SgRowInfo nxt{};
-        if (i + step < n) nxt = sg_row_info(next_id, in);
+        if (i + step < n) nxt = sg_row_info<PAIRED>(next_id, in);
         const uint32_t nn_id = i + 2 * step < n ? list[i + 2 * step] : 0u;
         body(cur);
         cur = nxt;
@@ -743,8 +787,8 @@ __device__ __forceinline__ void sg_rows(const uint32_t *__restrict__ list, uint3
 
 // Wave rows: one wave per row, at most 64 * KPL partials.  K: 32-bit sort keys
 // (half the LDS per row, more rows in flight) when B's columns allow.
-template <int KPL, typename K>
-__global__ __launch_bounds__(TB) void k_sg_wave(const uint32_t *__restrict__ list, const SgState *__restrict__ st,
+template <bool PAIRED, int KPL, typename K>
+__global__ __launch_bounds__(TB) void k_sg_wave(SgList<cl_wave(KPL)> list, const SgState *__restrict__ st,
                                                 SgIn in, SgOut out)
 {
     static_assert(64 * KPL <= WAVE_MAX, "generations fit their key bits");
@@ -754,9 +798,9 @@ __global__ __launch_bounds__(TB) void k_sg_wave(const uint32_t *__restrict__ lis
     __shared__ uint32_t s_ex[TB / 64][64], s_sb[TB / 64][64];
     __shared__ float s_va[TB / 64][64];
     const int w = threadIdx.x >> 6;
-    const uint32_t n = st->count[CL_WAVE + (KPL > 4) + (KPL > 8)];
-    sg_rows(list, n, blockIdx.x * (TB / 64) + w, gridDim.x * (TB / 64), in, [&](const SgRowInfo &ri) {
-        sg_row<64, WAVE_GB, K, KPL>(ri, in, out, key[w], val[w], hist[w], s_ex[w], s_sb[w], s_va[w], nullptr);
+    const uint32_t n = st->count[cl_wave(KPL)];
+    sg_rows<PAIRED>(list, n, blockIdx.x * (TB / 64) + w, gridDim.x * (TB / 64), in, [&](const SgRowInfo &ri) {
+        sg_row<PAIRED, 64, WAVE_GB, K, KPL>(ri, in, out, key[w], val[w], hist[w], s_ex[w], s_sb[w], s_va[w], nullptr);
     });
 }
 
@@ -767,9 +811,9 @@ __global__ __launch_bounds__(TB) void k_sg_wave(const uint32_t *__restrict__ lis
 // 90 and 106), and six keys are held to the 72 that let seven waves share a SIMD.
 // The four classes on 2M Poisson rows with 8 entries: 907 -> 866 us.  Loading the
 // next row's A entries a row ahead cost more registers than it gave (866 -> 912).
-template <int KPL>
-__global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(KPL == 6 ? 7 : 4))) void k_sg_team(const uint32_t *__restrict__ list, const SgState *__restrict__ st,
-                                                SgIn in, SgOut out)
+template <bool PAIRED, int KPL>
+__global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(KPL == 6 ? 7 : 4))) void k_sg_team(
+    SgList<cl_team(KPL)> list, const SgState *__restrict__ st, SgIn in, SgOut out)
 {
     constexpr int NTEAM = TB / TEAM;
     // per-team rows padded so the four teams of a wave start on different
@@ -783,17 +827,16 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(KPL == 6 ? 7
     __shared__ float s_va[NTEAM][TEAM];
     const int tm = threadIdx.x / TEAM;
     static_assert(KPL * TEAM <= TEAM_MAX, "a team row fits its LDS row");
-    const uint32_t n = st->count[CL_TEAM + KPL / 2 - 1];
-    sg_rows(list, n, blockIdx.x * NTEAM + tm, gridDim.x * NTEAM, in, [&](const SgRowInfo &ri) {
-        sg_row<TEAM, TEAM_GB, uint32_t, KPL>(ri, in, out, key[tm], val[tm], hist[tm], s_ex[tm], s_sb[tm], s_va[tm],
+    const uint32_t n = st->count[cl_team(KPL)];
+    sg_rows<PAIRED>(list, n, blockIdx.x * NTEAM + tm, gridDim.x * NTEAM, in, [&](const SgRowInfo &ri) {
+        sg_row<PAIRED, TEAM, TEAM_GB, uint32_t, KPL>(ri, in, out, key[tm], val[tm], hist[tm], s_ex[tm], s_sb[tm], s_va[tm],
                                              nullptr);
     });
 }
 
-// One workgroup of NT threads per row of class `cls`, at most MAXP partials.
-template <int NT, int GB, uint32_t MAXP, typename K>
-__global__ __launch_bounds__(NT) void k_sg_block(const uint32_t *__restrict__ list, const SgState *__restrict__ st,
-                                                 int cls, SgIn in, SgOut out)
+// One workgroup of NT threads per row of class CLS, at most MAXP partials.
+template <bool PAIRED, int CLS, int NT, int GB, uint32_t MAXP, typename K>
+__global__ __launch_bounds__(NT) void k_sg_block(SgList<CLS> list, const SgState *__restrict__ st, SgIn in, SgOut out)
 {
     constexpr int KPL = MAXP / NT;
     __shared__ __align__(16) K key[MAXP];
@@ -802,9 +845,9 @@ __global__ __launch_bounds__(NT) void k_sg_block(const uint32_t *__restrict__ li
     __shared__ uint32_t s_ex[NT], s_sb[NT];
     __shared__ float s_va[NT];
     __shared__ uint32_t lds_w[2 * NT / 64];
-    const uint32_t n = st->count[cls];
-    sg_rows(list, n, blockIdx.x, gridDim.x, in, [&](const SgRowInfo &ri) {
-        sg_row<NT, GB, K, KPL>(ri, in, out, key, val, hist, s_ex, s_sb, s_va, lds_w);
+    const uint32_t n = st->count[CLS];
+    sg_rows<PAIRED>(list, n, blockIdx.x, gridDim.x, in, [&](const SgRowInfo &ri) {
+        sg_row<PAIRED, NT, GB, K, KPL>(ri, in, out, key, val, hist, s_ex, s_sb, s_va, lds_w);
     });
 }
 
@@ -947,18 +990,51 @@ __global__ void k_sg_set_rows(uint32_t R, const uint32_t *__restrict__ Poff, con
 
 }  // namespace
 
-dcsr_status dcsr_spgemm(dcsr_handle A, dcsr_handle B, dcsr_handle C, dcsr_stream_t stream)
-{
-    if (!A || !B || !C || C == A || C == B) return DCSR_ERR_INVALID;
-    if (A->cols != B->rows || C->rows != A->rows || C->cols != B->cols) return DCSR_ERR_INVALID;
-    hipStream_t s = (hipStream_t)stream;
-    A->last_stream = B->last_stream = C->last_stream = s;
-    DCSR_TRY(refresh_replayed(A, s));
-    DCSR_TRY(refresh_replayed(B, s));
-    if (!A->state_known) DCSR_TRY(pull_state(A, s));
-    if (!B->state_known) DCSR_TRY(pull_state(B, s));
-    const uint32_t R = (uint32_t)A->rows;
+// Launches `kernel` over the rows of class CLS, `per` rows to a workgroup of nt
+// threads, on at most `most` workgroups (they stride over the rest).
+struct RowLaunch {
+    const SgState &hst;
+    const uint32_t *lists;
+    uint32_t R;
+    const SgState *st;
+    const SgIn &in;
+    const SgOut &out;
+    hipStream_t s;
+    template <int CLS>
+    void operator()(void (*kernel)(SgList<CLS>, const SgState *, SgIn, SgOut), uint32_t per, uint32_t most, int nt) const
+    {
+        const uint32_t want = (hst.count[CLS] + per - 1) / per;
+        if (want) kernel<<<want < most ? want : most, nt, 0, s>>>(SgList<CLS>(lists, R), st, in, out);
+    }
+};
 
+// The row kernels of every class; PAIRED as in SgIn.
+template <bool PAIRED>
+static void launch_rows(const RowLaunch &run, int64_t cols)
+{
+    run(k_sg_team<PAIRED, 2>, TB / TEAM, 8192, TB);
+    run(k_sg_team<PAIRED, 4>, TB / TEAM, 8192, TB);
+    run(k_sg_team<PAIRED, 6>, TB / TEAM, 8192, TB);
+    run(k_sg_team<PAIRED, 8>, TB / TEAM, 8192, TB);
+    if (cols <= WAVE_MAX_COLS32) {
+        run(k_sg_wave<PAIRED, 4, uint32_t>, 4, 8192, TB);
+        run(k_sg_wave<PAIRED, 8, uint32_t>, 4, 8192, TB);
+        run(k_sg_wave<PAIRED, 16, uint32_t>, 4, 8192, TB);
+    } else {
+        run(k_sg_wave<PAIRED, 4, uint64_t>, 4, 8192, TB);
+        run(k_sg_wave<PAIRED, 8, uint64_t>, 4, 8192, TB);
+        run(k_sg_wave<PAIRED, 16, uint64_t>, 4, 8192, TB);
+    }
+    if (cols <= BLOCK_MAX_COLS32) run(k_sg_block<PAIRED, CL_BLOCK, TB, BLOCK_GB, BLOCK_MAX, uint32_t>, 1, 4096, TB);
+    else run(k_sg_block<PAIRED, CL_BLOCK, TB, BLOCK_GB, BLOCK_MAX, uint64_t>, 1, 4096, TB);
+    if (cols <= BIG_MAX_COLS32) run(k_sg_block<PAIRED, CL_BIG, BIG_TB, BIG_GB, BIG_MAX32, uint32_t>, 1, 1024, BIG_TB);
+    else run(k_sg_block<PAIRED, CL_BIG, BIG_TB, BIG_GB, BIG_MAX64, uint64_t>, 1, 1024, BIG_TB);
+}
+
+// C = A * B (states known); paired: with the copies of SgIn, in C's workspace.
+static dcsr_status spgemm_run(dcsr_handle A, dcsr_handle B, dcsr_handle C, bool paired, hipStream_t s)
+{
+    const uint32_t R = (uint32_t)A->rows;
     uint32_t *P, *Poff, *cnt, *coff, *lists, *part;
     SgState *st;
     unsigned long long *bsum;
@@ -967,25 +1043,32 @@ dcsr_status dcsr_spgemm(dcsr_handle A, dcsr_handle B, dcsr_handle C, dcsr_stream
     DCSR_TRY(ws_get(C, WS_SG_POFF, (size_t)(R + 1) * 4, (void **)&Poff));
     DCSR_TRY(ws_get(C, WS_SG_CNT, (size_t)(R + 1) * 4, (void **)&cnt));
     DCSR_TRY(ws_get(C, WS_SG_COFF, (size_t)(R + 1) * 4, (void **)&coff));
-    DCSR_TRY(ws_get(C, WS_SG_LIST, (size_t)(R + 1) * 4 * NCLS, (void **)&lists));
+    DCSR_TRY(ws_get(C, WS_SG_LIST, (size_t)R * 4 * (NCLS / 2), (void **)&lists));
     DCSR_TRY(ws_get(C, WS_SG_STATE, sizeof(SgState), (void **)&st));
     DCSR_TRY(ws_get(C, WS_SG_BSUM, (size_t)nbR * 8, (void **)&bsum));
     DCSR_TRY(ws_get_zeroed(C, WS_PART, scan_part_words(R + 1, 2) * 4, (void **)&part, s));
 
-    DCSR_TRY(ensure_flat(A, s));
-    const uint32_t *a_foff = (const uint32_t *)A->ws.ptr[WS_FOFF];
-    const uint32_t *b_foff;
-    uint2 *b_ent, *ent;
-    DCSR_TRY(ws_get(C, WS_SG_BENT, (size_t)(B->nnz_h + 1) * 8, (void **)&b_ent));
-    DCSR_TRY(copy_rows_paired(B, b_ent, B->nnz_h, &b_foff, s));
-    DCSR_TRY(ws_get(C, WS_SG_ENT, (size_t)(A->nnz_h + 1) * 8, (void **)&ent));
+    SgIn in{P, Poff, A->row_start, A->row_len, A->pool_col, A->pool_val, B->row_start, B->row_len, B->pool_col,
+            B->pool_val, nullptr, nullptr, nullptr, nullptr};
+    uint2 *ent = nullptr;
+    if (paired) {
+        uint2 *b_ent;
+        DCSR_TRY(ensure_flat(A, s));
+        in.a_foff = (const uint32_t *)A->ws.ptr[WS_FOFF];
+        DCSR_TRY(ws_get(C, WS_SG_BENT, (size_t)(B->nnz_h + 1) * 8, (void **)&b_ent));
+        DCSR_TRY(copy_rows_paired(B, b_ent, B->nnz_h, &in.b_foff, s));
+        DCSR_TRY(ws_get(C, WS_SG_ENT, (size_t)(A->nnz_h + 1) * 8, (void **)&ent));
+        in.ent = ent;
+        in.b_ent = b_ent;
+    }
 
     // 1. partial counts, classes, offsets
     k_sg_state_zero<<<1, 1, 0, s>>>(st);
     if (R > 0) {
-        k_sg_count<<<grid_for(R, TB), TB, 0, s>>>(R, a_foff, A->row_start, A->pool_col, b_foff, ent, P);
-        k_sg_classify<<<nbR, TB, 0, s>>>(R, P, lists, R + 1, st, cnt, bsum, B->cols <= TEAM_MAX_COLS ? 1u : 0u,
-                                            B->cols <= BIG_MAX_COLS32 ? BIG_MAX32 : BIG_MAX64);
+        if (paired) k_sg_count<true><<<grid_for(R, TB), TB, 0, s>>>(R, in, ent, P);
+        else k_sg_count<false><<<grid_for(R, TB), TB, 0, s>>>(R, in, nullptr, P);
+        k_sg_classify<<<nbR, TB, 0, s>>>(R, P, lists, st, cnt, bsum, B->cols <= TEAM_MAX_COLS ? 1u : 0u,
+                                         B->cols <= BIG_MAX_COLS32 ? BIG_MAX32 : BIG_MAX64);
         k_sg_total<<<1, 1024, 0, s>>>(st, bsum, (int)nbR);
     }
     DCSR_HIP(scan_exclusive_u32(P, Poff, R, 1, part, Poff + R, s, fault_word(C)));
@@ -1005,38 +1088,13 @@ dcsr_status dcsr_spgemm(dcsr_handle A, dcsr_handle B, dcsr_handle C, dcsr_stream
     float *tval = C->pool_val;
 
     // 2. numeric phases
-    const SgIn in{P, Poff, A->row_start, A->row_len, a_foff, A->pool_val, ent, b_ent};
     const SgOut out{tcol, tval, cnt};
-    // launches `kernel` over the rows of class c, `per` rows to a workgroup of
-    // nt threads, on at most `most` workgroups (they stride over the rest)
-    auto run = [&](auto kernel, int c, uint32_t per, uint32_t most, int nt, auto... cls) {
-        const uint32_t want = (hst.count[c] + per - 1) / per;
-        if (want) kernel<<<want < most ? want : most, nt, 0, s>>>(lists + c * (uint64_t)(R + 1), st, cls..., in, out);
-    };
-    run(k_sg_team<2>, CL_TEAM + 0, TB / TEAM, 8192, TB);
-    run(k_sg_team<4>, CL_TEAM + 1, TB / TEAM, 8192, TB);
-    run(k_sg_team<6>, CL_TEAM + 2, TB / TEAM, 8192, TB);
-    run(k_sg_team<8>, CL_TEAM + 3, TB / TEAM, 8192, TB);
-    if (B->cols <= WAVE_MAX_COLS32) {
-        run(k_sg_wave<4, uint32_t>, CL_WAVE + 0, 4, 8192, TB);
-        run(k_sg_wave<8, uint32_t>, CL_WAVE + 1, 4, 8192, TB);
-        run(k_sg_wave<16, uint32_t>, CL_WAVE + 2, 4, 8192, TB);
-    } else {
-        run(k_sg_wave<4, uint64_t>, CL_WAVE + 0, 4, 8192, TB);
-        run(k_sg_wave<8, uint64_t>, CL_WAVE + 1, 4, 8192, TB);
-        run(k_sg_wave<16, uint64_t>, CL_WAVE + 2, 4, 8192, TB);
-    }
-    if (B->cols <= BLOCK_MAX_COLS32)
-        run(k_sg_block<TB, BLOCK_GB, BLOCK_MAX, uint32_t>, CL_BLOCK, 1, 4096, TB, (int)CL_BLOCK);
-    else
-        run(k_sg_block<TB, BLOCK_GB, BLOCK_MAX, uint64_t>, CL_BLOCK, 1, 4096, TB, (int)CL_BLOCK);
-    if (B->cols <= BIG_MAX_COLS32)
-        run(k_sg_block<BIG_TB, BIG_GB, BIG_MAX32, uint32_t>, CL_BIG, 1, 1024, BIG_TB, (int)CL_BIG);
-    else
-        run(k_sg_block<BIG_TB, BIG_GB, BIG_MAX64, uint64_t>, CL_BIG, 1, 1024, BIG_TB, (int)CL_BIG);
+    const RowLaunch run{hst, lists, R, st, in, out, s};
+    paired ? launch_rows<true>(run, B->cols) : launch_rows<false>(run, B->cols);
     if (hst.count[CL_HUB]) {
         const uint32_t hn = hst.count[CL_HUB];
-        const uint32_t *hlist = lists + CL_HUB * (uint64_t)(R + 1);
+        static_assert(CL_HUB % 2 == 0, "its list runs forward");
+        const uint32_t *hlist = SgList<CL_HUB>(lists, R).p;
         uint32_t *hpre_in, *hpre, *blen, *apos, *emit, *epos, *v0, *v1;
         uint64_t *k0, *k1;
         EA *ea;
@@ -1096,4 +1154,25 @@ dcsr_status dcsr_spgemm(dcsr_handle A, dcsr_handle B, dcsr_handle C, dcsr_stream
     C->flat_dirty = true;
     C->hubs_dirty = true;
     return DCSR_OK;
+}
+
+dcsr_status dcsr_spgemm(dcsr_handle A, dcsr_handle B, dcsr_handle C, dcsr_stream_t stream)
+{
+    if (!A || !B || !C || C == A || C == B) return DCSR_ERR_INVALID;
+    if (A->cols != B->rows || C->rows != A->rows || C->cols != B->cols) return DCSR_ERR_INVALID;
+    hipStream_t s = (hipStream_t)stream;
+    A->last_stream = B->last_stream = C->last_stream = s;
+    DCSR_TRY(refresh_replayed(A, s));
+    DCSR_TRY(refresh_replayed(B, s));
+    if (!A->state_known) DCSR_TRY(pull_state(A, s));
+    if (!B->state_known) DCSR_TRY(pull_state(B, s));
+    if (A->nnz_h + B->nnz_h >= C->sg_pair_min) {
+        const dcsr_status st = spgemm_run(A, B, C, true, s);
+        if (st != DCSR_ERR_OOM) return st;
+        // the copies leave no room for the rest (or find none): without them
+        (void)hipGetLastError();
+        DCSR_TRY(ws_release(C, WS_SG_BENT, s));
+        DCSR_TRY(ws_release(C, WS_SG_ENT, s));
+    }
+    return spgemm_run(A, B, C, false, s);
 }
