@@ -11,8 +11,7 @@
 // call on that device) and only that pointer is handed to kernels.  Every
 // call on one GPU shares that GPU's array and leaves its contents behind:
 // calls that overlap on one GPU (two streams, two threads) race, so callers
-// serialize them.  The only words that must start at zero (the update's
-// finish counters) are cleared by a fill kernel at the start of each call.
+// serialize them.  A call writes every word of it before it reads it.
 #include <mutex>
 
 #include "dcsr_internal.h"

@@ -57,7 +57,7 @@ struct SmallArgs {
 
 template <int IT>
 struct SmallLds {
-    static constexpr int NB = SU_TB * (IT < 8 ? (IT < 2 ? 2 : IT + (IT & 1)) : 8);  // buckets
+    static constexpr int NB = SU_TB * (IT < 2 ? 2 : IT + (IT & 1));  // buckets: whole counter words per thread
     static constexpr int HW = NB / 2 + 2 > SU_RADIX_WORDS ? NB / 2 + 2 : SU_RADIX_WORDS;
     uint64_t key[IT * SU_TB];   // in bucket order (sorted after the radix sort)
     uint16_t arr[IT * SU_TB];   // arrival index of key[i]

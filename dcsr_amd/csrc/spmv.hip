@@ -8,15 +8,18 @@
 // Design: merge-based ("flat") SpMV.  The rows' live lengths are
 // prefix-summed once per structural change (foff, natural row order).  Each
 // wave owns a fixed range of DCSR_SPMV_PW consecutive nonzeros of that flat
-// order, whatever rows they belong to, so power-law hubs and empty rows cost
-// the same per nonzero.  A wave walks its range 64 rows at a time: lanes find
-// their row by a 6-step search over the window's offsets in LDS, load
-// (col, val) from the row's pool chunk, gather x, and a DPP segmented scan
-// folds the products per row; four 64-wide chunks are in flight per
-// iteration.  A row that starts inside the range is written by that wave;
-// the partial of a row that started in an earlier wave is left in a carry
-// slot, and a second small kernel adds each row's carry chain in wave order.
-// All reductions have a fixed association order: y is bitwise reproducible.
+// order, whatever rows they belong to, so power-law hubs and empty rows
+// cost the same per nonzero.  With one column (k_flat1) the rows that start in
+// the range leave a bit each in a map of its entries, so an entry's row is a bit
+// count; a lane sums four consecutive products in double and one DPP segmented
+// scan folds the lanes' open sums.  With two or four (k_flat) a wave walks its
+// range 64 rows at a time, a 6-step search over the window's offsets per entry;
+// wider blocks (k_spmm_wide) stage the window's entries in LDS and give a lane
+// group a slice of them.  A row that starts inside the range is written by that
+// wave; the partial of a row that started in an earlier wave is left in a carry
+// slot, and a second small kernel adds each row's carry chain (in double for one
+// column).  All reductions have a fixed association order: y is bitwise
+// reproducible.
 #include <type_traits>
 #include "dcsr_internal.h"
 #include "lookback.h"

@@ -1659,6 +1659,8 @@ dcsr_status small_launch(dcsr_handle h, const int32_t *rows, const int32_t *cols
     } else if (n <= SMALL_FUSED) {
         k_upd_small<2, true><<<1, SU_TB, 0, s>>>(A);
     } else {
+        // five triples per thread where they hold the batch: 2 us of an update's 79 less
+        // than with seven; three, four or six in their ranges differ by less than the runs
         if (n <= 5 * SU_TB) k_upd_small<5, false><<<1, SU_TB, 0, s>>>(A);
         else k_upd_small<SU_IT_MAX, false><<<1, SU_TB, 0, s>>>(A);
         k_upd_bisect<P_SPLIT><<<grid_for(n, TB), TB, 0, s>>>(A);
