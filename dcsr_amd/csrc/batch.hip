@@ -30,7 +30,7 @@ namespace {
 // 16 waves and 73 KB of LDS: two workgroups fill a CU's waves.  A matrix is a
 // chain of short phases with a barrier between them, so what bounds a step is
 // how many rows are in flight per CU: 4,096 matrices (4.0M rows, 68M entries,
-// 2,000 triples each) take 1.1 ms per step; 4 waves per matrix with the records
+// 2,000 triples each) take 0.94 ms per step; 4 waves per matrix with the records
 // in memory and one lane per touched row took 2.44.  Everything is inlined: as a
 // function the update spilled its registers through memory (1.31 ms).
 constexpr int BT = 1024;
@@ -651,7 +651,8 @@ __device__ __forceinline__ void batch_spmv(uint32_t m, const uint32_t *__restric
     const uint32_t gbase = row_base[m];
     const uint32_t Rm = row_base[m + 1] - gbase;
     const float *xm = x + col_base[m];
-    const uint32_t t = threadIdx.x;
+    uint32_t t = threadIdx.x;
+    asm volatile("" : "+v"(t));  // not kept from matrix to matrix: 13 registers spilled, not 18
     const uint32_t tl = t % TEAM;
     for (uint32_t r0 = 0; r0 < Rm; r0 += BT / TEAM) {
         const uint32_t r = r0 + t / TEAM;
@@ -690,6 +691,10 @@ __device__ __forceinline__ void batch_spmv(uint32_t m, const uint32_t *__restric
         if (mine && tl == 0) y[gbase + r] = acc;
     }
     __syncthreads();
+    // loads that the rows above left behind would be waited for in every round below,
+    // and with them the row's store (100 matrices of 2,000 rows with 600 entries:
+    // 613 -> 563 us)
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
     const uint32_t nlong = S.sm[SM_LONG];
     for (uint32_t i = t >> 6; i < nlong; i += NW) {
         const uint32_t r = S.urc[i];
