@@ -30,7 +30,7 @@ namespace {
 // 16 waves and 73 KB of LDS: two workgroups fill a CU's waves.  A matrix is a
 // chain of short phases with a barrier between them, so what bounds a step is
 // how many rows are in flight per CU: 4,096 matrices (4.0M rows, 68M entries,
-// 2,000 triples each) take 0.94 ms per step; 4 waves per matrix with the records
+// 2,000 triples each) take 0.91 ms per step; 4 waves per matrix with the records
 // in memory and one lane per touched row took 2.44.  Everything is inlined: as a
 // function the update spilled its registers through memory (1.31 ms).
 constexpr int BT = 1024;
